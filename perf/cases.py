@@ -23,8 +23,8 @@ import sys
 import numpy as np
 import torch
 
-sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
-                                "unified-cache-management_amd"))
+# the package of the tree that is measured: the working folder is its root
+sys.path.insert(0, os.path.join(os.getcwd(), "unified-cache-management_amd"))
 
 from ucm_amd.sparse.decode_step import GSADecodeStep, GSADecodeStepMLA, SparseDecodeStep  # noqa: E402
 from ucm_amd.sparse.esa_retrieval_worker import dot_topk  # noqa: E402
