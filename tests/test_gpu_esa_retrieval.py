@@ -142,6 +142,50 @@ def test_many_equal_scores_are_bit_exact_in_list_order(max_n, k, values):
         assert np.array_equal(gi[b], indexes[b][order])
 
 
+@pytest.mark.parametrize("max_n", [1, 3, 255, 256, 257, 1023, 1024, 1025, 4095, 4096, 4097, 8192, 16383, 16384, 16385])
+@pytest.mark.parametrize("spread", ["even", "outlier", "crowded"])
+def test_selection_at_the_edges_of_its_row_lengths(max_n, spread):
+    """One instantiation per range of row lengths, one workgroup per so many places; a row whose scores
+    crowd into few of the equal-width bins (an outlier stretches their range, or 64 and more are equal)
+    takes the digit search instead.  dim 1 and query 1 make every score its data value, so the outputs
+    equal a stable sort exactly; every seventh entry is no candidate."""
+    rng = rng_for(max_n * 3 + len(spread))
+    data = rng.standard_normal((20000, 1)).astype(np.float32)
+    if spread == "outlier":
+        data[:50] *= 1e30
+    elif spread == "crowded":
+        data[:] = rng.integers(-2, 3, size=data.shape)
+    indexes = np.stack([rng.permutation(20000)[:max_n] for _ in range(2)]).astype(np.int32)
+    indexes[:, 6::7] = -1
+    indexes[1, 5:] = -1  # a row of at most five candidates beside a full one
+    for k in sorted({1, min(max_n, 4096), min(4096, max_n // 3 + 1)}):
+        gi, gs = gpu_dot_topk(data, np.ones((2, 1), np.float32), indexes, k)
+        for b in range(2):
+            pos = np.flatnonzero(indexes[b] >= 0)
+            order = pos[np.argsort(-data[indexes[b][pos], 0], kind="stable")][:k]
+            assert np.array_equal(gi[b, :len(order)], indexes[b][order])
+            assert np.array_equal(gs[b, :len(order)], data[indexes[b][order], 0])
+            assert (gi[b, len(order):] == -1).all() and (gs[b, len(order):] == 0).all()
+
+
+@pytest.mark.parametrize("dim", [4, 252, 256, 260, 508, 512, 768, 1020, 1024, 1028, 2300])
+def test_dot_products_at_the_edges_of_the_chunks(dim):
+    """Rows are read in groups of four, two and one 256-value chunks and a partial one, by waves of four
+    rows.  Integer-valued inputs make the sums exact; the query starts 4 bytes off a 16-byte line."""
+    rng = rng_for(dim)
+    data = rng.integers(-8, 9, size=(37, dim)).astype(np.float32)
+    store = torch.zeros(dim + 1, device="cuda")
+    store[1:] = torch.from_numpy(rng.integers(-8, 9, size=dim).astype(np.float32))
+    from ucm_amd.sparse.esa_retrieval_worker import dot_topk
+
+    idx = torch.from_numpy(rng.permutation(37).astype(np.int32)[None]).cuda()
+    gi, gs = dot_topk(torch.from_numpy(data).cuda(), store[1:][None], idx, 37)
+    exact = data @ store[1:].cpu().numpy()
+    order = np.argsort(-exact[idx[0].cpu().numpy()], kind="stable")
+    assert np.array_equal(gi[0].cpu().numpy(), idx[0].cpu().numpy()[order])
+    assert np.array_equal(gs[0].cpu().numpy(), exact[idx[0].cpu().numpy()[order]])
+
+
 def test_fewer_candidates_than_k_and_empty_rows():
     rng = rng_for(9)
     data = rng.standard_normal((100, 64)).astype(np.float32)

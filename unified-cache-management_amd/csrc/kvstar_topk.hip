@@ -220,9 +220,7 @@ __global__ __launch_bounds__(kStatThreads) void row_stats_kernel(const float* __
 __global__ __launch_bounds__(kStatThreads) void block_mass_kernel(const float* __restrict__ scores,
                                                                   const float* __restrict__ stats,
                                                                   int rows, int64_t S, int M,
-                                                                  float* __restrict__ mass,
-                                                                  uint32_t* __restrict__ keys,
-                                                                  int32_t* __restrict__ ident)
+                                                                  uint32_t* __restrict__ keys)
 {
     __shared__ float red[kStatThreads / 64];
     const int64_t n = blockIdx.x;
@@ -249,9 +247,7 @@ __global__ __launch_bounds__(kStatThreads) void block_mass_kernel(const float* _
     if (threadIdx.x == 0) {
         float t = 0.0f;
         for (int i = 0; i < kStatThreads / 64; ++i) t += red[i];
-        mass[n] = t;
         keys[n] = score_key(t);
-        ident[n] = (int32_t)n;
     }
 }
 
@@ -260,9 +256,7 @@ size_t align256k(size_t v) { return (v + 255) & ~(size_t)255; }
 struct KvstarWs {
     float* scores;
     float* stats;
-    float* mass;
     uint32_t* keys;
-    int32_t* ident;
     size_t bytes;
 };
 
@@ -274,12 +268,8 @@ KvstarWs carve_kvstar(void* base, int64_t rows, int64_t S, int64_t n_blocks)
     off += align256k((size_t)rows * S * 4);
     w.stats = (float*)((char*)base + off);
     off += align256k((size_t)rows * 8);
-    w.mass = (float*)((char*)base + off);
-    off += align256k((size_t)n_blocks * 4);
     w.keys = (uint32_t*)((char*)base + off);
-    off += align256k((size_t)n_blocks * 4);
-    w.ident = (int32_t*)((char*)base + off);
-    off += align256k((size_t)n_blocks * 4);
+    off += align256k((size_t)key_pitch(n_blocks) * 4);
     w.bytes = off;
     return w;
 }
@@ -339,11 +329,11 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     rc = ucm::launch_status("row_stats_kernel");
     if (rc != UCM_OK) return rc;
     hipLaunchKernelGGL(block_mass_kernel, dim3((unsigned)n_blocks), dim3(kStatThreads), 0, st, w.scores,
-                       w.stats, (int)rows, S, (int)M, w.mass, w.keys, w.ident);
+                       w.stats, (int)rows, S, (int)M, w.keys);
     rc = ucm::launch_status("block_mass_kernel");
     if (rc != UCM_OK) return rc;
     SortArgs s{};
-    s.keys = w.keys; s.scores = w.mass; s.idx = w.ident; s.max_n = (int)n_blocks; s.topk = topk;
+    s.keys = w.keys; s.pitch = key_pitch(n_blocks); s.max_n = (int)n_blocks; s.topk = topk;
     s.out_idx = out_idx; s.out_score = out_score;
-    return launch_topk_sort(s, 1, st);
+    return launch_topk(s, 1, st);
 }
