@@ -65,6 +65,39 @@ def test_matches_checker(X, Hq, Hkv, d, n, M, topk):
     check(q, k, None, topk)
 
 
+@pytest.mark.parametrize("X,Hq,Hkv,d,n,M,topk", [
+    (8, 8, 2, 32, 40, 31, 7),      # 32 query rows per KV head: whole tiles; one short of a tile of representatives
+    (9, 8, 2, 64, 40, 32, 7),      # a row more than a tile; a block is a tile of representatives
+    (3, 6, 2, 128, 9, 33, 9),      # a block of two tiles, the second with one representative
+    (2, 4, 2, 32, 300, 3, 20),     # ten blocks share a tile
+    (1, 2, 1, 64, 1, 100, 1),      # one block of several tiles
+    (2, 4, 4, 32, 33, 63, 33),     # an odd number of row tiles per workgroup pair, chunks that end inside a tile
+    (40, 64, 2, 32, 12, 2, 12),    # 2560 rows: statistics in two batches
+    (2, 4, 2, 24, 21, 16, 5),      # head dim of one and a half k-steps
+    (2, 4, 2, 256, 21, 16, 5),     # head dim above what is kept packed
+    (1, 2, 2, 32, 70, 256, 11),    # more tiles than two per wave and chunk
+])
+def test_edges_of_the_tiles(X, Hq, Hkv, d, n, M, topk):
+    q, k = make(X * 100 + n + d, X, Hq, Hkv, d, n, M)
+    check(q, k, None, topk)
+
+
+def test_far_scores_keep_their_order():
+    """Blocks whose every probability lies far below the largest (e^-60 to e^-95) keep the order of
+    their masses, down into the denormal range.  Relative tolerance: the scores' own rounding, 2^-24 of
+    their size (95), moves a probability by 95 * 2^-24 < 6e-6; below 1e-38 one step of a denormal."""
+    n, d = 36, 32
+    q = np.zeros((1, 1, d), np.float16)
+    q[0, 0, 0] = 8.0
+    k = np.zeros((n, 1, 1, d), np.float16)
+    k[:, 0, 0, 0] = -np.arange(n) * 2.65 / 8.0
+    gi, gs = run_gpu(q, k, None, n)
+    s = (q.astype(np.float64)[0, 0] @ k.astype(np.float64)[:, 0, 0].T)
+    ref = np.exp(s - s.max()) / np.exp(s - s.max()).sum()
+    assert gi.tolist() == list(range(n))
+    assert np.all(np.abs(gs - ref) <= 1e-5 * ref + 2e-45)
+
+
 def test_sharp_softmax():
     # larger logits: a few representatives take most of the mass
     q, k = make(11, 4, 8, 4, 64, 200, 2, scale=1.5)

@@ -10,13 +10,18 @@
 //      <= 1e-9, as the reference does);
 //   4. block score[n] = sum over x, H and the M representatives of block n;
 //   5. the topk blocks by descending score.
-// Kernels: qk_score_kernel (one thread per (s, kv head), the head's query rows broadcast from
-// LDS, K read once: the HBM-bound part), row_stats_kernel (max and sum of exponentials per
-// (x, H) row), block_mass_kernel (probabilities summed over rows in a fixed order, then over a
-// block's representatives: deterministic, no atomics) and the shared top-k selection.
-// Sums are taken in a different order than the reference's loops; the tolerance is stated
-// where the results are compared.  Equal scores come out in ascending block order (the
-// reference's heap pops them in descending block order).
+// Kernels: kvstar_stats_kernel (q.k on the matrix cores; maximum and sum of exponentials of every
+// (x, H) row over one chunk of the representatives), kvstar_mass_kernel (the chunks' pairs merged,
+// q.k once more, probabilities summed over rows and a block's representatives) and the shared top-k
+// selection.  The [X Hq, S] score matrix is never stored: writing it and reading it back twice moved
+// seven times the bytes of the keys themselves, and computing q.k a second time costs two matrix
+// instructions per 32 x 32 scores of 32 channels.  At 8 query tokens x 32 heads, 253 blocks x 64
+// representatives and 32 channels the four kernels that stored it took 32.9 us (13.6 q.k, 8.6 row
+// statistics, 6.1 block sums, 5.7 selection); these three take 17.8 us
+// (7.2, 8.3, 3.6; without the exponentials 6.0 and 7.3: what is left is launches and round trips).
+// Sums are taken in a different order than the reference's loops, the same one on every call (no
+// atomics); the tolerance is stated where the results are compared.  Equal scores come out in
+// ascending block order (the reference's heap pops them in descending block order).
 #include <hip/hip_fp16.h>
 
 #include "common.h"
@@ -24,254 +29,439 @@
 
 namespace {
 
-constexpr int kQkThreads = 256;  // the matrix-core kernel stages 32 query rows with 8 threads each
-constexpr int kStatThreads = 1024;
-constexpr int kRowTile = 16;  // query rows of one KV head scored per pass over a K vector
-
-struct QkArgs {
-    const __half* q;        // [X, Hq, d_orig]
-    const __half* k;        // [S, Hkv, d]
-    const int64_t* pruned;  // [Hkv, d] or null
-    int X, Hq, Hkv, g, d_orig, d;
-    int64_t S;
-    float* scores;          // [X * Hq, S]
-};
-
-// grid = (ceil(S / 256), Hkv, ceil(X * g / kRowTile)); LDS: kRowTile rows of d floats
-__global__ __launch_bounds__(kQkThreads) void qk_score_kernel(QkArgs a)
-{
-    extern __shared__ __align__(16) float qs[];  // [kRowTile][d]
-    __shared__ int orow[kRowTile];               // score row x * Hq + H of each query row, -1 = none
-    const int h = blockIdx.y;
-    const int row0 = blockIdx.z * kRowTile;  // first (x, gg) pair of this pass
-    const int rows = a.X * a.g;
-    if (threadIdx.x < kRowTile) {
-        const int rr = row0 + threadIdx.x;
-        orow[threadIdx.x] = rr < rows ? (rr / a.g) * a.Hq + h * a.g + rr % a.g : -1;
-    }
-    // stage the pass's query rows of KV head h: row r = x * g + gg  <->  q head H = h * g + gg
-    for (int i = threadIdx.x; i < kRowTile * a.d; i += kQkThreads) {
-        const int r = row0 + i / a.d, j = i % a.d;
-        float v = 0.0f;
-        if (r < rows) {
-            const int x = r / a.g, H = h * a.g + r % a.g;
-            int64_t src = a.pruned ? a.pruned[(int64_t)h * a.d + j] : j;
-            src = src < 0 ? 0 : (src >= a.d_orig ? a.d_orig - 1 : src);  // stay inside the row
-            v = __half2float(a.q[((int64_t)x * a.Hq + H) * a.d_orig + src]);
-        }
-        qs[i] = v;
-    }
-    __syncthreads();
-    const int64_t s = (int64_t)blockIdx.x * kQkThreads + threadIdx.x;
-    if (s >= a.S) return;
-    const __half* kv = a.k + (s * a.Hkv + h) * a.d;
-    float acc[kRowTile];
-#pragma unroll
-    for (int r = 0; r < kRowTile; ++r) acc[r] = 0.0f;
-    if ((a.d & 7) == 0) {  // 16-byte pieces of the K vector
-        for (int j = 0; j < a.d; j += 8) {
-            const uint4 raw = *reinterpret_cast<const uint4*>(kv + j);
-            __half hv[8];
-            __builtin_memcpy(hv, &raw, 16);
-            float kf[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) kf[i] = __half2float(hv[i]);
-#pragma unroll
-            for (int r = 0; r < kRowTile; ++r) {  // 16-byte LDS reads, the same address in all lanes
-                const float4 qa = *reinterpret_cast<const float4*>(qs + r * a.d + j);
-                const float4 qb = *reinterpret_cast<const float4*>(qs + r * a.d + j + 4);
-                float t = acc[r];
-                t = __builtin_fmaf(qa.x, kf[0], t);
-                t = __builtin_fmaf(qa.y, kf[1], t);
-                t = __builtin_fmaf(qa.z, kf[2], t);
-                t = __builtin_fmaf(qa.w, kf[3], t);
-                t = __builtin_fmaf(qb.x, kf[4], t);
-                t = __builtin_fmaf(qb.y, kf[5], t);
-                t = __builtin_fmaf(qb.z, kf[6], t);
-                t = __builtin_fmaf(qb.w, kf[7], t);
-                acc[r] = t;
-            }
-        }
-    } else {
-        for (int j = 0; j < a.d; ++j) {
-            const float kf = __half2float(kv[j]);
-#pragma unroll
-            for (int r = 0; r < kRowTile; ++r) acc[r] = __builtin_fmaf(qs[r * a.d + j], kf, acc[r]);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < kRowTile; ++r) {
-        const int o = orow[r];
-        if (o >= 0) a.scores[(int64_t)o * a.S + s] = acc[r];
-    }
-}
+constexpr int kThreads = 512;       // both kernels: eight waves
+constexpr int kStatItems = 2;       // row tiles a workgroup of the statistics kernel serves
+constexpr int kStatSubs = 4;        // waves that share a row tile's representatives there
+constexpr int kMaxChunks = 64;      // partial statistics per row
+constexpr int kMassRows = 2048;     // rows whose statistics the mass kernel holds in LDS at a time
+constexpr int kMassGroups = 512;    // its workgroups at most
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// q.k on the matrix cores for head dims that are multiples of 16: one workgroup per (128
-// representatives, KV head, 32 query rows); the query tile (channel-pruned) is gathered once
-// into LDS, then each wave takes 32 representatives: d / 16 v_mfma_f32_32x32x16_f16 with the
-// query tile as the A operand (lane: row lane % 32, eight channels of the k-step, one 16-byte
-// LDS read) and the representatives as the B operand (one 16-byte global load per lane and
-// k-step).  Accumulator v of a lane is
-// score[row 8 (v / 4) + 4 (lane / 32) + v % 4][representative lane % 32]: lanes 0..31 store 32
-// consecutive floats of one score row.  grid = (ceil(S / 128), Hkv, ceil(X g / 32));
-// LDS = 32 rows of (d + 8) halves.
-__global__ __launch_bounds__(kQkThreads) void qk_mfma_kernel(QkArgs a)
-{
-    extern __shared__ __align__(16) _Float16 qt[];  // [32][d + 8]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int h = blockIdx.y;
-    const int rows = a.X * a.g;
-    const int dp = a.d + 8;  // row pitch: 16 bytes of padding spread the rows over the banks
-    const _Float16* q = reinterpret_cast<const _Float16*>(a.q);
-    {
-        // eight threads per query row, each taking every eighth channel: one division per thread
-        const int rl = threadIdx.x >> 3;
-        const int rr = blockIdx.z * 32 + rl;
-        const bool ok = rr < rows;
-        const _Float16* qrow = q + ((int64_t)(ok ? rr / a.g : 0) * a.Hq + h * a.g + (ok ? rr % a.g : 0)) * a.d_orig;
-        for (int j = threadIdx.x & 7; j < a.d; j += 8) {
-            int64_t src = a.pruned ? a.pruned[(int64_t)h * a.d + j] : j;
-            src = src < 0 ? 0 : (src >= a.d_orig ? a.d_orig - 1 : src);  // stay inside the row
-            qt[rl * dp + j] = ok ? qrow[src] : (_Float16)0;
-        }
-    }
-    __syncthreads();
-    const int64_t s0 = ((int64_t)blockIdx.x * (kQkThreads / 64) + wave) * 32;
-    if (s0 >= a.S) return;  // wave-uniform, after the only barrier
-    int64_t s = s0 + (lane & 31);
-    const bool s_ok = s < a.S;
-    if (!s_ok) s = a.S - 1;
-    const int kb = (lane >> 5) * 8;  // channels kb .. kb + 7 of a k-step
-    const __half* kv = a.k + (s * a.Hkv + h) * a.d + kb;
-    const _Float16* qa_row = qt + (lane & 31) * dp + kb;
-    f32x16 acc = {0};
-    for (int c = 0; c < a.d; c += 16) {
-        const f16x8 qa = *reinterpret_cast<const f16x8*>(qa_row + c);
-        const f16x8 kk = *reinterpret_cast<const f16x8*>(kv + c);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(qa, kk, acc, 0, 0, 0);
-    }
-    // score row of query row lane % 32 (one division per lane, handed round by shuffles:
-    // sixteen divisions per lane in the store loop cost more than the matrix products)
-    const int r = blockIdx.z * 32 + (lane & 31);
-    const int orow = r < rows ? (r / a.g) * a.Hq + h * a.g + r % a.g : -1;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int o = __shfl(orow, 8 * (v / 4) + 4 * (lane >> 5) + (v % 4));
-        if (s_ok && o >= 0) a.scores[(int64_t)o * a.S + s] = acc[v];
-    }
-}
-
-// Running (max, sum of exp(x - max)) pairs merge associatively; a side that has seen nothing
-// carries max = -inf and sum = 0.
-__device__ __forceinline__ void merge_stats(float& m, float& sum, float om, float osum)
-{
-    const float nm = fmaxf(m, om);
-    if (nm == -INFINITY) return;
-    sum = sum * expf(m - nm) + osum * expf(om - nm);
-    m = nm;
-}
-
-// One workgroup per (x, H) row: max over s and sum of exp(score - max), in one pass over the
-// row (eight loads in flight per thread, running pairs merged at the end).
-__global__ __launch_bounds__(kStatThreads) void row_stats_kernel(const float* __restrict__ scores,
-                                                                 int64_t S, float* __restrict__ stats)
-{
-    __shared__ float red_m[kStatThreads / 64], red_s[kStatThreads / 64];
-    const float* row = scores + (int64_t)blockIdx.x * S;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    float m = -INFINITY, sum = 0.0f;
-    for (int64_t base = threadIdx.x; base < S; base += 8 * kStatThreads) {
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int64_t s = base + (int64_t)i * kStatThreads;
-            v[i] = s < S ? row[s] : -INFINITY;
-        }
-        float cm = v[0];
-#pragma unroll
-        for (int i = 1; i < 8; ++i) cm = fmaxf(cm, v[i]);
-        if (cm == -INFINITY) continue;
-        float cs = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) cs += expf(v[i] - cm);
-        merge_stats(m, sum, cm, cs);
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) merge_stats(m, sum, __shfl_xor(m, o), __shfl_xor(sum, o));
-    if (lane == 0) {
-        red_m[w] = m;
-        red_s[w] = sum;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float tm = red_m[0], ts = red_s[0];
-        for (int i = 1; i < kStatThreads / 64; ++i) merge_stats(tm, ts, red_m[i], red_s[i]);
-        stats[2 * blockIdx.x] = tm;
-        // the reference normalises only when the sum exceeds 1e-9
-        stats[2 * blockIdx.x + 1] = ts > 1e-9f ? 1.0f / ts : 1.0f;
-    }
-}
-
-// One workgroup per block n: probabilities of its M representatives summed over all rows, in a
-// fixed order (strided partial sums, xor-shuffle tree, then the waves in turn).
-__global__ __launch_bounds__(kStatThreads) void block_mass_kernel(const float* __restrict__ scores,
-                                                                  const float* __restrict__ stats,
-                                                                  int rows, int64_t S, int M,
-                                                                  uint32_t* __restrict__ keys)
-{
-    __shared__ float red[kStatThreads / 64];
-    const int64_t n = blockIdx.x;
-    const float* base = scores + n * M;
-    const int total = rows * M;
-    float part = 0.0f;
-    // element e = r * M + m; e advances by the workgroup size: (r, m) follow without a division
-    const int dr = kStatThreads / M, dm = kStatThreads % M;
-    int r = threadIdx.x / M, m = threadIdx.x % M;
-#pragma unroll 4
-    for (int e = threadIdx.x; e < total; e += kStatThreads) {
-        part += expf(base[(int64_t)r * S + m] - stats[2 * r]) * stats[2 * r + 1];
-        r += dr;
-        m += dm;
-        if (m >= M) {
-            m -= M;
-            ++r;
-        }
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) part += __shfl_xor(part, o);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0.0f;
-        for (int i = 0; i < kStatThreads / 64; ++i) t += red[i];
-        keys[n] = score_key(t);
-    }
-}
-
-size_t align256k(size_t v) { return (v + 255) & ~(size_t)255; }
-
-struct KvstarWs {
-    float* scores;
-    float* stats;
-    uint32_t* keys;
-    size_t bytes;
+// Sums of exponentials over parts of a row meet as (e, s) = s 2^e with a whole number e near the part's
+// maximum: merging two is a shift and an addition, not two more exponentials.
+struct Stat {
+    int e;
+    float s;
 };
 
-KvstarWs carve_kvstar(void* base, int64_t rows, int64_t S, int64_t n_blocks)
+// The X * g query rows of a KV head are cut into tiles of 32; item = h * tiles_q + tile.
+struct KvArgs {
+    const _Float16* q;      // [X, Hq, d_orig]
+    const _Float16* k;      // [S, Hkv, d]
+    const int64_t* pruned;  // [Hkv, d] or null
+    int X, Hq, Hkv, g, d_orig, d;
+    int64_t S;
+    int n_blocks, M;
+    int tiles_q, items;     // row tiles per KV head, and of all heads
+    int tiles_k, per_chunk; // tiles of 32 representatives: all, and per chunk of the statistics kernel
+    int chunks;
+    _Float16* qp;           // [items][32][d] query rows, channels pruned, zeros behind the last row (KS > 0)
+    Stat* part;             // [chunks][items * 32] sum of exponentials over a chunk
+    uint32_t* keys;         // [n_blocks]
+    int group_blocks;       // blocks a workgroup of the mass kernel handles together
+    int groups;
+};
+
+typedef _Float16 f16x8u __attribute__((ext_vector_type(8), aligned(2)));
+
+// Channels c .. c + 7 of a representative's row, zeros past d.
+__device__ __forceinline__ f16x8 load_k(const _Float16* row, int c, int d)
 {
-    KvstarWs w{};
+    f16x8 v = {0};
+    if (c + 8 <= d) {
+        v = *reinterpret_cast<const f16x8u*>(row + c);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = c + i < d ? row[c + i] : (_Float16)0;
+    }
+    return v;
+}
+
+// The query row of place r of an item: KV head h's row rr = x * g + gg belongs to query head h * g + gg.
+struct QRow {
+    const _Float16* row;
+    const int64_t* pruned;  // the KV head's channels, or null
+    bool ok;
+};
+
+__device__ __forceinline__ QRow q_row(const KvArgs& a, int item, int r)
+{
+    const int h = item / a.tiles_q;
+    const int rr = (item - h * a.tiles_q) * 32 + r;
+    QRow q;
+    q.ok = item < a.items && rr < a.X * a.g;
+    q.row = a.q + ((int64_t)(q.ok ? rr / a.g : 0) * a.Hq + (q.ok ? h * a.g + rr % a.g : 0)) * a.d_orig;
+    q.pruned = a.pruned ? a.pruned + (int64_t)(q.ok ? h : 0) * a.d : nullptr;
+    return q;
+}
+
+// Channel j of a query row; an index outside the row is moved to its ends.
+__device__ __forceinline__ int64_t q_channel(const QRow& q, int j, int d_orig)
+{
+    const int64_t src = q.pruned ? q.pruned[j] : j;
+    return src < 0 ? 0 : (src >= d_orig ? d_orig - 1 : src);
+}
+
+// Channels c .. c + 7 of a query row, zeros past d and for a row that does not exist.
+__device__ __forceinline__ f16x8 load_q(const QRow& q, int c, int d, int d_orig)
+{
+    f16x8 v;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = q.ok && c + i < d ? q.row[q_channel(q, c + i, d_orig)] : (_Float16)0;
+    return v;
+}
+
+constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596303e-8f;  // log2(e) in two pieces
+constexpr float kLn2 = 0.693147182f, kLn2Low = -1.90465421e-9f;   // ln(2) in two pieces
+
+// exp(x) for x far from overflow (here x <= 0 but for rounding): 2^(x log2 e) with the product's
+// rounding error carried along, whole and fractional part of the exponent taken apart so that results
+// down to the smallest denormal come out.  A NaN stays one.  12 instructions where expf() has 17 (it
+// tests both ends of its range): the two passes' exponentials are most of these kernels' instructions.
+__device__ __forceinline__ float exp_small(float x)
+{
+    x = __builtin_elementwise_maximum(x, -200.0f);  // also minus infinity; the result is 0 either way
+    const float t = x * kLog2e;
+    const float n = __builtin_rintf(t);
+    const float r = __builtin_fmaf(x, kLog2eLow, __builtin_fmaf(x, kLog2e, -t));
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - n) + r), (int)n);
+}
+
+__device__ __forceinline__ Stat to_stat(float m, float sum)  // sum of exp(x - m)
+{
+    if (m == -INFINITY) return Stat{-(1 << 28), 0.0f};  // nothing seen
+    const float e = __builtin_rintf(m * kLog2e);
+    const float d = __builtin_fmaf(-e, kLn2Low, __builtin_fmaf(-e, kLn2, m));
+    return Stat{(int)e, sum * expf(d)};
+}
+
+__device__ __forceinline__ Stat merge(Stat a, Stat b)
+{
+    const int e = a.e > b.e ? a.e : b.e;
+    return Stat{e, __builtin_amdgcn_ldexpf(a.s, a.e - e) + __builtin_amdgcn_ldexpf(b.s, b.e - e)};
+}
+
+// grid = (chunks, ceil(items / kStatItems)).  Wave w serves row tile w % kStatItems and every
+// kStatSubs-th tile of representatives of the chunk.  Representatives are the A operand (lane:
+// representative lane % 32, channels 8 (lane / 32) .. + 7 of the k-step), query rows the B operand:
+// accumulator v of a lane is the score of row lane % 32 against representative
+// 8 (v / 4) + 4 (lane / 32) + v % 4 of the tile, so a row's statistics are one lane's work and meet
+// once, at the end.  KS = d / 16 for 32, 64 and 128 channels: the loads of several tiles go out
+// together, in front of the gather of the query rows (which all waves share through LDS).  KS = 0: any d.
+template <int KS>
+__global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
+{
+    constexpr int U = KS == 0 || KS > 4 ? 1 : 2;  // tiles in flight per wave
+    constexpr int dp = KS * 16 + 8;  // row pitch: 16 bytes of padding spread the rows over the banks
+    __shared__ __align__(16) _Float16 qt[KS ? kStatItems * 32 * dp : 8];
+    __shared__ Stat red[kThreads / 64][32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = wave % kStatItems, sub = wave / kStatItems;
+    const int item = blockIdx.y * kStatItems + li;
+    const int h = item < a.items ? item / a.tiles_q : 0;
+    const int kb = (lane >> 5) * 8;
+    const int t0 = blockIdx.x * a.per_chunk + sub;
+    int t1 = (blockIdx.x + 1) * a.per_chunk;
+    t1 = item < a.items ? (t1 < a.tiles_k ? t1 : a.tiles_k) : 0;
+    auto k_row = [&](int t) {
+        int64_t s = (int64_t)t * 32 + (lane & 31);
+        s = s < a.S ? s : a.S - 1;
+        return a.k + (s * a.Hkv + h) * a.d;
+    };
+    f16x8 kk[U][KS ? KS : 1];
+    auto load_tiles = [&](int t) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const _Float16* row = k_row(t + u * kStatSubs < t1 ? t + u * kStatSubs : t);
+#pragma unroll
+            for (int c = 0; c < KS; ++c) kk[u][c] = *reinterpret_cast<const f16x8*>(row + c * 16 + kb);
+        }
+    };
+    if constexpr (KS > 0) {
+        load_tiles(t0 < a.tiles_k ? t0 : 0);
+        // eight threads per query row, each taking every eighth channel
+        const int rl = threadIdx.x >> 3;  // 0 .. 63: row rl % 32 of the workgroup's item rl / 32
+        const QRow q = q_row(a, blockIdx.y * kStatItems + (rl >> 5), rl & 31);
+        int64_t src[2 * KS];
+        _Float16 v[2 * KS];
+#pragma unroll
+        for (int i = 0; i < 2 * KS; ++i) src[i] = q_channel(q, (threadIdx.x & 7) + 8 * i, a.d_orig);
+#pragma unroll
+        for (int i = 0; i < 2 * KS; ++i) v[i] = q.row[src[i]];
+#pragma unroll
+        for (int i = 0; i < 2 * KS; ++i) qt[rl * dp + (threadIdx.x & 7) + 8 * i] = q.ok ? v[i] : (_Float16)0;
+        __syncthreads();
+        if (blockIdx.x == 0) {  // the gathered rows, for the mass kernel
+            for (int i = threadIdx.x; i < kStatItems * 32 * 2 * KS; i += kThreads) {
+                const int r = i / (2 * KS), c = (i % (2 * KS)) * 8;
+                const int64_t row = (int64_t)blockIdx.y * kStatItems * 32 + r;
+                if (row < (int64_t)a.items * 32)
+                    *reinterpret_cast<f16x8*>(a.qp + row * (KS * 16) + c) = *reinterpret_cast<const f16x8*>(qt + r * dp + c);
+            }
+        }
+    }
+    float m = -INFINITY, sum = 0.0f;
+    // the scores of U tiles (t, t + kStatSubs, ...) join the row's statistics
+    auto add_tiles = [&](const f32x16 (&acc)[U], int t) {
+        float x[U][16];
+        float nm = m;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t s0 = (int64_t)(t + u * kStatSubs) * 32;
+            const bool whole = t + u * kStatSubs < t1 && s0 + 32 <= a.S;  // uniform
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                x[u][v] = acc[u][v];
+                if (!whole && (t + u * kStatSubs >= t1 || s0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4 >= a.S))
+                    x[u][v] = -INFINITY;
+                nm = fmaxf(nm, x[u][v]);
+            }
+        }
+        if (nm == -INFINITY) return;
+        float cs = 0.0f;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) cs += exp_small(x[u][v] - nm);
+        sum = sum * exp_small(m - nm) + cs;
+        m = nm;
+    };
+    for (int t = t0; t < t1; t += U * kStatSubs) {
+        f32x16 acc[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc[u] = f32x16{0};
+        if constexpr (KS > 0) {
+            if (t != t0) load_tiles(t);
+            const _Float16* qrow = qt + (li * 32 + (lane & 31)) * dp + kb;
+#pragma unroll
+            for (int c = 0; c < KS; ++c) {
+                const f16x8 qq = *reinterpret_cast<const f16x8*>(qrow + c * 16);
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk[u][c], qq, acc[u], 0, 0, 0);
+            }
+        } else {
+            const _Float16* row = k_row(t);
+            const QRow q = q_row(a, item, lane & 31);
+            for (int c = 0; c < a.d; c += 16)
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(load_k(row, c + kb, a.d),
+                                                                load_q(q, c + kb, a.d, a.d_orig), acc[0], 0, 0, 0);
+        }
+        add_tiles(acc, t);
+    }
+    Stat st = to_stat(m, sum);
+    st = merge(st, Stat{__shfl_xor(st.e, 32), __shfl_xor(st.s, 32)});  // the row's other representatives
+    if (lane < 32) red[wave][lane] = st;
+    __syncthreads();
+    if (sub == 0 && lane < 32 && item < a.items) {
+#pragma unroll
+        for (int i = 1; i < kStatSubs; ++i) st = merge(st, red[li + i * kStatItems][lane]);
+        a.part[(int64_t)blockIdx.x * a.items * 32 + item * 32 + lane] = st;
+    }
+}
+
+// One workgroup per group of blocks (a block of 32 and more representatives, or as many small blocks as
+// 32 representatives make): the rows' statistics merged from the chunks' pairs, then each wave takes
+// every eighth row tile against the group's representatives, now as the B operand: accumulator v of a
+// lane is row 8 (v / 4) + 4 (lane / 32) + v % 4 against representative lane % 32, whose probabilities
+// add up in the lane.  Partial sums meet in a fixed order: accumulators, row tiles of a wave, lane
+// halves, waves, representatives.
+template <int KS>
+__global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
+{
+    constexpr int kWaves = kThreads / 64;
+    __shared__ __align__(16) float2 stat[kMassRows];  // (shift, 1 / sum of exponentials) of a row
+    __shared__ Stat halves[kThreads];
+    __shared__ float red[kWaves][32];
+    __shared__ float rep[32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int kb = (lane >> 5) * 8;
+    const int rows = a.items * 32;
+    const int batches = (rows + kMassRows - 1) / kMassRows;
+    const int real = a.X * a.g;  // query rows of a KV head
+    for (int grp = blockIdx.x; grp < a.groups; grp += gridDim.x) {
+        const int64_t s0 = (int64_t)grp * a.group_blocks * a.M;  // the group's first representative
+        const int64_t left = a.S - s0;
+        const int64_t want = (int64_t)a.group_blocks * a.M;
+        const int ns = (int)(left < want ? left : want);
+        float tot = 0.0f;
+        for (int batch = 0; batch < batches; ++batch) {
+            const int r0 = batch * kMassRows;
+            const int nr = rows - r0 < kMassRows ? rows - r0 : kMassRows;
+            if (batches > 1 || grp == (int)blockIdx.x) {
+                // two threads per row where the rows leave half of the workgroup idle
+                const bool split = nr <= kThreads / 2;
+                const int step = split ? kThreads / 2 : kThreads;
+                const int half = split ? threadIdx.x / (kThreads / 2) : 0;
+                const int c_mid = split ? (a.chunks + 1) / 2 : a.chunks;
+                const int c0 = half ? c_mid : 0, c1 = half ? a.chunks : c_mid;
+                for (int r = split ? threadIdx.x % (kThreads / 2) : threadIdx.x; r < (split ? step : nr); r += step) {
+                    Stat st{-(1 << 28), 0.0f};
+                    if (r < nr) {
+                        const Stat* p = a.part + r0 + r;
+                        for (int c = c0; c < c1; c += 16) {
+                            Stat v[16];
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) v[i] = p[(int64_t)(c + i < c1 ? c + i : c1 - 1) * rows];
+                            int e = st.e;
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) e = e > v[i].e ? e : v[i].e;
+                            float sum = __builtin_amdgcn_ldexpf(st.s, st.e - e);
+#pragma unroll
+                            for (int i = 0; i < 16; ++i)
+                                sum += c + i < c1 ? __builtin_amdgcn_ldexpf(v[i].s, v[i].e - e) : 0.0f;
+                            st = Stat{e, sum};
+                        }
+                    }
+                    if (split) {
+                        halves[threadIdx.x] = st;
+                        __syncthreads();
+                        if (half == 0) st = merge(st, halves[threadIdx.x + kThreads / 2]);
+                    }
+                    if (half == 0 && r < nr) {
+                        // the shift e ln 2 rounded, its rounding error moved into the factor
+                        const float e = (float)st.e, shift = e * kLn2;
+                        const float d = __builtin_fmaf(-e, kLn2Low, __builtin_fmaf(-e, kLn2, shift));
+                        // the reference normalises only when the sum exceeds 1e-9
+                        stat[r] = make_float2(shift, st.s > 1e-9f ? expf(d) / st.s : 1.0f);
+                    }
+                }
+                __syncthreads();
+            }
+            const int items = nr / 32;
+            for (int it = wave; it < items; it += kWaves) {
+                const int item = r0 / 32 + it;
+                const int h = item / a.tiles_q;
+                const int valid = real - (item - h * a.tiles_q) * 32;  // rows of the tile that exist
+                const _Float16* qrow = a.qp + ((int64_t)item * 32 + (lane & 31)) * (KS * 16) + kb;
+                f16x8 qq[KS ? KS : 1];
+#pragma unroll
+                for (int c = 0; c < KS; ++c) qq[c] = *reinterpret_cast<const f16x8*>(qrow + c * 16);
+                auto add_tile = [&](const f32x16& acc, int t) {
+                    float p = 0.0f;
+#pragma unroll
+                    for (int v4 = 0; v4 < 4; ++v4) {
+                        const int row = 8 * v4 + 4 * (lane >> 5);
+                        const float4 sa = *reinterpret_cast<const float4*>(&stat[it * 32 + row]);
+                        const float4 sb = *reinterpret_cast<const float4*>(&stat[it * 32 + row + 2]);
+                        const float mm[4] = {sa.x, sa.z, sb.x, sb.z}, inv[4] = {sa.y, sa.w, sb.y, sb.w};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float e = exp_small(acc[v4 * 4 + i] - mm[i]) * inv[i];
+                            p += valid >= 32 || row + i < valid ? e : 0.0f;
+                        }
+                    }
+                    if (t * 32 + (lane & 31) < ns) tot += p;
+                };
+                for (int t = 0; t * 32 < ns; t += 2) {
+                    if constexpr (KS > 0) {
+                        f16x8 kk[2][KS];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            const int s = (t + u) * 32 + (lane & 31);
+                            const _Float16* row = a.k + ((s0 + (s < ns ? s : ns - 1)) * a.Hkv + h) * a.d;
+#pragma unroll
+                            for (int c = 0; c < KS; ++c) kk[u][c] = *reinterpret_cast<const f16x8*>(row + c * 16 + kb);
+                        }
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            if ((t + u) * 32 >= ns) break;
+                            f32x16 acc = {0};
+#pragma unroll
+                            for (int c = 0; c < KS; ++c)
+                                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(qq[c], kk[u][c], acc, 0, 0, 0);
+                            add_tile(acc, t + u);
+                        }
+                    } else {
+                        for (int u = 0; u < 2 && (t + u) * 32 < ns; ++u) {
+                            const int s = (t + u) * 32 + (lane & 31);
+                            const _Float16* row = a.k + ((s0 + (s < ns ? s : ns - 1)) * a.Hkv + h) * a.d;
+                            const QRow q = q_row(a, item, lane & 31);
+                            f32x16 acc = {0};
+                            for (int c = 0; c < a.d; c += 16)
+                                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(load_q(q, c + kb, a.d, a.d_orig),
+                                                                             load_k(row, c + kb, a.d), acc, 0, 0, 0);
+                            add_tile(acc, t + u);
+                        }
+                    }
+                }
+            }
+            if (batches > 1) __syncthreads();  // the next batch overwrites the statistics
+        }
+        tot += __shfl_xor(tot, 32);
+        if (lane < 32) red[wave][lane] = tot;
+        __syncthreads();
+        if (wave == 0) {
+            float t = 0.0f;
+            if (lane < 32) {
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w) t += red[w][lane];
+                rep[lane] = t;
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (a.M >= 32) {
+                // every lane's representatives belong to the one block
+#pragma unroll
+                for (int o = 16; o >= 1; o >>= 1) t += __shfl_xor(t, o);
+                if (lane == 0) a.keys[grp] = score_key(t);
+            } else {
+                const int blk = grp * a.group_blocks + lane;
+                if (lane < a.group_blocks && blk < a.n_blocks) {
+                    float s = 0.0f;
+                    for (int i = 0; i < a.M; ++i) s += rep[lane * a.M + i];
+                    a.keys[blk] = score_key(s);
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+constexpr int kPackedDim = 128;  // the largest head dimension whose query rows are kept packed
+
+// How the representatives are shared out.
+void plan_chunks(KvArgs& a)
+{
+    a.S = (int64_t)a.n_blocks * a.M;
+    a.tiles_k = (int)ucm::ceil_div(a.S, 32);
+    // two tiles per wave at least.  kMaxChunks: 32 leave half of the chip idle at 8 KV heads (statistics
+    // 8.9 us instead of 7.2), and every workgroup of the mass kernel reads all chunks' pairs of its rows
+    a.per_chunk = (int)ucm::ceil_div(a.tiles_k, kMaxChunks);
+    if (a.per_chunk < 2 * kStatSubs) a.per_chunk = 2 * kStatSubs;
+    a.chunks = (int)ucm::ceil_div(a.tiles_k, a.per_chunk);
+    a.group_blocks = a.M >= 32 ? 1 : 32 / a.M;
+    a.groups = (int)ucm::ceil_div(a.n_blocks, a.group_blocks);
+}
+
+// Addresses of the workspace's parts; the sizes hold for every number of KV heads and every head
+// dimension (the caller asks with neither).
+size_t carve_kvstar(KvArgs& a, void* base)
+{
+    const size_t rows = (size_t)a.Hq * (a.X + 31);  // at most 31 rows of padding per KV head
+    char* p = (char*)base;
     size_t off = 0;
-    w.scores = (float*)((char*)base + off);
-    off += align256k((size_t)rows * S * 4);
-    w.stats = (float*)((char*)base + off);
-    off += align256k((size_t)rows * 8);
-    w.keys = (uint32_t*)((char*)base + off);
-    off += align256k((size_t)key_pitch(n_blocks) * 4);
-    w.bytes = off;
-    return w;
+    a.qp = (_Float16*)(p + off);
+    off += align256(rows * kPackedDim * 2);
+    a.part = (Stat*)(p + off);
+    off += align256((size_t)a.chunks * rows * 8);
+    a.keys = (uint32_t*)(p + off);
+    off += align256((size_t)key_pitch(a.n_blocks) * 4);
+    return off;
+}
+
+template <int KS>
+int launch_kvstar(const KvArgs& a, hipStream_t st)
+{
+    const dim3 grid((unsigned)a.chunks, (unsigned)ucm::ceil_div(a.items, kStatItems));
+    hipLaunchKernelGGL(kvstar_stats_kernel<KS>, grid, dim3(kThreads), 0, st, a);
+    const int rc = ucm::launch_status("kvstar_stats_kernel");
+    if (rc != UCM_OK) return rc;
+    hipLaunchKernelGGL(kvstar_mass_kernel<KS>, dim3((unsigned)(a.groups < kMassGroups ? a.groups : kMassGroups)),
+                       dim3(kThreads), 0, st, a);
+    return ucm::launch_status("kvstar_mass_kernel");
 }
 
 }  // namespace
@@ -279,7 +469,11 @@ KvstarWs carve_kvstar(void* base, int64_t rows, int64_t S, int64_t n_blocks)
 extern "C" size_t ucm_kvstar_topk_workspace_bytes(int32_t X, int32_t Hq, int64_t n_blocks, int32_t M)
 {
     if (X <= 0 || Hq <= 0 || n_blocks <= 0 || M <= 0) return 256;
-    return carve_kvstar(nullptr, (int64_t)X * Hq, n_blocks * M, n_blocks).bytes;
+    if (n_blocks > INT32_MAX || n_blocks * M > INT32_MAX) return 256;  // refused by the call
+    KvArgs a{};
+    a.X = X; a.Hq = Hq; a.n_blocks = (int)n_blocks; a.M = M;
+    plan_chunks(a);
+    return carve_kvstar(a, nullptr);
 }
 
 extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t d_orig,
@@ -297,43 +491,29 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
                 "Dimension mismatch: No dPrunedIndex, but Q and K head dims differ.");
     UCM_REQUIRE(topk > 0, "topk %d must be positive", topk);
     if (topk > kMaxTopk) return ucm::fail(UCM_EUNSUPPORTED, "topk %d above %d", topk, kMaxTopk);
-    UCM_REQUIRE((size_t)kRowTile * d * 4 <= 64 * 1024, "head dim %d above 1024", d);
+    UCM_REQUIRE(d <= 1024, "head dim %d above 1024", d);
     UCM_REQUIRE(n_blocks <= INT32_MAX && n_blocks * M <= INT32_MAX, "too many block representatives");
-    const int64_t rows = (int64_t)X * Hq, S = n_blocks * M;
+    const int64_t rows = (int64_t)X * Hq;
     UCM_REQUIRE(rows <= 65535 && rows * M <= INT32_MAX, "too many query rows");
     UCM_REQUIRE(workspace && workspace_bytes >= ucm_kvstar_topk_workspace_bytes(X, Hq, n_blocks, M),
                 "workspace too small");
     UCM_REQUIRE((((uintptr_t)blk_repre | (uintptr_t)workspace) & 15) == 0, "block representatives must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    const KvstarWs w = carve_kvstar(workspace, rows, S, n_blocks);
-    QkArgs a{};
-    a.q = (const __half*)query; a.k = (const __half*)blk_repre; a.pruned = pruned_index;
-    a.X = X; a.Hq = Hq; a.Hkv = Hkv; a.g = Hq / Hkv; a.d_orig = d_orig; a.d = d; a.S = S;
-    a.scores = w.scores;
-    const dim3 grid((unsigned)ucm::ceil_div(S, kQkThreads), (unsigned)Hkv,
-                    (unsigned)ucm::ceil_div((int64_t)X * a.g, kRowTile));
-    UCM_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "too many heads or query rows");
-    int rc;
-    if (d % 16 == 0 && d <= 512) {
-        const dim3 mgrid((unsigned)ucm::ceil_div(S, 32 * (kQkThreads / 64)), (unsigned)Hkv,
-                         (unsigned)ucm::ceil_div((int64_t)X * a.g, 32));
-        UCM_REQUIRE(mgrid.z <= 65535, "too many query rows");
-        hipLaunchKernelGGL(qk_mfma_kernel, mgrid, dim3(kQkThreads), (size_t)32 * (d + 8) * 2, st, a);
-        rc = ucm::launch_status("qk_mfma_kernel");
-    } else {
-        hipLaunchKernelGGL(qk_score_kernel, grid, dim3(kQkThreads), (size_t)kRowTile * d * 4, st, a);
-        rc = ucm::launch_status("qk_score_kernel");
-    }
-    if (rc != UCM_OK) return rc;
-    hipLaunchKernelGGL(row_stats_kernel, dim3((unsigned)rows), dim3(kStatThreads), 0, st, w.scores, S, w.stats);
-    rc = ucm::launch_status("row_stats_kernel");
-    if (rc != UCM_OK) return rc;
-    hipLaunchKernelGGL(block_mass_kernel, dim3((unsigned)n_blocks), dim3(kStatThreads), 0, st, w.scores,
-                       w.stats, (int)rows, S, (int)M, w.keys);
-    rc = ucm::launch_status("block_mass_kernel");
+    KvArgs a{};
+    a.q = (const _Float16*)query; a.k = (const _Float16*)blk_repre; a.pruned = pruned_index;
+    a.X = X; a.Hq = Hq; a.Hkv = Hkv; a.g = Hq / Hkv; a.d_orig = d_orig; a.d = d;
+    a.n_blocks = (int)n_blocks; a.M = M;
+    a.tiles_q = (int)ucm::ceil_div((int64_t)X * a.g, 32);
+    a.items = Hkv * a.tiles_q;
+    plan_chunks(a);
+    carve_kvstar(a, workspace);
+    const int rc = d == 32 ? launch_kvstar<2>(a, st)
+                 : d == 64 ? launch_kvstar<4>(a, st)
+                 : d == kPackedDim ? launch_kvstar<8>(a, st)
+                                   : launch_kvstar<0>(a, st);
     if (rc != UCM_OK) return rc;
     SortArgs s{};
-    s.keys = w.keys; s.pitch = key_pitch(n_blocks); s.max_n = (int)n_blocks; s.topk = topk;
+    s.keys = a.keys; s.pitch = key_pitch(n_blocks); s.max_n = (int)n_blocks; s.topk = topk;
     s.out_idx = out_idx; s.out_score = out_score;
     return launch_topk(s, 1, st);
 }
