@@ -373,3 +373,53 @@ def test_unpack_hash_roundtrip():
     c = enc.compute_hash(x.to(torch.bfloat16).cuda())
     pm = enc._unpack_hash(c).cpu()
     assert pm[0, 3] == 1 and pm[1, 100] == 1 and pm.sum() == 2 - (256 - 2)
+
+
+@pytest.mark.parametrize("T,N,H,n_w,slots", [
+    (1281, 512, 1, 1, "i64"),    # 32-column slices, a last tile of one row
+    (2049, 512, 1, 1, "i32"),    # 64-column slices
+    (4097, 512, 1, 1, "i64"),    # 128-column slices, one tile per workgroup
+    (8321, 512, 1, 1, "paged"),  # the same, a second tile for some
+    (2300, 256, 2, 2, "paged"),  # a projection per head
+    (30000, 96, 1, 1, "i32"),    # column count only 32 divides, several tiles per workgroup
+    (30001, 192, 1, 1, "dense"), # ... only 64 divides
+    (3000, 320, 2, 1, "i64"),
+])
+def test_rows_of_512_values_at_the_edges_of_slices_and_tiles(T, N, H, n_w, slots):
+    """One instantiation per slice width; one or several row tiles per workgroup; rows that do not exist,
+    are skipped or hold NaN."""
+    rng = rng_for(T + N + H)
+    K, BS = 512, 64
+    x32 = rng.standard_normal((T, H, K)).astype(np.float32)
+    x32[T // 3] = 0.0
+    x32[T // 2, :, 5] = np.nan
+    x = torch.from_numpy(x32).to(torch.bfloat16)
+    W = torch.from_numpy(rng.standard_normal((n_w, K, N)).astype(np.float32)).to(torch.bfloat16)
+    enc = make_encoder(K, N, torch.bfloat16, W if n_w > 1 else W[0], n_w=n_w, hpw=1)
+    nb = -(-T // BS)
+    ids = rng.permutation(nb).astype(np.int32)
+    slot = ids[np.arange(T) // BS].astype(np.int64) * BS + np.arange(T) % BS
+    cache = torch.zeros((nb, BS, H, N // 32 + 1), dtype=torch.int32, device="cuda")  # rows of other codes between
+    view = cache[..., 1:]
+    if slots == "paged":
+        kv = torch.zeros((nb * BS, H, K), dtype=torch.bfloat16)
+        kv[torch.from_numpy(slot)] = x
+        enc.compute_hash_from_paged_cache(kv.view(nb, BS, H, K).cuda(), torch.from_numpy(ids).cuda(), T, view, block_size=BS)
+    elif slots == "dense":
+        got = enc.compute_hash(x.cuda(), per_head=True).cpu().numpy().reshape(T, H, N // 8)
+    else:
+        slot[7::11] = -1  # rows that are skipped
+        enc.compute_hash_and_cache(x.cuda(), torch.from_numpy(slot).to(torch.int64 if slots == "i64" else torch.int32).cuda(),
+                                   view, block_size=BS)
+    if slots != "dense":
+        flat = cache.cpu().numpy().reshape(nb * BS, H, N // 32 + 1)
+        assert not flat[:, :, 0].any()
+        unused = np.setdiff1d(np.arange(nb * BS), slot)
+        assert not flat[unused].any()
+        got = np.ascontiguousarray(flat[np.maximum(slot, 0)][:, :, 1:]).view(np.uint8)
+    keep = np.flatnonzero(slot >= 0)
+    nan = keep[keep == T // 2]
+    assert not got[nan].any() and not got[keep[keep == T // 3]].any()  # NaN > 0 and 0 > 0 are false
+    rows = keep[keep != T // 2]
+    for h in range(H):
+        assert_codes_match(got[rows, h], x[rows, h].float().numpy(), W[min(h, n_w - 1)].float().numpy())

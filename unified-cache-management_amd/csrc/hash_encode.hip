@@ -22,6 +22,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 
@@ -557,6 +558,135 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
             encode_rows(tile, slot_target(tile, sl));
         }
     }
+}
+
+// ---------------------------------------------------------------------------------------
+// Rows of 512 values (latent vectors), any row count above the latency path's.
+//
+// A workgroup keeps a slice of 32 NT hash columns of the projection in LDS (transposed) and walks
+// row tiles of 128: a wave owns 32 rows whose 32 operands it loads straight into registers.  All NT
+// column tiles advance together, so an operand register is free after its k-step and takes the next
+// row tile's value there: the rows of the next tile travel while this one is multiplied, without
+// registers of their own.
+//
+// What bounds it: for up to one row tile per workgroup the loads in front of the first matrix
+// instruction (128 KiB of rows and 32 NT KiB of projection through one compute unit's address unit;
+// 8192 rows x 512 bits: 10.3 us, of which 1.9 us are matrix instructions), then the matrix pipe at the
+// clock the power limit leaves (4 us a tile of 128 x 128).  The slices of a row tile are workgroups of one
+// XCD where the number of row streams is a multiple of 8, so its rows come from HBM once.  512 bits
+// before (133 KiB slices in front of four tiles a workgroup, rows through LDS) and now: 2048 rows 9.8
+// and 7.1 us, 4096 rows 15.4 and 7.7 us, 8192 rows 23.7 and 10.3 us, 32,768 rows 30.3 and 24.3 us.
+// ---------------------------------------------------------------------------------------
+constexpr int kSliceKS = 32;                    // 512 / 16 k-steps
+constexpr int kSlicePitch = kSliceKS * 16 + kPad;
+
+template <typename V, int NT>
+__global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 1 : 2, NT == 4 ? 1 : 2))) void encode_slice_kernel(EncArgs a)
+{
+    constexpr int K = kSliceKS * 16, KP = kSlicePitch;
+    extern __shared__ uint16_t wt[];  // [32 NT][KP], k contiguous
+    const int h = blockIdx.z;
+    const int n0 = blockIdx.y * NT * 32;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, kb = lane >> 5;
+    const int64_t tiles = (a.T + kRowsPerWg - 1) / kRowsPerWg;
+
+    auto token_of = [&](int64_t tile) {  // rows past T re-read the last one; they are not stored
+        const int64_t t = tile * kRowsPerWg + wave * kRowsPerWave + r;
+        return t < a.T ? t : a.T - 1;
+    };
+    auto row_ptr = [&](int64_t t) { return (const uint16_t*)a.x + src_offset(a, t, h) + kb * 8; };
+
+    // The slice in 8 x 8 patches, transposed in registers; its loads and those of the first rows go out
+    // together.  Two neighbouring lanes take 16 columns of one k-group and the next six lanes the three
+    // k-groups behind it: the eight 16-byte LDS writes of eight lanes then fall on different banks.
+    constexpr int kRounds = (K / 8) * (NT * 4) / kMfmaThreads;
+    const uint16_t* wsrc = (const uint16_t*)a.w + (int64_t)weight_index(a, h) * K * a.N + n0;
+    auto patch_of = [&](int it, int& kq, int& j) {
+        const int idx = it * kMfmaThreads + threadIdx.x;
+        j = (idx & 1) | ((idx >> 3) % (NT * 2)) << 1;
+        kq = ((idx >> 1) & 3) | ((idx >> 3) / (NT * 2)) << 2;
+    };
+    u32x4 row[kRounds][8];
+#pragma unroll
+    for (int it = 0; it < kRounds; ++it) {
+        int kq, j;
+        patch_of(it, kq, j);
+        const uint16_t* src = wsrc + (int64_t)(kq * 8) * a.N + 8 * j;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) row[it][i] = *reinterpret_cast<const u32x4*>(src + (int64_t)i * a.N);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    V av[kSliceKS];
+    int64_t tile = blockIdx.x;
+    {
+        const uint16_t* xr = row_ptr(token_of(tile));
+#pragma unroll
+        for (int ks = 0; ks < kSliceKS; ++ks) av[ks] = *reinterpret_cast<const V*>(xr + ks * 16);
+    }
+    RawSlot raw = fetch_slot_flat(a, token_of(tile));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int it = 0; it < kRounds; ++it) {
+        int kq, j;
+        patch_of(it, kq, j);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
+            u32x4 o;
+            o.x = __builtin_amdgcn_perm(row[it][1][c >> 1], row[it][0][c >> 1], sel);
+            o.y = __builtin_amdgcn_perm(row[it][3][c >> 1], row[it][2][c >> 1], sel);
+            o.z = __builtin_amdgcn_perm(row[it][5][c >> 1], row[it][4][c >> 1], sel);
+            o.w = __builtin_amdgcn_perm(row[it][7][c >> 1], row[it][6][c >> 1], sel);
+            *reinterpret_cast<u32x4*>(wt + (8 * j + c) * KP + kq * 8) = o;
+        }
+    }
+    __syncthreads();
+
+    const uint16_t* bp = wt + r * KP + kb * 8;
+    auto pass = [&](int64_t cur, int64_t next, auto more_) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_)::value;
+        const int64_t t = cur * kRowsPerWg + wave * kRowsPerWave + r;
+        uint32_t* dst = t < a.T && lane < 32 ? slot_dst(a, slot_value(a, raw, t), h) : nullptr;
+        const uint16_t* nx = MORE ? row_ptr(token_of(next)) : nullptr;
+        if constexpr (MORE) raw = fetch_slot_flat(a, token_of(next));
+        f32x16 acc[NT];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) acc[q] = acc_start();
+        V bv[2][NT];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) bv[0][q] = *reinterpret_cast<const V*>(bp + q * 32 * KP);
+#pragma unroll
+        for (int ks = 0; ks < kSliceKS; ++ks) {
+            if (ks + 1 < kSliceKS) {
+#pragma unroll
+                for (int q = 0; q < NT; ++q)
+                    bv[(ks + 1) & 1][q] = *reinterpret_cast<const V*>(bp + q * 32 * KP + (ks + 1) * 16);
+            }
+#pragma unroll
+            for (int q = 0; q < NT; ++q) acc[q] = Mfma<V>::run(bv[ks & 1][q], av[ks], acc[q]);
+            if constexpr (MORE) av[ks] = *reinterpret_cast<const V*>(nx + ks * 16);
+            __builtin_amdgcn_sched_barrier(0);  // loads hoisted out of their k-step cost more registers than there are
+        }
+        uint32_t words[NT];
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+            const uint32_t half = pack_half(acc[q]);
+            words[q] = join_halves(kb ? half << 4 : half);
+        }
+        if (dst) {
+            uint32_t* d = dst + n0 / 32;
+            if (NT == 4 && (((uintptr_t)d) & 15) == 0) {
+                *reinterpret_cast<u32x4*>(d) = u32x4{words[0], words[1 % NT], words[2 % NT], words[3 % NT]};
+            } else {
+#pragma unroll
+                for (int q = 0; q < NT; ++q) d[q] = words[q];
+            }
+        }
+    };
+    for (; tile + gridDim.x < tiles; tile += gridDim.x) pass(tile, tile + gridDim.x, std::true_type{});
+    pass(tile, tile, std::false_type{});
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1759,6 +1889,51 @@ int launch_mfma(EncArgs a, hipStream_t st)
     return ucm::fail(UCM_EUNSUPPORTED, "no LDS slice fits K=%d", K);
 }
 
+int stream_workgroups();
+
+template <typename V, int NT>
+int launch_slice_nt(const EncArgs& a, hipStream_t st)
+{
+    constexpr size_t lds = (size_t)NT * 32 * kSlicePitch * 2;
+    if (lds > 64 * 1024) {
+        static int opted = 0;  // 0 = not tried, 1 = allowed, -1 = refused by the runtime
+        if (opted == 0) {
+            const hipError_t e = hipFuncSetAttribute((const void*)encode_slice_kernel<V, NT>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) (void)hipGetLastError();
+            opted = (e == hipSuccess) ? 1 : -1;
+        }
+        if (opted < 0) return UCM_EUNSUPPORTED;
+    }
+    const int64_t tiles = ucm::ceil_div(a.T, kRowsPerWg);
+    const int64_t units = (int64_t)(a.N / (32 * NT)) * a.H;
+    int64_t streams = (int64_t)stream_workgroups() * (NT == 4 ? 1 : 2) / units;
+    if (streams < 1) streams = 1;
+    if (streams > tiles) streams = tiles;
+    hipLaunchKernelGGL((encode_slice_kernel<V, NT>), dim3((unsigned)streams, (unsigned)(a.N / (32 * NT)), (unsigned)a.H),
+                       dim3(kMfmaThreads), lds, st, a);
+    return ucm::launch_status("encode_slice_kernel");
+}
+
+template <typename V>
+int launch_slice(const EncArgs& a, hipStream_t st)
+{
+    // Narrow slices while they leave every compute unit at most one workgroup: the time in front of the
+    // first matrix instruction grows with the slice (1 to 256 workgroups: 32 columns 7 us, 64 columns
+    // 7.5 us, 128 columns 9.5 to 10.3 us; two workgroups of 64 columns on a compute unit 13 us).
+    const int nt = a.N / 32;
+    const int64_t tiles = ucm::ceil_div(a.T, kRowsPerWg) * a.H;
+    if (nt % 4 == 0 && tiles * (nt / 2) > stream_workgroups()) {
+        const int rc = launch_slice_nt<V, 4>(a, st);
+        if (rc != UCM_EUNSUPPORTED) return rc;  // no large-LDS opt-in: a narrower slice
+    }
+    if (nt % 2 == 0 && tiles * nt > stream_workgroups()) {
+        const int rc = launch_slice_nt<V, 2>(a, st);
+        if (rc != UCM_EUNSUPPORTED) return rc;
+    }
+    return launch_slice_nt<V, 1>(a, st);
+}
+
 template <typename V>
 int dispatch_mfma(const EncArgs& a, hipStream_t st)
 {
@@ -1766,7 +1941,7 @@ int dispatch_mfma(const EncArgs& a, hipStream_t st)
         case 64: return launch_mfma<V, 4>(a, st);
         case 128: return launch_mfma<V, 8>(a, st);
         case 256: return launch_mfma<V, 16>(a, st);
-        case 512: return launch_mfma<V, 32>(a, st);
+        case 512: return launch_slice<V>(a, st);
         default: return ucm::fail(UCM_ERROR, "internal: K %d has no MFMA kernel", a.K);
     }
 }
@@ -1792,12 +1967,10 @@ bool mfma_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 // the tiled kernel (65,536 rows: 14.8 against 12.4 us; 1M rows: 67.6 against 71.8 us; 4M rows: 225
 // against 262 us)
 constexpr int64_t kStreamMinRows = (int64_t)1 << 20;
-// the wide (K = 512) kernel pays for itself earlier: it replaces a tiled kernel that re-reads the
-// rows once per slice of the projection (256 bits: 16,384 rows 19 against 26 us, 262,144 rows 74
-// against 164 us; 512 bits: 32,768 rows 36 against 34 us, 65,536 rows 52 against 65 us, 262,144 rows
-// 155 against 301 us)
-constexpr int64_t kWideMinRows256 = (int64_t)1 << 14;
-constexpr int64_t kWideMinRows512 = (int64_t)1 << 16;
+// the wide (K = 512) kernel against the slice kernel: 256 bits: 65,536 rows 26.9 against 26.1 us, 131,072
+// rows 42.5 against 50.8 us; 512 bits: 65,536 rows 54 against 42 us, 131,072 rows 84 against 86 us
+constexpr int64_t kWideMinRows256 = (int64_t)3 << 15;
+constexpr int64_t kWideMinRows512 = (int64_t)1 << 17;
 // 0 = the defaults above; set per calling thread (a test hook must not move other threads' encodes)
 thread_local int64_t t_stream_min_rows = 0;
 thread_local unsigned long long* t_clock_probe = nullptr;  // see ucm_hash_encode_set_clock_probe()
@@ -2099,9 +2272,10 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
 // Which matrix-core kernel: the wave-per-tile kernel costs about 4 us plus 12.5 ps per wave and
 // k value (each wave gathers its own operand columns from L2); the LDS kernel has a floor of
 // about 6 us plus 0.13 us per KiB of projection slice that every workgroup stages before its
-// first tile (7 us at 64 x 64, 10 us at 128 x 128, 23-24 us for a 133 KiB slice), after which it
-// streams rows at HBM rate.  Measured crossovers this reproduces: 128 -> 128 bits with 8 heads at
-// ~4000 rows, 256 -> 256 with 4 heads and 512 -> 512 at ~5000-6000 rows, 64 -> 64 never below
+// first tile (7 us at 64 x 64, 10 us at 128 x 128), after which it streams rows at HBM rate.  Rows of
+// 512 values have the slice kernel: 7 us until it fills the chip.  Measured crossovers this
+// reproduces: 128 -> 128 bits with 8 heads at ~4000 rows, 256 -> 256 with 4 heads at ~5000-6000 rows,
+// 512 -> 512 at ~1100 rows (1000: 6.3 against 6.8 us, 1500: 8.3 against 7.0 us), 64 -> 64 never below
 // 16,384 rows.
 bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 {
@@ -2111,7 +2285,7 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype)
     const int bn = pick_slice(a.N, a.K, (size_t)160 * 1024 - kStage);
     if (bn == 0) return true;
     const double slice_kib = (double)bn * (a.K + kPad) * 2 / 1024.0;
-    const double lds_floor_us = 6.0 + 0.13 * slice_kib;
+    const double lds_floor_us = a.K == 16 * kSliceKS ? 7.5 : 6.0 + 0.13 * slice_kib;
     const double small_us = 4.0 + (double)small_waves(a) * a.K * 12.5e-6;
     return small_us < lds_floor_us;
 }
