@@ -21,6 +21,8 @@ OBJ_DIR = os.path.join(HERE, "build")
 LIB = os.path.join(LIB_DIR, "libucm_hip.so")
 TORCH_OPS_SRC = os.path.join(HERE, "csrc", "torch_ops.cpp")
 TORCH_OPS_LIB = os.path.join(LIB_DIR, "libucm_torch_ops.so")
+NATIVE_SRC = os.path.join(HERE, "csrc", "native_calls.cpp")
+NATIVE_LIB = os.path.join(LIB_DIR, "ucm_native.so")
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -70,12 +72,25 @@ def build(verbose=True, only_changed=False):
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB], verbose)
     if not only_changed or _stale(TORCH_OPS_SRC, TORCH_OPS_LIB):
         build_torch_ops(verbose)
+    if not only_changed or _stale(NATIVE_SRC, NATIVE_LIB):
+        build_native(verbose)
     return LIB
 
 
 def build_torch_ops(verbose=True):
-    """libucm_torch_ops.so: the TORCH_LIBRARY registration (torch.ops.ucm_amd.*) over the C ABI.  Host
-    code only (g++), linked against libucm_hip.so and the installed PyTorch."""
+    """libucm_torch_ops.so: the TORCH_LIBRARY registration (torch.ops.ucm_amd.*) over the C ABI."""
+    return _build_host(TORCH_OPS_SRC, TORCH_OPS_LIB, [], verbose)
+
+
+def build_native(verbose=True):
+    """ucm_native.so: the Python module with the per-step calls' native fronts."""
+    import sysconfig
+
+    return _build_host(NATIVE_SRC, NATIVE_LIB, ["-I" + sysconfig.get_paths()["include"], "-ltorch_python"], verbose)
+
+
+def _build_host(src, lib, extra, verbose):
+    """Host code only (g++), linked against libucm_hip.so and the installed PyTorch."""
     import torch
     from torch.utils import cpp_extension as ce
 
@@ -84,10 +99,10 @@ def build_torch_ops(verbose=True):
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
            "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(HERE, "csrc")]
     cmd += ["-I" + p for p in ce.include_paths()] + ["-I/opt/rocm/include", "-w"]
-    cmd += [TORCH_OPS_SRC, "-o", TORCH_OPS_LIB, "-L" + LIB_DIR, "-lucm_hip", "-L" + tlib, "-ltorch", "-ltorch_cpu",
-            "-lc10", "-lc10_hip", "-ltorch_hip", "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + tlib]
+    cmd += [src, "-o", lib, "-L" + LIB_DIR, "-lucm_hip", "-L" + tlib, "-ltorch", "-ltorch_cpu",
+            "-lc10", "-lc10_hip", "-ltorch_hip"] + extra + ["-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + tlib]
     _run(cmd, verbose)
-    return TORCH_OPS_LIB
+    return lib
 
 
 if __name__ == "__main__":

@@ -4,6 +4,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "lib", "libucm_hip.so")
+NATIVE_PATH = os.path.join(os.path.dirname(LIB_PATH), "ucm_native.so")
 
 UCM_OK = 0
 UCM_ERROR = -1
@@ -19,6 +20,7 @@ TOPK_REDUCE_HEADS, TOPK_RETURN_PHYSICAL, TOPK_SCORE_ORDER, TOPK_DISTANCE = 1, 2,
 TRANS_CE, TRANS_SM = 0, 1
 
 _lib = None
+_native = None
 
 i32, i64, u32, u64 = C.c_int32, C.c_int64, C.c_uint32, C.c_uint64
 vp, sz, ci = C.c_void_p, C.c_size_t, C.c_int
@@ -152,6 +154,24 @@ def lib():
             fn.argtypes = args
         _lib = l
     return _lib
+
+
+def native():
+    """The module of native fronts (csrc/native_calls.cpp): a front takes the plain case of a call and
+    returns None for any other, which is the caller's general path's."""
+    global _native
+    if _native is None:
+        import importlib.machinery
+        import importlib.util
+
+        lib()  # libucm_hip.so and torch first: the module binds to what is loaded
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"{NATIVE_PATH} is missing: run unified-cache-management_amd/build.py")
+        loader = importlib.machinery.ExtensionFileLoader("ucm_native", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("ucm_native", loader))
+        loader.exec_module(mod)
+        _native = mod
+    return _native
 
 
 def last_dispatch():

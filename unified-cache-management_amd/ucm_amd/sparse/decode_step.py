@@ -78,8 +78,14 @@ class SparseDecodeStep:
         """new_keys [T,Hkv,K] + slot_mapping [T] (T may be 0), queries [B,Hq,K],
         k_hash_cache int32 [NB,BS,Hkv,N/32], block_table int32 [B,max_blocks], seq_lens int32 [B].
         Returns (indices, scores) int32 [B, Hkv or 1, k]: views of buffers reused by every call."""
-        args = self._arguments(new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens)
-        _lib.check(_lib.lib().ucm_sparse_decode_step(*args, _lib.stream_ptr(queries.device)))
+        rc = _lib.native().sparse_step(
+            self.w, self.q_codes, self.out_idx, self.out_score, self.workspace, self.Hq, self.Hkv, self.B, self.K,
+            self.N, self.max_blocks, self.BS, self.k, self.sink, self.recent, self.flags,
+            new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens)
+        if rc is None:
+            args = self._arguments(new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens)
+            rc = _lib.lib().ucm_sparse_decode_step(*args, _lib.stream_ptr(queries.device))
+        _lib.check(rc)
         return self.out_idx, self.out_score
 
     def bind(self, new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens):
@@ -240,8 +246,14 @@ class GSADecodeStep:
 
     def step(self, new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens):
         """Returns (new_block_table [B, width], new_seq_lens [B]): buffers reused by every call."""
-        args = self._arguments(new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens)
-        _lib.check(_lib.lib().ucm_gsa_decode_step(*args, _lib.stream_ptr(queries.device)))
+        rc = _lib.native().gsa_step(
+            self.w, self.q_codes, self.new_table, self.new_lens, self.workspace, self.Hq, self.Hkv, self.B, self.K,
+            self.N, self.width, self.BS, self.topk, self.sink, self.recent, self.threshold,
+            new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens)
+        if rc is None:
+            args = self._arguments(new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens)
+            rc = _lib.lib().ucm_gsa_decode_step(*args, _lib.stream_ptr(queries.device))
+        _lib.check(rc)
         return self.new_table, self.new_lens
 
     def bind(self, new_keys, slot_mapping, queries, k_hash_cache, block_table, seq_lens):
@@ -300,6 +312,13 @@ class GSADecodeStepMLA:
         [B,Hq,K_nope], q_rope [B,Hq,K_rope] (all Hq heads: the reduction happens inside);
         k_hash_cache int32 [NB,BS,Wd]; block_table int32 [B,width]; seq_lens int32 [B].
         Returns (new_block_table [B, width], new_seq_lens [B]): buffers reused by every call."""
+        rc = _lib.native().gsa_step_mla(
+            self.wn, self.wr, self.q_codes, self.new_table, self.new_lens, self.workspace, self.Hq, self.R, self.B,
+            self.width, self.BS, self.topk, self.sink, self.recent, self.threshold,
+            new_nope, new_rope, slot_mapping, q_nope, q_rope, k_hash_cache, block_table, seq_lens)
+        if rc is not None:
+            _lib.check(rc)
+            return self.new_table, self.new_lens
         dt = self.wn.dtype
         T = 0 if new_nope is None else int(new_nope.shape[0])
         for t in (q_nope, q_rope) + ((new_nope, new_rope) if T else ()):

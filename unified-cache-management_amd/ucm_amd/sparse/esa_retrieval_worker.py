@@ -18,6 +18,11 @@ from .. import _lib
 def dot_topk(data, query, indexes, topk, workspace=None):
     """data fp32 [n, dim], query fp32 [B, dim], indexes int32 [B, max_n] (all on one GPU) ->
     (indices int32 [B, topk], scores fp32 [B, topk]) on torch's current stream."""
+    out = _lib.native().dot_topk(data, query, indexes, topk, workspace)
+    if out is not None:
+        if type(out) is int:
+            _lib.check(out)
+        return out
     if data.dtype != torch.float32 or query.dtype != torch.float32 or indexes.dtype != torch.int32:
         raise ValueError("data and query must be float32, indexes int32")
     if data.device.type != "cuda" or query.device != data.device or indexes.device != data.device:

@@ -151,6 +151,11 @@ class HashEncoder:
         """Encode x [T,H,K] and store each code at k_hash_cache[slot // BS, slot % BS, h, :].
         Slots < 0 or >= NB*BS are skipped.  Returns k_hash_cache.  Tile-size keyword arguments
         of the reference's Triton launcher are accepted and ignored."""
+        rc = _lib.native().encode_cache(self._w, self.hash_weights, self.heads_per_weight if self.num_weights > 1 else 0,
+                                        block_size, x, slot_mapping, k_hash_cache) if self.hash_bits % 32 == 0 else None
+        if rc is not None:
+            _lib.check(rc)
+            return k_hash_cache
         if x.ndim != 3:
             raise ValueError(f"x must be [T,H,K], got {x.shape}")
         if slot_mapping.ndim != 1:
@@ -203,6 +208,12 @@ class HashEncoder:
         (`kv_cache[0][0][prefix_block_ids]`, reshape, compute_hash_and_cache with the prefix
         slot mapping, gsa_on_device.py:574-588); slot(i) = block_ids[i // BS] * BS + i % BS
         as in rebuild_prefix_cache_info_for_req (:1142-1174).  Returns k_hash_cache."""
+        rc = _lib.native().encode_paged(self._w, self.hash_weights, self.heads_per_weight if self.num_weights > 1 else 0,
+                                        block_size, k_cache, block_ids, num_tokens,
+                                        k_hash_cache) if self.hash_bits % 32 == 0 else None
+        if rc is not None:
+            _lib.check(rc)
+            return k_hash_cache
         if k_cache.ndim != 4:
             raise ValueError(f"k_cache must be [NB,BS,H,K], got {k_cache.shape}")
         if k_hash_cache.ndim != 4:

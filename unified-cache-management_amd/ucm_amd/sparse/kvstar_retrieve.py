@@ -54,6 +54,11 @@ def kvstar_topk(query_group, blk_repre, pruned_index, topk, workspace=None):
     """query_group fp16 [x, Hq, d_orig], blk_repre fp16 [n, M, Hkv, d], pruned_index int64
     [Hkv, d] or None, all on one GPU -> (block numbers int32 [min(topk, n)], scores fp32) on
     torch's current stream."""
+    out = _lib.native().kvstar_topk(query_group, blk_repre, pruned_index, topk, workspace)
+    if out is not None:
+        if type(out) is int:
+            _lib.check(out)
+        return out
     if query_group.dtype != torch.float16 or blk_repre.dtype != torch.float16:
         raise ValueError("query_group and blk_repre must be float16")
     if query_group.device.type != "cuda" or blk_repre.device != query_group.device:
