@@ -423,3 +423,43 @@ def test_rows_of_512_values_at_the_edges_of_slices_and_tiles(T, N, H, n_w, slots
     rows = keep[keep != T // 2]
     for h in range(H):
         assert_codes_match(got[rows, h], x[rows, h].float().numpy(), W[min(h, n_w - 1)].float().numpy())
+
+
+@pytest.mark.parametrize("K,N,H,T,paged", [
+    (128, 128, 8, 1025, True),    # one row tile per workgroup, the last with one row
+    (128, 128, 2, 6001, False),
+    (64, 64, 8, 1500, True),
+    (64, 128, 4, 12300, False),   # just past three workgroups a compute unit: four tiles each
+    (128, 128, 8, 12500, True),
+    (128, 256, 1, 98400, False),
+    (128, 128, 8, 65700, True),   # eight tiles each
+    (64, 64, 8, 10300, False),    # the streaming kernel's first sizes at 64 x 64
+])
+def test_row_tiles_per_workgroup(K, N, H, T, paged):
+    """One instantiation per number of row tiles a workgroup encodes, at the edges of their ranges; a sample
+    of rows (the first, the last, every tile position) against the oracle."""
+    rng = rng_for(T + N)
+    BS, nb = 64, -(-T // 64)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(nb * BS, H, K, generator=g, device="cuda").to(torch.bfloat16)
+    W = torch.from_numpy(rng.standard_normal((K, N)).astype(np.float32)).to(torch.bfloat16)
+    enc = make_encoder(K, N, torch.bfloat16, W)
+    ids = torch.from_numpy(rng.permutation(nb).astype(np.int32)).cuda()
+    cache = torch.zeros((nb, BS, H, N // 32), dtype=torch.int32, device="cuda")
+    t = torch.arange(T, device="cuda")
+    slot = ids[t // BS].long() * BS + t % BS
+    if paged:
+        enc.compute_hash_from_paged_cache(x.view(nb, BS, H, K), ids, T, cache, block_size=BS)
+        x = x[slot]
+    else:
+        enc.compute_hash_and_cache(x[:T], slot, cache, block_size=BS)
+    flat = cache.view(nb * BS, H, N // 32)
+    rest = torch.ones(nb * BS, dtype=torch.bool, device="cuda")
+    rest[slot] = False
+    assert not flat[rest].any()
+    rows = np.unique(np.concatenate([np.arange(130), T - 1 - np.arange(130), rng.integers(0, T, 1500)]))
+    pick = torch.from_numpy(rows).cuda()
+    got = flat[slot[pick]].cpu().numpy().view(np.uint8)
+    xs = x[pick].float().cpu().numpy()
+    for h in range(H):
+        assert_codes_match(got[:, h], xs[:, h], W.float().numpy())

@@ -33,7 +33,6 @@ constexpr int kRowsPerWave = 32;
 constexpr int kMfmaThreads = 256;                                // encode_mfma_kernel workgroup
 constexpr int kMfmaWaves = kMfmaThreads / 64;
 constexpr int kRowsPerWg = kMfmaWaves * kRowsPerWave;            // 128 rows per workgroup tile
-constexpr int kTilesPerWg = 4;                                   // row tiles a workgroup encodes
 constexpr int kStageBytes = kRowsPerWave * 128;                  // per wave: one 128-byte line of 32 rows
 constexpr int kPad = 8;  // elements of padding per LDS row (16 bytes)
 
@@ -284,13 +283,13 @@ struct Mfma<f16x8> {
 // handled per group (divides the slice's tile count; 4 gives one 16-byte store per row).  NG:
 // groups per slice when known at compile time (the group loop is then unrolled, which keeps
 // the compiler from draining all outstanding loads in front of it), 0 = run-time count.
-// grid = (groups of kTilesPerWg row tiles, column slices, heads); a workgroup stages its W slice
+// grid = (groups of TPW row tiles, column slices, heads); a workgroup stages its W slice
 // in LDS once and then encodes its run of row tiles (128 rows each, 32 per wave).  Two waves
 // per SIMD: the register budget holds two row tiles in flight per wave next to the one being
 // computed.  The pipelined path is straight-line code with the same loads on every path, so
 // that the compiler can count outstanding loads exactly and never waits for a prefetch it has
 // just issued.
-template <typename V, int KS, int NQ, int NG>
+template <typename V, int KS, int NQ, int NG, int TPW>
 __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2, 3))) void encode_mfma_kernel(EncArgs a)
 {
     extern __shared__ uint16_t wt[];  // [BN][K + kPad], k contiguous; then the waves' staging
@@ -306,7 +305,7 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
     const int r = lane & 31, kb = lane >> 5;
     const uint16_t* xbase = (const uint16_t*)a.x + (int64_t)h * a.x_stride_h;
     const int64_t tiles = (a.T + kRowsPerWg - 1) / kRowsPerWg;
-    const int64_t first = (int64_t)blockIdx.x * kTilesPerWg;  // this workgroup's run of tiles
+    const int64_t first = (int64_t)blockIdx.x * TPW;  // this workgroup's run of tiles
 
     // Rows are fetched one 128-byte line at a time: a load instruction covers 8 rows x 128
     // contiguous bytes (lane l: row 8j + l/8, 16-byte chunk l%8), so every cache line is touched
@@ -430,11 +429,11 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
     };
     constexpr bool kPipelined = kPrefetch && NG > 0;
     // paged input: the block ids of the wave's rows in each of the workgroup's tiles, up front
-    int sblk[kTilesPerWg] = {0, 0, 0, 0};
+    int sblk[TPW] = {0};
     if constexpr (kPipelined) {
         if (a.src_blocks) {
 #pragma unroll
-            for (int i = 0; i < kTilesPerWg; ++i)
+            for (int i = 0; i < TPW; ++i)
                 sblk[i] = wave_block(first + i < tiles ? first + i : tiles - 1);
         }
     }
@@ -450,7 +449,7 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
             patch_load(idx, row);
             if (it == 0) {
                 load_tile(first, sblk[0], raw0, first < tiles);
-                load_tile(first + 1, sblk[1], raw1, first + 1 < tiles);
+                if constexpr (TPW > 1) load_tile(first + 1, sblk[1 % TPW], raw1, first + 1 < tiles);
             }
             patch_store(idx, row);
         }
@@ -534,25 +533,26 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
         RawSlot slot0 = tile_slot(first < tiles ? first : tiles - 1);
         RawSlot slot1 = tile_slot(first + 1 < tiles ? first + 1 : tiles - 1);
 #pragma unroll
-        for (int i = 0; i < kTilesPerWg; i += 2) {
+        for (int i = 0; i < TPW; i += 2) {
             const int64_t t0 = first + i, t1 = first + i + 1;
             to_operands(raw0, av);
             uint32_t* dst = t0 < tiles ? slot_target(t0, slot0) : nullptr;
-            if (i + 2 < kTilesPerWg) {
+            if (i + 2 < TPW) {
                 slot0 = tile_slot(t0 + 2 < tiles ? t0 + 2 : tiles - 1);
-                load_tile(t0 + 2, sblk[(i + 2) % kTilesPerWg], raw0, t0 + 2 < tiles);
+                load_tile(t0 + 2, sblk[(i + 2) % TPW], raw0, t0 + 2 < tiles);
             }
             encode_rows(t0, dst);
+            if (i + 1 >= TPW) break;
             to_operands(raw1, av);
             dst = t1 < tiles ? slot_target(t1, slot1) : nullptr;
-            if (i + 3 < kTilesPerWg) {
+            if (i + 3 < TPW) {
                 slot1 = tile_slot(t1 + 2 < tiles ? t1 + 2 : tiles - 1);
-                load_tile(t1 + 2, sblk[(i + 3) % kTilesPerWg], raw1, t1 + 2 < tiles);
+                load_tile(t1 + 2, sblk[(i + 3) % TPW], raw1, t1 + 2 < tiles);
             }
             encode_rows(t1, dst);
         }
     } else {
-        for (int64_t tile = first; tile < first + kTilesPerWg && tile < tiles; ++tile) {
+        for (int64_t tile = first; tile < first + TPW && tile < tiles; ++tile) {
             const RawSlot sl = tile_slot(tile);
             load_operands(tile, av);
             encode_rows(tile, slot_target(tile, sl));
@@ -1844,23 +1844,44 @@ int pick_slice(int N, int K, size_t cap)
     return 0;
 }
 
-template <typename V, int KS, int NQ, int NG>
-int launch_mfma_q(const EncArgs& a, size_t lds, const dim3& grid, hipStream_t st)
+int stream_workgroups();
+
+template <typename V, int KS, int NQ, int NG, int TPW>
+int launch_mfma_t(const EncArgs& a, size_t lds, const dim3& grid, hipStream_t st)
 {
     // 0 = not tried, 1 = large LDS allocations allowed, -1 = refused by the runtime
     static int big_lds = 0;
     if (lds > 64 * 1024) {
         if (big_lds == 0) {
             const hipError_t e =
-                hipFuncSetAttribute((const void*)encode_mfma_kernel<V, KS, NQ, NG>,
+                hipFuncSetAttribute((const void*)encode_mfma_kernel<V, KS, NQ, NG, TPW>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) (void)hipGetLastError();
             big_lds = (e == hipSuccess) ? 1 : -1;
         }
         if (big_lds < 0) return UCM_EUNSUPPORTED;
     }
-    hipLaunchKernelGGL((encode_mfma_kernel<V, KS, NQ, NG>), grid, dim3(kMfmaThreads), lds, st, a);
+    hipLaunchKernelGGL((encode_mfma_kernel<V, KS, NQ, NG, TPW>), grid, dim3(kMfmaThreads), lds, st, a);
     return ucm::launch_status("encode_mfma_kernel");
+}
+
+template <typename V, int KS, int NQ, int NG>
+int launch_mfma_q(const EncArgs& a, size_t lds, hipStream_t st)
+{
+    const int64_t tiles = ucm::ceil_div(a.T, kRowsPerWg);
+    const int64_t all = tiles * (a.N / a.BN) * a.H;
+    auto grid = [&](int tpw) { return dim3((unsigned)ucm::ceil_div(tiles, tpw), (unsigned)(a.N / a.BN), (unsigned)a.H); };
+    if constexpr (KS <= 8 && NG > 0) {
+        // Row tiles per workgroup.  One while that leaves no more than three workgroups to a compute
+        // unit: a run of four on a part of the chip costs four tiles' time (128 -> 128 bits, 8 heads,
+        // runs of one against four: 2048 tokens 4.8 and 9.6 us, 8192: 7.5 and 10.1, 12,000: 10.2 and
+        // 11.2, 16,384: 12.6 and 12.1).  Eight once those fill the chip twice over: half the projection
+        // slices staged (65,536 tokens 31.9 against 35.6 us, 32,768: 19.6 against 19.3).
+        const int64_t cus = stream_workgroups();
+        if (all <= 3 * cus) return launch_mfma_t<V, KS, NQ, NG, 1>(a, lds, grid(1), st);
+        if (all >= 16 * cus) return launch_mfma_t<V, KS, NQ, NG, 8>(a, lds, grid(8), st);
+    }
+    return launch_mfma_t<V, KS, NQ, NG, 4>(a, lds, grid(4), st);
 }
 
 template <typename V, int KS>
@@ -1872,24 +1893,19 @@ int launch_mfma(EncArgs a, hipStream_t st)
         a.BN = pick_slice(a.N, K, cap - kStage);
         if (a.BN == 0) return ucm::fail(UCM_EUNSUPPORTED, "no LDS slice fits K=%d", K);
         const size_t lds = (size_t)a.BN * (K + kPad) * 2 + kStage;
-        const int64_t tiles = (a.T + kRowsPerWg - 1) / kRowsPerWg;
-        const int slices = a.N / a.BN;
-        const dim3 grid((unsigned)ucm::ceil_div(tiles, kTilesPerWg), (unsigned)slices, (unsigned)a.H);
         const int nt = a.BN / 32;
-        const int rc = nt == 4       ? launch_mfma_q<V, KS, 4, 1>(a, lds, grid, st)
-                       : nt == 8     ? launch_mfma_q<V, KS, 4, 2>(a, lds, grid, st)
-                       : nt % 4 == 0 ? launch_mfma_q<V, KS, 4, 0>(a, lds, grid, st)
-                       : nt == 2     ? launch_mfma_q<V, KS, 2, 1>(a, lds, grid, st)
-                       : nt == 1     ? launch_mfma_q<V, KS, 1, 1>(a, lds, grid, st)
-                       : nt % 2 == 0 ? launch_mfma_q<V, KS, 2, 0>(a, lds, grid, st)
-                                     : launch_mfma_q<V, KS, 1, 0>(a, lds, grid, st);
+        const int rc = nt == 4       ? launch_mfma_q<V, KS, 4, 1>(a, lds, st)
+                       : nt == 8     ? launch_mfma_q<V, KS, 4, 2>(a, lds, st)
+                       : nt % 4 == 0 ? launch_mfma_q<V, KS, 4, 0>(a, lds, st)
+                       : nt == 2     ? launch_mfma_q<V, KS, 2, 1>(a, lds, st)
+                       : nt == 1     ? launch_mfma_q<V, KS, 1, 1>(a, lds, st)
+                       : nt % 2 == 0 ? launch_mfma_q<V, KS, 2, 0>(a, lds, st)
+                                     : launch_mfma_q<V, KS, 1, 0>(a, lds, st);
         // a refused large-LDS opt-in falls back to the slice that fits the default 64 KiB
         if (rc != UCM_EUNSUPPORTED || lds <= 64 * 1024) return rc;
     }
     return ucm::fail(UCM_EUNSUPPORTED, "no LDS slice fits K=%d", K);
 }
-
-int stream_workgroups();
 
 template <typename V, int NT>
 int launch_slice_nt(const EncArgs& a, hipStream_t st)
@@ -1962,11 +1978,13 @@ bool mfma_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 }
 
 // ---- streaming kernel: eligibility and launch ----
-// rows x heads from which the streaming kernel is used: below about a million rows its fixed
-// cost (every wave stages a projection matrix of its own, 256 persistent workgroups) loses against
-// the tiled kernel (65,536 rows: 14.8 against 12.4 us; 1M rows: 67.6 against 71.8 us; 4M rows: 225
-// against 262 us)
-constexpr int64_t kStreamMinRows = (int64_t)1 << 20;
+// rows x heads from which the streaming kernel is used: below, its fixed cost (every wave stages a
+// projection matrix of its own, 256 persistent workgroups) loses against the tiled kernel.  128 -> 128
+// bits, 8 heads: 524,288 rows 32.7 against 30.5 us, 800,000 rows 46.4 against 53.2; one head: 500,000 rows
+// 34.3 against 33.1; 64 -> 128: 524,288 rows 21.3 against 20.1 us, 800,000 rows 28.7 against 35.8.  64 -> 64
+// bits, an eighth of the projection: 65,536 rows 5.8 against 5.6 us, 96,000 rows 6.4 against 7.1,
+// 262,144 rows 9.6 against 11.0, 524,288 rows 15.1 against 16.7.
+int64_t stream_min_rows(const EncArgs& a) { return a.K == 64 && a.N == 64 ? (int64_t)5 << 14 : (int64_t)3 << 18; }
 // the wide (K = 512) kernel against the slice kernel: 256 bits: 65,536 rows 26.9 against 26.1 us, 131,072
 // rows 42.5 against 50.8 us; 512 bits: 65,536 rows 54 against 42 us, 131,072 rows 84 against 86 us
 constexpr int64_t kWideMinRows256 = (int64_t)3 << 15;
@@ -1994,7 +2012,7 @@ bool stream_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 {
     if (!mfma_eligible(a, x_dtype, w_dtype) || a.src_blocks) return false;
     if (!((a.K == 128 && (a.N == 128 || a.N == 64)) || (a.K == 64 && (a.N == 128 || a.N == 64)))) return false;
-    if (a.T * a.H < (t_stream_min_rows > 0 ? t_stream_min_rows : kStreamMinRows)) return false;
+    if (a.T * a.H < (t_stream_min_rows > 0 ? t_stream_min_rows : stream_min_rows(a))) return false;
     if (a.slot && ((uintptr_t)a.slot & 3)) return false;
     // one shift per slot, one 16-byte store per four-word code (set_block_shift() has run)
     if (a.bs_shift < 0) return false;
@@ -2270,13 +2288,14 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
 }
 
 // Which matrix-core kernel: the wave-per-tile kernel costs about 4 us plus 12.5 ps per wave and
-// k value (each wave gathers its own operand columns from L2); the LDS kernel has a floor of
-// about 6 us plus 0.13 us per KiB of projection slice that every workgroup stages before its
-// first tile (7 us at 64 x 64, 10 us at 128 x 128), after which it streams rows at HBM rate.  Rows of
-// 512 values have the slice kernel: 7 us until it fills the chip.  Measured crossovers this
-// reproduces: 128 -> 128 bits with 8 heads at ~4000 rows, 256 -> 256 with 4 heads at ~5000-6000 rows,
-// 512 -> 512 at ~1100 rows (1000: 6.3 against 6.8 us, 1500: 8.3 against 7.0 us), 64 -> 64 never below
-// 16,384 rows.
+// k value (each wave gathers its own operand columns from L2); the LDS kernel with one row tile per
+// workgroup has a floor of about 4.2 us plus 0.027 us per KiB of projection slice that a workgroup stages
+// first (64 x 64: 4.4 us, 128 x 128: 5.1 us).  Measured: 128 -> 128 bits, 8 heads, 300 tokens 4.2 against
+// 4.7 us, 1024 tokens 5.6 against 4.6, 2048 tokens 7.3 against 4.8; one head, 4096 tokens 4.1 against 4.5,
+// 8192 tokens 5.2 against 4.6; 64 -> 64 bits, 8 heads, 600 tokens 3.6 against 3.9, 2048 tokens 4.7 against
+// 4.0.  Rows of 256 values are not pipelined and run four tiles a workgroup: 6 us plus 0.13 us per KiB
+// (256 -> 256 with 4 heads: equal at ~5000-6000 rows).  Rows of 512 values have the slice kernel: 7 us until
+// it fills the chip (512 -> 512: equal at ~1100 rows; 1000: 6.3 against 6.8 us, 1500: 8.3 against 7.0 us).
 bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 {
     if (!mfma_eligible(a, x_dtype, w_dtype) || small_waves(a) > 0x7fffffff) return false;
@@ -2285,7 +2304,7 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype)
     const int bn = pick_slice(a.N, a.K, (size_t)160 * 1024 - kStage);
     if (bn == 0) return true;
     const double slice_kib = (double)bn * (a.K + kPad) * 2 / 1024.0;
-    const double lds_floor_us = a.K == 16 * kSliceKS ? 7.5 : 6.0 + 0.13 * slice_kib;
+    const double lds_floor_us = a.K == 16 * kSliceKS ? 7.5 : a.K <= 128 ? 4.2 + 0.027 * slice_kib : 6.0 + 0.13 * slice_kib;
     const double small_us = 4.0 + (double)small_waves(a) * a.K * 12.5e-6;
     return small_us < lds_floor_us;
 }
