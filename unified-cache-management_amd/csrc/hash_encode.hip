@@ -2296,7 +2296,11 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
 // 4.0.  Rows of 256 values are not pipelined and run four tiles a workgroup: 6 us plus 0.13 us per KiB
 // (256 -> 256 with 4 heads: equal at ~5000-6000 rows).  Rows of 512 values have the slice kernel: 7 us until
 // it fills the chip (512 -> 512: equal at ~1100 rows; 1000: 6.3 against 6.8 us, 1500: 8.3 against 7.0 us).
-bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype)
+//
+// alone = false: a job of a decode step, where the other kernels are a launch more for every job (new keys
+// and queries of one or two projections share one here) and a group's mean is this kernel's anyway: it
+// stays with it up to 10 us (K = 128) and 23 us (K = 512) of its own.
+bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype, bool alone = true)
 {
     if (!mfma_eligible(a, x_dtype, w_dtype) || small_waves(a) > 0x7fffffff) return false;
     if (a.T <= kSmallRows && a.K <= 256) return true;
@@ -2304,7 +2308,7 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype)
     const int bn = pick_slice(a.N, a.K, (size_t)160 * 1024 - kStage);
     if (bn == 0) return true;
     const double slice_kib = (double)bn * (a.K + kPad) * 2 / 1024.0;
-    const double lds_floor_us = a.K == 16 * kSliceKS ? 7.5 : a.K <= 128 ? 4.2 + 0.027 * slice_kib : 6.0 + 0.13 * slice_kib;
+    const double lds_floor_us = !alone ? 6.0 + 0.13 * slice_kib : a.K == 16 * kSliceKS ? 7.5 : a.K <= 128 ? 4.2 + 0.027 * slice_kib : 6.0 + 0.13 * slice_kib;
     const double small_us = 4.0 + (double)small_waves(a) * a.K * 12.5e-6;
     return small_us < lds_floor_us;
 }
@@ -2594,8 +2598,8 @@ int build_pair(const PairSpec& p, EncArgs& kk, EncArgs& kq, bool& has_keys)
 
 bool pair_is_small(const PairSpec& p, const EncArgs& kk, const EncArgs& kq, bool has_keys)
 {
-    return has_keys && p.B > 0 && small_eligible(kk, p.x_dtype, p.w_dtype) &&
-           small_eligible(kq, p.x_dtype, p.w_dtype);
+    return has_keys && p.B > 0 && small_eligible(kk, p.x_dtype, p.w_dtype, false) &&
+           small_eligible(kq, p.x_dtype, p.w_dtype, false);
 }
 
 // The queries alone through the small-row kernel (the only one that averages query groups).
