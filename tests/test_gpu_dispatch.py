@@ -231,3 +231,24 @@ def test_latent_scorer_clock_probe(Wd, G):
         assert L.ucm_hamming_topk_set_clock_probe(probe.data_ptr() + 4) == _lib.UCM_EPARAM
     finally:
         _lib.check(L.ucm_hamming_topk_set_clock_probe(None))
+
+
+@pytest.mark.parametrize("Wd,G", [(18, 16), (8, 16)])
+@pytest.mark.parametrize("B,blocks", [(1, 4096), (1, 4097), (5, 1640), (9, 1400)])
+def test_latent_scorer_blocks_per_wave(Wd, G, B, blocks):
+    """A wave of the latent scorers takes one to four blocks by the launch's size: the edges of those ranges,
+    requests that end inside a wave's blocks, inside a workgroup's and before its first, both modes."""
+    from ucm_amd import _lib
+    from ucm_amd.sparse import hamming_score, hamming_topk
+
+    lens = [64 * blocks - 5] + [(64 * blocks * i) // B + 1 for i in range(1, B)]
+    q, kc, table, lens = make_paged_case(31 + blocks + Wd, B, G, 1, Wd, 64, lens)
+    k = 40
+    idx, sc = hamming_topk(_dev(q), _dev(kc), _dev(table), _dev(lens), k, 64, 128)
+    assert _lib.last_dispatch().startswith("block_score_strip%d+" % Wd)
+    oi, os_ = c_api.hamming_topk(q, kc, table, lens, k, 64, 128, 0)
+    assert np.array_equal(sc.cpu().numpy(), os_) and np.array_equal(idx.cpu().numpy(), oi)
+    msl = 64 * blocks - 3
+    tok = hamming_score(_dev(kc), _dev(q), _dev(table), _dev(lens), msl, 64, 128, False, out_int32=True)
+    assert _lib.last_dispatch() == "token_score_strip<%d,0>" % Wd
+    assert np.array_equal(tok.cpu().numpy(), c_api.hamming_score(q, kc, table, lens, msl, 64, 128, False))

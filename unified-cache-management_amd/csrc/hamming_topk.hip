@@ -46,7 +46,7 @@ struct ScoreArgs {
     int table_stride, max_blocks;
     const int32_t* lens;
     int B, Hq, G, sink, recent;
-    int TB;                  // logical blocks per workgroup
+    int TB;                  // logical blocks per workgroup; strip scorers: per wave, at most strip_run()
     int reduce_out;          // block_score_one / block_score_rows: write the maximum over the
                              // KV heads, scores then is [B][1][max_blocks]
     const uint32_t* planes;  // [B][Hkv][PMAX][Wd], planes mode only
@@ -1625,6 +1625,14 @@ constexpr int kStripWaves = 8;  // waves per workgroup
 constexpr int kStripRun = 4;    // blocks per wave
 constexpr int kStripSlots = 2;  // blocks of a wave in LDS
 constexpr int strip_run(int wd) { return wd == 18 ? kStripRun : 4; }  // blocks per wave
+// Blocks per wave of a launch over `blocks` blocks of B requests: the run while that makes two workgroups
+// for every one of the 256 compute units, fewer where compute units would stand idle (2 x 313 blocks: 20
+// workgroups of runs of four 7.3 us, 80 of single blocks 5.0 us).
+inline int strip_blocks(int wd, int B, int blocks)
+{
+    const int64_t n = ucm::ceil_div((int64_t)B * blocks, kStripWaves * 512);
+    return n < 1 ? 1 : (n < strip_run(wd) ? (int)n : strip_run(wd));
+}
 constexpr int kStripFirst = 0;  // of those, a building wave requests before the weight build (at most kStripSlots)
 
 // One block of NL KiB (+ half a KiB when TAIL) from `base` into LDS at byte address `lds`.
@@ -1720,7 +1728,8 @@ __device__ __forceinline__ void strip_body(const ScoreArgs& a, int max_seq_len, 
     __shared__ int cpiece[2 * (WD / 2)];
     const int b = blockIdx.y;
     const int lane = lane_id(), wid = wave_id();
-    const int j0 = (blockIdx.x * kStripWaves + wid) * RUN;
+    const int most = a.TB;  // blocks of a wave
+    const int j0 = (blockIdx.x * kStripWaves + wid) * most;
     // first round of reads: those that need the kernel arguments only
     const int len = a.lens[b];
     int my_entry;  // lane i: table entry of block j0 + i
@@ -1808,13 +1817,13 @@ __device__ __forceinline__ void strip_body(const ScoreArgs& a, int max_seq_len, 
         const _Float16 none_h[4] = {(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
 #pragma unroll
         for (int i = 0; i < RUN; ++i)
-            if (i >= first_i) emit(i, false, none_i, none_h);
+            if (i >= first_i && i < most) emit(i, false, none_i, none_h);
     };
-    if ((int)blockIdx.x * kStripWaves * RUN >= nblk) {  // the whole workgroup
+    if ((int)blockIdx.x * kStripWaves * most >= nblk) {  // the whole workgroup
         if (TOKENS) emit_unread(0);
         return;
     }
-    const int run = nblk - j0 < RUN ? nblk - j0 : RUN;  // <= 0: nothing to score
+    const int run = nblk - j0 < most ? nblk - j0 : most;  // <= 0: nothing to score
     int entry[RUN];
 #pragma unroll
     for (int i = 0; i < RUN; ++i) entry[i] = __builtin_amdgcn_readlane(my_entry, i);
@@ -3202,7 +3211,8 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
         if (planes_inside && a.G >= 16 && a.G <= 128) {
             // the weighted bit sums on the matrix unit, as for 18-word codes
             note_score("block_score_strip8");
-            const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * strip_run(8)), (unsigned)B);
+            a.TB = strip_blocks(8, B, max_blocks);
+            const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
             launch_score_threads(block_score_strip<8>, g64, kStripWaves * kWave, 0, st, a);
         } else if (planes_inside) {
             // one nibble digit of the per-bit counts up to 15 query heads, two up to 255
@@ -3220,7 +3230,8 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
             }
         } else if (planes_in_lanes && Wd == 18) {
             note_score("block_score_strip18");
-            const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * kStripRun), (unsigned)B);
+            a.TB = strip_blocks(18, B, max_blocks);
+            const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
             launch_score_threads(block_score_strip<18>, g64, kStripWaves * kWave, 0, st, a);
         } else if (planes_in_lanes) {
             note_score("block_score_lanes_run", Wd / 2, pmax);
@@ -4161,7 +4172,8 @@ extern "C" int ucm_hamming_score(const uint32_t* q_codes, int64_t q_stride_b, in
         }
         if (run18 || run8) {
             // the weighted bit sums of every 8-byte piece on the matrix unit; no plane kernel, no workspace
-            const dim3 rgrid((unsigned)ucm::ceil_div(nblk, kStripWaves * strip_run(Wd)), (unsigned)B);
+            a.TB = strip_blocks(Wd, B, nblk);
+            const dim3 rgrid((unsigned)ucm::ceil_div(nblk, kStripWaves * a.TB), (unsigned)B);
             const dim3 threads(kStripWaves * kWave);
             note_score("token_score_strip", Wd, out_is_f16 ? 1 : 0);
             if (Wd == 18) {
