@@ -113,10 +113,11 @@ PyObject* front(F&& f)
 template <class F>
 int without_gil(F&& f)
 {
-    PyThreadState* s = PyEval_SaveThread();
-    const int rc = f();
-    PyEval_RestoreThread(s);
-    return rc;
+    struct Released {  // taken again also where reading a tensor throws
+        PyThreadState* s = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(s); }
+    } released;
+    return f();
 }
 
 // The tensors of a grouped-query step, checked like the step's own _arguments().
