@@ -1877,6 +1877,9 @@ int launch_mfma_q(const EncArgs& a, size_t lds, hipStream_t st)
         // runs of one against four: 2048 tokens 4.8 and 9.6 us, 8192: 7.5 and 10.1, 12,000: 10.2 and
         // 11.2, 16,384: 12.6 and 12.1).  Eight once those fill the chip twice over: half the projection
         // slices staged (65,536 tokens 31.9 against 35.6 us, 32,768: 19.6 against 19.3).
+        // Runs of two and three between those were tried: 12,700 tokens of two 11.9 against 12.2 us and 24,576
+        // 15.1 against 16.7, but 20,000 15.9 against 15.5 and 64 -> 128 bits, 13,000 tokens 13.8 against 11.0;
+        // three (held to 168 registers, which spills) 32,691 tokens 24.4 against 19.1.
         const int64_t cus = stream_workgroups();
         if (all <= 3 * cus) return launch_mfma_t<V, KS, NQ, NG, 1>(a, lds, grid(1), st);
         if (all >= 16 * cus) return launch_mfma_t<V, KS, NQ, NG, 8>(a, lds, grid(8), st);
