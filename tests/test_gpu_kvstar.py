@@ -98,6 +98,57 @@ def test_far_scores_keep_their_order():
     assert np.all(np.abs(gs - ref) <= 1e-5 * ref + 2e-45)
 
 
+@pytest.mark.parametrize("base", [-1.8e8, -1.92e8, -3.2e8, -4.0e9, 1.4e9, 1.6e9, 4.0e9])
+@pytest.mark.parametrize("d,M", [(32, 1), (32, 3), (64, 40), (24, 3)])
+def test_scores_of_any_finite_size(base, d, M):
+    """Rows whose scores all lie near `base` (finite fp16 inputs reach 4.3e9 in one channel), beside a row of
+    ordinary ones.  One channel makes the base, one adds steps of one fp32 unit of it: every product and sum
+    is exact in any order, so the rows compare with the checker's at the usual tolerance."""
+    n, rng = 45, np.random.default_rng(int(abs(base)) % 1000 + d)
+    ulp = float(np.spacing(np.float32(abs(base))))
+    a = 64.0 * round(abs(base) / 64 / 61440)         # times 61440 = 2^12 * 15: a multiple of 2^18
+    q = np.zeros((2, 2, d), np.float16)
+    q[:, :, 0], q[:, :, 1] = np.copysign(a, base), ulp
+    q[1, 1, 0], q[1, 1, 1] = 0.0, 0.25               # an ordinary row
+    k = np.zeros((n, M, 1, d), np.float16)
+    k[..., 0] = 61440.0
+    k[..., 1] = rng.integers(0, 4, (n, M, 1))
+    assert a * 61440.0 + 3 * ulp != a * 61440.0 and abs(a * 61440 / abs(base) - 1) < 0.01
+    check(q, k, None, n)
+
+
+@pytest.mark.parametrize("n,M,d", [(40, 1, 32), (33, 3, 32), (30, 64, 64), (70, 20, 128), (40, 3, 24), (33, 33, 96)])
+@pytest.mark.parametrize("what", ["nan", "+inf", "-inf", "all_-inf"])
+def test_infinite_and_undefined_scores(what, n, M, d):
+    """As the checker has it: exponentials of the distance to the row's largest score, which passes over NaN
+    (the checker's also does unless its first score is one); a row whose sum is NaN is not normalised; a row
+    of minus infinities has NaN everywhere.  Blocks with a NaN score come last, in block order."""
+    q, k = make(n + M + d, 2, 4, 2, d, n, M)
+    q = np.abs(q) + np.float16(0.125)                # no zero times infinity
+    flat = k.reshape(n * M, 2, d)
+    S = n * M
+    for s in (S // 3, S - 1):
+        if what == "nan":
+            flat[s, 0, 3] = np.nan                   # KV head 0 only: the other head's rows stay normalised
+        elif what == "+inf":
+            flat[s, 0, 3] = np.inf
+        elif what == "-inf":
+            flat[s, 0, 3] = -np.inf
+        else:
+            flat[:, 0, 3] = -np.inf
+    gi, gs = run_gpu(q, k, None, n)
+    _, _, ref = c_api.kvstar_topk(q, k, n)
+    undefined = np.isnan(ref)
+    assert undefined.any() == (what != "-inf") and (undefined.all() == (what == "all_-inf"))
+    got = np.zeros(n, np.float32)
+    got[gi] = gs
+    assert sorted(gi.tolist()) == list(range(n)) and np.array_equal(np.isnan(got), undefined)
+    ok = ~undefined
+    assert np.all(np.abs(got[ok] - ref[ok]) <= ATOL + RTOL * np.abs(ref[ok]))
+    tail = gi[int(ok.sum()):]
+    assert tail.tolist() == np.flatnonzero(undefined).tolist()
+
+
 def test_sharp_softmax():
     # larger logits: a few representatives take most of the mass
     q, k = make(11, 4, 8, 4, 64, 200, 2, scale=1.5)

@@ -39,10 +39,11 @@ constexpr int kMassGroups = 512;    // its workgroups at most
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Sums of exponentials over parts of a row meet as (e, s) = s 2^e with a whole number e near the part's
-// maximum: merging two is a shift and an addition, not two more exponentials.
+// Largest score of a part of a row and the sum of exp(score - m) over it; (-inf, 0) where nothing was seen.
+// Scores reach 4.4e12 for finite inputs (1024 channels), where fp32 steps are 2^18: only the difference of
+// two scores, which is exact when they are close, is ever an exponent.
 struct Stat {
-    int e;
+    float m;
     float s;
 };
 
@@ -114,7 +115,6 @@ __device__ __forceinline__ f16x8 load_q(const QRow& q, int c, int d, int d_orig)
 }
 
 constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596303e-8f;  // log2(e) in two pieces
-constexpr float kLn2 = 0.693147182f, kLn2Low = -1.90465421e-9f;   // ln(2) in two pieces
 
 // exp(x) for x far from overflow (here x <= 0 but for rounding): 2^(x log2 e) with the product's
 // rounding error carried along, whole and fractional part of the exponent taken apart so that results
@@ -129,18 +129,29 @@ __device__ __forceinline__ float exp_small(float x)
     return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - n) + r), (int)n);
 }
 
-__device__ __forceinline__ Stat to_stat(float m, float sum)  // sum of exp(x - m)
+// What a part's maximum is measured from: 0 where the largest one is minus infinity, whose exponentials are 0.
+__device__ __forceinline__ float stat_base(float m) { return m == -INFINITY ? 0.0f : m; }
+
+// The factor exp(x) of a part whose maximum lies x <= 0 off the largest.  Rounding the exponent moves it by
+// |x| 2^-24 of itself, at most 2^-25 of the row's sum, which holds a term of 1: that error need not be carried
+// as in exp_small (1.1 us more at the example's shape), only log2(e)'s own, which has the same sign in every part.
+__device__ __forceinline__ float part_weight(float x)
 {
-    if (m == -INFINITY) return Stat{-(1 << 28), 0.0f};  // nothing seen
-    const float e = __builtin_rintf(m * kLog2e);
-    const float d = __builtin_fmaf(-e, kLn2Low, __builtin_fmaf(-e, kLn2, m));
-    return Stat{(int)e, sum * expf(d)};
+    return __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, x * kLog2eLow));
 }
 
-__device__ __forceinline__ Stat merge(Stat a, Stat b)
+// `st` and the first `count` of the parts v.
+template <int N>
+__device__ __forceinline__ Stat merge(Stat st, const Stat (&v)[N], int count = N)
 {
-    const int e = a.e > b.e ? a.e : b.e;
-    return Stat{e, __builtin_amdgcn_ldexpf(a.s, a.e - e) + __builtin_amdgcn_ldexpf(b.s, b.e - e)};
+    float m = st.m;
+#pragma unroll
+    for (int i = 0; i < N; ++i) m = fmaxf(m, i < count ? v[i].m : -INFINITY);
+    const float base = stat_base(m);
+    float sum = st.s * part_weight(st.m - base);
+#pragma unroll
+    for (int i = 0; i < N; ++i) sum += i < count ? v[i].s * part_weight(v[i].m - base) : 0.0f;
+    return Stat{m, sum};
 }
 
 // grid = (chunks, ceil(items / kStatItems)).  Wave w serves row tile w % kStatItems and every
@@ -156,7 +167,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
     constexpr int U = KS == 0 || KS > 4 ? 1 : 2;  // tiles in flight per wave
     constexpr int dp = KS * 16 + 8;  // row pitch: 16 bytes of padding spread the rows over the banks
     __shared__ __align__(16) _Float16 qt[KS ? kStatItems * 32 * dp : 8];
-    __shared__ Stat red[kThreads / 64][32];
+    __shared__ Stat red[kThreads / 64][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = wave % kStatItems, sub = wave / kStatItems;
     const int item = blockIdx.y * kStatItems + li;
@@ -250,14 +261,13 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
         }
         add_tiles(acc, t);
     }
-    Stat st = to_stat(m, sum);
-    st = merge(st, Stat{__shfl_xor(st.e, 32), __shfl_xor(st.s, 32)});  // the row's other representatives
-    if (lane < 32) red[wave][lane] = st;
+    red[wave][lane] = Stat{m, sum};  // a row is lanes r and r + 32 of kStatSubs waves
     __syncthreads();
     if (sub == 0 && lane < 32 && item < a.items) {
+        Stat v[2 * kStatSubs];
 #pragma unroll
-        for (int i = 1; i < kStatSubs; ++i) st = merge(st, red[li + i * kStatItems][lane]);
-        a.part[(int64_t)blockIdx.x * a.items * 32 + item * 32 + lane] = st;
+        for (int i = 0; i < 2 * kStatSubs; ++i) v[i] = red[li + i / 2 * kStatItems][lane + 32 * (i & 1)];
+        a.part[(int64_t)blockIdx.x * a.items * 32 + item * 32 + lane] = merge(Stat{-INFINITY, 0.0f}, v);
     }
 }
 
@@ -271,7 +281,7 @@ template <int KS>
 __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
 {
     constexpr int kWaves = kThreads / 64;
-    __shared__ __align__(16) float2 stat[kMassRows];  // (shift, 1 / sum of exponentials) of a row
+    __shared__ __align__(16) float2 stat[kMassRows];  // (largest score, 1 / sum of exponentials) of a row
     __shared__ Stat halves[kThreads];
     __shared__ float red[kWaves][32];
     __shared__ float rep[32];
@@ -293,39 +303,30 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
                 // two threads per row where the rows leave half of the workgroup idle
                 const bool split = nr <= kThreads / 2;
                 const int step = split ? kThreads / 2 : kThreads;
-                const int half = split ? threadIdx.x / (kThreads / 2) : 0;
+                const int half = split ? __builtin_amdgcn_readfirstlane(threadIdx.x / (kThreads / 2)) : 0;
                 const int c_mid = split ? (a.chunks + 1) / 2 : a.chunks;
                 const int c0 = half ? c_mid : 0, c1 = half ? a.chunks : c_mid;
                 for (int r = split ? threadIdx.x % (kThreads / 2) : threadIdx.x; r < (split ? step : nr); r += step) {
-                    Stat st{-(1 << 28), 0.0f};
+                    Stat st{-INFINITY, 0.0f};
                     if (r < nr) {
                         const Stat* p = a.part + r0 + r;
                         for (int c = c0; c < c1; c += 16) {
                             Stat v[16];
 #pragma unroll
                             for (int i = 0; i < 16; ++i) v[i] = p[(int64_t)(c + i < c1 ? c + i : c1 - 1) * rows];
-                            int e = st.e;
-#pragma unroll
-                            for (int i = 0; i < 16; ++i) e = e > v[i].e ? e : v[i].e;
-                            float sum = __builtin_amdgcn_ldexpf(st.s, st.e - e);
-#pragma unroll
-                            for (int i = 0; i < 16; ++i)
-                                sum += c + i < c1 ? __builtin_amdgcn_ldexpf(v[i].s, v[i].e - e) : 0.0f;
-                            st = Stat{e, sum};
+                            st = merge(st, v, c1 - c);
                         }
                     }
                     if (split) {
                         halves[threadIdx.x] = st;
                         __syncthreads();
-                        if (half == 0) st = merge(st, halves[threadIdx.x + kThreads / 2]);
+                        if (half == 0) {
+                            const Stat other[1] = {halves[threadIdx.x + kThreads / 2]};
+                            st = merge(st, other);
+                        }
                     }
-                    if (half == 0 && r < nr) {
-                        // the shift e ln 2 rounded, its rounding error moved into the factor
-                        const float e = (float)st.e, shift = e * kLn2;
-                        const float d = __builtin_fmaf(-e, kLn2Low, __builtin_fmaf(-e, kLn2, shift));
-                        // the reference normalises only when the sum exceeds 1e-9
-                        stat[r] = make_float2(shift, st.s > 1e-9f ? expf(d) / st.s : 1.0f);
-                    }
+                    // the reference normalises only when the sum exceeds 1e-9
+                    if (half == 0 && r < nr) stat[r] = make_float2(st.m, st.s > 1e-9f ? 1.0f / st.s : 1.0f);
                 }
                 __syncthreads();
             }
