@@ -118,7 +118,7 @@ def test_scores_of_any_finite_size(base, d, M):
 
 
 @pytest.mark.parametrize("n,M,d", [(40, 1, 32), (33, 3, 32), (30, 64, 64), (70, 20, 128), (40, 3, 24), (33, 33, 96)])
-@pytest.mark.parametrize("what", ["nan", "+inf", "-inf", "all_-inf"])
+@pytest.mark.parametrize("what", ["nan", "+inf", "-inf", "nan_lane", "all_-inf"])
 def test_infinite_and_undefined_scores(what, n, M, d):
     """As the checker has it: exponentials of the distance to the row's largest score, which passes over NaN
     (the checker's also does unless its first score is one); a row whose sum is NaN is not normalised; a row
@@ -130,6 +130,9 @@ def test_infinite_and_undefined_scores(what, n, M, d):
     for s in (S // 3, S - 1):
         if what == "nan":
             flat[s, 0, 3] = np.nan                   # KV head 0 only: the other head's rows stay normalised
+        elif what == "nan_lane":
+            t = max(32, s - s % 32)                  # a tile of representatives, not the first: all scores of a lane
+            flat[t:t + 32, 0, 3] = np.nan
         elif what == "+inf":
             flat[s, 0, 3] = np.inf
         elif what == "-inf":

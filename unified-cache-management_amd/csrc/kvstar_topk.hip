@@ -230,13 +230,15 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
                 nm = fmaxf(nm, x[u][v]);
             }
         }
-        if (nm == -INFINITY) return;
+        // a lane that has seen no number yet measures from 0: minus infinities add 0, a NaN (which the
+        // maximum passes over) still makes the row's sum one
+        const float base = stat_base(nm);
         float cs = 0.0f;
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) cs += exp_small(x[u][v] - nm);
-        sum = sum * exp_small(m - nm) + cs;
+            for (int v = 0; v < 16; ++v) cs += exp_small(x[u][v] - base);
+        sum = sum * exp_small(m - base) + cs;
         m = nm;
     };
     for (int t = t0; t < t1; t += U * kStatSubs) {
