@@ -152,6 +152,28 @@ def test_infinite_and_undefined_scores(what, n, M, d):
     assert tail.tolist() == np.flatnonzero(undefined).tolist()
 
 
+@pytest.mark.parametrize("d", [8, 17, 31, 32, 33, 48, 64, 80, 95, 96, 100, 112, 128, 130, 256, 512, 513, 1024])
+@pytest.mark.parametrize("M", [3, 40])
+def test_head_dimensions(d, M):
+    """Every remainder of the k-steps (groups of four, two, one and a partial one), a query row of more
+    channels than the keys have, and rows that start at odd multiples of two bytes."""
+    Hkv, d_orig = 2, d + 5
+    rng = np.random.default_rng(d)
+    q, k = make(d * 10 + M, 3, 6, Hkv, d, 41, M, scale=0.5 if d < 200 else 0.25 if d < 500 else 0.15, d_orig=d_orig)
+    pr = np.stack([np.sort(rng.permutation(d_orig)[:d]) for _ in range(Hkv)]).astype(np.int64)
+    check(q, k, pr, 13)
+    check(np.ascontiguousarray(q[..., :d]), k, None, 13)
+
+
+@pytest.mark.parametrize("d", [32, 64, 100, 128, 256])
+def test_probabilities_add_up_at_large_scores(d):
+    """Scores of several 10,000 are steps of 2^-9 apart: the kernels that sum a row's exponentials and the
+    block's probabilities take the same q.k, or rows would add up to e^(2^-9) and not to 1."""
+    q, k = make(d, 4, 8, 2, d, 30, 40, scale=60.0)
+    _, gs = run_gpu(q, k, None, 30)
+    assert abs(gs.astype(np.float64).sum() - 32) < 32 * 1e-5
+
+
 def test_sharp_softmax():
     # larger logits: a few representatives take most of the mass
     q, k = make(11, 4, 8, 4, 64, 200, 2, scale=1.5)

@@ -24,14 +24,21 @@
 // ascending block order (the reference's heap pops them in descending block order).
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "float_topk.h"
 
 namespace {
 
 constexpr int kThreads = 512;       // both kernels: eight waves
-constexpr int kStatItems = 2;       // row tiles a workgroup of the statistics kernel serves
-constexpr int kStatSubs = 4;        // waves that share a row tile's representatives there
+constexpr int kAnyDim = 0;          // KS of the statistics kernel for other dimensions than 32, 64 and 128, up to
+constexpr int kAnyDimMost = 512;    // this (32 rows in LDS), and
+constexpr int kPacked = -1;         // for those above it, whose query rows kvstar_pack_kernel has gathered
+constexpr int stat_items(int ks) { return ks > 0 ? 2 : 1; }  // row tiles a workgroup of it serves
+constexpr int kEarly = 8;           // k-steps that kernels for any dimension request ahead of their other work,
+constexpr int kEarlyMost = 256;     // in rows up to this (512 channels, 16 representatives: 0.8 us more with it)
+constexpr int kLongDim = 128;       // above it loads take more of both kernels' time than the statistics' merging
 constexpr int kMaxChunks = 64;      // partial statistics per row
 constexpr int kMassRows = 2048;     // rows whose statistics the mass kernel holds in LDS at a time
 constexpr int kMassGroups = 512;    // its workgroups at most
@@ -58,7 +65,8 @@ struct KvArgs {
     int tiles_q, items;     // row tiles per KV head, and of all heads
     int tiles_k, per_chunk; // tiles of 32 representatives: all, and per chunk of the statistics kernel
     int chunks;
-    _Float16* qp;           // [items][32][d] query rows, channels pruned, zeros behind the last row (KS > 0)
+    int dp;                 // d in whole steps of 16 channels
+    _Float16* qp;           // [items][32][dp] query rows, channels pruned, zeros behind the last row and channel
     Stat* part;             // [chunks][items * 32] sum of exponentials over a chunk
     uint32_t* keys;         // [n_blocks]
     int group_blocks;       // blocks a workgroup of the mass kernel handles together
@@ -154,23 +162,83 @@ __device__ __forceinline__ Stat merge(Stat st, const Stat (&v)[N], int count = N
     return Stat{m, sum};
 }
 
-// grid = (chunks, ceil(items / kStatItems)).  Wave w serves row tile w % kStatItems and every
-// kStatSubs-th tile of representatives of the chunk.  Representatives are the A operand (lane:
+// Any head dimension: U tiles of representatives against a row tile, up to eight k-steps' loads in flight (16
+// bytes each, representatives of an odd dimension from any even address).  The steps are added in ascending
+// order, as where their number is known: both kernels get the same score to the last bit.  QA: the query rows
+// are the A operand.  c: the first channel to add.
+template <bool QA, int U>
+__device__ __forceinline__ void dots_any(const _Float16* qrow, const _Float16* const (&row)[U], int kb, int c, int d,
+                                         f32x16 (&acc)[U])
+{
+    auto mul = [&](const f16x8& q, const f16x8& k, f32x16& c) {
+        c = QA ? __builtin_amdgcn_mfma_f32_32x32x16_f16(q, k, c, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_f16(k, q, c, 0, 0, 0);
+    };
+    auto steps = [&](int c, auto n_) {
+        constexpr int N = decltype(n_)::value;
+        f16x8 q[N], k[U][N];
+#pragma unroll
+        for (int u = 0; u < U; ++u)  // a row's pieces one after the other: four of them share a cache line
+#pragma unroll
+            for (int i = 0; i < N; ++i) k[u][i] = *reinterpret_cast<const f16x8u*>(row[u] + c + i * 16 + kb);
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = *reinterpret_cast<const f16x8*>(qrow + c + i * 16 + kb);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int u = 0; u < U; ++u) mul(q[i], k[u][i], acc[u]);
+    };
+    for (; c + 128 <= d; c += 128) steps(c, std::integral_constant<int, 8>{});
+    if (c + 64 <= d) {
+        steps(c, std::integral_constant<int, 4>{});
+        c += 64;
+    }
+    if (c + 32 <= d) {
+        steps(c, std::integral_constant<int, 2>{});
+        c += 32;
+    }
+    if (c + 16 <= d) {
+        steps(c, std::integral_constant<int, 1>{});
+        c += 16;
+    }
+    if (c < d) {
+        const f16x8 q = *reinterpret_cast<const f16x8*>(qrow + c + kb);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mul(q, load_k(row[u], c + kb, d), acc[u]);
+    }
+}
+
+// The query rows gathered, 8 channels per thread, where they are too long for the statistics kernel to do it.
+__global__ __launch_bounds__(kThreads) void kvstar_pack_kernel(KvArgs a)
+{
+    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    const int per_row = a.dp / 8;
+    const int64_t row = i / per_row;
+    if (row >= (int64_t)a.items * 32) return;
+    const int c = (int)(i - row * per_row) * 8;
+    *reinterpret_cast<f16x8*>(a.qp + row * a.dp + c) = load_q(q_row(a, (int)(row >> 5), (int)(row & 31)), c, a.d, a.d_orig);
+}
+
+// grid = (chunks, ceil(items / kItems)).  Wave w serves row tile w % kItems and every
+// kSubs-th tile of representatives of the chunk.  Representatives are the A operand (lane:
 // representative lane % 32, channels 8 (lane / 32) .. + 7 of the k-step), query rows the B operand:
 // accumulator v of a lane is the score of row lane % 32 against representative
 // 8 (v / 4) + 4 (lane / 32) + v % 4 of the tile, so a row's statistics are one lane's work and meet
 // once, at the end.  KS = d / 16 for 32, 64 and 128 channels: the loads of several tiles go out
-// together, in front of the gather of the query rows (which all waves share through LDS).  KS = 0: any d.
+// together, in front of the gather of the query rows (which all waves share through LDS).  Any other d: one
+// row tile per workgroup, as many k-steps as the registers take at a time.  Query rows gathered by every lane in
+// front of every tile cost 2 to 6 times the call: 8 x 32 query rows, 253 blocks of 64, 96 channels 66 us, gathered
+// once 27 us; blocks of 16, 512 channels 208 and 35 us.
 template <int KS>
 __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
 {
-    constexpr int U = KS == 0 || KS > 4 ? 1 : 2;  // tiles in flight per wave
-    constexpr int dp = KS * 16 + 8;  // row pitch: 16 bytes of padding spread the rows over the banks
-    __shared__ __align__(16) _Float16 qt[KS ? kStatItems * 32 * dp : 8];
+    constexpr int kItems = stat_items(KS), kSubs = kThreads / 64 / kItems;  // kSubs waves share a row tile's representatives
+    constexpr int U = KS == 2 || KS == 4 ? 2 : 1;  // tiles in flight per wave
+    extern __shared__ __align__(16) _Float16 qt[];  // [kItems * 32][pitch], but for kPacked
+    const int pitch = (KS > 0 ? KS * 16 : a.dp) + 8;  // 16 bytes of padding spread the rows over the banks
     __shared__ Stat red[kThreads / 64][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int li = wave % kStatItems, sub = wave / kStatItems;
-    const int item = blockIdx.y * kStatItems + li;
+    const int li = wave % kItems, sub = wave / kItems;
+    const int item = blockIdx.y * kItems + li;
     const int h = item < a.items ? item / a.tiles_q : 0;
     const int kb = (lane >> 5) * 8;
     const int t0 = blockIdx.x * a.per_chunk + sub;
@@ -181,11 +249,13 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
         s = s < a.S ? s : a.S - 1;
         return a.k + (s * a.Hkv + h) * a.d;
     };
-    f16x8 kk[U][KS ? KS : 1];
+    f16x8 early[kEarly];  // of the first tile, requested in front of the gather
+    const bool hurry = a.d <= kEarlyMost;
+    f16x8 kk[U][KS > 0 ? KS : 1];
     auto load_tiles = [&](int t) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const _Float16* row = k_row(t + u * kStatSubs < t1 ? t + u * kStatSubs : t);
+            const _Float16* row = k_row(t + u * kSubs < t1 ? t + u * kSubs : t);
 #pragma unroll
             for (int c = 0; c < KS; ++c) kk[u][c] = *reinterpret_cast<const f16x8*>(row + c * 16 + kb);
         }
@@ -194,7 +264,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
         load_tiles(t0 < a.tiles_k ? t0 : 0);
         // eight threads per query row, each taking every eighth channel
         const int rl = threadIdx.x >> 3;  // 0 .. 63: row rl % 32 of the workgroup's item rl / 32
-        const QRow q = q_row(a, blockIdx.y * kStatItems + (rl >> 5), rl & 31);
+        const QRow q = q_row(a, blockIdx.y * kItems + (rl >> 5), rl & 31);
         int64_t src[2 * KS];
         _Float16 v[2 * KS];
 #pragma unroll
@@ -202,30 +272,54 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
 #pragma unroll
         for (int i = 0; i < 2 * KS; ++i) v[i] = q.row[src[i]];
 #pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) qt[rl * dp + (threadIdx.x & 7) + 8 * i] = q.ok ? v[i] : (_Float16)0;
+        for (int i = 0; i < 2 * KS; ++i) qt[rl * pitch + (threadIdx.x & 7) + 8 * i] = q.ok ? v[i] : (_Float16)0;
+    } else if constexpr (KS == kAnyDim) {
+        const _Float16* row = k_row(t0 < a.tiles_k ? t0 : 0);
+#pragma unroll
+        for (int i = 0; i < kEarly; ++i) {
+            early[i] = f16x8{0};
+            if (hurry && 16 * i + 16 <= a.d) early[i] = *reinterpret_cast<const f16x8u*>(row + 16 * i + kb);
+        }
+        // sixteen threads per query row, each taking every sixteenth channel
+        const int rl = threadIdx.x >> 4;
+        const QRow q = q_row(a, blockIdx.y, rl);
+        for (int c = threadIdx.x & 15; c < a.dp; c += 16 * 8) {
+            int64_t src[8];
+            _Float16 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) src[i] = q_channel(q, c + 16 * i < a.d ? c + 16 * i : 0, a.d_orig);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = q.row[src[i]];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (c + 16 * i < a.dp) qt[rl * pitch + c + 16 * i] = q.ok && c + 16 * i < a.d ? v[i] : (_Float16)0;
+        }
+    }
+    if constexpr (KS != kPacked) {
         __syncthreads();
         if (blockIdx.x == 0) {  // the gathered rows, for the mass kernel
-            for (int i = threadIdx.x; i < kStatItems * 32 * 2 * KS; i += kThreads) {
-                const int r = i / (2 * KS), c = (i % (2 * KS)) * 8;
-                const int64_t row = (int64_t)blockIdx.y * kStatItems * 32 + r;
+            const int per_row = KS > 0 ? 2 * KS : a.dp / 8;
+            for (int i = threadIdx.x; i < kItems * 32 * per_row; i += kThreads) {
+                const int r = i / per_row, c = (i % per_row) * 8;
+                const int64_t row = (int64_t)blockIdx.y * kItems * 32 + r;
                 if (row < (int64_t)a.items * 32)
-                    *reinterpret_cast<f16x8*>(a.qp + row * (KS * 16) + c) = *reinterpret_cast<const f16x8*>(qt + r * dp + c);
+                    *reinterpret_cast<f16x8*>(a.qp + row * a.dp + c) = *reinterpret_cast<const f16x8*>(qt + r * pitch + c);
             }
         }
     }
     float m = -INFINITY, sum = 0.0f;
-    // the scores of U tiles (t, t + kStatSubs, ...) join the row's statistics
+    // the scores of U tiles (t, t + kSubs, ...) join the row's statistics
     auto add_tiles = [&](const f32x16 (&acc)[U], int t) {
         float x[U][16];
         float nm = m;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t s0 = (int64_t)(t + u * kStatSubs) * 32;
-            const bool whole = t + u * kStatSubs < t1 && s0 + 32 <= a.S;  // uniform
+            const int64_t s0 = (int64_t)(t + u * kSubs) * 32;
+            const bool whole = t + u * kSubs < t1 && s0 + 32 <= a.S;  // uniform
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 x[u][v] = acc[u][v];
-                if (!whole && (t + u * kStatSubs >= t1 || s0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4 >= a.S))
+                if (!whole && (t + u * kSubs >= t1 || s0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4 >= a.S))
                     x[u][v] = -INFINITY;
                 nm = fmaxf(nm, x[u][v]);
             }
@@ -241,13 +335,13 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
         sum = sum * exp_small(m - base) + cs;
         m = nm;
     };
-    for (int t = t0; t < t1; t += U * kStatSubs) {
+    for (int t = t0; t < t1; t += U * kSubs) {
         f32x16 acc[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) acc[u] = f32x16{0};
         if constexpr (KS > 0) {
             if (t != t0) load_tiles(t);
-            const _Float16* qrow = qt + (li * 32 + (lane & 31)) * dp + kb;
+            const _Float16* qrow = qt + (li * 32 + (lane & 31)) * pitch + kb;
 #pragma unroll
             for (int c = 0; c < KS; ++c) {
                 const f16x8 qq = *reinterpret_cast<const f16x8*>(qrow + c * 16);
@@ -255,20 +349,33 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
                 for (int u = 0; u < U; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk[u][c], qq, acc[u], 0, 0, 0);
             }
         } else {
-            const _Float16* row = k_row(t);
-            const QRow q = q_row(a, item, lane & 31);
-            for (int c = 0; c < a.d; c += 16)
-                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(load_k(row, c + kb, a.d),
-                                                                load_q(q, c + kb, a.d, a.d_orig), acc[0], 0, 0, 0);
+            const _Float16* row[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) row[u] = k_row(t + u * kSubs < t1 ? t + u * kSubs : t);
+            if constexpr (KS == kPacked) {
+                dots_any<false>(a.qp + ((int64_t)item * 32 + (lane & 31)) * a.dp, row, kb, 0, a.d, acc);
+            } else {
+                const _Float16* qrow = qt + (lane & 31) * pitch;
+                int c = 0;
+                if (hurry && t == t0) {
+#pragma unroll
+                    for (int i = 0; i < kEarly; ++i) {
+                        if (16 * i + 16 > a.d) break;
+                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(early[i], *reinterpret_cast<const f16x8*>(qrow + 16 * i + kb), acc[0], 0, 0, 0);
+                        c = 16 * i + 16;
+                    }
+                }
+                dots_any<false>(qrow, row, kb, c, a.d, acc);
+            }
         }
         add_tiles(acc, t);
     }
-    red[wave][lane] = Stat{m, sum};  // a row is lanes r and r + 32 of kStatSubs waves
+    red[wave][lane] = Stat{m, sum};  // a row is lanes r and r + 32 of kSubs waves
     __syncthreads();
     if (sub == 0 && lane < 32 && item < a.items) {
-        Stat v[2 * kStatSubs];
+        Stat v[2 * kSubs];
 #pragma unroll
-        for (int i = 0; i < 2 * kStatSubs; ++i) v[i] = red[li + i / 2 * kStatItems][lane + 32 * (i & 1)];
+        for (int i = 0; i < 2 * kSubs; ++i) v[i] = red[li + i / 2 * kItems][lane + 32 * (i & 1)];
         a.part[(int64_t)blockIdx.x * a.items * 32 + item * 32 + lane] = merge(Stat{-INFINITY, 0.0f}, v);
     }
 }
@@ -279,7 +386,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
 // lane is row 8 (v / 4) + 4 (lane / 32) + v % 4 against representative lane % 32, whose probabilities
 // add up in the lane.  Partial sums meet in a fixed order: accumulators, row tiles of a wave, lane
 // halves, waves, representatives.
-template <int KS>
+template <int KS, bool EARLY>
 __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
 {
     constexpr int kWaves = kThreads / 64;
@@ -298,6 +405,18 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
         const int64_t want = (int64_t)a.group_blocks * a.M;
         const int ns = (int)(left < want ? left : want);
         float tot = 0.0f;
+        auto rep_row = [&](int t, int h) {  // representative lane % 32 of tile t of the group
+            const int s = t * 32 + (lane & 31);
+            return a.k + ((s0 + (s < ns ? s : ns - 1)) * a.Hkv + h) * a.d;
+        };
+        f16x8 early[2][EARLY ? kEarly : 1];  // of the first two tiles, requested in front of the statistics
+        if constexpr (EARLY) {
+            const int h = wave < a.items ? wave / a.tiles_q : 0;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < kEarly; ++i) early[u][i] = *reinterpret_cast<const f16x8u*>(rep_row(u, h) + 16 * i + kb);
+        }
         for (int batch = 0; batch < batches; ++batch) {
             const int r0 = batch * kMassRows;
             const int nr = rows - r0 < kMassRows ? rows - r0 : kMassRows;
@@ -337,10 +456,10 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
                 const int item = r0 / 32 + it;
                 const int h = item / a.tiles_q;
                 const int valid = real - (item - h * a.tiles_q) * 32;  // rows of the tile that exist
-                const _Float16* qrow = a.qp + ((int64_t)item * 32 + (lane & 31)) * (KS * 16) + kb;
-                f16x8 qq[KS ? KS : 1];
+                const _Float16* qrow = a.qp + ((int64_t)item * 32 + (lane & 31)) * (KS > 0 ? KS * 16 : a.dp);
+                f16x8 qq[KS > 0 ? KS : 1];
 #pragma unroll
-                for (int c = 0; c < KS; ++c) qq[c] = *reinterpret_cast<const f16x8*>(qrow + c * 16);
+                for (int c = 0; c < KS; ++c) qq[c] = *reinterpret_cast<const f16x8*>(qrow + c * 16 + kb);
                 auto add_tile = [&](const f32x16& acc, int t) {
                     float p = 0.0f;
 #pragma unroll
@@ -362,8 +481,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
                         f16x8 kk[2][KS];
 #pragma unroll
                         for (int u = 0; u < 2; ++u) {
-                            const int s = (t + u) * 32 + (lane & 31);
-                            const _Float16* row = a.k + ((s0 + (s < ns ? s : ns - 1)) * a.Hkv + h) * a.d;
+                            const _Float16* row = rep_row(t + u, h);
 #pragma unroll
                             for (int c = 0; c < KS; ++c) kk[u][c] = *reinterpret_cast<const f16x8*>(row + c * 16 + kb);
                         }
@@ -377,16 +495,35 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
                             add_tile(acc, t + u);
                         }
                     } else {
-                        for (int u = 0; u < 2 && (t + u) * 32 < ns; ++u) {
-                            const int s = (t + u) * 32 + (lane & 31);
-                            const _Float16* row = a.k + ((s0 + (s < ns ? s : ns - 1)) * a.Hkv + h) * a.d;
-                            const QRow q = q_row(a, item, lane & 31);
-                            f32x16 acc = {0};
-                            for (int c = 0; c < a.d; c += 16)
-                                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(load_q(q, c + kb, a.d, a.d_orig),
-                                                                             load_k(row, c + kb, a.d), acc, 0, 0, 0);
-                            add_tile(acc, t + u);
-                        }
+                        auto tiles = [&](auto n_) {
+                            constexpr int U = decltype(n_)::value;
+                            const _Float16* row[U];
+                            f32x16 acc[U];
+#pragma unroll
+                            for (int u = 0; u < U; ++u) {
+                                row[u] = rep_row(t + u, h);
+                                acc[u] = f32x16{0};
+                            }
+                            int c = 0;
+                            if constexpr (EARLY) {
+                                if (t == 0 && item == wave) {
+                                    f16x8 q[kEarly];
+#pragma unroll
+                                    for (int i = 0; i < kEarly; ++i) q[i] = *reinterpret_cast<const f16x8*>(qrow + 16 * i + kb);
+#pragma unroll
+                                    for (int i = 0; i < kEarly; ++i)
+#pragma unroll
+                                        for (int u = 0; u < U; ++u)
+                                            acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(q[i], early[u][i], acc[u], 0, 0, 0);
+                                    c = 16 * kEarly;
+                                }
+                            }
+                            dots_any<true>(qrow, row, kb, c, a.d, acc);
+#pragma unroll
+                            for (int u = 0; u < U; ++u) add_tile(acc[u], t + u);
+                        };
+                        if ((t + 1) * 32 < ns) tiles(std::integral_constant<int, 2>{});
+                        else tiles(std::integral_constant<int, 1>{});
                     }
                 }
             }
@@ -423,19 +560,26 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-constexpr int kPackedDim = 128;  // the largest head dimension whose query rows are kept packed
+constexpr int kMaxDim = 1024;
 
-// How the representatives are shared out.
+// How the representatives are shared out: the larger d, the more chunks.
 void plan_chunks(KvArgs& a)
 {
     a.S = (int64_t)a.n_blocks * a.M;
     a.tiles_k = (int)ucm::ceil_div(a.S, 32);
-    // two tiles per wave at least.  kMaxChunks: 32 leave half of the chip idle at 8 KV heads (statistics
-    // 8.9 us instead of 7.2), and every workgroup of the mass kernel reads all chunks' pairs of its rows
+    // kMaxChunks: 32 leave half of the chip idle at 8 KV heads (statistics 8.9 us instead of 7.2), and every
+    // workgroup of the mass kernel reads all chunks' pairs of its rows.  Fewer than eight tiles to a workgroup
+    // of the statistics kernel, and fewer than 32 representatives to one of the mass kernel, only make more
+    // pairs to merge (1000 blocks of one representative, 32 channels: 15.0 us, in 256 groups 16.3) unless rows
+    // are long and compute units idle (512 channels, 253 blocks of 16: 40.6 us, like this 34.9; 256 channels,
+    // 64 blocks of 16, two heads: 19.2 and 17.0).
+    const bool longer = a.d > kLongDim;
     a.per_chunk = (int)ucm::ceil_div(a.tiles_k, kMaxChunks);
-    if (a.per_chunk < 2 * kStatSubs) a.per_chunk = 2 * kStatSubs;
+    if (a.per_chunk < (longer ? 4 : 8)) a.per_chunk = longer ? 4 : 8;
     a.chunks = (int)ucm::ceil_div(a.tiles_k, a.per_chunk);
     a.group_blocks = a.M >= 32 ? 1 : 32 / a.M;
+    if (longer)
+        while (a.group_blocks > 1 && ucm::ceil_div(a.n_blocks, a.group_blocks) < 256) a.group_blocks /= 2;
     a.groups = (int)ucm::ceil_div(a.n_blocks, a.group_blocks);
 }
 
@@ -447,7 +591,7 @@ size_t carve_kvstar(KvArgs& a, void* base)
     char* p = (char*)base;
     size_t off = 0;
     a.qp = (_Float16*)(p + off);
-    off += align256(rows * kPackedDim * 2);
+    off += align256(rows * kMaxDim * 2);
     a.part = (Stat*)(p + off);
     off += align256((size_t)a.chunks * rows * 8);
     a.keys = (uint32_t*)(p + off);
@@ -458,12 +602,25 @@ size_t carve_kvstar(KvArgs& a, void* base)
 template <int KS>
 int launch_kvstar(const KvArgs& a, hipStream_t st)
 {
-    const dim3 grid((unsigned)a.chunks, (unsigned)ucm::ceil_div(a.items, kStatItems));
-    hipLaunchKernelGGL(kvstar_stats_kernel<KS>, grid, dim3(kThreads), 0, st, a);
-    const int rc = ucm::launch_status("kvstar_stats_kernel");
+    int rc;
+    if (KS == kPacked) {
+        hipLaunchKernelGGL(kvstar_pack_kernel, dim3((unsigned)ucm::ceil_div((int64_t)a.items * 4 * a.dp, kThreads)), dim3(kThreads), 0, st, a);
+        rc = ucm::launch_status("kvstar_pack_kernel");
+        if (rc != UCM_OK) return rc;
+    }
+    const size_t lds = KS == kPacked ? 0 : (size_t)stat_items(KS) * 32 * (a.dp + 8) * 2;
+    hipLaunchKernelGGL(kvstar_stats_kernel<KS>, dim3((unsigned)a.chunks, (unsigned)ucm::ceil_div(a.items, stat_items(KS))),
+                       dim3(kThreads), lds, st, a);
+    rc = ucm::launch_status("kvstar_stats_kernel");
     if (rc != UCM_OK) return rc;
-    hipLaunchKernelGGL(kvstar_mass_kernel<KS>, dim3((unsigned)(a.groups < kMassGroups ? a.groups : kMassGroups)),
-                       dim3(kThreads), 0, st, a);
+    const dim3 groups((unsigned)(a.groups < kMassGroups ? a.groups : kMassGroups));
+    // Early loads where a block has two tiles and long rows and one generation of workgroups has nothing else to
+    // hide them behind (253 blocks of 64, 192 channels: 38.1 and 36.3 us); elsewhere their registers cost more
+    // (1024 blocks of 32, 96 channels: 59.5 and 69.4 us).
+    if (KS == kAnyDim && a.M > 32 && a.d >= 16 * kEarly && a.groups <= 256)
+        hipLaunchKernelGGL((kvstar_mass_kernel<kAnyDim, true>), groups, dim3(kThreads), 0, st, a);
+    else
+        hipLaunchKernelGGL((kvstar_mass_kernel<(KS > 0 ? KS : kAnyDim), false>), groups, dim3(kThreads), 0, st, a);
     return ucm::launch_status("kvstar_mass_kernel");
 }
 
@@ -474,7 +631,7 @@ extern "C" size_t ucm_kvstar_topk_workspace_bytes(int32_t X, int32_t Hq, int64_t
     if (X <= 0 || Hq <= 0 || n_blocks <= 0 || M <= 0) return 256;
     if (n_blocks > INT32_MAX || n_blocks * M > INT32_MAX) return 256;  // refused by the call
     KvArgs a{};
-    a.X = X; a.Hq = Hq; a.n_blocks = (int)n_blocks; a.M = M;
+    a.X = X; a.Hq = Hq; a.n_blocks = (int)n_blocks; a.M = M; a.d = kMaxDim;
     plan_chunks(a);
     return carve_kvstar(a, nullptr);
 }
@@ -494,7 +651,7 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
                 "Dimension mismatch: No dPrunedIndex, but Q and K head dims differ.");
     UCM_REQUIRE(topk > 0, "topk %d must be positive", topk);
     if (topk > kMaxTopk) return ucm::fail(UCM_EUNSUPPORTED, "topk %d above %d", topk, kMaxTopk);
-    UCM_REQUIRE(d <= 1024, "head dim %d above 1024", d);
+    UCM_REQUIRE(d <= kMaxDim, "head dim %d above %d", d, kMaxDim);
     UCM_REQUIRE(n_blocks <= INT32_MAX && n_blocks * M <= INT32_MAX, "too many block representatives");
     const int64_t rows = (int64_t)X * Hq;
     UCM_REQUIRE(rows <= 65535 && rows * M <= INT32_MAX, "too many query rows");
@@ -504,7 +661,7 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     hipStream_t st = (hipStream_t)stream;
     KvArgs a{};
     a.q = (const _Float16*)query; a.k = (const _Float16*)blk_repre; a.pruned = pruned_index;
-    a.X = X; a.Hq = Hq; a.Hkv = Hkv; a.g = Hq / Hkv; a.d_orig = d_orig; a.d = d;
+    a.X = X; a.Hq = Hq; a.Hkv = Hkv; a.g = Hq / Hkv; a.d_orig = d_orig; a.d = d; a.dp = (int)ucm::ceil_div(d, 16) * 16;
     a.n_blocks = (int)n_blocks; a.M = M;
     a.tiles_q = (int)ucm::ceil_div((int64_t)X * a.g, 32);
     a.items = Hkv * a.tiles_q;
@@ -512,8 +669,9 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     carve_kvstar(a, workspace);
     const int rc = d == 32 ? launch_kvstar<2>(a, st)
                  : d == 64 ? launch_kvstar<4>(a, st)
-                 : d == kPackedDim ? launch_kvstar<8>(a, st)
-                                   : launch_kvstar<0>(a, st);
+                 : d == 128 ? launch_kvstar<8>(a, st)
+                                   : d <= kAnyDimMost ? launch_kvstar<kAnyDim>(a, st)
+                                 : launch_kvstar<kPacked>(a, st);
     if (rc != UCM_OK) return rc;
     SortArgs s{};
     s.keys = a.keys; s.pitch = key_pitch(n_blocks); s.max_n = (int)n_blocks; s.topk = topk;
