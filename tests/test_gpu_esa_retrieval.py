@@ -168,6 +168,45 @@ def test_selection_at_the_edges_of_its_row_lengths(max_n, spread):
             assert (gi[b, len(order):] == -1).all() and (gs[b, len(order):] == 0).all()
 
 
+@pytest.mark.parametrize("max_n", [63, 64, 65, 200, 511, 512, 513, 1024, 1025, 4096, 4097, 8192, 8193, 16384, 16500])
+@pytest.mark.parametrize("spread", ["far", "inf", "both_inf", "nan", "decades", "two_far", "clusters", "ties_below", "all_equal"])
+def test_selection_of_uneven_rows(max_n, spread):
+    """Rows whose scores crowd into few equal-width bins of their range, because of one score or one side of
+    it (the crowded bins are divided once more) or still after that (digit search: dense clusters and ties,
+    which need no ordering where they lie at the threshold).  dim 1 and query 1 as above; NaN comes last."""
+    rng = rng_for(max_n * 5 + len(spread))
+    data = rng.standard_normal((20000, 1)).astype(np.float32)
+    perm = np.stack([rng.permutation(20000)[:max_n] for _ in range(2)]).astype(np.int32)
+    some = perm[:, max_n // 2]
+    if spread == "far":
+        data[some] = 300.0
+    elif spread in ("inf", "both_inf"):
+        data[some] = np.inf
+        if spread == "both_inf":
+            data[perm[:, 3]] = -np.inf
+    elif spread == "nan":
+        data[perm[:, 5:9]] = np.nan
+    elif spread == "decades":
+        data = np.exp(3 * data).astype(np.float32)
+    elif spread == "two_far":
+        data[some], data[perm[:, 1]] = 3e38, -3e38   # a range wider than the largest float
+    elif spread == "clusters":
+        data = (data * 1e-3 + rng.integers(0, 2, data.shape) * 50).astype(np.float32)
+    elif spread == "ties_below":
+        data[rng.random(20000) < 0.8] = -5.0
+        data[some] = 1e20
+    else:
+        data[:] = 0.25
+    for k in sorted({1, min(max_n, 4096), min(4096, max_n // 3 + 1)}):
+        gi, gs = gpu_dot_topk(data, np.ones((2, 1), np.float32), perm, k)
+        for b in range(2):
+            v = data[perm[b], 0]
+            order = np.argsort(np.where(np.isnan(v), np.inf, -v) + 0.0, kind="stable")
+            order = np.concatenate([order[~np.isnan(v[order])], order[np.isnan(v[order])]])[:k]
+            assert np.array_equal(gi[b], perm[b][order])
+            assert np.array_equal(gs[b], data[perm[b][order], 0], equal_nan=True)
+
+
 @pytest.mark.parametrize("dim", [4, 252, 256, 260, 508, 512, 768, 1020, 1024, 1028, 2300])
 def test_dot_products_at_the_edges_of_the_chunks(dim):
     """Rows are read in groups of four, two and one 256-value chunks and a partial one, by waves of four

@@ -8,7 +8,7 @@
 //   * dot_score_kernel — HBM-bound gather: one wave per kRowsPerWave candidate rows, 16-byte loads;
 //     writes one order-preserving 32-bit key per candidate (candidates that are -1 or outside the
 //     matrix get a key below every number);
-//   * topk_kernel (float_topk.h) — one workgroup per request.  Equal scores come out in list order;
+//   * launch_topk() (float_topk.h) — one launch selects and orders.  Equal scores come out in list order;
 //     the reference leaves ties unspecified.
 // Scores differ from the reference's in the last bits (the partial sums are added in a
 // different order); the tolerance is stated where the results are compared.

@@ -1,7 +1,7 @@
 // Selection shared by the float retrieval paths: the k best of a row of fp32 scores in
-// descending order, equal scores in list order.  One workgroup per row; a score travels as an
-// order-preserving 32-bit key that can be turned back into the score, so a row is one word per
-// candidate.  Included by the translation units that launch it.
+// descending order, equal scores in list order.  One workgroup per row, or several that order a share of
+// its places each; a score travels as an order-preserving 32-bit key that can be turned back into the
+// score, so a row is one word per candidate.  Included by the translation units that launch it.
 #pragma once
 
 #include "common.h"
@@ -28,10 +28,11 @@ __device__ __forceinline__ float key_score(uint32_t k)
     return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
 }
 
-// A finite number that orders like the key, for dividing the rows' range into equal widths.
+// A number that orders like the key, for dividing the rows' range into equal widths.  Both ends lie at half of
+// the largest float, so that the range is finite.
 __device__ __forceinline__ float key_place(uint32_t k)
 {
-    const float big = 3.402823466e38f;
+    const float big = 1.7e38f;
     const float v = key_score(k);
     return k == 1u ? -big : (v > big ? big : (v < -big ? -big : v));
 }
@@ -88,124 +89,299 @@ __device__ __forceinline__ int scan_wg(int v, int* wsum, int* total)
     return base + inc - v;
 }
 
+// What a score is output as: a NaN of one kind, whichever it was.
+__device__ __forceinline__ float out_of(uint32_t k) { return k == 1u ? __uint_as_float(0x7fc00000u) : key_score(k); }
+
+// Bins of equal width over the scores between two keys, best first.
+template <int BINS>
+struct Bins {
+    float top, scale;
+    __device__ __forceinline__ Bins(uint32_t hi, uint32_t lo) : top(key_place(hi))
+    {
+        const float width = top - key_place(lo);
+        scale = width > 0.0f ? (float)(BINS - 1) / width : 0.0f;
+    }
+    __device__ __forceinline__ int of(uint32_t k) const
+    {
+        const float at = (top - key_place(k)) * scale;  // not a number where the scale is infinite: bin 0
+        return at > 0.0f ? (int)(at < (float)(BINS - 1) ? at : (float)(BINS - 1)) : 0;
+    }
+};
+
 // Direct path.  The row's range of scores is divided into 4 NT bins of equal width, the keys are
 // counted per bin, a prefix sum over the bins (best first) says where each bin's entries go, and the
 // entries of the bins that start before place k are put there and ranked among the few that share
-// their bin.  Returns false, with nothing written, when such a bin holds more than kCrowd entries
-// (many equal scores, or a range stretched by outliers).
+// their bin.  Where such a bin holds more than kCrowd entries (a few scores far from the rest stretch the
+// range: an infinity, one block that holds most of the mass), the entries from the first crowded bin to the
+// last are divided again over their own range, up to kAgain times.  Returns false, with nothing written, when
+// bins are crowded still (many equal scores, several dense clusters).
 // What bounds it is its chain of barriers and LDS round trips, not bytes: one pass over the keys
 // replaces the search for the k-th key digit by digit, the compaction and the ordering (4 + 2 + 3
 // passes of counting, scanning and placing).  8000 candidates, k = 3000, two rows: 21.0 us for the
-// digit search, 8.1 us like this on one workgroup per row, 6.8 us with the places shared by three.
+// digit search, 8.1 us like this on one workgroup per row, 6.8 us with the places shared by three.  The whole
+// call over 128-value rows: even rows 10.9 us, with one infinite score 16.3 (29.8 when the search followed the
+// first crowded division).
 template <int NT, int PER>
-__device__ __forceinline__ bool topk_direct(const SortArgs& a, const uint32_t (&kreg)[PER], uint32_t* bins,
-                                            unsigned long long* win, int* wsum, uint32_t (*range)[NT / 64],
-                                            int* s_two)
-{
-    constexpr int kBins = 4 * NT;
-    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    uint32_t hi = 0u, lo = 0u;  // largest key and largest complement of a key
+struct Direct {
+    static constexpr int kBins = 4 * NT, kAgain = 2;
+    const SortArgs& a;
+    const uint32_t (&kreg)[PER];
+    uint32_t* bins;           // kBins words for every division
+    unsigned long long* win;  // NT + kCrowd entries
+    int* wsum;
+    uint32_t (*range)[NT / 64];
+    int* s_int;               // ends of the bins in front of this workgroup's places and of its own; first and last crowded bin
+    const int b, tid, lane, w;
+    // an entry's bin, counted through all divisions, and its place in the bin << 16; in one word where 16 keys
+    // leave no registers for two (at 8 keys and less two words are 0.2 us faster)
+    static constexpr bool kOneWord = PER > 8;
+    uint32_t slot[PER], at[kOneWord ? 1 : PER];
+    int n_valid, kk;
+
+    __device__ __forceinline__ int bin(int e) const { return (int)(kOneWord ? slot[e] & 0xffffu : slot[e]); }
+    __device__ __forceinline__ int place_of(int e) const { return (int)((kOneWord ? slot[e] : at[e]) >> 16); }
+    __device__ __forceinline__ void set(int e, uint32_t bin, uint32_t place)
+    {
+        slot[e] = kOneWord ? place << 16 | bin : bin;
+        if constexpr (!kOneWord) at[e] = place << 16;
+    }
+
+    __device__ __forceinline__ Direct(const SortArgs& args, const uint32_t (&k)[PER], uint32_t* lds, int* ws,
+                                      uint32_t (*r)[NT / 64], int* si)
+        : a(args), kreg(k), bins(lds), win(reinterpret_cast<unsigned long long*>(lds + (1 + kAgain) * kBins)), wsum(ws), range(r),
+          s_int(si), b(blockIdx.x), tid(threadIdx.x), lane(threadIdx.x & 63), w(threadIdx.x >> 6)
+    {
+    }
+
+    // Largest and smallest key of the entries for which in(e), behind a barrier.
+    template <class In>
+    __device__ __forceinline__ void range_of(In&& in, uint32_t& hi, uint32_t& lo)
+    {
+        hi = 0u;
+        uint32_t l = 0u;  // the smallest as the largest complement
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-        hi = kreg[e] > hi ? kreg[e] : hi;
-        lo = kreg[e] != 0u && ~kreg[e] > lo ? ~kreg[e] : lo;
-    }
-    hi = wave_max(hi);
-    lo = wave_max(lo);
-    if (lane == 0) {
-        range[0][w] = hi;
-        range[1][w] = lo;
-    }
-    reinterpret_cast<uint4*>(bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
-    if (tid < 2) s_two[tid] = 0;
-    __syncthreads();
+        for (int e = 0; e < PER; ++e) {
+            if (kreg[e] == 0u || !in(e)) continue;
+            hi = kreg[e] > hi ? kreg[e] : hi;
+            l = ~kreg[e] > l ? ~kreg[e] : l;
+        }
+        hi = wave_max(hi);
+        l = wave_max(l);
+        if (lane == 0) {
+            range[0][w] = hi;
+            range[1][w] = l;
+        }
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NT / 64; ++i) {
-        hi = range[0][i] > hi ? range[0][i] : hi;
-        lo = range[1][i] > lo ? range[1][i] : lo;
+        for (int i = 0; i < NT / 64; ++i) {
+            hi = range[0][i] > hi ? range[0][i] : hi;
+            l = range[1][i] > l ? range[1][i] : l;
+        }
+        lo = ~l;
     }
-    const float top = key_place(hi), width = top - key_place(~lo);
-    // an infinite width (range over the float limits) puts everything into one bin: the other path's case
-    const float scale = width > 0.0f ? (float)(kBins - 1) / width : 0.0f;
-    auto bin_of = [&](uint32_t k) {
-        const float at = (top - key_place(k)) * scale;  // not a number where the range is infinite: bin 0
-        return at > 0.0f ? (int)(at < (float)(kBins - 1) ? at : (float)(kBins - 1)) : 0;
-    };
-    int bin[PER], at[PER];
+
+    // The counts of a division's bins turned into (first place << 16 | entries) words; both fit: a row on this
+    // path has at most 16384 candidates.  Behind a barrier, returns whether a bin is crowded.
+    __device__ __forceinline__ bool place(int division, int base, uint32_t (&packed)[4])
+    {
+        uint4* mine = reinterpret_cast<uint4*>(bins + division * kBins) + tid;
+        const uint4 c = *mine;
+        const uint32_t cnt[4] = {c.x, c.y, c.z, c.w};
+        int total, first = base + scan_wg<NT>((int)(c.x + c.y + c.z + c.w), wsum, &total);
+        if (division == 0) {
+            n_valid = total;
+            kk = n_valid < a.topk ? n_valid : a.topk;
+        }
+        bool crowded = false;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-        bin[e] = bin_of(kreg[e]);
-        at[e] = 0;
-        if (kreg[e] != 0u) at[e] = (int)atomicAdd(&bins[bin[e]], 1u);
+        for (int i = 0; i < 4; ++i) {
+            packed[i] = (uint32_t)first << 16 | cnt[i];
+            crowded |= first < kk && cnt[i] > (uint32_t)kCrowd;
+            first += (int)cnt[i];
+        }
+        *mine = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+        if (division == 0) mark_ends(packed, 0, 1, 0);
+        return __syncthreads_or(crowded);
     }
-    __syncthreads();
-    const uint4 c = reinterpret_cast<const uint4*>(bins)[tid];
-    int n_valid;
-    const int before = scan_wg<NT>((int)(c.x + c.y + c.z + c.w), wsum, &n_valid);
-    const int kk = n_valid < a.topk ? n_valid : a.topk;
-    // (first place << 16 | entries) per bin; both fit: a row on this path has at most 16384 candidates
-    const uint32_t cnt[4] = {c.x, c.y, c.z, c.w};
-    uint32_t packed[4];
-    // this workgroup's share of the places: the entries of the bins that start in [lo_at, hi_at)
-    const int share = (kk + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int lo_at = (int)blockIdx.y * share;
-    const int hi_at = lo_at >= kk ? lo_at : (lo_at + share < kk ? lo_at + share : kk);
-    int first = before, end_lo = -1, end_hi = -1;
-    bool crowded = false;
+
+    // First and last crowded bin of a division, behind a barrier.
+    __device__ __forceinline__ void crowd(const uint32_t (&packed)[4], int division, int& f, int& l)
+    {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        packed[i] = (uint32_t)first << 16 | cnt[i];
-        crowded |= first < kk && cnt[i] > (uint32_t)kCrowd;
-        if (first < lo_at) end_lo = first + (int)cnt[i];
-        if (first < hi_at) end_hi = first + (int)cnt[i];
-        first += (int)cnt[i];
+        for (int i = 0; i < 4; ++i) {
+            if ((int)(packed[i] >> 16) < kk && (packed[i] & 0xffffu) > (uint32_t)kCrowd) {
+                atomicMin(&s_int[2], division * kBins + 4 * tid + i);
+                atomicMax(&s_int[3], division * kBins + 4 * tid + i);
+            }
+        }
+        __syncthreads();
+        f = s_int[2];
+        l = s_int[3];
     }
-    reinterpret_cast<uint4*>(bins)[tid] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-    // where the last bins that start before lo_at and before hi_at end; one thread has each
-    if (before < lo_at && first >= lo_at) s_two[0] = end_lo;
-    if (before < hi_at && first >= hi_at) s_two[1] = end_hi;
-    if (__syncthreads_or(crowded)) return false;
+
+    // This workgroup's share of the places: the entries of the bins that start in [lo_at, hi_at).
+    __device__ __forceinline__ void share(int& lo_at, int& hi_at) const
+    {
+        const int n = (kk + (int)gridDim.y - 1) / (int)gridDim.y;
+        lo_at = (int)blockIdx.y * n < kk ? (int)blockIdx.y * n : kk;
+        hi_at = lo_at + n < kk ? lo_at + n : kk;
+    }
+
+    // Where the bins end that hold the places in front of lo_at and of hi_at: one thread has each.  b0 .. b1: bins
+    // that are divided again.
+    __device__ __forceinline__ void mark_ends(const uint32_t (&packed)[4], int division, int b0, int b1) const
+    {
+        int lo_at, hi_at;
+        share(lo_at, hi_at);
+        const int from = (int)(packed[0] >> 16), to = (int)(packed[3] >> 16) + (int)(packed[3] & 0xffffu);
+        if (!((from < lo_at && lo_at <= to) || (from < hi_at && hi_at <= to))) return;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-        if (kreg[e] == 0u) continue;
-        const int f = (int)(bins[bin[e]] >> 16);
-        if (f >= lo_at && f < hi_at) win[f - lo_at + at[e]] = ((unsigned long long)kreg[e] << 32) | (uint32_t)(~(uint32_t)(tid * PER + e));
-    }
-    __syncthreads();
-    const int end = s_two[1];
-    for (int i = s_two[0] + tid; i < end; i += NT) {
-        const unsigned long long x = win[i - lo_at];
-        const uint32_t k = (uint32_t)(x >> 32);
-        const int pos = (int)(~(uint32_t)x);
-        const int32_t id = a.idx ? a.idx[(int64_t)b * a.max_n + pos] : pos;
-        const uint32_t p = bins[bin_of(k)];
-        const int f = (int)(p >> 16), n = (int)(p & 0xffffu);
-        int rank = f;  // entries of the bin that go before this one come first
-        for (int j = 0; j < n; ++j) rank += win[f - lo_at + j] > x;
-        if (rank < kk) {
-            a.out_idx[(int64_t)b * a.topk + rank] = id;
-            a.out_score[(int64_t)b * a.topk + rank] = k == 1u ? __uint_as_float(0x7fc00000u) : key_score(k);
+        for (int i = 0; i < 4; ++i) {
+            const int j = division * kBins + 4 * tid + i;
+            if (j >= b0 && j <= b1) continue;
+            const int first = (int)(packed[i] >> 16), end = first + (int)(packed[i] & 0xffffu);
+            if (first < lo_at && lo_at <= end) s_int[0] = end;
+            if (first < hi_at && hi_at <= end) s_int[1] = end;
         }
     }
-    for (int t = kk + (int)blockIdx.y * NT + tid; t < a.topk; t += NT * (int)gridDim.y) {
-        a.out_idx[(int64_t)b * a.topk + t] = -1;
-        a.out_score[(int64_t)b * a.topk + t] = 0.0f;
-    }
-    return true;
-}
 
-// Any row.  Four 8-bit radix passes find the k-th largest key, winners go to LDS at slots from one
-// prefix sum (keys above the threshold, then the ties in list order), and (key, position) pairs are
-// ordered: equal-width buckets over [threshold, largest key], or bitonic networks and pairwise merges
-// where a bucket is crowded.  PER = 0: keys are re-read from memory in every phase (rows longer than
-// the registers hold).
+    // Entries to their bins' places, ranked there, and out.  bin_of(key): the entry's bin.
+    template <class BinOf>
+    __device__ __forceinline__ void finish(BinOf&& bin_of) const
+    {
+        int lo_at, hi_at;
+        share(lo_at, hi_at);
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            if (kreg[e] == 0u) continue;
+            const int f = (int)(bins[bin(e)] >> 16);
+            if (f >= lo_at && f < hi_at) win[f - lo_at + place_of(e)] = ((unsigned long long)kreg[e] << 32) | (uint32_t)(~(uint32_t)(tid * PER + e));
+        }
+        __syncthreads();
+        const int end = s_int[1];
+        for (int i = s_int[0] + tid; i < end; i += NT) {
+            const unsigned long long x = win[i - lo_at];
+            const uint32_t k = (uint32_t)(x >> 32);
+            const int pos = (int)(~(uint32_t)x);
+            const int32_t id = a.idx ? a.idx[(int64_t)b * a.max_n + pos] : pos;
+            const uint32_t p = bins[bin_of(k)];
+            const int f = (int)(p >> 16), n = (int)(p & 0xffffu);
+            int rank = f;  // entries of the bin that go before this one come first
+            for (int j = 0; j < n; ++j) rank += win[f - lo_at + j] > x;
+            if (rank < kk) {
+                a.out_idx[(int64_t)b * a.topk + rank] = id;
+                a.out_score[(int64_t)b * a.topk + rank] = out_of(k);
+            }
+        }
+        for (int t = kk + (int)blockIdx.y * NT + tid; t < a.topk; t += NT * (int)gridDim.y) {
+            a.out_idx[(int64_t)b * a.topk + t] = -1;
+            a.out_score[(int64_t)b * a.topk + t] = 0.0f;
+        }
+    }
+
+    __device__ __forceinline__ bool run()
+    {
+        reinterpret_cast<uint4*>(bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
+        if (tid < 4) s_int[tid] = tid == 2 ? (1 + kAgain) * kBins : (tid == 3 ? -1 : 0);
+        uint32_t hi, lo;
+        range_of([](int) { return true; }, hi, lo);
+        const Bins<kBins> whole(hi, lo);
+        // 64 lanes adding to one LDS word serialise: where the wave's first keys share a bin, so may the others,
+        // and one lane adds for all that have its own (a row that one infinite score crowds into a bin: 4 us less)
+#pragma unroll
+        for (int e = 0; e < PER; ++e) set(e, (uint32_t)whole.of(kreg[e]), 0u);
+        const int bin0 = __builtin_amdgcn_readfirstlane(bin(0));
+        if (__ballot(kreg[0] != 0u && bin(0) == bin0) == ~0ull) {
+            const unsigned long long before = (1ull << lane) - 1;
+#pragma unroll
+            for (int e = 0; e < PER; ++e) {
+                const unsigned long long same = __ballot(kreg[e] != 0u && bin(e) == bin0);
+                uint32_t base = 0u;
+                if (lane == 0) base = atomicAdd(&bins[bin0], (uint32_t)__popcll(same));
+                base = __builtin_amdgcn_readfirstlane(base);
+                if (same >> lane & 1) set(e, (uint32_t)bin(e), base + (uint32_t)__popcll(same & before));
+                else if (kreg[e] != 0u) set(e, (uint32_t)bin(e), atomicAdd(&bins[bin(e)], 1u));
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < PER; ++e)
+                if (kreg[e] != 0u) set(e, (uint32_t)bin(e), atomicAdd(&bins[bin(e)], 1u));
+        }
+        __syncthreads();
+        uint32_t packed[4];
+        if (place(0, 0, packed)) return run_again(whole, packed);
+        finish([&](uint32_t k) { return whole.of(k); });
+        return true;
+    }
+
+    __device__ __forceinline__ bool run_again(const Bins<kBins>& whole, const uint32_t (&packed0)[4])
+    {
+        uint32_t packed[1 + kAgain][4];
+        int b0[1 + kAgain], b1[1 + kAgain];  // per division: its bins that are divided again
+        Bins<kBins> part[1 + kAgain] = {whole, whole, whole};
+        static_assert(kAgain == 2, "");
+#pragma unroll
+        for (int i = 0; i < 4; ++i) packed[0][i] = packed0[i];
+        bool crowded = true;
+#pragma unroll
+        for (int d = 1; d <= kAgain; ++d) {
+            b0[d] = (1 + kAgain) * kBins;
+            b1[d] = -1;
+            if (!crowded) continue;
+            int f, l;
+            crowd(packed[d - 1], d - 1, f, l);
+            b0[d - 1] = f;
+            b1[d - 1] = l;
+            reinterpret_cast<uint4*>(bins + d * kBins)[tid] = make_uint4(0u, 0u, 0u, 0u);
+            uint32_t hi, lo;
+            range_of([&](int e) { return bin(e) >= f && bin(e) <= l; }, hi, lo);
+            if (hi == lo) return false;  // ties
+            part[d] = Bins<kBins>(hi, lo);
+            // every thread has read the last two: range_of() has a barrier
+            if (tid < 4) s_int[tid] = tid == 2 ? (1 + kAgain) * kBins : (tid == 3 ? -1 : 0);
+#pragma unroll
+            for (int e = 0; e < PER; ++e) {
+                if (kreg[e] == 0u || bin(e) < f || bin(e) > l) continue;
+                const uint32_t j = (uint32_t)(d * kBins + part[d].of(kreg[e]));
+                set(e, j, atomicAdd(&bins[j], 1u));
+            }
+            __syncthreads();
+            crowded = place(d, (int)(bins[f] >> 16), packed[d]);
+        }
+        if (crowded) return false;
+#pragma unroll
+        for (int d = 0; d <= kAgain; ++d)
+            if (d == 0 || b0[d - 1] <= b1[d - 1]) mark_ends(packed[d], d, b0[d], b1[d]);
+        finish([&](uint32_t k) {
+            int j = whole.of(k);
+#pragma unroll
+            for (int d = 1; d <= kAgain; ++d)
+                if (j >= b0[d - 1] && j <= b1[d - 1]) j = d * kBins + part[d].of(k);
+            return j;
+        });
+        return true;
+    }
+};
+
+// Any row.  Radix passes of 10 or 11 bits find the k-th largest key, winners go to LDS at slots from one
+// prefix sum (keys above the threshold, then the ties in list order), and the (key, position) pairs above the
+// threshold are ordered: equal-width buckets over (threshold, largest key], or bitonic networks and pairwise
+// merges where a bucket is crowded.  PER = 0: keys are re-read from memory in every phase (rows longer than
+// the registers hold).  Where the direct path was tried in vain, three passes instead of four of 8 bits, no
+// ordering of the ties and no second count of the candidates pay for it: two rows of 4000 candidates, k = 1200,
+// all scores equal 16.5 us for the call (34.4 with four passes and no attempt in front), four different ones
+// 35.5 (35.9).
+// lds: 4 NT words, then the winners (a.cap of 8 bytes).  n_valid: candidates of the row, -1 = not known.
 template <int NT, int PER>
-__device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER : 1], uint32_t* lds,
-                            unsigned long long* win, int* wsum, int* s_two)
+__device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER : 1], uint32_t* lds, int* wsum, int* s_two,
+                            int n_valid)
 {
     constexpr bool REG = PER > 0;
     constexpr int kBuckets = NT;  // one per thread
-    int* hist = reinterpret_cast<int*>(lds);        // 256
+    constexpr int kDigitBits = NT >= 512 ? 11 : 10, kPerThread = (1 << kDigitBits) / NT;
+    static_assert(kPerThread >= 1 && (1 << kDigitBits) <= 4 * NT, "");
+    unsigned long long* win = reinterpret_cast<unsigned long long*>(lds + 4 * NT);
+    int* hist = reinterpret_cast<int*>(lds);
     int* bcount = reinterpret_cast<int*>(lds);      // kBuckets each, after the search
     int* bfill = bcount + kBuckets;
     int* bbase = bfill + kBuckets;
@@ -226,22 +402,24 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
         }
     };
 
-    // candidates present
-    int mine = 0;
-    for_chunks([&](int, uint32_t k) { mine += k != 0u; });
-    int n_valid;
-    (void)scan_wg<NT>(mine, wsum, &n_valid);
+    if (n_valid < 0) {
+        int mine = 0;
+        for_chunks([&](int, uint32_t k) { mine += k != 0u; });
+        (void)scan_wg<NT>(mine, wsum, &n_valid);
+    }
     const int kk = n_valid < a.topk ? n_valid : a.topk;
 
-    // ---- radix search, 8 bits a pass, for the kk-th largest key among the candidates ----
+    // ---- radix search for the kk-th largest key among the candidates ----
     uint32_t prefix = 0, mask = 0;
     int need = kk;
-    for (int shift = 24; shift >= 0 && kk > 0; shift -= 8) {
-        if (tid < 256) hist[tid] = 0;
+    for (int below = 32; below > 0 && kk > 0;) {  // bits not known yet
+        const int bits = below < kDigitBits ? below : kDigitBits, shift = below - bits, last = (1 << bits) - 1;
+#pragma unroll
+        for (int j = 0; j < kPerThread; ++j) hist[tid + j * NT] = 0;
         __syncthreads();
         for_chunks([&](int, uint32_t k) {
             const bool in = k != 0u && (k & mask) == prefix;
-            const int d = (k >> shift) & 255;
+            const int d = (k >> shift) & last;
             // scores of one magnitude share their leading digits: when a whole wave holds one
             // digit its first lane adds the count (64 lanes adding to one LDS word serialise)
             const unsigned long long act = __ballot(in);
@@ -256,19 +434,29 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
             }
         });
         __syncthreads();
-        // digits in descending order, one per thread: the chosen digit is where the running
+        // digits in descending order, kPerThread to a thread: the chosen digit is where the running
         // count first reaches `need`
-        const int cnt = tid < 256 ? hist[255 - tid] : 0;
-        int all;
-        const int before = scan_wg<NT>(cnt, wsum, &all);
-        if (tid < 256 && before < need && before + cnt >= need) {
-            s_two[0] = 255 - tid;
-            s_two[1] = need - before;  // still to take among keys with this digit
+        int cnt[kPerThread], sum = 0, all;
+#pragma unroll
+        for (int j = 0; j < kPerThread; ++j) {
+            const int d = last - (tid * kPerThread + j);
+            cnt[j] = d >= 0 ? hist[d] : 0;
+            sum += cnt[j];
+        }
+        int before = scan_wg<NT>(sum, wsum, &all);
+#pragma unroll
+        for (int j = 0; j < kPerThread; ++j) {
+            if (before < need && before + cnt[j] >= need) {
+                s_two[0] = last - (tid * kPerThread + j);
+                s_two[1] = need - before;  // still to take among keys with this digit
+            }
+            before += cnt[j];
         }
         __syncthreads();
         prefix |= (uint32_t)s_two[0] << shift;
-        mask |= 255u << shift;
+        mask |= (uint32_t)last << shift;
         need = s_two[1];
+        below = shift;
         __syncthreads();
     }
     const uint32_t thr = prefix;  // the kk-th largest key; `need` of the keys equal to it are taken
@@ -322,110 +510,62 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
     }
     __syncthreads();
 
-    // ---- order the winners, descending: larger key first, then smaller position ----
-    // The winners' keys lie in [thr, kmax]; equal-width buckets over that range (descending), a
-    // prefix sum over the bucket counts, every winner dropped into its bucket, then ranked among the
-    // few entries that share it.
-    constexpr int kPer = REG && NT * PER < kMaxTopk ? PER : kMaxTopk / NT;  // entries per thread at the largest cap
-    uint32_t kmax = 0u;
-    unsigned long long x[kPer];
-#pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-        const int i = tid + e * NT;
-        x[e] = i < kk ? win[i] : 0ull;
-        const uint32_t k = (uint32_t)(x[e] >> 32);
-        kmax = k > kmax ? k : kmax;
-    }
-    kmax = wave_max(kmax);
-    bcount[tid] = 0;
-    bfill[tid] = 0;
-    if (lane == 0) wsum[tid >> 6] = (int)kmax;
-    __syncthreads();
-    for (int w = 0; w < NT / 64; ++w) kmax = (uint32_t)wsum[w] > kmax ? (uint32_t)wsum[w] : kmax;
-    const uint32_t range = kmax > thr ? kmax - thr : 0u;
-    const int bits = range ? 32 - __builtin_clz(range) : 0;
-    constexpr int kBucketBits = __builtin_ctz(kBuckets);
-    const int bshift = bits > kBucketBits ? bits - kBucketBits : 0;
-    int bucket[kPer];
-#pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-        const int i = tid + e * NT;
-        bucket[e] = -1;
-        if (i < kk) {
-            bucket[e] = (kBuckets - 1) - (int)(((uint32_t)(x[e] >> 32) - thr) >> bshift);
-            atomicAdd(&bcount[bucket[e]], 1);
-        }
-    }
-    __syncthreads();
-    const int my_count = bcount[tid];
-    int all_winners;
-    const int my_base = scan_wg<NT>(my_count, wsum, &all_winners);
-    const bool crowded = __syncthreads_or(my_count > kBucketMax);
-    if (!crowded) {
-        bbase[tid] = my_base;
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < kPer; ++e)
-            if (bucket[e] >= 0) win[bbase[bucket[e]] + atomicAdd(&bfill[bucket[e]], 1)] = x[e];
-        __syncthreads();
-        int dst[kPer];
+    // ---- order the winners above the threshold, descending: larger key first, then smaller position (the
+    //      ties behind them are in list order already) ----
+    // Their keys lie in (thr, kmax]; equal-width buckets over that range (descending), a prefix sum over the
+    // bucket counts, every winner dropped into its bucket, then ranked among the few entries that share it.
+    if (n_gt > 1) {
+        constexpr int kPer = REG && NT * PER < kMaxTopk ? PER : kMaxTopk / NT;  // entries per thread at the largest cap
+        uint32_t kmax = 0u;
+        unsigned long long x[kPer];
 #pragma unroll
         for (int e = 0; e < kPer; ++e) {
-            dst[e] = -1;
-            if (bucket[e] >= 0) {
-                const int first = bbase[bucket[e]], n = bcount[bucket[e]];
-                int ahead = 0;  // entries of the bucket that go before this one
-                for (int j = 0; j < n; ++j) ahead += win[first + j] > x[e];
-                dst[e] = first + ahead;
-            }
+            const int i = tid + e * NT;
+            x[e] = i < n_gt ? win[i] : 0ull;
+            const uint32_t k = (uint32_t)(x[e] >> 32);
+            kmax = k > kmax ? k : kmax;
         }
+        kmax = wave_max(kmax);
+        bcount[tid] = 0;
+        bfill[tid] = 0;
+        if (lane == 0) wsum[tid >> 6] = (int)kmax;
         __syncthreads();
+        for (int w = 0; w < NT / 64; ++w) kmax = (uint32_t)wsum[w] > kmax ? (uint32_t)wsum[w] : kmax;
+        const uint32_t range = kmax > thr ? kmax - thr : 0u;
+        const int bits = range ? 32 - __builtin_clz(range) : 0;
+        constexpr int kBucketBits = __builtin_ctz(kBuckets);
+        const int bshift = bits > kBucketBits ? bits - kBucketBits : 0;
+        int bucket[kPer];
 #pragma unroll
-        for (int e = 0; e < kPer; ++e)
-            if (dst[e] >= 0) win[dst[e]] = x[e];
-        __syncthreads();
-    } else {
-        // (a) bitonic networks over aligned segments of 256 entries, every segment descending;
-        // (b) sorted runs merged pairwise: an entry's place in the merged run is its place in its
-        //     own run plus the number of entries of the sibling run that go before it (binary
-        //     search; the left run wins ties, which only the empty slots have).  For 4096 entries
-        //     that is 36 + 2 * 4 barriers where one network over everything takes 78.
-        const int seg = a.cap < 256 ? a.cap : 256;
-        for (int size = 2; size <= seg; size <<= 1) {
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                for (int t = tid; t < a.cap / 2; t += NT) {
-                    const int lo = 2 * t - (t & (stride - 1));
-                    const int hi = lo + stride;
-                    const bool desc = size == seg || (lo & size) == 0;
-                    const unsigned long long p = win[lo], q = win[hi];
-                    if ((p < q) == desc) {
-                        win[lo] = q;
-                        win[hi] = p;
-                    }
-                }
-                __syncthreads();
+        for (int e = 0; e < kPer; ++e) {
+            const int i = tid + e * NT;
+            bucket[e] = -1;
+            if (i < n_gt) {
+                bucket[e] = (kBuckets - 1) - (int)(((uint32_t)(x[e] >> 32) - thr) >> bshift);
+                atomicAdd(&bcount[bucket[e]], 1);
             }
         }
-        for (int run = seg; run < a.cap; run <<= 1) {
+        __syncthreads();
+        const int my_count = bcount[tid];
+        int all_winners;
+        const int my_base = scan_wg<NT>(my_count, wsum, &all_winners);
+        const bool crowded = __syncthreads_or(my_count > kBucketMax);
+        if (!crowded) {
+            bbase[tid] = my_base;
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < kPer; ++e)
+                if (bucket[e] >= 0) win[bbase[bucket[e]] + atomicAdd(&bfill[bucket[e]], 1)] = x[e];
+            __syncthreads();
             int dst[kPer];
-            const int sh = __builtin_ctz(run);
 #pragma unroll
             for (int e = 0; e < kPer; ++e) {
-                const int i = tid + e * NT;
                 dst[e] = -1;
-                if (i < a.cap) {
-                    x[e] = win[i];
-                    const int r = i >> sh, at = i & (run - 1);
-                    const unsigned long long* sib = win + (r ^ 1) * run;
-                    const bool left = (r & 1) == 0;
-                    int lo = 0, hi = run;  // entries of the sibling run that go before x[e]
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        const unsigned long long o = sib[mid];
-                        if (o > x[e] || (!left && o == x[e])) lo = mid + 1;
-                        else hi = mid;
-                    }
-                    dst[e] = (r >> 1) * 2 * run + at + lo;
+                if (bucket[e] >= 0) {
+                    const int first = bbase[bucket[e]], n = bcount[bucket[e]];
+                    int ahead = 0;  // entries of the bucket that go before this one
+                    for (int j = 0; j < n; ++j) ahead += win[first + j] > x[e];
+                    dst[e] = first + ahead;
                 }
             }
             __syncthreads();
@@ -433,6 +573,58 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
             for (int e = 0; e < kPer; ++e)
                 if (dst[e] >= 0) win[dst[e]] = x[e];
             __syncthreads();
+        } else {
+            // (a) bitonic networks over aligned segments of 256 entries, every segment descending;
+            // (b) sorted runs merged pairwise: an entry's place in the merged run is its place in its
+            //     own run plus the number of entries of the sibling run that go before it (binary
+            //     search; the left run wins ties, which only the empty slots have).  For 4096 entries
+            //     that is 36 + 2 * 4 barriers where one network over everything takes 78.
+            int cap = 2;  // entries of the networks: the ties that fall inside stay behind all others, in their order
+            while (cap < n_gt) cap <<= 1;
+            const int seg = cap < 256 ? cap : 256;
+            for (int size = 2; size <= seg; size <<= 1) {
+                for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                    for (int t = tid; t < cap / 2; t += NT) {
+                        const int lo = 2 * t - (t & (stride - 1));
+                        const int hi = lo + stride;
+                        const bool desc = size == seg || (lo & size) == 0;
+                        const unsigned long long p = win[lo], q = win[hi];
+                        if ((p < q) == desc) {
+                            win[lo] = q;
+                            win[hi] = p;
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
+            for (int run = seg; run < cap; run <<= 1) {
+                int dst[kPer];
+                const int sh = __builtin_ctz(run);
+#pragma unroll
+                for (int e = 0; e < kPer; ++e) {
+                    const int i = tid + e * NT;
+                    dst[e] = -1;
+                    if (i < cap) {
+                        x[e] = win[i];
+                        const int r = i >> sh, at = i & (run - 1);
+                        const unsigned long long* sib = win + (r ^ 1) * run;
+                        const bool left = (r & 1) == 0;
+                        int lo = 0, hi = run;  // entries of the sibling run that go before x[e]
+                        while (lo < hi) {
+                            const int mid = (lo + hi) >> 1;
+                            const unsigned long long o = sib[mid];
+                            if (o > x[e] || (!left && o == x[e])) lo = mid + 1;
+                            else hi = mid;
+                        }
+                        dst[e] = (r >> 1) * 2 * run + at + lo;
+                    }
+                }
+                __syncthreads();
+#pragma unroll
+                for (int e = 0; e < kPer; ++e)
+                    if (dst[e] >= 0) win[dst[e]] = x[e];
+                __syncthreads();
+            }
         }
     }
 
@@ -443,55 +635,100 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
             const int pos = (int)(~(uint32_t)(win[t] & 0xffffffffull));
             const uint32_t k = (uint32_t)(win[t] >> 32);
             oi = a.idx ? a.idx[(int64_t)b * a.max_n + pos] : pos;
-            os = k == 1u ? __uint_as_float(0x7fc00000u) : key_score(k);
+            os = out_of(k);
         }
         a.out_idx[(int64_t)b * a.topk + t] = oi;
         a.out_score[(int64_t)b * a.topk + t] = os;
     }
 }
 
-// grid = (rows, workgroups per row); dynamic LDS: the winners' array.  Thread t holds list positions t * PER ..
+// Short rows: every candidate counts those that come before it in the output order (larger key, or equal key
+// and earlier position) and writes itself at that rank.  Its time does not depend on the values.  A workgroup
+// ranks 64 candidates; its four waves compare them with every fourth 64 entries of the row, which a wave holds
+// in a register and hands round lane by lane.  grid = (rows, ceil(max_n / 64)).
+constexpr int kRankRow = 512;
+__global__ __launch_bounds__(256) void topk_rank_kernel(SortArgs a)
+{
+    __shared__ int part[4][64], valid[4];
+    const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, mine_at = blockIdx.y;
+    const uint32_t* keys = a.keys + b * a.pitch;
+    const int pos = mine_at * 64 + lane;
+    const uint32_t mine = pos < a.max_n ? keys[pos] : 0u;
+    const int32_t id = w == 0 && a.idx && pos < a.max_n ? a.idx[(int64_t)b * a.max_n + pos] : pos;
+    int rank = 0, have = 0;
+    for (int piece = w; piece * 64 < a.max_n; piece += 4) {
+        const uint32_t k = piece * 64 + lane < a.max_n ? keys[piece * 64 + lane] : 0u;
+        have += __popcll(__ballot(k != 0u));
+        if (piece == mine_at) {
+#pragma unroll
+            for (int j = 0; j < 64; ++j) {
+                const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)k, j);
+                rank += o > mine || (o == mine && j < lane);
+            }
+        } else {
+            // equal keys come first where they lie in front: o >= mine is o > mine - 1 (mine is 0 for nothing only)
+            const uint32_t above = mine - (piece < mine_at ? 1u : 0u);
+#pragma unroll
+            for (int j = 0; j < 64; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)k, j) > above;
+        }
+    }
+    part[w][lane] = rank;
+    if (lane == 0) valid[w] = have;
+    __syncthreads();
+    if (w != 0) return;
+    rank = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+    if (mine != 0u && rank < a.topk) {
+        a.out_idx[(int64_t)b * a.topk + rank] = id;
+        a.out_score[(int64_t)b * a.topk + rank] = out_of(mine);
+    }
+    for (int t = valid[0] + valid[1] + valid[2] + valid[3] + pos; t < a.topk; t += 64 * (int)gridDim.y) {
+        a.out_idx[(int64_t)b * a.topk + t] = -1;
+        a.out_score[(int64_t)b * a.topk + t] = 0.0f;
+    }
+}
+
+// LDS of topk_kernel: bins and winners, as the two paths lay them out.
+constexpr size_t direct_lds(int nt) { return (size_t)nt * 48 + (size_t)(nt + kCrowd) * 8; }
+constexpr size_t search_lds(int nt, int cap) { return (size_t)nt * 16 + (size_t)cap * 8; }
+
+// grid = (rows, workgroups per row).  Thread t holds list positions t * PER ..
 // t * PER + PER - 1 (consecutive, so that one prefix sum over per-thread counts orders the list).
 template <int NT, int PER>
 __global__ __launch_bounds__(NT) void topk_kernel(SortArgs a)
 {
-    extern __shared__ unsigned long long win[];  // [cap] (key << 32) | ~position
-    __shared__ __align__(16) uint32_t bins[4 * NT];
+    extern __shared__ __align__(16) uint32_t lds[];
     __shared__ int wsum[NT / 64];
     __shared__ uint32_t range[2][NT / 64];
-    __shared__ int s_two[2];
+    __shared__ int s_int[4];
     if constexpr (PER > 0) {
-        static_assert(PER == 1 || PER % 4 == 0, "16-byte loads");
+        static_assert(PER % 4 == 0, "16-byte loads");
         uint32_t kreg[PER];
         const uint32_t* keys = a.keys + blockIdx.x * a.pitch;
         const int first = threadIdx.x * PER;
-        if constexpr (PER == 1) {
-            kreg[0] = first < a.max_n ? keys[first] : 0u;
-        } else {
 #pragma unroll
-            for (int e = 0; e < PER; e += 4) {
-                uint4 v = make_uint4(0u, 0u, 0u, 0u);  // a row's last piece may reach into its padding
-                if (first + e < a.max_n) v = *reinterpret_cast<const uint4*>(keys + first + e);
-                kreg[e] = v.x;
-                kreg[e + 1] = first + e + 1 < a.max_n ? v.y : 0u;
-                kreg[e + 2] = first + e + 2 < a.max_n ? v.z : 0u;
-                kreg[e + 3] = first + e + 3 < a.max_n ? v.w : 0u;
-            }
+        for (int e = 0; e < PER; e += 4) {
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);  // a row's last piece may reach into its padding
+            if (first + e < a.max_n) v = *reinterpret_cast<const uint4*>(keys + first + e);
+            kreg[e] = v.x;
+            kreg[e + 1] = first + e + 1 < a.max_n ? v.y : 0u;
+            kreg[e + 2] = first + e + 2 < a.max_n ? v.z : 0u;
+            kreg[e + 3] = first + e + 3 < a.max_n ? v.w : 0u;
         }
-        if (topk_direct<NT, PER>(a, kreg, bins, win, wsum, range, s_two)) return;
+        Direct<NT, PER> direct(a, kreg, lds, wsum, range, s_int);
+        if (direct.run()) return;
         if (blockIdx.y != 0) return;  // every workgroup of the row sees the same bins; one searches
         __syncthreads();
-        topk_search<NT, PER>(a, kreg, bins, win, wsum, s_two);
+        topk_search<NT, PER>(a, kreg, lds, wsum, s_int, direct.n_valid);
     } else {
         const uint32_t none[1] = {0u};
-        topk_search<NT, 0>(a, none, bins, win, wsum, s_two);
+        topk_search<NT, 0>(a, none, lds, wsum, s_int, -1);
     }
 }
 
 template <int NT, int PER>
 inline int launch_topk_as(SortArgs s, int rows, hipStream_t st)
 {
-    // the search sorts a power of two of entries; the direct path needs room for the bin that crosses place k
+    // the search sorts a power of two of entries
     const int most = s.topk < s.max_n ? s.topk : s.max_n;
     int cap = 2;
     while (cap < most) cap <<= 1;
@@ -499,18 +736,25 @@ inline int launch_topk_as(SortArgs s, int rows, hipStream_t st)
     // Workgroups per row: one for every NT places.  Each counts the whole row (the keys come from the L2)
     // and orders its share of the places, one entry per thread.
     const int split = PER > 0 ? (int)ucm::ceil_div(most, NT) : 1;
-    hipLaunchKernelGGL((topk_kernel<NT, PER>), dim3((unsigned)rows, (unsigned)split), dim3(NT),
-                       (size_t)(cap > NT + kCrowd ? cap : NT + kCrowd) * 8, st, s);
+    const size_t need = search_lds(NT, cap), direct = PER > 0 ? direct_lds(NT) : 0;
+    static_assert(search_lds(NT, kMaxTopk) + 512 <= 64 * 1024 && direct_lds(NT) + 512 <= 64 * 1024, "");
+    hipLaunchKernelGGL((topk_kernel<NT, PER>), dim3((unsigned)rows, (unsigned)split), dim3(NT), need > direct ? need : direct, st, s);
     return ucm::launch_status("topk_kernel");
 }
 
+// Rows of up to 512 candidates are ranked: as fast as the direct path on an even row (two rows, whole call: 253
+// candidates 6.0 against 5.8 us, 400: 6.7 and 6.4, 700: 7.5 and 6.9) and faster on one that crowds (400: 8.9 with a
+// second division, 11 to 18 with the search).
 // Threads by row length: few where the row fits (a barrier of 4 waves costs less than one of 16: 1000
 // candidates as 256 x 4 keys 6.5 us for the whole retrieval call of two short rows, as 1024 x 1 7.1 us;
 // 4000 as 512 x 8 and as 1024 x 4 8.3 and 8.5 us), 1024 from where 512 would hold 16 keys each (8000:
 // 11.2 us of selection against 8.1 us).
 inline int launch_topk(const SortArgs& s, int rows, hipStream_t st)
 {
-    if (s.max_n <= 256) return launch_topk_as<256, 1>(s, rows, st);
+    if (s.max_n <= kRankRow) {
+        hipLaunchKernelGGL(topk_rank_kernel, dim3((unsigned)rows, (unsigned)ucm::ceil_div(s.max_n, 64)), dim3(256), 0, st, s);
+        return ucm::launch_status("topk_rank_kernel");
+    }
     if (s.max_n <= 1024) return launch_topk_as<256, 4>(s, rows, st);
     if (s.max_n <= 4096) return launch_topk_as<512, 8>(s, rows, st);
     if (s.max_n <= 8192) return launch_topk_as<1024, 8>(s, rows, st);
