@@ -89,10 +89,19 @@ int ucm_hash_encode_cache(const void* x, int x_dtype, int64_t T, int32_t H, int3
  * Tuning and test hook, no counterpart in the reference.  Inputs of at least `rows` rows (tokens x
  * heads) with 64 or 128 input dimensions and 64 or 128 hash bits take the streaming kernel
  * (persistent waves, projection matrix in registers, rows loaded straight into LDS); smaller ones
- * take the tiled kernel.  Both give identical codes.  rows <= 0 restores the default (2^20).  The
- * setting belongs to the calling thread: encodes issued by other threads are not affected.
+ * take the tiled kernel.  Both give identical codes.  rows <= 0 restores the defaults (81,920 for 64 dimensions
+ * and 64 bits, 786,432 for the others).  The setting belongs to the calling thread: encodes issued by other threads are not affected.
  */
 int ucm_hash_encode_set_stream_threshold(int64_t rows);
+
+/*
+ * Test hook, no counterpart in the reference.  Writes the name of the kernel that the last ucm_hash_encode,
+ * ucm_hash_encode_cache or ucm_hash_encode_paged on the calling thread launched, e.g. "encode_small",
+ * "encode_mfma<4,1,8>" (column tiles per group, groups per slice, row tiles per workgroup) or
+ * "encode_slice<2>" (column tiles per slice), cut to cap - 1 characters.  Returns the full length.  The kernels
+ * give the same codes at very different speeds; this lets a test pin which one a shape takes.
+ */
+int64_t ucm_hash_encode_last_dispatch(char* buf, size_t cap);
 
 /*
  * Measurement aid, no counterpart in the reference.  While a non-null address is set, every launch

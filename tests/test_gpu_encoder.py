@@ -463,3 +463,23 @@ def test_row_tiles_per_workgroup(K, N, H, T, paged):
     xs = x[pick].float().cpu().numpy()
     for h in range(H):
         assert_codes_match(got[:, h], xs[:, h], W.float().numpy())
+
+
+def _encode_route(K, N, H, T):
+    """The kernel that a plain encode into a paged cache takes."""
+    from ucm_amd import _lib
+
+    enc = make_encoder(K, N, torch.bfloat16, torch.ones(K, N, dtype=torch.bfloat16))
+    nb = -(-T // 64)
+    cache = torch.zeros((nb, 64, H, N // 32), dtype=torch.int32, device="cuda")
+    enc.compute_hash_and_cache(torch.ones(T, H, K, dtype=torch.bfloat16, device="cuda"), torch.arange(T, device="cuda"), cache,
+                               block_size=64)
+    return _lib.last_encode()
+
+
+@pytest.mark.parametrize("K,N,T", [(64, 96, 1300), (64, 192, 1700), (64, 320, 1300), (64, 512, 800), (128, 96, 2200),
+                                   (128, 160, 1000), (128, 192, 2200), (128, 224, 1700), (128, 384, 1300), (128, 512, 2500)])
+def test_column_counts_without_a_one_tile_form_keep_the_small_kernel(K, N, T):
+    """The tiled kernel has one row tile per workgroup for slices of 32, 64, 128 and 256 columns only; with four
+    it took 1.3 to 2.9 times the small kernel's time at these sizes."""
+    assert _encode_route(K, N, 8, T) == "encode_small"

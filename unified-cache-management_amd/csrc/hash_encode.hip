@@ -1835,6 +1835,14 @@ __global__ __launch_bounds__(kThreads) void code_scatter_kernel(const uint32_t* 
     }
 }
 
+// Which kernel the last encode on this thread launched (ucm_hash_encode_last_dispatch).
+struct EncNote {
+    const char* family;
+    int p[3];  // -1 = unused
+};
+thread_local EncNote t_note = {nullptr, {-1, -1, -1}};
+void note_encode(const char* family, int a = -1, int b = -1, int c = -1) { t_note = EncNote{family, {a, b, c}}; }
+
 // Widest slice of hash columns (a multiple of 32 that divides N) whose transposed LDS image
 // stays within `cap` bytes; 0 when not even 32 columns fit.
 int pick_slice(int N, int K, size_t cap)
@@ -1843,6 +1851,9 @@ int pick_slice(int N, int K, size_t cap)
         if (N % bn == 0 && (size_t)bn * (K + kPad) * 2 <= cap) return bn;
     return 0;
 }
+
+// Whether launch_mfma_q() has one row tile per workgroup to offer for slices of bn columns.
+bool one_tile_form(int K, int bn) { return K <= 128 && (bn == 32 || bn == 64 || bn == 128 || bn == 256); }
 
 int stream_workgroups();
 
@@ -1861,6 +1872,7 @@ int launch_mfma_t(const EncArgs& a, size_t lds, const dim3& grid, hipStream_t st
         }
         if (big_lds < 0) return UCM_EUNSUPPORTED;
     }
+    note_encode("encode_mfma", NQ, NG, TPW);
     hipLaunchKernelGGL((encode_mfma_kernel<V, KS, NQ, NG, TPW>), grid, dim3(kMfmaThreads), lds, st, a);
     return ucm::launch_status("encode_mfma_kernel");
 }
@@ -1929,6 +1941,7 @@ int launch_slice_nt(const EncArgs& a, hipStream_t st)
     int64_t streams = (int64_t)stream_workgroups() * (NT == 4 ? 1 : 2) / units;
     if (streams < 1) streams = 1;
     if (streams > tiles) streams = tiles;
+    note_encode("encode_slice", NT);
     hipLaunchKernelGGL((encode_slice_kernel<V, NT>), dim3((unsigned)streams, (unsigned)(a.N / (32 * NT)), (unsigned)a.H),
                        dim3(kMfmaThreads), lds, st, a);
     return ucm::launch_status("encode_slice_kernel");
@@ -2048,6 +2061,7 @@ int launch_stream_a(const EncArgs& a, hipStream_t st)
     if ((wgs * kStreamWaves) % a.H) return UCM_EUNSUPPORTED;
     const int nstreams = wgs * kStreamWaves / a.H;
     const int64_t ntiles = ucm::ceil_div(a.T, kRowsPerWave);
+    note_encode("encode_stream");
     hipLaunchKernelGGL((encode_stream_kernel<V, KS, NT, SLOT, ACCS, HC>), dim3((unsigned)wgs), dim3(kStreamThreads),
                        lds, st, a, ntiles, nstreams);
     return ucm::launch_status("encode_stream_kernel");
@@ -2123,6 +2137,7 @@ int launch_wide_s(const EncArgs& a, hipStream_t st)
     const int64_t ntiles = ucm::ceil_div(a.T, kRowsPerWave);
     // one workgroup per compute unit and slice of 256 hash columns; a second slice is a second pass
     // over the rows (two slices side by side, meeting in L2, measured the same)
+    note_encode("encode_wide");
     for (int c = 0; c < ncol; ++c)
         hipLaunchKernelGGL((encode_wide_kernel<V, SLOT>), dim3((unsigned)wgs), dim3(kWideThreads), kWideLds, st, a,
                            ntiles, wgs, c, t_clock_probe);
@@ -2146,6 +2161,7 @@ template <typename V>
 int launch_small(const EncJobs& js, int64_t waves, int K, hipStream_t st)
 {
     const dim3 grid((unsigned)waves);
+    note_encode("encode_small");
     switch (K) {
         case 64: hipLaunchKernelGGL((encode_small_kernel<V, 4>), grid, dim3(64), 0, st, js); break;
         case 128: hipLaunchKernelGGL((encode_small_kernel<V, 8>), grid, dim3(64), 0, st, js); break;
@@ -2284,6 +2300,7 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
 {
     const int tn = a.N % 128 == 0 ? 128 : (a.N % 64 == 0 ? 64 : 32);
     const dim3 grid((unsigned)ucm::ceil_div(a.T, 64), (unsigned)(a.N / tn), (unsigned)a.H);
+    note_encode("encode_tiled", tn);
     if (tn == 128) hipLaunchKernelGGL((encode_tiled_kernel<DT, 128>), grid, dim3(kThreads), 0, st, a);
     else if (tn == 64) hipLaunchKernelGGL((encode_tiled_kernel<DT, 64>), grid, dim3(kThreads), 0, st, a);
     else hipLaunchKernelGGL((encode_tiled_kernel<DT, 32>), grid, dim3(kThreads), 0, st, a);
@@ -2296,8 +2313,10 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
 // first (64 x 64: 4.4 us, 128 x 128: 5.1 us).  Measured: 128 -> 128 bits, 8 heads, 300 tokens 4.2 against
 // 4.7 us, 1024 tokens 5.6 against 4.6, 2048 tokens 7.3 against 4.8; one head, 4096 tokens 4.1 against 4.5,
 // 8192 tokens 5.2 against 4.6; 64 -> 64 bits, 8 heads, 600 tokens 3.6 against 3.9, 2048 tokens 4.7 against
-// 4.0.  Rows of 256 values are not pipelined and run four tiles a workgroup: 6 us plus 0.13 us per KiB
-// (256 -> 256 with 4 heads: equal at ~5000-6000 rows).  Rows of 512 values have the slice kernel: 7 us until
+// 4.0.  Where the kernel is not pipelined (rows of 256 values; slices of other than 32, 64, 128 and 256 columns,
+// see launch_mfma_q) it runs four tiles a workgroup: 6 us plus 0.13 us per KiB (256 -> 256 with 4 heads: equal at
+// ~5000-6000 rows; 128 -> 192, 8 heads: 1000 tokens 6.0 against 12.2 us, 4000 14.0 against 13.9; 128 -> 512: 1000
+// 9.8 against 21.9, 3000 20.2 against 23.5).  Rows of 512 values have the slice kernel: 7 us until
 // it fills the chip (512 -> 512: equal at ~1100 rows; 1000: 6.3 against 6.8 us, 1500: 8.3 against 7.0 us).
 //
 // alone = false: a job of a decode step, where the other kernels are a launch more for every job (new keys
@@ -2311,7 +2330,9 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype, bool alone = tru
     const int bn = pick_slice(a.N, a.K, (size_t)160 * 1024 - kStage);
     if (bn == 0) return true;
     const double slice_kib = (double)bn * (a.K + kPad) * 2 / 1024.0;
-    const double lds_floor_us = !alone ? 6.0 + 0.13 * slice_kib : a.K == 16 * kSliceKS ? 7.5 : a.K <= 128 ? 4.2 + 0.027 * slice_kib : 6.0 + 0.13 * slice_kib;
+    double lds_floor_us = 6.0 + 0.13 * slice_kib;
+    if (alone && a.K == 16 * kSliceKS) lds_floor_us = 7.5;
+    else if (alone && one_tile_form(a.K, bn)) lds_floor_us = 4.2 + 0.027 * slice_kib;
     const double small_us = 4.0 + (double)small_waves(a) * a.K * 12.5e-6;
     return small_us < lds_floor_us;
 }
@@ -2418,6 +2439,7 @@ int encode_common(EncArgs a, int x_dtype, int w_dtype, hipStream_t st)
     const int64_t total = a.T * a.H * (a.N / 32);
     int64_t blocks = ucm::ceil_div(total, kThreads);
     if (blocks > 65535 * 16) blocks = 65535 * 16;
+    note_encode("encode_fma");
     hipLaunchKernelGGL(encode_fma_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, a, x_dtype,
                        w_dtype);
     return ucm::launch_status("encode_fma_kernel");
@@ -2473,6 +2495,16 @@ extern "C" int ucm_hash_encode_debug_trip_stream_latch(void)
     ucm::clear_error();
     g_latch_forced[latch_device()].store(1, std::memory_order_relaxed);
     return UCM_OK;
+}
+
+extern "C" int64_t ucm_hash_encode_last_dispatch(char* buf, size_t cap)
+{
+    char tmp[64];
+    int n = snprintf(tmp, sizeof(tmp), "%s", t_note.family ? t_note.family : "");
+    for (int i = 0; i < 3 && t_note.p[i] >= 0; ++i) n += snprintf(tmp + n, sizeof(tmp) - n, "%c%d", i == 0 ? '<' : ',', t_note.p[i]);
+    if (t_note.p[0] >= 0) n += snprintf(tmp + n, sizeof(tmp) - n, ">");
+    if (buf && cap) snprintf(buf, cap, "%s", tmp);
+    return n;
 }
 
 extern "C" int ucm_hash_encode_set_stream_threshold(int64_t rows)

@@ -47,6 +47,7 @@ _SIGNATURES = {
     "ucm_hamming_topk_set_profile_events": (ci, [vp, vp]),
     "ucm_hamming_topk_set_clock_probe": (ci, [vp]),
     "ucm_hamming_last_dispatch": (i64, [C.c_char_p, sz]),
+    "ucm_hash_encode_last_dispatch": (i64, [C.c_char_p, sz]),
     "ucm_sparse_decode_step": (ci, [vp, i64, i64, i64, vp, ci, vp, i64, i64, ci, i32, vp, ci, i32, i32,
                                     vp, i64, i32, i32, i64, i64, i64, vp, i32, i32, vp, i32, i32, i32,
                                     i32, i32, u32, vp, vp, vp, vp, sz, vp]),
@@ -178,6 +179,13 @@ def last_dispatch():
     """Kernels launched by the last top-k / score call on this thread (ucm_hamming_last_dispatch)."""
     buf = C.create_string_buffer(256)
     lib().ucm_hamming_last_dispatch(buf, 256)
+    return buf.value.decode()
+
+
+def last_encode():
+    """Kernel launched by the last encode call on this thread (ucm_hash_encode_last_dispatch)."""
+    buf = C.create_string_buffer(64)
+    lib().ucm_hash_encode_last_dispatch(buf, 64)
     return buf.value.decode()
 
 
