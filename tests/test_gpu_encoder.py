@@ -483,3 +483,14 @@ def test_column_counts_without_a_one_tile_form_keep_the_small_kernel(K, N, T):
     """The tiled kernel has one row tile per workgroup for slices of 32, 64, 128 and 256 columns only; with four
     it took 1.3 to 2.9 times the small kernel's time at these sizes."""
     assert _encode_route(K, N, 8, T) == "encode_small"
+
+
+@pytest.mark.parametrize("K,N,H,T,small", [
+    (128, 128, 8, 700, True), (128, 128, 8, 1300, False), (128, 128, 1, 6000, True), (128, 128, 1, 12000, False),
+    (128, 64, 8, 1000, True), (128, 64, 8, 1700, False), (128, 256, 8, 700, True), (128, 256, 8, 1300, False),
+    (64, 128, 8, 1000, True), (64, 128, 8, 3000, False), (64, 64, 8, 1700, True), (64, 64, 8, 4000, False),
+    (64, 32, 8, 6000, True), (128, 32, 8, 6000, False), (64, 256, 1, 5000, True), (64, 256, 8, 3000, False),
+])
+def test_small_kernel_up_to_where_the_tiled_one_is_as_fast(K, N, H, T, small):
+    """Sizes on both sides of the equal times, some way off them."""
+    assert (_encode_route(K, N, H, T) == "encode_small") == small

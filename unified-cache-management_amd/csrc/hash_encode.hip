@@ -2307,13 +2307,15 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
     return ucm::launch_status("encode_tiled_kernel");
 }
 
-// Which matrix-core kernel: the wave-per-tile kernel costs about 4 us plus 12.5 ps per wave and
-// k value (each wave gathers its own operand columns from L2); the LDS kernel with one row tile per
-// workgroup has a floor of about 4.2 us plus 0.027 us per KiB of projection slice that a workgroup stages
-// first (64 x 64: 4.4 us, 128 x 128: 5.1 us).  Measured: 128 -> 128 bits, 8 heads, 300 tokens 4.2 against
-// 4.7 us, 1024 tokens 5.6 against 4.6, 2048 tokens 7.3 against 4.8; one head, 4096 tokens 4.1 against 4.5,
-// 8192 tokens 5.2 against 4.6; 64 -> 64 bits, 8 heads, 600 tokens 3.6 against 3.9, 2048 tokens 4.7 against
-// 4.0.  Where the kernel is not pipelined (rows of 256 values; slices of other than 32, 64, 128 and 256 columns,
+// Which matrix-core kernel.  The wave-per-tile kernel (each wave gathers its own operand columns from L2) costs
+// 4 us plus 12.5 ps per wave and k value once its waves are many, and a microsecond less below 1500 waves.  The
+// LDS kernel with one row tile per workgroup costs 3.5 us and what the staging of its projection slice takes, to 4.7
+// us for 128 x 128 and 6.4 for 128 x 256, and 1.2 us more where there are more workgroups than compute units.  The prices
+// below are on the first one's scale.  Kernel times, small against tiled, 8 heads: 128 -> 128 bits 700 tokens 4.3 and
+// 4.7 us, 1000: 4.8 and 4.6, 3000: 8.4 and 4.7; 128 -> 64 1300: 4.0 and 4.5, 1700: 4.6 and 4.4; 128 -> 256 800: 6.4
+// and 6.4; 64 -> 64 2200: 3.9 and 4.0, 4000: 5.5 and 4.1; 64 -> 256 800: 4.6 and 4.6; 64 -> 32 3000: 3.5 and 3.4, 6000
+// (376 workgroups): 4.0 and 4.5.
+// Where the kernel is not pipelined (rows of 256 values; slices of other than 32, 64, 128 and 256 columns,
 // see launch_mfma_q) it runs four tiles a workgroup: 6 us plus 0.13 us per KiB (256 -> 256 with 4 heads: equal at
 // ~5000-6000 rows; 128 -> 192, 8 heads: 1000 tokens 6.0 against 12.2 us, 4000 14.0 against 13.9; 128 -> 512: 1000
 // 9.8 against 21.9, 3000 20.2 against 23.5).  Rows of 512 values have the slice kernel: 7 us until
@@ -2332,7 +2334,8 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype, bool alone = tru
     const double slice_kib = (double)bn * (a.K + kPad) * 2 / 1024.0;
     double lds_floor_us = 6.0 + 0.13 * slice_kib;
     if (alone && a.K == 16 * kSliceKS) lds_floor_us = 7.5;
-    else if (alone && one_tile_form(a.K, bn)) lds_floor_us = 4.2 + 0.027 * slice_kib;
+    else if (alone && one_tile_form(a.K, bn))
+        lds_floor_us = 4.72 + 0.0002 * slice_kib * a.K + (ucm::ceil_div(a.T, kRowsPerWg) * (a.N / bn) * a.H > stream_workgroups() ? 1.2 : 0.0);
     const double small_us = 4.0 + (double)small_waves(a) * a.K * 12.5e-6;
     return small_us < lds_floor_us;
 }
