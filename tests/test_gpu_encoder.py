@@ -429,10 +429,11 @@ def test_rows_of_512_values_at_the_edges_of_slices_and_tiles(T, N, H, n_w, slots
     (128, 128, 8, 1025, True),    # one row tile per workgroup, the last with one row
     (128, 128, 2, 6001, False),
     (64, 64, 8, 1500, True),
-    (64, 128, 4, 12300, False),   # just past three workgroups a compute unit: four tiles each
+    (64, 128, 4, 24600, False),   # just past three workgroups a compute unit: four tiles each
     (128, 128, 8, 12500, True),
     (128, 256, 1, 98400, False),
     (128, 128, 8, 65700, True),   # eight tiles each
+    (64, 128, 8, 65700, True),    # ... of 64 values
     (64, 64, 8, 10300, False),    # the streaming kernel's first sizes at 64 x 64
 ])
 def test_row_tiles_per_workgroup(K, N, H, T, paged):
@@ -494,3 +495,13 @@ def test_column_counts_without_a_one_tile_form_keep_the_small_kernel(K, N, T):
 def test_small_kernel_up_to_where_the_tiled_one_is_as_fast(K, N, H, T, small):
     """Sizes on both sides of the equal times, some way off them."""
     assert (_encode_route(K, N, H, T) == "encode_small") == small
+
+
+@pytest.mark.parametrize("K,N,H,T,tiles", [
+    (128, 128, 8, 12288, 1), (128, 128, 8, 12400, 4), (64, 128, 4, 24600, 4), (64, 64, 8, 10000, 1), (128, 256, 1, 65536, 1),
+    (128, 256, 1, 66000, 4), (64, 256, 8, 12288, 1), (128, 128, 1, 98304, 1), (128, 128, 8, 65700, 8), (64, 32, 8, 65700, 8),
+])
+def test_row_tiles_per_workgroup_by_the_number_of_workgroups(K, N, H, T, tiles):
+    """One row tile up to three workgroups a compute unit (two where a slice fills the LDS), eight from sixteen."""
+    route = _encode_route(K, N, H, T)
+    assert route.startswith("encode_mfma<") and route.endswith(",%d>" % tiles), route

@@ -1892,8 +1892,10 @@ int launch_mfma_q(const EncArgs& a, size_t lds, hipStream_t st)
         // Runs of two and three between those were tried: 12,700 tokens of two 11.9 against 12.2 us and 24,576
         // 15.1 against 16.7, but 20,000 15.9 against 15.5 and 64 -> 128 bits, 13,000 tokens 13.8 against 11.0;
         // three (held to 168 registers, which spills) 32,691 tokens 24.4 against 19.1.
+        // Two generations only where a slice leaves room for one workgroup (128 -> 256 bits, 84 KiB, one head: 40,000
+        // tokens 12.3 and 13.5 us, 90,000 18.2 and 14.5).
         const int64_t cus = stream_workgroups();
-        if (all <= 3 * cus) return launch_mfma_t<V, KS, NQ, NG, 1>(a, lds, grid(1), st);
+        if (all <= (lds > 80 * 1024 ? 2 : 3) * cus) return launch_mfma_t<V, KS, NQ, NG, 1>(a, lds, grid(1), st);
         if (all >= 16 * cus) return launch_mfma_t<V, KS, NQ, NG, 8>(a, lds, grid(8), st);
     }
     return launch_mfma_t<V, KS, NQ, NG, 4>(a, lds, grid(4), st);
