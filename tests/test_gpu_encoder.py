@@ -383,6 +383,9 @@ def test_unpack_hash_roundtrip():
     (2300, 256, 2, 2, "paged"),  # a projection per head
     (30000, 96, 1, 1, "i32"),    # column count only 32 divides, several tiles per workgroup
     (30001, 192, 1, 1, "dense"), # ... only 64 divides
+    (70001, 96, 1, 1, "paged"),  # past the slices: four row tiles a workgroup, 96-column and
+    (17000, 224, 1, 1, "i64"),   # 32-column slices
+    (60001, 192, 1, 1, "dense"),
     (3000, 320, 2, 1, "i64"),
 ])
 def test_rows_of_512_values_at_the_edges_of_slices_and_tiles(T, N, H, n_w, slots):
@@ -505,3 +508,11 @@ def test_row_tiles_per_workgroup_by_the_number_of_workgroups(K, N, H, T, tiles):
     """One row tile up to three workgroups a compute unit (two where a slice fills the LDS), eight from sixteen."""
     route = _encode_route(K, N, H, T)
     assert route.startswith("encode_mfma<") and route.endswith(",%d>" % tiles), route
+
+
+@pytest.mark.parametrize("N,T,slices", [(96, 49152, True), (96, 70000, False), (160, 16384, True), (160, 24576, False), (192, 32768, True),
+                                        (192, 60000, False), (192, 70000, True), (416, 8192, False), (288, 16384, True),
+                                        (320, 65536, True)])
+def test_slices_of_512_values_up_to_where_they_read_the_rows_too_often(N, T, slices):
+    route = _encode_route(512, N, 1, T)
+    assert route.startswith("encode_slice<" if slices else "encode_mfma<"), route

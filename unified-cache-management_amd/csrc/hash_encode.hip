@@ -1957,6 +1957,17 @@ int launch_slice(const EncArgs& a, hipStream_t st)
     // 7.5 us, 128 columns 9.5 to 10.3 us; two workgroups of 64 columns on a compute unit 13 us).
     const int nt = a.N / 32;
     const int64_t tiles = ucm::ceil_div(a.T, kRowsPerWg) * a.H;
+    // Column counts that 64 or 128 do not divide make many narrow slices, whose workgroups each read the rows
+    // again: from some number of them on encode_mfma_kernel is faster, with slices of 32 columns and three
+    // workgroups to a compute unit, or with slices of 96.  Slice kernel against that one: 160 columns, 480 workgroups
+    // 11.6 and 18.9 us, 640: 17.4 and 19.2, 960: 23.1 and 19.3, 1280: 31.3 and 20.4; 416 columns, 832 workgroups 21.9
+    // and 18.5; 96 columns, 1152: 27.8 and 28.7, 1536: 35.8 and 33.8, 3072: 68.4 and 41.5.  With slices of 64, of two
+    // to every 96 columns, while one generation of that kernel serves all rows: 192 columns, 65,536 rows 37.2 and
+    // 33.9 us, 98,304 rows 53.9 and 65.0.
+    const int64_t units = tiles * nt, cus = stream_workgroups();
+    if (nt % 2 != 0 && (nt % 3 == 0 ? units > 5 * cus : 4 * units > 11 * cus)) return launch_mfma<V, kSliceKS>(a, st);
+    if (nt % 4 == 2 && nt % 3 == 0 && units > 9 * cus && ucm::ceil_div(a.T, 4 * kRowsPerWg) * (nt / 3) * a.H <= cus)
+        return launch_mfma<V, kSliceKS>(a, st);
     if (nt % 4 == 0 && tiles * (nt / 2) > stream_workgroups()) {
         const int rc = launch_slice_nt<V, 4>(a, st);
         if (rc != UCM_EUNSUPPORTED) return rc;  // no large-LDS opt-in: a narrower slice
