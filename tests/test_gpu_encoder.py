@@ -516,3 +516,8 @@ def test_row_tiles_per_workgroup_by_the_number_of_workgroups(K, N, H, T, tiles):
 def test_slices_of_512_values_up_to_where_they_read_the_rows_too_often(N, T, slices):
     route = _encode_route(512, N, 1, T)
     assert route.startswith("encode_slice<" if slices else "encode_mfma<"), route
+
+
+@pytest.mark.parametrize("N,T,wide", [(256, 65535, False), (256, 65536, True), (512, 131071, False), (512, 131072, True)])
+def test_rows_from_which_512_values_take_the_persistent_kernel(N, T, wide):
+    assert (_encode_route(512, N, 1, T) == "encode_wide") == wide

@@ -2014,9 +2014,9 @@ bool mfma_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 // bits, an eighth of the projection: 65,536 rows 5.8 against 5.6 us, 96,000 rows 6.4 against 7.1,
 // 262,144 rows 9.6 against 11.0, 524,288 rows 15.1 against 16.7.
 int64_t stream_min_rows(const EncArgs& a) { return a.K == 64 && a.N == 64 ? (int64_t)5 << 14 : (int64_t)3 << 18; }
-// the wide (K = 512) kernel against the slice kernel: 256 bits: 65,536 rows 26.9 against 26.1 us, 131,072
-// rows 42.5 against 50.8 us; 512 bits: 65,536 rows 54 against 42 us, 131,072 rows 84 against 86 us
-constexpr int64_t kWideMinRows256 = (int64_t)3 << 15;
+// the wide (K = 512) kernel against the slice kernel: 256 bits: 49,152 rows 22.8 against 20.1 us, 65,536 rows 26.5
+// against 28.1, 98,304 rows 34.0 against 40.4; 512 bits: 65,536 rows 54 against 42 us, 131,072 rows 84 against 86
+constexpr int64_t kWideMinRows256 = (int64_t)1 << 16;
 constexpr int64_t kWideMinRows512 = (int64_t)1 << 17;
 // 0 = the defaults above; set per calling thread (a test hook must not move other threads' encodes)
 thread_local int64_t t_stream_min_rows = 0;
