@@ -512,7 +512,7 @@ def test_row_tiles_per_workgroup_by_the_number_of_workgroups(K, N, H, T, tiles):
 
 @pytest.mark.parametrize("N,T,slices", [(96, 49152, True), (96, 70000, False), (160, 16384, True), (160, 24576, False), (192, 32768, True),
                                         (192, 60000, False), (192, 70000, True), (416, 8192, False), (288, 16384, True),
-                                        (320, 65536, True)])
+                                        (320, 65536, True), (32, 131072, True)])
 def test_slices_of_512_values_up_to_where_they_read_the_rows_too_often(N, T, slices):
     route = _encode_route(512, N, 1, T)
     assert route.startswith("encode_slice<" if slices else "encode_mfma<"), route

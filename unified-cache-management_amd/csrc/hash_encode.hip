@@ -1963,9 +1963,9 @@ int launch_slice(const EncArgs& a, hipStream_t st)
     // 11.6 and 18.9 us, 640: 17.4 and 19.2, 960: 23.1 and 19.3, 1280: 31.3 and 20.4; 416 columns, 832 workgroups 21.9
     // and 18.5; 96 columns, 1152: 27.8 and 28.7, 1536: 35.8 and 33.8, 3072: 68.4 and 41.5.  With slices of 64, of two
     // to every 96 columns, while one generation of that kernel serves all rows: 192 columns, 65,536 rows 37.2 and
-    // 33.9 us, 98,304 rows 53.9 and 65.0.
+    // 33.9 us, 98,304 rows 53.9 and 65.0.  (A single slice of 32: 131,072 rows 28.2 and 32.3.)
     const int64_t units = tiles * nt, cus = stream_workgroups();
-    if (nt % 2 != 0 && (nt % 3 == 0 ? units > 5 * cus : 4 * units > 11 * cus)) return launch_mfma<V, kSliceKS>(a, st);
+    if (nt > 1 && nt % 2 != 0 && (nt % 3 == 0 ? units > 5 * cus : 4 * units > 11 * cus)) return launch_mfma<V, kSliceKS>(a, st);
     if (nt % 4 == 2 && nt % 3 == 0 && units > 9 * cus && ucm::ceil_div(a.T, 4 * kRowsPerWg) * (nt / 3) * a.H <= cus)
         return launch_mfma<V, kSliceKS>(a, st);
     if (nt % 4 == 0 && tiles * (nt / 2) > stream_workgroups()) {
