@@ -234,7 +234,7 @@ def test_latent_scorer_clock_probe(Wd, G):
 
 
 @pytest.mark.parametrize("Wd,G", [(18, 16), (8, 16)])
-@pytest.mark.parametrize("B,blocks", [(1, 4096), (1, 4097), (5, 1640), (9, 1400)])
+@pytest.mark.parametrize("B,blocks", [(1, 4096), (1, 4097), (5, 1640), (9, 1400), (1, 2048), (1, 2049), (3, 2049), (2, 4096)])
 def test_latent_scorer_blocks_per_wave(Wd, G, B, blocks):
     """A wave of the latent scorers takes one to four blocks by the launch's size: the edges of those ranges,
     requests that end inside a wave's blocks, inside a workgroup's and before its first, both modes."""

@@ -1625,12 +1625,17 @@ constexpr int kStripWaves = 8;  // waves per workgroup
 constexpr int kStripRun = 4;    // blocks per wave
 constexpr int kStripSlots = 2;  // blocks of a wave in LDS
 constexpr int strip_run(int wd) { return wd == 18 ? kStripRun : 4; }  // blocks per wave
-// Blocks per wave of a launch over `blocks` blocks of B requests: the run while that makes two workgroups
-// for every one of the 256 compute units, fewer where compute units would stand idle (2 x 313 blocks: 20
-// workgroups of runs of four 7.3 us, 80 of single blocks 5.0 us).
-inline int strip_blocks(int wd, int B, int blocks)
+// Blocks per wave of a launch over `blocks` blocks of B requests: fewer than the run where compute units would
+// stand idle (2 x 313 blocks: 20 workgroups of runs of four 7.3 us, 80 of single blocks 5.0 us).  The block scores
+// of 18-word codes take as few as leave one workgroup to each of the 256 compute units, whose weight build is
+// what a second one pays again (top-128 call, 16 query heads: 8 x 512 blocks singly 10.5, in twos 10.0 us; 8 x 768 in
+// twos 12.6, in threes 11.3; 8 x 1024 in twos 13.0, in fours 12.3), and past that, like the others, as leave two
+// (8 x 1536 in threes 16.6, in fours 17.6; per-token scores 8 x 1024 in twos 9.2, in fours 10.1).
+inline int strip_blocks(int wd, int B, int blocks, bool tokens)
 {
-    const int64_t n = ucm::ceil_div((int64_t)B * blocks, kStripWaves * 512);
+    const int64_t all = (int64_t)B * blocks;
+    const int wgs = wd == 18 && !tokens && all <= 256 * kStripWaves * kStripRun ? 256 : 512;
+    const int64_t n = ucm::ceil_div(all, kStripWaves * wgs);
     return n < 1 ? 1 : (n < strip_run(wd) ? (int)n : strip_run(wd));
 }
 constexpr int kStripFirst = 0;  // of those, a building wave requests before the weight build (at most kStripSlots)
@@ -3211,7 +3216,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
         if (planes_inside && a.G >= 16 && a.G <= 128) {
             // the weighted bit sums on the matrix unit, as for 18-word codes
             note_score("block_score_strip8");
-            a.TB = strip_blocks(8, B, max_blocks);
+            a.TB = strip_blocks(8, B, max_blocks, false);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
             launch_score_threads(block_score_strip<8>, g64, kStripWaves * kWave, 0, st, a);
         } else if (planes_inside) {
@@ -3230,7 +3235,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
             }
         } else if (planes_in_lanes && Wd == 18) {
             note_score("block_score_strip18");
-            a.TB = strip_blocks(18, B, max_blocks);
+            a.TB = strip_blocks(18, B, max_blocks, false);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
             launch_score_threads(block_score_strip<18>, g64, kStripWaves * kWave, 0, st, a);
         } else if (planes_in_lanes) {
@@ -4172,7 +4177,7 @@ extern "C" int ucm_hamming_score(const uint32_t* q_codes, int64_t q_stride_b, in
         }
         if (run18 || run8) {
             // the weighted bit sums of every 8-byte piece on the matrix unit; no plane kernel, no workspace
-            a.TB = strip_blocks(Wd, B, nblk);
+            a.TB = strip_blocks(Wd, B, nblk, true);
             const dim3 rgrid((unsigned)ucm::ceil_div(nblk, kStripWaves * a.TB), (unsigned)B);
             const dim3 threads(kStripWaves * kWave);
             note_score("token_score_strip", Wd, out_is_f16 ? 1 : 0);
