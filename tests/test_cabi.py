@@ -151,3 +151,23 @@ def test_torch_operator_library_registers_its_operators():
     z = torch.zeros((1, 1, 4), dtype=torch.int32)
     with pytest.raises((NotImplementedError, RuntimeError)):
         ops.hamming_topk(z, z.view(1, 1, 1, 4), z.view(1, 4)[:, :1], z.view(-1)[:1], 1, 0, 0, 0)
+
+
+@pytest.mark.parametrize("module", ["missing", "not_a_library"])
+def test_calls_work_without_the_module_of_native_fronts(module, monkeypatch, tmp_path):
+    """libucm_hip.so alone is enough: the general path takes every call, after one warning."""
+    import torch
+
+    from ucm_amd import _lib
+    from ucm_amd.sparse.esa_retrieval_worker import dot_topk
+
+    path = tmp_path / "ucm_native.so"
+    if module == "not_a_library":
+        path.write_bytes(b"no library")
+    monkeypatch.setattr(_lib, "NATIVE_PATH", str(path))
+    monkeypatch.setattr(_lib, "_native", None)
+    x = torch.zeros(2, 2)
+    with pytest.warns(RuntimeWarning, match="without their native fronts"):
+        with pytest.raises(ValueError, match="one GPU"):  # the general path's answer for host tensors
+            dot_topk(x, x, x.int(), 1)
+    assert _lib.native().dot_topk(x, x, x.int(), 1, None) is None and _lib.native() is _lib.native()

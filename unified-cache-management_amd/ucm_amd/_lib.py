@@ -157,20 +157,32 @@ def lib():
     return _lib
 
 
+class _NoFronts:
+    """Stands in for the module of native fronts: every call is the general path's."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def native():
     """The module of native fronts (csrc/native_calls.cpp): a front takes the plain case of a call and
-    returns None for any other, which is the caller's general path's."""
+    returns None for any other, which is the caller's general path's.  The general path launches the same
+    kernels, some microseconds of host time later: without the module, or with one that was built for another
+    interpreter or torch, it takes every call."""
     global _native
     if _native is None:
         import importlib.machinery
         import importlib.util
+        import warnings
 
         lib()  # libucm_hip.so and torch first: the module binds to what is loaded
-        if not os.path.exists(NATIVE_PATH):
-            raise RuntimeError(f"{NATIVE_PATH} is missing: run unified-cache-management_amd/build.py")
-        loader = importlib.machinery.ExtensionFileLoader("ucm_native", NATIVE_PATH)
-        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("ucm_native", loader))
-        loader.exec_module(mod)
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("ucm_native", NATIVE_PATH)
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("ucm_native", loader))
+            loader.exec_module(mod)
+        except ImportError as e:
+            warnings.warn(f"calls go without their native fronts ({e}): run unified-cache-management_amd/build.py", RuntimeWarning)
+            mod = _NoFronts()
         _native = mod
     return _native
 
