@@ -95,7 +95,8 @@ bool shape_is(const Tensor& t, std::initializer_list<int64_t> s) { return t.size
 
 bool is_index(const Tensor& t) { return t.scalar_type() == at::kInt || t.scalar_type() == at::kLong; }
 
-// Body of a front: runs f, which returns a new reference or null for "not plain".
+// Body of a front: runs f, which returns a new reference or null: for "not plain", or with a Python error set
+// (an output that could not be wrapped; its kernels have been issued).
 template <class F>
 PyObject* front(F&& f)
 {
@@ -106,7 +107,7 @@ PyObject* front(F&& f)
         PyErr_Clear();
         r = nullptr;
     }
-    if (!r) Py_RETURN_NONE;
+    if (!r && !PyErr_Occurred()) Py_RETURN_NONE;
     return r;
 }
 
