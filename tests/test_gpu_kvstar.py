@@ -73,6 +73,7 @@ def test_matches_checker(X, Hq, Hkv, d, n, M, topk):
     (1, 2, 1, 64, 1, 100, 1),      # one block of several tiles
     (2, 4, 4, 32, 33, 63, 33),     # an odd number of row tiles per workgroup pair, chunks that end inside a tile
     (40, 64, 2, 32, 12, 2, 12),    # 2560 rows: statistics in two batches
+    (40, 64, 2, 130, 9, 40, 9),    # ... of long rows
     (2, 4, 2, 24, 21, 16, 5),      # head dim of one and a half k-steps
     (2, 4, 2, 256, 21, 16, 5),     # head dim above what is kept packed
     (1, 2, 2, 32, 70, 256, 11),    # more tiles than two per wave and chunk

@@ -209,6 +209,42 @@ def test_front_and_general_path_agree(name, variant):
         assert g.dtype == w.dtype and g.shape == w.shape and torch.equal(g, w)
 
 
+def _tensors(call):
+    for cell in call.__closure__:
+        v = cell.cell_contents
+        for t in v if isinstance(v, list) else [v]:
+            if isinstance(t, torch.Tensor):
+                yield t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(CALLS))
+def test_fronts_issue_on_the_current_stream(name):
+    """The inputs hold zeros until work that takes a few milliseconds has run on the current stream: a launch on
+    any other stream would read those."""
+    with general_path():
+        want = _outcome(CALLS[name], "plain")
+    call = CALLS[name]("plain")
+    later = [(t, t.clone()) for t in _tensors(call)]
+    assert len(later) >= 3
+    for t, _ in later:
+        t.zero_()
+    busy = torch.randn(4096, 4096, device="cuda")
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(20):
+            busy = busy @ busy
+            busy /= busy.abs().max()
+        for t, good in later:
+            t.copy_(good)
+        out = call()
+        assert not side.query()  # still busy: the call did not wait
+    side.synchronize()
+    for g, w in zip(out if isinstance(out, (list, tuple)) else [out], want):
+        assert torch.equal(g.cpu(), w)
+
+
 @pytest.mark.gpu
 def test_plain_calls_take_the_front():
     calls = {n: m("plain") for n, m in CALLS.items()}
