@@ -73,7 +73,6 @@ def test_matches_checker(X, Hq, Hkv, d, n, M, topk):
     (1, 2, 1, 64, 1, 100, 1),      # one block of several tiles
     (2, 4, 4, 32, 33, 63, 33),     # an odd number of row tiles per workgroup pair, chunks that end inside a tile
     (40, 64, 2, 32, 12, 2, 12),    # 2560 rows: statistics in two batches
-    (40, 64, 2, 130, 9, 40, 9),    # ... of long rows
     (2, 4, 2, 24, 21, 16, 5),      # head dim of one and a half k-steps
     (2, 4, 2, 256, 21, 16, 5),     # head dim above what is kept packed
     (1, 2, 2, 32, 70, 256, 11),    # more tiles than two per wave and chunk
@@ -199,6 +198,14 @@ def test_against_float64_formulation_at_llama_shape():
     kth = np.sort(ref)[::-1][63]
     assert np.all(ref[gi] >= kth - (ATOL + RTOL * kth))
     assert gs.sum() <= 8 * 32 * (1 + 1e-5)
+
+
+def test_long_rows_in_two_batches_of_statistics():
+    # 2560 query rows; against float64, as the checker adds a block's 102,400 probabilities one by one
+    q, k = make(40, 40, 64, 2, 130, 9, 40, scale=0.5)
+    gi, gs = run_gpu(q, k, None, 9)
+    ref = brute.kvstar_block_scores(q, k)
+    assert np.allclose(gs, ref[gi], rtol=RTOL, atol=ATOL) and np.all(np.diff(gs) <= 0)
 
 
 def test_equal_scores_come_out_in_ascending_block_order():

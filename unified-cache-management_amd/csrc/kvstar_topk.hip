@@ -124,10 +124,9 @@ __device__ __forceinline__ f16x8 load_q(const QRow& q, int c, int d, int d_orig)
 
 constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596303e-8f;  // log2(e) in two pieces
 
-// exp(x) for x far from overflow (here x <= 0 but for rounding): 2^(x log2 e) with the product's
-// rounding error carried along, whole and fractional part of the exponent taken apart so that results
-// down to the smallest denormal come out.  A NaN stays one.  12 instructions where expf() has 17 (it
-// tests both ends of its range): the two passes' exponentials are most of these kernels' instructions.
+// exp(x) for x far from overflow (here x <= 0 but for rounding): 2^(x log2 e) with log2 e in two pieces and the
+// product's rounding error carried along (Dekker's exact product, by a fused multiply-add), whole and fractional
+// part of the exponent taken apart so that results down to the smallest denormal come out.  A NaN stays one.
 __device__ __forceinline__ float exp_small(float x)
 {
     x = __builtin_elementwise_maximum(x, -200.0f);  // also minus infinity; the result is 0 either way
@@ -654,6 +653,7 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     UCM_REQUIRE(d <= kMaxDim, "head dim %d above %d", d, kMaxDim);
     UCM_REQUIRE(n_blocks <= INT32_MAX && n_blocks * M <= INT32_MAX, "too many block representatives");
     const int64_t rows = (int64_t)X * Hq;
+    // row tiles are a grid dimension; the second bound is the entry point's own, no index comes near it
     UCM_REQUIRE(rows <= 65535 && rows * M <= INT32_MAX, "too many query rows");
     UCM_REQUIRE(workspace && workspace_bytes >= ucm_kvstar_topk_workspace_bytes(X, Hq, n_blocks, M),
                 "workspace too small");
