@@ -430,10 +430,17 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
                     Stat st{-INFINITY, 0.0f};
                     if (r < nr) {
                         const Stat* p = a.part + r0 + r;
-                        for (int c = c0; c < c1; c += 16) {
+                        int c = c0;
+                        for (; c + 16 <= c1; c += 16) {
                             Stat v[16];
 #pragma unroll
-                            for (int i = 0; i < 16; ++i) v[i] = p[(int64_t)(c + i < c1 ? c + i : c1 - 1) * rows];
+                            for (int i = 0; i < 16; ++i) v[i] = p[(int64_t)(c + i) * rows];
+                            st = merge(st, v);
+                        }
+                        for (; c < c1; c += 8) {
+                            Stat v[8];
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) v[i] = p[(int64_t)(c + i < c1 ? c + i : c1 - 1) * rows];
                             st = merge(st, v, c1 - c);
                         }
                     }
