@@ -16,9 +16,9 @@
 // selection.  The [X Hq, S] score matrix is never stored: writing it and reading it back twice moved
 // seven times the bytes of the keys themselves, and computing q.k a second time costs two matrix
 // instructions per 32 x 32 scores of 32 channels.  At 8 query tokens x 32 heads, 253 blocks x 64
-// representatives and 32 channels the four kernels that stored it took 32.9 us (13.6 q.k, 8.6 row
-// statistics, 6.1 block sums, 5.7 selection); these three take 17.8 us
-// (7.2, 8.3, 3.6; without the exponentials 6.0 and 7.3: what is left is launches and round trips).
+// representatives and 32 channels the four kernels that stored it took 33.1 us (13.6 q.k, 8.6 row
+// statistics, 6.1 block sums, 5.7 selection); these three take 18.3 us
+// (7.4, 8.8, 3.2; 1.2 and 1.0 of the first two for the exponentials: what is left is launches and round trips).
 // Sums are taken in a different order than the reference's loops, the same one on every call (no
 // atomics); the tolerance is stated where the results are compared.  Equal scores come out in
 // ascending block order (the reference's heap pops them in descending block order).
