@@ -214,3 +214,32 @@ def test_errors(device):
         sm.PagedGatherAsync([t.data_ptr()], [8], [0, -1], t.data_ptr())
     with pytest.raises(ValueError):  # beyond the cache's extent
         sm.PagedScatterAsync(t.data_ptr(), [t.data_ptr()], [8], [0, 8], num_cache_blocks=8)
+
+
+@pytest.mark.parametrize("n_cols,col_bytes,n_ids", [
+    (2, 4096, 1), (2, 4096, 496), (2, 4096, 497), (2, 48, 1984), (2, 48, 1985),  # a launch, two, four, the table
+    (1, 70001, 7), (3, 4112, 5), (3, 100, 9),          # tails, columns that start at any byte
+    (128, 64, 244), (128, 64, 245), (129, 64, 4),      # the most columns the arguments hold, and one more
+])
+def test_paged_copy_of_equal_columns(device, n_cols, col_bytes, n_ids):
+    """Where the ids travel as kernel arguments: how many fit a launch, how many launches there are, ids that
+    repeat and columns out of address order."""
+    rng = rng_for(n_cols * 10007 + n_ids)
+    NB = n_ids + 3
+    pool = torch.from_numpy(rng.integers(0, 256, size=(n_cols, NB, col_bytes), dtype=np.uint8)).cuda()
+    order = rng.permutation(n_cols)
+    base = np.array([pool[c].data_ptr() for c in order], np.uint64)
+    sizes = np.full(n_cols, col_bytes, np.uint64)
+    ids = rng.integers(0, NB, n_ids).astype(np.int32)
+    flat = torch.zeros((n_ids + 1, n_cols, col_bytes), dtype=torch.uint8, device="cuda")
+    stream = device.MakeSMStream()
+    torch.cuda.synchronize()
+    stream.PagedGatherAsync(base, sizes, ids, flat.data_ptr(), num_cache_blocks=NB)
+    stream.Synchronized()
+    want = pool.cpu().numpy()
+    got = flat.cpu().numpy()
+    assert np.array_equal(got[:n_ids], want[order][:, ids].transpose(1, 0, 2)) and not got[n_ids].any()
+    fresh = rng.permutation(NB)[:n_ids].astype(np.int32)
+    stream.PagedScatterAsync(flat.data_ptr(), base, sizes, fresh, sync=True, num_cache_blocks=NB)
+    want[order[:, None], fresh[None, :]] = got[:n_ids].transpose(1, 0, 2)
+    assert np.array_equal(pool.cpu().numpy(), want)

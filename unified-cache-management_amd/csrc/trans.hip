@@ -110,6 +110,38 @@ __global__ __launch_bounds__(kThreads) void paged_copy_kernel(const uint64_t* __
     }
 }
 
+// What a copy of equal columns needs, as kernel arguments: the columns' addresses, then the launch's block ids
+// (int32) behind them.  2 KiB of arguments cost 0.1 to 0.3 us of host time more than a few bytes.
+constexpr size_t kArgWords = 250;
+constexpr size_t kArgCols = 128;    // columns at most: half of the words stay for ids
+constexpr size_t kArgLaunches = 4;  // launches at most
+constexpr size_t kArgBytes = (size_t)512 << 20;  // bytes at most
+
+struct ColumnArgs {
+    uint8_t* flat;      // flat row of the first id
+    uint64_t col_bytes;
+    uint64_t row_bytes;
+    int n_cols, to_cache;
+    uint64_t words[kArgWords];
+};
+
+// paged_copy_kernel for columns of one size, without a table in memory.  What bounded small copies was neither
+// bytes nor the copy: the upload of the table and the event that guards its staging slot are 10 us of host time
+// and a round trip per call, where a launch is 2.  Segment, column and block are the grid's three dimensions: no
+// division in front of the load, one round of scalar reads behind the arguments.
+// Out and back, with the wait at the end: 153 blocks x 2 columns of 32 KiB 36.3 -> 26.5 us, 122 x 64 of 4 KiB
+// 52.8 -> 40.0, 32 x 64 of 256 KiB 381 -> 355.
+__global__ __launch_bounds__(kThreads) void column_copy_kernel(ColumnArgs a)
+{
+    const size_t off = (size_t)blockIdx.x * kSeg;
+    const size_t bytes = a.col_bytes - off < kSeg ? a.col_bytes - off : kSeg;
+    const int32_t* ids = reinterpret_cast<const int32_t*>(a.words + a.n_cols);
+    uint8_t* cache_p = (uint8_t*)(a.words[blockIdx.y] + (uint64_t)ids[blockIdx.z] * a.col_bytes) + off;
+    uint8_t* flat_p = a.flat + blockIdx.z * a.row_bytes + blockIdx.y * a.col_bytes + off;
+    if (a.to_cache) wg_copy(flat_p, cache_p, bytes);
+    else wg_copy(cache_p, flat_p, bytes);
+}
+
 struct Slot {
     void* host = nullptr;  // pinned staging for tables
     void* dev = nullptr;
@@ -465,6 +497,34 @@ extern "C" int ucm_trans_paged_copy(ucm_trans_stream_t* s, const uint64_t* base,
         row_bytes += col_bytes[c];
         segs_per_row += (col_bytes[c] + kSeg - 1) / kSeg;
     }
+    const bool host_end = is_host_memory(flat);
+    // Columns of one size between device memory, few enough for the arguments of a few launches.  Beyond that
+    // the upload, paid once, is the cheaper form; a host end is bound by its link.  From 512 MiB on the form
+    // with the table is the faster one: its workgroups come to their loads later, and with fewer of them in
+    // flight the memory turns less often between reads and writes (1 GiB of 64 columns each way: 319 and 345 us
+    // out and back, column_copy_kernel 348 and 366, with five of its workgroups to a unit instead of eight 332
+    // and 346, which is slower than eight below 256 MiB).
+    bool equal = true;
+    for (int c = 1; c < n_cols; ++c) equal = equal && col_bytes[c] == col_bytes[0];
+    const size_t segs_per_col = segs_per_row / n_cols;
+    if (equal && !host_end && (size_t)n_cols <= kArgCols && segs_per_col <= (1u << 20) &&
+        (size_t)n_blocks <= kArgBytes / row_bytes) {
+        const size_t per_launch = (kArgWords - n_cols) * 2;
+        if ((size_t)n_blocks <= per_launch * kArgLaunches) {
+            ColumnArgs a;
+            a.col_bytes = col_bytes[0]; a.row_bytes = row_bytes; a.n_cols = n_cols; a.to_cache = to_cache;
+            std::memcpy(a.words, base, (size_t)n_cols * 8);
+            for (size_t first = 0; first < (size_t)n_blocks; first += per_launch) {
+                const size_t n = (size_t)n_blocks - first < per_launch ? (size_t)n_blocks - first : per_launch;
+                a.flat = (uint8_t*)flat + first * row_bytes;
+                std::memcpy(a.words + n_cols, block_ids + first, n * 4);
+                hipLaunchKernelGGL(column_copy_kernel, dim3((unsigned)segs_per_col, (unsigned)n_cols, (unsigned)n),
+                                   dim3(kThreads), 0, s->stream, a);
+            }
+            const int rc = ucm::launch_status("column_copy_kernel");
+            return rc != UCM_OK ? rc : finish(s, sync);
+        }
+    }
     const size_t meta_words = 3 * (size_t)n_cols + segs_per_row;
     const size_t bytes = meta_words * 8 + (size_t)n_blocks * 4;
     Slot* sl = nullptr;
@@ -481,7 +541,6 @@ extern "C" int ucm_trans_paged_copy(ucm_trans_stream_t* s, const uint64_t* base,
     }
     std::memcpy(h + meta_words, block_ids, (size_t)n_blocks * 4);
     UCM_HIP_TRY(hipMemcpyAsync(sl->dev, sl->host, bytes, hipMemcpyHostToDevice, s->stream));
-    const bool host_end = is_host_memory(flat);
     if (host_end && row_bytes <= kStageBytes) {
         // two stages per piece of whole blocks, as in table_copy()
         const size_t per_piece = kStageBytes / row_bytes;
