@@ -13,13 +13,22 @@ import numpy as np
 from . import _lib
 
 
+def _address(arr):
+    """Address of a contiguous array's values; through the buffer protocol 0.3 us, as `arr.ctypes.data`, which
+    read-only and empty arrays need, 1.4 us - three of them were half of a small paged copy's host time."""
+    try:
+        return C.addressof(C.c_char.from_buffer(arr))
+    except (TypeError, ValueError, BufferError):
+        return arr.ctypes.data
+
+
 def _table(obj):
     """-> (address, on_device, keepalive)"""
     if isinstance(obj, np.ndarray):
         if obj.dtype != np.uint64:
             raise ValueError("pointer tables must be numpy uint64 arrays")
         arr = np.ascontiguousarray(obj)
-        return arr.ctypes.data, 0, arr
+        return _address(arr), 0, arr
     return int(obj), 1, None
 
 
@@ -116,8 +125,8 @@ class Stream:
         ids = np.ascontiguousarray(block_ids, dtype=np.int32).reshape(-1)
         if base.shape != cb.shape:
             raise ValueError("base_ptrs and col_bytes must have the same length")
-        _lib.check(_lib.lib().ucm_trans_paged_copy(self._h, base.ctypes.data, cb.ctypes.data,
-                                                   base.shape[0], ids.ctypes.data, ids.shape[0],
+        _lib.check(_lib.lib().ucm_trans_paged_copy(self._h, _address(base), _address(cb),
+                                                   base.shape[0], _address(ids), ids.shape[0],
                                                    int(num_cache_blocks), int(flat), to_cache,
                                                    int(bool(sync))))
 
