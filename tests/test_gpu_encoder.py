@@ -140,6 +140,26 @@ def test_few_tokens_many_heads_one_projection(B, H, K, N, n_w):
     assert np.array_equal(cache.cpu().numpy().view(np.uint32), expect)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,K,N,n_w", [
+    (224, 1, 512, 512, 1), (225, 1, 512, 512, 1), (256, 1, 256, 128, 1),  # seven row tiles, eight
+    (8, 33, 512, 64, 1), (16, 33, 256, 96, 1),   # nine and seventeen row tiles of pairs; columns no power of two
+    (40, 8, 512, 128, 8), (5, 12, 256, 64, 4),   # a projection per head or per three heads: two row tiles each, one
+])
+def test_split_row_tiles(dtype, B, H, K, N, n_w):
+    """Rows of 256 and 512 values, few enough for the kernel whose waves share a row tile: the order in which row
+    and column tiles go out, rows past the last, rows that lie apart (a strided view)."""
+    rng = rng_for(B * 131 + H * 7 + K + N)
+    wide = torch.from_numpy(rng.standard_normal((B, H, K + 24)).astype(np.float32)).to(dtype)
+    W = torch.from_numpy(rng.standard_normal((n_w, K, N)).astype(np.float32)).to(dtype)
+    enc = make_encoder(K, N, dtype, W if n_w > 1 else W[0], n_w=n_w, hpw=H // n_w)
+    codes = enc.compute_hash(wide.cuda()[..., 8:8 + K], per_head=True).cpu().numpy()
+    assert _encode_route(K, N, H, B).startswith("encode_small")
+    x = wide[..., 8:8 + K].float().numpy()
+    for h in range(H):
+        assert_codes_match(codes[:, h], x[:, h], W[h // (H // n_w)].float().numpy())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("slot_dtype", [torch.int32, torch.int64])
 def test_compute_hash_and_cache(dtype, slot_dtype):
