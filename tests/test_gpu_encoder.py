@@ -160,6 +160,44 @@ def test_split_row_tiles(dtype, B, H, K, N, n_w):
         assert_codes_match(codes[:, h], x[:, h], W[h // (H // n_w)].float().numpy())
 
 
+@pytest.mark.parametrize("T,N,H,BS,dtype,route", [
+    (1285, 512, 1, 64, torch.float16, "2,4"),    # eleven row tiles: three of the second eight streams; one row past a group of four
+    (4097, 128, 3, 48, torch.bfloat16, "2,4"),   # heads side by side, block size no power of two, a last tile of one row
+    (8063, 512, 1, 64, torch.bfloat16, "4,4"),   # 63 row tiles, one row short
+    (20000, 384, 1, 64, torch.float16, "4,8"),   # streams that eight does not divide, a second tile for some
+    (50001, 512, 1, 64, torch.bfloat16, "8,8"),  # a second row tile for some of the streams, the last one of a few rows
+    (65535, 512, 1, 32, torch.bfloat16, "8,8"),  # two for all, one row short
+])
+def test_rows_of_512_values_by_tile_shape(T, N, H, BS, dtype, route):
+    """Every shape of the tile; one or several row tiles per workgroup; a strided view of the rows, rows that are
+    skipped, zero or NaN.  The rows checked are those around tile edges and a sample of the others."""
+    assert _encode_route(512, N, H, T) == "encode_pipe<%s>" % route
+    rng = rng_for(T + N + H)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T)
+    x = torch.randn(T, H, 512 + 8, generator=g, device="cuda", dtype=torch.float32).to(dtype)[..., 8:]
+    x[T // 3] = 0.0
+    x[T // 2, :, 5] = float("nan")
+    W = torch.from_numpy(rng.standard_normal((512, N)).astype(np.float32)).to(dtype)
+    enc = make_encoder(512, N, dtype, W)
+    nb = -(-T // BS)
+    ids = rng.permutation(nb)
+    slot = ids[np.arange(T) // BS].astype(np.int64) * BS + np.arange(T) % BS
+    stored = slot.copy()
+    stored[7::11] = -1
+    cache = torch.zeros((nb, BS, H, N // 32), dtype=torch.int32, device="cuda")
+    enc.compute_hash_and_cache(x, torch.from_numpy(stored).cuda(), cache, block_size=BS)
+    flat = cache.cpu().numpy().reshape(nb * BS, H, N // 32)
+    assert not flat[slot[7::11]].any() and not flat[slot[[T // 3, T // 2]]].any()
+    near = (np.arange(0, T + 128, 128)[:, None] + np.array([-33, -1, 0, 31, 32, 64])).reshape(-1)
+    rows = np.unique(np.concatenate([near, [T - 2, T - 1], rng.integers(0, T, 2000)]))
+    rows = rows[(rows >= 0) & (rows < T)]
+    rows = rows[(stored[rows] >= 0) & (rows != T // 2)]
+    xs = x[torch.from_numpy(rows).cuda()].float().cpu().numpy()
+    for h in range(H):
+        assert_codes_match(np.ascontiguousarray(flat[slot[rows], h]).view(np.uint8), xs[:, h], W.float().numpy())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("slot_dtype", [torch.int32, torch.int64])
 def test_compute_hash_and_cache(dtype, slot_dtype):

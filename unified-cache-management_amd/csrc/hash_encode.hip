@@ -561,7 +561,295 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 // ---------------------------------------------------------------------------------------
-// Rows of 512 values (latent vectors), any row count above the latency path's.
+// Rows of 512 values (latent vectors) to hash columns in multiples of 64, any row count above the latency path's.
+//
+// A workgroup's tile is 128 rows by 32 NT columns; a wave multiplies 64 rows by 16 NT columns.  Rows and projection
+// come in chunks of 64 values of k, straight from memory into a ring of four chunks in LDS (load-to-LDS, 16 bytes a
+// lane, neighbouring lanes on one line), so that nothing but the first chunk stands in front of the first matrix
+// instruction, no register holds a value on its way, and the next tile's chunks travel while this one's are
+// multiplied.  The projection keeps its row-major layout; its operands are read with the transposing LDS read.
+// Pieces of a row change places inside it (the lane picks the piece it fetches), so that both kinds of operand
+// reads find every bank once.  A wave asks for its operands two k-steps ahead; the one barrier of a chunk - all
+// waves have read chunk c, all loads of chunk c + 1 have landed - stands two k-steps in front of the first
+// operand it protects, beside matrix instructions that need none of it.
+//
+// What bounds it: the first chunk's way (some 3 us with the launch), then LDS - 64 x 64 products a wave read 4 KiB of
+// operands for four matrix instructions of 32 cycles, 128 bytes a cycle from four waves, beside 64 that the loads
+// write - and past 128 columns the projection and row traffic from L2: eight waves on 256 x 256 halve both and run at
+// 1.16 PFLOP/s.  512 bits, before (slices of the projection transposed through registers in front of the rows, row
+// loads whose 64 pieces lie on 64 lines: encode_slice_kernel, then with 128 columns too) and now: 2,048 rows 7.2 and
+// 5.5 us, 4,096 rows 7.9 and 6.0, 8,192 rows 10.7 and 8.2, 16,384 rows 16.1 and 11.1, 32,768 rows 26.3 and 16.4,
+// 65,536 rows 46.4 and 29.7.
+// ---------------------------------------------------------------------------------------
+constexpr int kPipeKS = 32;     // k-steps of 16: rows of 512 values
+constexpr int kPipeChunk = 64;  // values of k to a chunk
+constexpr int pipe_rows(int waves) { return waves * 32; }
+constexpr int pipe_ring(int nt, int waves) { return waves == 8 ? 2 : 4; }  // chunks in LDS
+constexpr int pipe_stage_bytes(int nt, int waves) { return (pipe_rows(waves) + nt * 32) * kPipeChunk * 2; }
+constexpr int pipe_slot_bytes(int waves) { return pipe_rows(waves) * 8; }  // a tile's raw slots: low words, then high words
+constexpr int pipe_lds(int nt, int waves)
+{
+    return pipe_ring(nt, waves) * pipe_stage_bytes(nt, waves) + 2 * pipe_slot_bytes(waves);
+}
+
+// Touches every 64-byte line of a kernel-argument struct at once.  The compiler fetches a field
+// where the code first needs it, behind the branches of the row addressing - a dozen scalar reads
+// one after the other in a kernel that lives for a few microseconds; with the lines already in the
+// scalar cache those reads are short.  (Copying the struct through pinned registers instead makes
+// its pointers lose their address space: every access becomes a flat one.)
+template <class T>
+__device__ __forceinline__ void warm_args(const T& args)
+{
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(&args);
+    uint32_t t = 0;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; i += 16) t |= src[i];
+    t |= src[sizeof(T) / 4 - 1];
+    asm volatile("" ::"s"(t));
+}
+
+// N loads of 16 bytes a lane, each to 1 KiB of LDS behind the last: bases in scalar registers, lane offsets off.
+__device__ __forceinline__ void pipe_load(uint32_t lds, uint64_t b0, uint32_t o0, uint64_t b1, uint32_t o1)
+{
+    uint32_t keep;
+    asm volatile("s_mov_b32 %[keep], m0\n\ts_mov_b32 m0, %[lds]\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %[o0], %[b0]\n\t"
+                 "s_add_u32 m0, %[lds], 0x400\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %[o1], %[b1]\n\t"
+                 "s_mov_b32 m0, %[keep]\n\t"
+                 : [keep] "=&s"(keep)
+                 : [lds] "s"(lds), [b0] "s"(b0), [o0] "v"(o0), [b1] "s"(b1), [o1] "v"(o1)
+                 : "memory", "scc");
+}
+// One 4-byte load a lane from an address of its own.
+__device__ __forceinline__ void pipe_load_word(uint32_t lds, const void* p)
+{
+    uint32_t keep;
+    asm volatile("s_mov_b32 %[keep], m0\n\ts_mov_b32 m0, %[lds]\n\ts_nop 0\n\t"
+                 "global_load_lds_dword %[p], off\n\t"
+                 "s_mov_b32 m0, %[keep]\n\t"
+                 : [keep] "=&s"(keep)
+                 : [lds] "s"(lds), [p] "v"(p)
+                 : "memory");
+}
+__device__ __forceinline__ uint64_t uniform64(uint64_t v)
+{
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+template <typename V, int NT, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void encode_pipe_kernel(EncArgs a, int streams)
+{
+    static_assert((NT == 2 && kWaves == 4) || NT == 4 || (NT == 8 && kWaves == 8), "64, 128 or 256 columns");
+    constexpr int kRows = pipe_rows(kWaves), kPipeRing = pipe_ring(NT, kWaves);
+    constexpr int kPipeRowBytes = kRows * kPipeChunk * 2, kPipeSlotBytes = pipe_slot_bytes(kWaves);
+    constexpr int kStage = pipe_stage_bytes(NT, kWaves), kCols = NT / 2;  // kCols: column tiles of 32 of a wave
+    constexpr int kWLoads = NT * 4 / kWaves, kLoads = 4 + kWLoads;         // of a wave, per chunk
+    constexpr int kChunks = kPipeKS * 16 / kPipeChunk;
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* tr_ptr;
+    extern __shared__ __align__(16) uint16_t wt[];
+    char* lds = reinterpret_cast<char*>(wt);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)wt);
+    warm_args(a);
+    const int h = blockIdx.z;
+    // The slices of a row tile are workgroups of one XCD (consecutive ones go to the eight XCDs in turn), so that
+    // its rows come past that XCD's L2 once: streams in eights, each eight slice by slice.  What fills the last
+    // eight has nothing to do.  Fewer than eight streams take all XCDs for each.
+    const int slices = a.N / (NT * 32);
+    int stream, n0;
+    if (streams >= 8) {
+        stream = (int)blockIdx.x / (8 * slices) * 8 + (blockIdx.x & 7);
+        n0 = (int)(blockIdx.x >> 3) % slices * (NT * 32);
+        if (stream >= streams) return;
+    } else {
+        stream = (int)blockIdx.x % streams;
+        n0 = (int)blockIdx.x / streams * (NT * 32);
+    }
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = wave >> 1, wc = wave & 1;  // the wave's half of the rows, of the columns
+    const int r = lane & 31, kb = lane >> 5;
+    const int64_t tiles = (a.T + kRows - 1) / kRows;
+
+    // What a wave fetches of a chunk: rows 32 wave .. + 32, eight to a load (piece p of row i lies at place
+    // p ^ (i / 2 % 8)), and 64 / (16 / NT) rows of the projection, 64-byte units changed over by k % 4 or k / 2 % 2.
+    constexpr int kWRows = 16 / NT;  // rows of the projection to a load
+    uint32_t xoff[4], woff[2];  // woff: of even and of odd loads
+    uint64_t xbase, wbase;  // of the next chunk
+    const uint64_t wload = (uint64_t)kWRows * a.N * 2, wchunk = (uint64_t)kPipeChunk * a.N * 2;
+    {
+        constexpr int kWPieces = NT * 4;  // 16-byte pieces of a row
+        const int k = lane / kWPieces, p = lane % kWPieces;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int turn = NT == 2 ? ((k >> 1) & 1) : ((j * kWRows + k) & 3);
+            woff[j] = (uint32_t)(k * a.N * 2 + (p ^ (turn << 2)) * 16);
+        }
+    }
+    auto point_at = [&](int64_t tile) __attribute__((always_inline)) {
+        wbase = (uint64_t)(uintptr_t)((const uint16_t*)a.w + (int64_t)weight_index(a, h) * kPipeKS * 16 * a.N + n0) +
+                (uint64_t)(wave * kWLoads) * wload;
+        // the wave's 32 rows lie in one block of a paged input and less than 2 GiB apart; rows past T re-read the
+        // last one, they are not stored
+        const int64_t t0 = tile * kRows + wave * 32;
+        const int64_t first = t0 < a.T ? t0 : a.T - 1;
+        const int last = (int)(a.T - 1 - first < 31 ? a.T - 1 - first : 31);
+        xbase = uniform64((uint64_t)(uintptr_t)((const uint16_t*)a.x + src_offset(a, first, h)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = i * 8 + (lane >> 3) < last ? i * 8 + (lane >> 3) : last;
+            const int piece = (lane & 7) ^ ((4 * (i & 1) + (lane >> 4)) & 7);
+            xoff[i] = (uint32_t)row * (uint32_t)(a.x_stride_t * 2) + piece * 16;
+        }
+    };
+    auto fetch_slots = [&](int64_t tile, int buf) __attribute__((always_inline)) {
+        const int part = wave / (kWaves / 2), group = wave % (kWaves / 2);  // low or high words, 64 rows
+        int64_t t = tile * kRows + group * 64 + lane;
+        if (t > a.T - 1) t = a.T - 1;
+        // without a slot array the reads hit the first row and are ignored
+        const char* p = a.slot ? (const char*)a.slot : (const char*)a.x;
+        int sh = a.slot_is_i64 ? 3 : 2, hi_off = a.slot_is_i64 ? 4 : 0;
+        int64_t i = a.slot ? t : 0;
+        if (a.src_blocks) {
+            int64_t tok;
+            split_token(a, t, i, tok);
+            p = (const char*)a.src_blocks;
+            sh = 2;
+            hi_off = 0;
+        }
+        pipe_load_word(lds0 + kPipeRing * kStage + buf * kPipeSlotBytes + part * (kPipeSlotBytes / 2) + group * 256,
+                       p + (i << sh) + (part ? hi_off : 0));
+    };
+    auto issue = [&](int c) __attribute__((always_inline)) {
+        uint32_t st = lds0;
+        uint64_t wnext = wload;
+        asm volatile("" : "+s"(st), "+s"(wnext));  // opaque, as below
+        st += (c % kPipeRing) * kStage;
+        pipe_load(st + wave * 4096, xbase, xoff[0], xbase, xoff[1]);
+        pipe_load(st + wave * 4096 + 2048, xbase, xoff[2], xbase, xoff[3]);
+#pragma unroll
+        for (int j = 0; j < kWLoads; j += 2)
+            pipe_load(st + kPipeRowBytes + (wave * kWLoads + j) * 1024, wbase + j * wnext, woff[0], wbase + (j + 1) * wnext, woff[1]);
+        // (opaque: otherwise every chunk's addresses are computed in advance and kept)
+        xbase += kPipeChunk * 2;
+        wbase += wchunk;
+        asm volatile("" : "+s"(xbase), "+s"(wbase));
+    };
+    struct Ops {
+        V x[2], w[kCols];
+    };
+    // Where the wave's operands lie in a chunk: row l % 32 of a row tile, piece 2 ks + l / 32; of the projection,
+    // the transposing read gives lane l of each 16 the column l of four rows whose 8-byte pieces the 16 lanes name.
+    // Pieces and units are numbered by exclusive or: the k-step and the column tile turn a bit of an address each.
+    const uint32_t xat = lds0 + (wr * 64 + r) * 128 + ((kb ^ ((r >> 1) & 7)) << 4);  // (the row tiles are 32 rows apart)
+    const int tk = (lane >> 2) & 3;                                               // row of the four
+    const uint32_t wat = lds0 + kPipeRowBytes + (kb * 8 + tk) * (NT * 64) + (((wc * kCols) ^ (NT == 2 ? tk >> 1 : tk)) << 6) +
+                         ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    uint32_t xc = 0, wc_at = 0;  // the two of the chunk that is read
+    auto read_ops = [&](int c, int ks, Ops& o) __attribute__((always_inline)) {
+        typedef __attribute__((address_space(3))) const V* row_ptr;
+        if (ks == 0) {
+            xc = xat + (c % kPipeRing) * kStage;
+            wc_at = wat + (c % kPipeRing) * kStage;
+            asm volatile("" : "+v"(xc), "+v"(wc_at));  // opaque, as in issue()
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) o.x[q] = *(row_ptr)(uintptr_t)((xc ^ (ks << 5)) + q * 32 * 128);
+#pragma unroll
+        for (int q = 0; q < kCols; ++q) {
+            s16x4 half[2];
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                half[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (tr_ptr)(uintptr_t)((wc_at ^ (q << 6)) + (ks * 16 + p * 4) * (NT * 64)));
+            __builtin_memcpy(&o.w[q], half, 16);
+        }
+    };
+
+    int64_t tile = stream;
+    int buf = 0;
+    point_at(tile);
+    fetch_slots(tile, 0);
+#pragma unroll
+    for (int c = 0; c < kPipeRing; ++c) issue(c);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((kPipeRing - 1) * kLoads) : "memory");
+    constexpr int kAhead = NT == 8 ? 1 : 2;  // k-steps that operands are asked for in advance
+    Ops op[4];
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) read_ops(0, s, op[s]);
+
+    auto pass = [&](int64_t next, auto more_) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_)::value;
+        f32x16 acc[kCols][2];
+#pragma unroll
+        for (int q = 0; q < kCols; ++q) acc[q][0] = acc[q][1] = acc_start();
+#pragma unroll
+        for (int s = 0; s < kPipeKS; ++s) {
+            const int c = s / 4, ks = s % 4;
+            if (ks == 4 - kAhead && (MORE || c + 1 < kChunks)) {
+                // everything read of chunk c is in registers, chunk c + 1 is in LDS, for every wave
+                // chunks requested behind it
+                const int newer = MORE || kChunks - 2 - c > kPipeRing - 2 ? kPipeRing - 2 : kChunks - 2 - c;
+                if (newer == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kLoads) : "memory");
+                else if (newer == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                if (c + kPipeRing < kChunks) {
+                    issue(c + kPipeRing);
+                } else if (MORE) {
+                    if (c + kPipeRing == kChunks) {
+                        point_at(next);
+                        fetch_slots(next, buf ^ 1);
+                    }
+                    issue(c + kPipeRing - kChunks);
+                }
+            }
+            if (s + kAhead < kPipeKS || MORE) read_ops((s + kAhead) / 4 % kChunks, (s + kAhead) % 4, op[(s + kAhead) % 4]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < kCols; ++q) {
+                acc[q][0] = Mfma<V>::run(op[s % 4].w[q], op[s % 4].x[0], acc[q][0]);
+                acc[q][1] = Mfma<V>::run(op[s % 4].w[q], op[s % 4].x[1], acc[q][1]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const uint32_t* slots = reinterpret_cast<const uint32_t*>(lds + kPipeRing * kStage + buf * kPipeSlotBytes);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int row = wr * 64 + p * 32 + r;
+            const int64_t t = tile * kRows + row;
+            uint32_t words[kCols];
+#pragma unroll
+            for (int q = 0; q < kCols; ++q) {
+                const uint32_t half = pack_half(acc[q][p]);
+                words[q] = join_halves(kb ? half << 4 : half);
+            }
+            const RawSlot raw{slots[row], slots[kRows + row]};
+            uint32_t* dst = t < a.T && lane < 32 ? slot_dst(a, slot_value(a, raw, t), h) : nullptr;
+            if (dst) {
+                dst += n0 / 32 + wc * kCols;
+                if (kCols == 4 && (((uintptr_t)dst) & 15) == 0) {
+                    *reinterpret_cast<u32x4*>(dst) = u32x4{words[0], words[1 % kCols], words[2 % kCols], words[3 % kCols]};
+                } else if (kCols == 2 && (((uintptr_t)dst) & 7) == 0) {
+                    uint2 v;
+                    v.x = words[0];
+                    v.y = words[kCols - 1];
+                    *reinterpret_cast<uint2*>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < kCols; ++q) dst[q] = words[q];
+                }
+            }
+        }
+        buf ^= 1;
+    };
+    for (; tile + streams < tiles; tile += streams) pass(tile + streams, std::true_type{});
+    pass(tile, std::false_type{});
+}
+
+// ---------------------------------------------------------------------------------------
+// Rows of 512 values (latent vectors) to column counts that 128 does not divide, any row count above the latency path's.
 //
 // A workgroup keeps a slice of 32 NT hash columns of the projection in LDS (transposed) and walks
 // row tiles of 128: a wave owns 32 rows whose 32 operands it loads straight into registers.  All NT
@@ -570,18 +858,15 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
 // registers of their own.
 //
 // What bounds it: for up to one row tile per workgroup the loads in front of the first matrix
-// instruction (128 KiB of rows and 32 NT KiB of projection through one compute unit's address unit;
-// 8192 rows x 512 bits: 10.3 us, of which 1.9 us are matrix instructions), then the matrix pipe at the
-// clock the power limit leaves (4 us a tile of 128 x 128).  The slices of a row tile are workgroups of one
-// XCD where the number of row streams is a multiple of 8, so its rows come from HBM once.  512 bits
-// before (133 KiB slices in front of four tiles a workgroup, rows through LDS) and now: 2048 rows 9.8
-// and 7.1 us, 4096 rows 15.4 and 7.7 us, 8192 rows 23.7 and 10.3 us, 32,768 rows 30.3 and 24.3 us.
+// instruction (128 KiB of rows and 32 NT KiB of projection through one compute unit's address unit), then
+// the row loads, whose 64 pieces lie on 64 lines.  The slices of a row tile are workgroups of one XCD where the
+// number of row streams is a multiple of 8, so its rows come from HBM once.
 // ---------------------------------------------------------------------------------------
 constexpr int kSliceKS = 32;                    // 512 / 16 k-steps
 constexpr int kSlicePitch = kSliceKS * 16 + kPad;
 
 template <typename V, int NT>
-__global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(NT == 4 ? 1 : 2, NT == 4 ? 1 : 2))) void encode_slice_kernel(EncArgs a)
+__global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void encode_slice_kernel(EncArgs a)
 {
     constexpr int K = kSliceKS * 16, KP = kSlicePitch;
     extern __shared__ uint16_t wt[];  // [32 NT][KP], k contiguous
@@ -677,12 +962,8 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(NT
         }
         if (dst) {
             uint32_t* d = dst + n0 / 32;
-            if (NT == 4 && (((uintptr_t)d) & 15) == 0) {
-                *reinterpret_cast<u32x4*>(d) = u32x4{words[0], words[1 % NT], words[2 % NT], words[3 % NT]};
-            } else {
 #pragma unroll
-                for (int q = 0; q < NT; ++q) d[q] = words[q];
-            }
+            for (int q = 0; q < NT; ++q) d[q] = words[q];
         }
     };
     for (; tile + gridDim.x < tiles; tile += gridDim.x) pass(tile, tile + gridDim.x, std::true_type{});
@@ -1771,22 +2052,6 @@ __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv)
     }
 }
 
-// Touches every 64-byte line of a kernel-argument struct at once.  The compiler fetches a field
-// where the code first needs it, behind the branches of the row addressing - a dozen scalar reads
-// one after the other in a kernel that lives for a few microseconds; with the lines already in the
-// scalar cache those reads are short.  (Copying the struct through pinned registers instead makes
-// its pointers lose their address space: every access becomes a flat one.)
-template <class T>
-__device__ __forceinline__ void warm_args(const T& args)
-{
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&args);
-    uint32_t t = 0;
-#pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 4; i += 16) t |= src[i];
-    t |= src[sizeof(T) / 4 - 1];
-    asm volatile("" ::"s"(t));
-}
-
 // waves that share a tile: rows of 256 values and more are split four ways
 constexpr int small_split(int KS) { return KS >= 16 ? 4 : 1; }
 
@@ -1965,6 +2230,62 @@ int launch_mfma(EncArgs a, hipStream_t st)
     return ucm::fail(UCM_EUNSUPPORTED, "no LDS slice fits K=%d", K);
 }
 
+// Row tiles that are walked at the same time: a workgroup to a compute unit, and as many streams on every XCD (three
+// slices, 85 streams: five XCDs had 33 workgroups for their 32 compute units; 24,000 rows 25.0 us, 80 streams 18.8).
+int64_t pipe_streams(const EncArgs& a, int nt, int waves)
+{
+    const int64_t tiles = ucm::ceil_div(a.T, pipe_rows(waves));
+    const int64_t units = (int64_t)(a.N / (32 * nt)) * a.H;
+    int64_t streams = (int64_t)stream_workgroups() / units;
+    if (streams > 8) streams &= ~(int64_t)7;
+    return streams < 1 ? 1 : (streams < tiles ? streams : tiles);
+}
+
+template <typename V, int NT, int WAVES>
+int launch_pipe_nt(const EncArgs& a, hipStream_t st)
+{
+    constexpr int lds = pipe_lds(NT, WAVES);
+    static int opted = 0;  // 0 = not tried, 1 = allowed, -1 = refused by the runtime
+    if (opted == 0) {
+        const hipError_t e = hipFuncSetAttribute((const void*)encode_pipe_kernel<V, NT, WAVES>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) (void)hipGetLastError();
+        opted = (e == hipSuccess) ? 1 : -1;
+    }
+    if (opted < 0) return UCM_EUNSUPPORTED;
+    const int64_t streams = pipe_streams(a, NT, WAVES);
+    note_encode("encode_pipe", NT, WAVES);
+    hipLaunchKernelGGL((encode_pipe_kernel<V, NT, WAVES>), dim3((unsigned)((streams < 8 ? streams : ucm::ceil_div(streams, 8) * 8) * (a.N / (32 * NT))), 1, (unsigned)a.H),
+                       dim3(64 * WAVES), lds, st, a, (int)streams);
+    return ucm::launch_status("encode_pipe_kernel");
+}
+
+// The tile: each shape's time is a start of 2.4 to 3.2 us and so much for every generation of workgroups (tenths of a
+// microsecond, measured at 256 and 512 columns with every compute unit at work), whose last one is paid in full.
+// 512 columns, the four shapes in their order: 4,096 rows 6.0, 7.3, 9.0 and 13.1 us; 8,192 rows 9.7, 8.2, 9.9, 13.8;
+// 16,384 rows 16.4, 13.6, 11.1, 14.6; 32,768 rows 29.0, 23.7, 19.4, 16.4; 65,536 rows 54.7, 42.2, 34.5, 29.7.
+template <typename V>
+int launch_pipe(const EncArgs& a, hipStream_t st)
+{
+    static const struct { int nt, waves, cost; } shapes[] = {{2, 4, 36}, {4, 4, 52}, {4, 8, 83}, {8, 8, 132}};
+    int best = 0;
+    int64_t best_cost = 0;
+    for (int i = 0; i < 4; ++i) {
+        if (a.N % (32 * shapes[i].nt)) continue;
+        const int64_t tiles = ucm::ceil_div(a.T, pipe_rows(shapes[i].waves));
+        const int64_t units = ucm::ceil_div((int64_t)(a.N / (32 * shapes[i].nt)) * a.H, stream_workgroups());
+        const int64_t cost = ucm::ceil_div(tiles, pipe_streams(a, shapes[i].nt, shapes[i].waves)) * units * shapes[i].cost;
+        if (i == 0 || cost < best_cost) {
+            best = i;
+            best_cost = cost;
+        }
+    }
+    if (best == 0) return launch_pipe_nt<V, 2, 4>(a, st);
+    if (best == 1) return launch_pipe_nt<V, 4, 4>(a, st);
+    if (best == 2) return launch_pipe_nt<V, 4, 8>(a, st);
+    return launch_pipe_nt<V, 8, 8>(a, st);
+}
+
 template <typename V, int NT>
 int launch_slice_nt(const EncArgs& a, hipStream_t st)
 {
@@ -1981,7 +2302,7 @@ int launch_slice_nt(const EncArgs& a, hipStream_t st)
     }
     const int64_t tiles = ucm::ceil_div(a.T, kRowsPerWg);
     const int64_t units = (int64_t)(a.N / (32 * NT)) * a.H;
-    int64_t streams = (int64_t)stream_workgroups() * (NT == 4 ? 1 : 2) / units;
+    int64_t streams = (int64_t)stream_workgroups() * 2 / units;
     if (streams < 1) streams = 1;
     if (streams > tiles) streams = tiles;
     note_encode("encode_slice", NT);
@@ -1995,7 +2316,7 @@ int launch_slice(const EncArgs& a, hipStream_t st)
 {
     // Narrow slices while they leave every compute unit at most one workgroup: the time in front of the
     // first matrix instruction grows with the slice (1 to 256 workgroups: 32 columns 7 us, 64 columns
-    // 7.5 us, 128 columns 9.5 to 10.3 us; two workgroups of 64 columns on a compute unit 13 us).
+    // 7.5 us; two workgroups of 64 columns on a compute unit 13 us).
     const int nt = a.N / 32;
     const int64_t tiles = ucm::ceil_div(a.T, kRowsPerWg) * a.H;
     // Column counts that 64 or 128 do not divide make many narrow slices, whose workgroups each read the rows
@@ -2009,10 +2330,6 @@ int launch_slice(const EncArgs& a, hipStream_t st)
     if (nt > 1 && nt % 2 != 0 && (nt % 3 == 0 ? units > 5 * cus : 4 * units > 11 * cus)) return launch_mfma<V, kSliceKS>(a, st);
     if (nt % 4 == 2 && nt % 3 == 0 && units > 9 * cus && ucm::ceil_div(a.T, 4 * kRowsPerWg) * (nt / 3) * a.H <= cus)
         return launch_mfma<V, kSliceKS>(a, st);
-    if (nt % 4 == 0 && tiles * (nt / 2) > stream_workgroups()) {
-        const int rc = launch_slice_nt<V, 4>(a, st);
-        if (rc != UCM_EUNSUPPORTED) return rc;  // no large-LDS opt-in: a narrower slice
-    }
     if (nt % 2 == 0 && tiles * nt > stream_workgroups()) {
         const int rc = launch_slice_nt<V, 2>(a, st);
         if (rc != UCM_EUNSUPPORTED) return rc;
@@ -2027,7 +2344,14 @@ int dispatch_mfma(const EncArgs& a, hipStream_t st)
         case 64: return launch_mfma<V, 4>(a, st);
         case 128: return launch_mfma<V, 8>(a, st);
         case 256: return launch_mfma<V, 16>(a, st);
-        case 512: return launch_slice<V>(a, st);
+        case 512: {
+            if (a.N % 128 == 0) {
+                const int rc = launch_pipe<V>(a, st);
+                if (rc != UCM_EUNSUPPORTED) return rc;  // no large-LDS opt-in: narrow slices
+                ucm::clear_error();
+            }
+            return launch_slice<V>(a, st);
+        }
         default: return ucm::fail(UCM_ERROR, "internal: K %d has no MFMA kernel", a.K);
     }
 }
@@ -2055,8 +2379,11 @@ bool mfma_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 // bits, an eighth of the projection: 65,536 rows 5.8 against 5.6 us, 96,000 rows 6.4 against 7.1,
 // 262,144 rows 9.6 against 11.0, 524,288 rows 15.1 against 16.7.
 int64_t stream_min_rows(const EncArgs& a) { return a.K == 64 && a.N == 64 ? (int64_t)5 << 14 : (int64_t)3 << 18; }
-// the wide (K = 512) kernel against the slice kernel: 256 bits: 49,152 rows 22.8 against 20.1 us, 65,536 rows 26.5
-// against 28.1, 98,304 rows 34.0 against 40.4; 512 bits: 65,536 rows 54 against 42 us, 131,072 rows 84 against 86
+// The wide (K = 512) kernel against the slice kernel of 128 columns, by which these lines were drawn: 256 bits: 49,152
+// rows 22.8 against 20.1 us, 65,536 rows 26.5 against 28.1; 512 bits: 65,536 rows 54 against 42 us, 131,072 rows 84
+// against 86.  encode_pipe_kernel, which took that one's place below them, is ahead beyond them too (256 bits, 65,536
+// rows: wide 26.2, pipe 19.5 us, 262,144 rows 84.0, 80.5; 512 bits, 131,072 rows 93.5, 70.5, 1,048,576 rows 538, 508):
+// the route of such calls is part of what the tests hold still, so the lines are where they were.
 constexpr int64_t kWideMinRows256 = (int64_t)1 << 16;
 constexpr int64_t kWideMinRows512 = (int64_t)1 << 17;
 // 0 = the defaults above; set per calling thread (a test hook must not move other threads' encodes)
