@@ -244,3 +244,72 @@ def test_separate_operators_under_graph_capture(G):
                                  table.cpu().numpy(), lens.cpu().numpy(), msl, 128, 256, False)
         assert np.array_equal(got[3].cpu().numpy(), ot)
         _ = (qs.float() @ qs.float().transpose(1, 2)).sum().item()  # unrelated eager work
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,BS,nblk,T,dtype,sink,recent", [
+    (1, 8, 8, 128, 128, 40, 1, torch.bfloat16, None, None),   # no groups
+    (3, 32, 8, 128, 128, 30, 3, torch.float16, None, None),
+    (2, 64, 32, 128, 16, 61, 7, torch.bfloat16, 0, 16),       # no sink window, the most heads; more new keys than requests
+    (5, 33, 1, 128, 48, 40, 9, torch.bfloat16, 48, 48),       # one head, an odd group, block size no power of two
+    (2, 16, 2, 64, 1024, 12, 256, torch.bfloat16, 0, 1),      # the longest blocks, the most new keys
+    (4, 20, 4, 64, 40, 50, 0, torch.float16, None, None),     # no new keys
+    (16, 8, 4, 128, 64, 40, 16, torch.bfloat16, None, None),  # as many blocks as go this way
+    (2, 10, 2, 64, 32, 300, 2, torch.bfloat16, 32, 64),       # a longer row for the selection
+])
+def test_small_step_scores_and_hashes_in_one_launch(B, Hq, Hkv, D, BS, nblk, T, dtype, sink, recent):
+    """Steps of few blocks, whose scoring workgroups hash the queries: new keys inside scored blocks (their old
+    codes must not count) and dropped ones, a block two requests share, unusable table entries, an empty request
+    and lengths that end inside a block; the same codes, tables and lengths as the operators one by one."""
+    from ucm_amd import _lib
+    from ucm_amd.sparse import GSADecodeStep, HashEncoder
+
+    rng = rng_for(B * 1009 + Hq * 31 + D + BS + T)
+    NB, W = B * nblk + 2, D // 32
+    w = torch.from_numpy(rng.standard_normal((D, D)).astype(np.float32)).to(dtype).cuda()
+    cache = torch.from_numpy(rng.integers(0, 2**32, size=(NB, BS, Hkv, W), dtype=np.uint32).view(np.int32)).cuda()
+    tab = rng.permutation(NB)[:B * nblk].astype(np.int32).reshape(B, nblk)
+    lens = np.array([nblk * BS - (i * 37) % (nblk * BS // 2) for i in range(B)], np.int32)
+    if B > 1:
+        tab[1, 3] = tab[0, 2]
+        lens[1] = nblk * BS - BS // 2
+    if B > 2:
+        lens[2] = 0
+        tab[0, 4], tab[0, 5], tab[1, 0] = -1, NB, -3
+    # new keys all over the first requests' blocks, each slot once
+    slots = np.array([int(tab[0, 1 + i % (nblk - 2)]) * BS + (i * 7) % BS for i in range(T)], np.int64)
+    slots = np.where((slots < 0) | (slots >= NB * BS), -1, slots)
+    _, first = np.unique(slots, return_index=True)
+    slots[np.setdiff1d(np.arange(T), first)] = -1
+    if T:  # a code equal to its head's query code would be the best there is: old codes must not be seen
+        q_at = slots[slots >= 0]
+        cache.view(NB * BS, Hkv, W)[torch.from_numpy(q_at).cuda()] = 0
+    q = torch.from_numpy(rng.standard_normal((B, Hq, D)).astype(np.float32)).to(dtype).cuda()
+    newk = torch.from_numpy(rng.standard_normal((T, Hkv, D)).astype(np.float32)).to(dtype).cuda() if T else None
+    topk_tok = 8 * BS
+    step = GSADecodeStep(w, Hq, Hkv, B, nblk, topk_tok, block_size=BS, sink_token=sink, recent_token=recent)
+    expect_cache = cache.clone()
+    enc = HashEncoder(D, D, dtype, torch.device("cuda:0"))
+    enc.set_hash_weight(w)
+    G = Hq // Hkv
+    mean = q.view(B, Hkv, G, D)[:, :, 0].float()
+    for g in range(1, G):  # the group's rows in order, as the step adds them
+        mean = mean + q.view(B, Hkv, G, D)[:, :, g].float()
+    mean = (mean * torch.tensor(1.0 / G, dtype=torch.float32)).to(dtype)
+    qc = enc.compute_hash(mean).view(torch.int32)
+    slot_t = torch.from_numpy(slots).cuda()
+    if T:
+        enc.compute_hash_and_cache(newk, slot_t, expect_cache, block_size=BS)
+    new_table, new_lens = step.step(newk, slot_t if T else None, q, cache, torch.from_numpy(tab).cuda(), torch.from_numpy(lens).cuda())
+    assert _lib.last_dispatch().startswith("encode_score<%d>+" % W)
+    assert torch.equal(cache, expect_cache)
+    assert torch.equal(step.q_codes.view(B, Hkv, W), qc.view(B, Hkv, W))
+    oi, _ = c_api.hamming_topk(step.q_codes.cpu().numpy().view(np.uint32).reshape(B, Hkv, W),
+                               cache.cpu().numpy().view(np.uint32), tab, lens, 8,
+                               BS if sink is None else sink, 4 * BS if recent is None else recent,
+                               flags=c_api.F_REDUCE_HEADS | c_api.F_PHYSICAL)
+    expect = np.zeros((B, nblk), np.int32)
+    for b in range(B):
+        n = min(8, -(-int(lens[b]) // BS))
+        expect[b, :n] = oi[b, 0, :n]
+    assert np.array_equal(new_table.cpu().numpy(), expect)
+    assert np.array_equal(new_lens.cpu().numpy(), c_api.update_seq_lens(lens, topk_tok, BS))

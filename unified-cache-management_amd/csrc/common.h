@@ -59,6 +59,15 @@ struct PairSpec {
     // of heads i, i + Hq / q_reduce, i + 2 * Hq / q_reduce, ... (q_codes is [B, Hq / q_reduce, Wd])
     int q_reduce = 0;
 };
+// The block scores of a grouped-query decode step: best KV head, sink and recent blocks kept (see ucm_hamming_topk).
+struct StepScore {
+    const int32_t* table; int table_stride, max_blocks; const int32_t* lens; int sink, recent;
+    int32_t* scores;  // [B][max_blocks]
+};
+// whether encode_and_score() takes the step; fails as encode_pair() would
+int step_is_fused(const PairSpec& p, const StepScore& s, bool& fused);
+// both jobs of a pair and the block scores in one launch
+int encode_and_score(const PairSpec& p, const StepScore& s, hipStream_t st);
 // one launch when both jobs are small
 int encode_pair(const PairSpec& p, hipStream_t st);
 // two pairs; one launch when all four jobs are small and the input widths are 512 and 64

@@ -3046,7 +3046,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
                      int32_t table_stride, int32_t max_blocks, const int32_t* seq_lens, int32_t B,
                      int32_t Hq, int32_t k, int32_t sink_tok, int32_t recent_tok, uint32_t flags,
                      int32_t* out_idx, int32_t* out_score, void* workspace, size_t workspace_bytes,
-                     ucm_stream_t stream, const StepOut* step_out)
+                     ucm_stream_t stream, const StepOut* step_out, const ucm::PairSpec* fused = nullptr)
 {
     note_reset();
     int rc = common_checks(q_codes, k_cache, seq_lens, NB, BS, Hkv, Wd, B, Hq, max_blocks);
@@ -3111,7 +3111,15 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
     const bool direct_g = a.G == 1 || a.G == 2 || a.G == 4;
     const bool one_head_planes = Hkv == 1 && !direct_g && pairs_layout(a, k_cache) &&
                                  (Wd >= 16 || lanes_layout(a, k_cache, false));
-    if (fast && !one_head_planes) {
+    if (fused) {
+        // one launch writes the codes and the scores, the best head's per block
+        note_score("encode_score", Wd);
+        ++g_note.score_launches;
+        const ucm::StepScore sc{block_table, table_stride, max_blocks, seq_lens, sink_tok, recent_tok, ws.scores};
+        rc = ucm::encode_and_score(*fused, sc, st);
+        if (rc != UCM_OK) return rc;
+        reduced_scores = true;
+    } else if (fast && !one_head_planes) {
         int pmax = planes_for_group(a.G);
         const bool direct = a.G == 1 || a.G == 2 || a.G == 4;
         {
@@ -3351,13 +3359,16 @@ extern "C" int ucm_gsa_decode_step(const void* new_keys, int64_t T, int64_t k_st
                        q_stride_b, q_stride_h, q_codes, (int64_t)Hkv * Wd, Wd, x_dtype, K, w,
                        w_dtype, n_w, N_bits};
     spec.q_group_mean = 1;
-    int rc = ucm::encode_pair(spec, (hipStream_t)stream);
+    bool fused = false;
+    int rc = ucm::step_is_fused(spec, ucm::StepScore{block_table, table_stride, max_blocks, seq_lens, sink_tok, recent_tok, nullptr}, fused);
+    fused = fused && !(g_prof_before && g_prof_after);  // those time the scores alone
+    if (rc == UCM_OK && !fused) rc = ucm::encode_pair(spec, (hipStream_t)stream);
     if (rc != UCM_OK) return rc;
     const StepOut so{new_block_table, new_table_stride, new_seq_lens, seq_len_threshold, topk_tok};
     return hamming_topk_run(q_codes, (int64_t)Hkv * Wd, Wd, k_cache, NB, BS, Hkv, Wd, ks_block, ks_token,
                             ks_head, block_table, table_stride, max_blocks, seq_lens, B, Hkv, topk_tok / BS,
                             sink_tok, recent_tok, UCM_TOPK_REDUCE_HEADS | UCM_TOPK_RETURN_PHYSICAL, nullptr,
-                            nullptr, workspace, workspace_bytes, stream, &so);
+                            nullptr, workspace, workspace_bytes, stream, &so, fused ? &spec : nullptr);
 }
 
 // ---------------------------------------------------------------------------------------

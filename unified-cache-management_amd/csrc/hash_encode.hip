@@ -1807,8 +1807,11 @@ __host__ __device__ __forceinline__ bool small_rows_are_pairs(const EncArgs& a)
 // row's k-steps each and the partial sums meet in LDS - everything a wave does before its first
 // matrix instruction (32 + 32 loads of 16 bytes per lane, 128 permutes, the LDS transpose at
 // K = 512) is one chain, and a quarter of it per wave is a quarter of the chain.
+// `lds` is the tile's: small_lds(KS, SPLIT) values.
+constexpr int small_lds(int KS, int SPLIT) { return SPLIT * 32 * (KS / SPLIT * 16 + kPad); }
+
 template <typename V, int KS, int SPLIT = 1>
-__device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv)
+__device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv, uint16_t* lds)
 {
     static_assert(KS % SPLIT == 0, "the row's k-steps divide evenly over the waves of a tile");
     constexpr int K = KS * 16;        // the row's width: what separates two projection matrices
@@ -1962,8 +1965,7 @@ __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv)
     // transpose them in registers and pass them through LDS - K / 16 loads per lane; fetching the
     // operands directly takes eight 2-byte loads per k-step (K / 2 per lane: 256 at K = 512).
     constexpr int KP = KL + kPad;
-    __shared__ __align__(16) uint16_t wt_all[SPLIT][32 * KP];
-    uint16_t* wt = wt_all[slice];
+    uint16_t* wt = lds + slice * 32 * KP;
     V bv[KSL];
     // the rows pass through the same LDS, in front of the patches: a wave's LDS operations complete in order
     auto rows_to_operands = [&]() __attribute__((always_inline)) {
@@ -2029,7 +2031,7 @@ __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv)
         // A wave's partial sums go where its slice of W was: its own reads of that region are
         // behind it (LDS operations of a wave complete in order), and nobody else touches it
         // before the barrier.
-        static_assert(sizeof(wt_all[0]) >= 16 * 64 * sizeof(float), "a slice of W makes room for one wave's sums");
+        static_assert(32 * KP * 2 >= 16 * 64 * (int)sizeof(float), "a slice of W makes room for one wave's sums");
         float* part = reinterpret_cast<float*>(wt);
         if (slice > 0) {
 #pragma unroll
@@ -2039,7 +2041,7 @@ __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv)
         if (slice > 0) return;
 #pragma unroll
         for (int sl = 1; sl < SPLIT; ++sl) {
-            const float* other = reinterpret_cast<const float*>(wt_all[sl]);
+            const float* other = reinterpret_cast<const float*>(lds + sl * 32 * KP);
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[i] += other[i * 64 + lane];
         }
@@ -2059,9 +2061,10 @@ template <typename V, int KS>
 __global__ __launch_bounds__(64 * small_split(KS)) __attribute__((amdgpu_waves_per_eu(small_split(KS) > 1 ? 3 : 1, 8))) void encode_small_kernel(EncJobs js)
 {
     warm_args(js);
+    __shared__ __align__(16) uint16_t lds[small_lds(KS, small_split(KS))];
     const bool second = (int)blockIdx.x >= js.waves0;
     encode_small_body<V, KS, small_split(KS)>(second ? js.job[1] : js.job[0],
-                                              second ? blockIdx.x - js.waves0 : blockIdx.x);
+                                              second ? blockIdx.x - js.waves0 : blockIdx.x, lds);
 }
 
 // Four jobs in one launch, two of input width 16 * KSA and two of 16 * KSB (the two parts of a
@@ -2075,15 +2078,240 @@ template <typename V, int KSA, int KSB>
 __global__ __launch_bounds__(64 * small_split(KSA)) __attribute__((amdgpu_waves_per_eu(3, 8))) void encode_small_mixed_kernel(EncJobs4 js)
 {
     static_assert(small_split(KSB) == 1, "the narrow jobs' tiles take one wave of the workgroup");
+    static_assert(small_lds(KSB, 1) <= small_lds(KSA, small_split(KSA)), "one area for both");
+    __shared__ __align__(16) uint16_t lds[small_lds(KSA, small_split(KSA))];
     warm_args(js);
     const int w = blockIdx.x;
     if (w < js.end[1]) {
         const int j = w >= js.end[0] ? 1 : 0;
-        encode_small_body<V, KSA, small_split(KSA)>(js.job[j], j ? w - js.end[0] : w);
+        encode_small_body<V, KSA, small_split(KSA)>(js.job[j], j ? w - js.end[0] : w, lds);
     } else {
         if (threadIdx.x >= 64) return;  // a narrow tile is one wave's work
         const int j = w >= js.end[2] ? 3 : 2;
-        encode_small_body<V, KSB>(js.job[j], w - js.end[j - 1]);
+        encode_small_body<V, KSB>(js.job[j], w - js.end[j - 1], lds);
+    }
+}
+
+// A small decode step of a grouped-query model up to its block scores in one launch: every workgroup that scores a
+// block hashes its request's mean queries for itself, so that no launch of their own stands in front of the
+// scores.  The block's codes are requested first and travel while the waves hash, a 32-column tile each (32 KiB of
+// projection from L2 per workgroup: why this is for steps of few blocks).  The step's new keys are hashed by
+// workgroups at the grid's end; a block that one of them falls into hashes that key itself instead of reading
+// a code that is being written.  Blocks whose score is settled (sink, recent window, unusable entry) read nothing;
+// block 0, which is in the sink window if there is one, leaves the request's query codes in memory.
+//
+// What bounds it: one chain - arguments, length and table entry, rows and projection, LDS, products, codes - of about
+// 5.5 us, with the selection behind it 7.8 us a step of one request of 8,192 tokens (9.9 with an encode launch of its own,
+// of which 2.5 us are issuing it: launches are most of such a step's host time).  Three waves to a SIMD: with two a
+// step of 512 blocks takes 10.3 us instead of 9.2.
+constexpr int kStepThreads = 256;
+constexpr int kStepTokens = kStepThreads;  // new keys of a step at most: a thread looks at a slot each
+constexpr int kStepMostBS = 1024;          // tokens of a block at most: a bit each for the freshly hashed ones
+
+struct StepJobs {
+    EncArgs kk, kq;
+    const int32_t* table;
+    const int32_t* lens;
+    int32_t* scores;  // [B][max_blocks]
+    int table_stride, max_blocks, sink, recent;
+    int tokens;  // new keys
+};
+
+template <typename V, int KS, int WD>
+__global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3, 8))) void encode_score_kernel(StepJobs js)
+{
+    static_assert(WD == 4 || WD == 2, "128- or 64-bit codes");
+    constexpr int kAhead = 4;  // codes of a thread requested in front of the hashing
+    constexpr int KP = KS * 16 + kPad, N = WD * 32;
+    constexpr int kRowPieces = KS * 2;  // 16-byte pieces of a row
+    typedef uint32_t Code __attribute__((ext_vector_type(WD)));
+    __shared__ __align__(16) uint16_t wt[WD][32 * KP];
+    __shared__ __align__(16) uint16_t rows[32 * KP];
+    __shared__ __align__(16) Code qcode[32], ncode[32];
+    __shared__ uint32_t fresh[kStepMostBS / 32];
+    __shared__ int hits[kStepTokens];
+    __shared__ int nhits;
+    __shared__ int low[kStepThreads / 64];
+    warm_args(js);
+    const int lane = threadIdx.x & 63, tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const EncArgs& kk = js.kk;
+    const int BS = js.kq.BS, h_shift = js.kq.h_shift, heads = js.kq.H;
+    const int full = 32 * WD;
+    const int b = blockIdx.y, j = blockIdx.x;
+    // past the blocks: a new key each
+    const bool is_key = j >= js.max_blocks;
+    const int64_t my_key = is_key ? (int64_t)(j - js.max_blocks) * gridDim.y + b : 0;
+    if (is_key && my_key >= js.tokens) return;
+    const int len = is_key ? 0 : js.lens[b];
+    const int64_t entry = is_key ? -1 : (js.table ? js.table[(int64_t)b * js.table_stride + j] : (int64_t)b * js.max_blocks + j);
+    const int64_t pos0 = (int64_t)j * BS;
+    if (!is_key && pos0 >= len && j > 0) return;
+    const bool usable = entry >= 0 && entry < js.kq.NBsrc;
+    const int64_t p1 = pos0 + BS < len ? pos0 + BS : len;
+    const bool forced = pos0 < js.sink || p1 > len - js.recent;
+    const bool read = usable && !forced && pos0 < len;
+    int32_t* score = js.scores + (int64_t)b * js.max_blocks + (is_key ? 0 : j);
+    if (!is_key && !read && j > 0) {
+        if (tid == 0) *score = usable ? full : -1;
+        return;
+    }
+    const int codes = read ? BS << h_shift : 0;
+    const Code* base = reinterpret_cast<const Code*>(js.kq.cache + (read ? entry : 0) * js.kq.xs_block);
+    Code kv[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+        const int i = u * kStepThreads + tid;
+        if (i < codes) kv[u] = base[i];
+    }
+    // the wave's 32 columns of the projection, an 8 x 8 patch a lane
+    u32x4 wrow[8];
+    const int patch = lane % (kRowPieces * 4), kq = patch >> 2, jc = patch & 3;
+    static_assert(kRowPieces * 4 <= 64, "a patch a lane");
+    if (wave < WD) {
+        const uint16_t* src = (const uint16_t*)js.kq.w + (int64_t)(kq * 8) * N + wave * 32 + 8 * jc;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) wrow[i] = *reinterpret_cast<const u32x4*>(src + i * N);
+    }
+    // rows of a job into LDS, 16 bytes a thread; a query group's mean to a row, rounded as in encode_small_body
+    auto stage = [&](const EncArgs& a, int64_t t, bool mean) __attribute__((always_inline)) {
+        for (int i = tid; i < heads * kRowPieces; i += kStepThreads) {
+            const int h = i / kRowPieces, c = i % kRowPieces * 8;
+            const uint16_t* src = (const uint16_t*)a.x + t * a.x_stride_t + (int64_t)h * a.x_stride_h + c;
+            V m = *reinterpret_cast<const V*>(src);
+            if (mean && a.gmean > 1) {
+                float sum[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sum[e] = (float)m[e];
+                auto add_rows = [&](int g, auto n_) __attribute__((always_inline)) {
+                    constexpr int R = decltype(n_)::value;
+                    V v[R];
+#pragma unroll
+                    for (int n = 0; n < R; ++n) v[n] = *reinterpret_cast<const V*>(src + (int64_t)(g + n) * a.x_stride_g);
+#pragma unroll
+                    for (int n = 0; n < R; ++n)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) sum[e] += (float)v[n][e];
+                };
+                int g = 1;
+                for (; g + 7 <= a.gmean; g += 7) add_rows(g, std::integral_constant<int, 7>{});
+                for (; g + 3 <= a.gmean; g += 3) add_rows(g, std::integral_constant<int, 3>{});
+                for (; g < a.gmean; ++g) add_rows(g, std::integral_constant<int, 1>{});
+                const float inv = 1.0f / (float)a.gmean;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) m[e] = (typename Mfma<V>::elem)(sum[e] * inv);
+            }
+            *reinterpret_cast<V*>(rows + h * KP + c) = m;
+        }
+    };
+    if (is_key) stage(kk, my_key, false);
+    else stage(js.kq, b, true);
+    // which of the new keys fall into this block
+    if (tid == 0) nhits = 0;
+    if (tid < kStepMostBS / 32) fresh[tid] = 0;
+    __syncthreads();
+    auto slot_of = [&](int64_t t, int64_t& blk, int64_t& tok) {
+        const int64_t s = slot_value(kk, fetch_slot(kk, t), t);
+        blk = -1;
+        tok = 0;
+        if (s >= 0) split_token(kk, s, blk, tok);
+    };
+    if (read && tid < js.tokens) {
+        int64_t blk, tok;
+        slot_of(tid, blk, tok);
+        if (blk == entry) {
+            hits[atomicAdd(&nhits, 1)] = tid;
+            atomicOr(&fresh[tok >> 5], 1u << (tok & 31));
+        }
+    }
+    // the projection as operands, by way of LDS as in encode_small_body
+    V bv[KS];
+    if (wave < WD) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
+            u32x4 o;
+            o.x = __builtin_amdgcn_perm(wrow[1][c >> 1], wrow[0][c >> 1], sel);
+            o.y = __builtin_amdgcn_perm(wrow[3][c >> 1], wrow[2][c >> 1], sel);
+            o.z = __builtin_amdgcn_perm(wrow[5][c >> 1], wrow[4][c >> 1], sel);
+            o.w = __builtin_amdgcn_perm(wrow[7][c >> 1], wrow[6][c >> 1], sel);
+            *reinterpret_cast<u32x4*>(wt[wave] + (8 * jc + c) * KP + kq * 8) = o;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            bv[ks] = *reinterpret_cast<const V*>(wt[wave] + (lane & 31) * KP + ks * 16 + (lane >> 5) * 8);
+    }
+    // codes of the staged rows, one a head (rows past the heads hold anything and are not stored)
+    auto hash = [&](Code* out) __attribute__((always_inline)) {
+        if (wave < WD) {
+            f32x16 acc = acc_start();
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                acc = Mfma<V>::run(bv[ks], *reinterpret_cast<const V*>(rows + (lane & 31) * KP + ks * 16 + (lane >> 5) * 8), acc);
+            const uint32_t half = pack_half(acc);
+            const uint32_t word = join_halves(lane >> 5 ? half << 4 : half);
+            if (lane < heads) reinterpret_cast<uint32_t*>(out + lane)[wave] = word;
+        }
+        __syncthreads();
+    };
+    hash(qcode);
+    const uint32_t* words = reinterpret_cast<const uint32_t*>(qcode);
+    if (is_key) {
+        if (tid < heads * WD) {
+            uint32_t* dst = row_dst(kk, my_key, tid / WD);
+            if (dst) dst[tid % WD] = words[tid];
+        }
+        return;
+    }
+    if (j == 0 && tid < heads * WD)
+        js.kq.out[(int64_t)b * js.kq.out_stride_t + (tid / WD) * js.kq.out_stride_h + tid % WD] = words[tid];
+    if (!read) {  // block 0, in the sink window or unusable, or of an empty request
+        if (tid == 0 && pos0 < len) *score = usable ? full : -1;
+        return;
+    }
+    int best = 0x7fffffff;
+    auto distance = [&](const Code& c, int h) {
+        int d = 0;
+#pragma unroll
+        for (int w = 0; w < WD; ++w) d += __popc(c[w] ^ qcode[h][w]);
+        return d;
+    };
+    const int seen = nhits;
+    auto add = [&](const Code& c, int i) {
+        const int tok = i >> h_shift;
+        const int d = distance(c, i & (heads - 1));
+        if (pos0 + tok < len && !(seen > 0 && ((fresh[tok >> 5] >> (tok & 31)) & 1)) && d < best) best = d;
+    };
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+        const int i = u * kStepThreads + tid;
+        if (i < codes) add(kv[u], i);
+    }
+    for (int i = kAhead * kStepThreads + tid; i < codes; i += kStepThreads) add(base[i], i);
+    for (int n = 0; n < seen; ++n) {
+        const int t = __builtin_amdgcn_readfirstlane(hits[n]);
+        stage(kk, t, false);
+        __syncthreads();
+        hash(ncode);
+        int64_t blk, tok;
+        slot_of(t, blk, tok);
+        if (tid < heads && pos0 + tok < len) {
+            const int d = distance(ncode[tid], tid);
+            best = d < best ? d : best;
+        }
+    }
+#pragma unroll
+    for (int st = 1; st < 64; st <<= 1) {
+        const int o = __shfl_xor(best, st);
+        best = o < best ? o : best;
+    }
+    if (lane == 0) low[wave] = best;
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+        for (int w = 1; w < kStepThreads / 64; ++w) best = low[w] < best ? low[w] : best;
+        *score = full - best;
     }
 }
 
@@ -3015,6 +3243,13 @@ int build_pair(const PairSpec& p, EncArgs& kk, EncArgs& kq, bool& has_keys)
     return check_cache(p.slot, p.cache, p.NB, p.BS);
 }
 
+// Blocks of a step up to which its scoring workgroups hash the queries themselves: about as many as are on the chip at
+// once (three workgroups to a compute unit with 128-bit codes, six with 64), every further generation hashes
+// again.  Step with that kernel and with the separate launches, 8 heads, blocks of 128 tokens: 128 bits, 64 blocks 7.8 and
+// 9.9 us, 512 blocks 9.2 and 10.4, 768 blocks 11.4 and 11.2, 1,024 blocks 15.4 and 12.0; 64 bits, 64 blocks 7.3 and 10.9, 512
+// blocks 8.0 and 11.7, 1,024 blocks 9.6 and 13.8, 2,048 blocks 14.8 and 16.0 (4 heads x 64 tokens 12.8 and 12.5).
+int64_t step_most_blocks(int words) { return words == 4 ? (int64_t)stream_workgroups() * 5 / 2 : (int64_t)stream_workgroups() * 6; }
+
 bool pair_is_small(const PairSpec& p, const EncArgs& kk, const EncArgs& kq, bool has_keys)
 {
     return has_keys && p.B > 0 && small_eligible(kk, p.x_dtype, p.w_dtype, false) &&
@@ -3063,6 +3298,62 @@ int launch_pair(const PairSpec& p, EncArgs& kk, EncArgs& kq, bool has_keys, hipS
     return encode_common(kq, p.x_dtype, p.w_dtype, st);
 }
 }  // namespace
+
+int step_is_fused(const PairSpec& p, const StepScore& s, bool& fused)
+{
+    EncArgs kk, kq;
+    bool has_keys;
+    fused = false;
+    int rc = stream_latch_check();
+    if (rc != UCM_OK) return rc;
+    rc = build_pair(p, kk, kq, has_keys);
+    if (rc != UCM_OK) return rc;
+    const int wd = p.N_bits / 32;
+    const bool bits = (p.K == 128 && p.N_bits == 128) || (p.K == 64 && p.N_bits == 64);
+    const bool heads = p.Hkv <= 32 && (p.Hkv & (p.Hkv - 1)) == 0;
+    const bool rows = p.cs_head == wd && p.cs_token == (int64_t)p.Hkv * wd && p.cs_block % wd == 0 &&
+                      ((uintptr_t)p.cache & (4 * wd - 1)) == 0;
+    fused = p.q_group_mean && bits && heads && rows && p.n_w == 1 && p.B > 0 && p.B <= 65535 && p.T <= kStepTokens &&
+            p.BS <= kStepMostBS && s.max_blocks > 0 && (int64_t)p.B * s.max_blocks <= step_most_blocks(wd) &&
+            small_eligible(kq, p.x_dtype, p.w_dtype, false) && (!has_keys || small_eligible(kk, p.x_dtype, p.w_dtype, false));
+    return UCM_OK;
+}
+
+int encode_and_score(const PairSpec& p, const StepScore& s, hipStream_t st)
+{
+    StepJobs js{};
+    bool has_keys;
+    int rc = build_pair(p, js.kk, js.kq, has_keys);
+    if (rc != UCM_OK) return rc;
+    if (has_keys) {
+        set_block_shift(js.kk);
+        js.tokens = (int)p.T;
+    }
+    uint32_t* codes = js.kq.out;
+    set_block_shift(js.kq);
+    // the kernel stores the query codes itself: the query job's cache fields are the code cache's
+    js.kq.out = codes;
+    js.kq.cache = p.cache;
+    js.kq.xs_block = p.cs_block;
+    js.kq.NBsrc = p.NB;
+    js.kq.BS = p.BS;
+    js.table = s.table;
+    js.table_stride = s.table_stride;
+    js.max_blocks = s.max_blocks;
+    js.lens = s.lens;
+    js.scores = s.scores;
+    js.sink = s.sink;
+    js.recent = s.recent;
+    const int keys = (int)ceil_div(js.tokens, p.B);
+    const dim3 grid((unsigned)(s.max_blocks + keys), (unsigned)p.B);
+    note_encode("encode_score", p.N_bits / 32);
+    const bool bf = p.x_dtype == UCM_DT_BF16;
+    if (p.K == 128 && bf) hipLaunchKernelGGL((encode_score_kernel<bf16x8, 8, 4>), grid, dim3(kStepThreads), 0, st, js);
+    else if (p.K == 128) hipLaunchKernelGGL((encode_score_kernel<f16x8, 8, 4>), grid, dim3(kStepThreads), 0, st, js);
+    else if (bf) hipLaunchKernelGGL((encode_score_kernel<bf16x8, 4, 2>), grid, dim3(kStepThreads), 0, st, js);
+    else hipLaunchKernelGGL((encode_score_kernel<f16x8, 4, 2>), grid, dim3(kStepThreads), 0, st, js);
+    return launch_status("encode_score_kernel");
+}
 
 int encode_pair(const PairSpec& p, hipStream_t st)
 {
