@@ -198,6 +198,86 @@ def test_rows_of_512_values_by_tile_shape(T, N, H, BS, dtype, route):
         assert_codes_match(np.ascontiguousarray(flat[slot[rows], h]).view(np.uint8), xs[:, h], W.float().numpy())
 
 
+@pytest.mark.parametrize("D,H,BS,T,dtype", [
+    (128, 1, 32, 1, torch.bfloat16), (128, 8, 128, 130, torch.bfloat16), (64, 3, 96, 1000, torch.float16),
+    (128, 3, 32, 8001, torch.float16), (64, 8, 64, 17000, torch.bfloat16),   # one tile a wave, two for some
+    (128, 2, 128, 200001, torch.bfloat16),                                    # several tiles a wave, waves side by side
+    (128, 8, 128, 530000, torch.bfloat16),                                    # more than the 64 whose blocks a wave holds
+])
+def test_rehash_of_rows_side_by_side(D, H, BS, T, dtype):
+    """The streaming rehash: block ids outside the cache, a last block part full, zero and NaN rows, an untouched
+    rest of the code cache.  Rows checked are the first, the last and a sample."""
+    from ucm_amd import _lib
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + D)
+    nb = -(-T // BS)
+    kv = torch.randn(nb + 1, BS, H, D, generator=g, device="cuda", dtype=dtype)
+    W = torch.from_numpy(rng_for(D + T).standard_normal((D, D)).astype(np.float32)).to(dtype)
+    ids = torch.randperm(nb + 1, generator=g, device="cuda")[:nb].to(torch.int32)
+    used = ids.cpu().numpy().copy()
+    if nb > 5:
+        ids[2], ids[4] = -1, nb + 1
+        used[[2, 4]] = -1
+        kv[int(used[1]), 1] = 0.0
+        kv[int(used[1]), 2, :, 3] = float("nan")
+    enc = make_encoder(D, D, dtype, W)
+    fill = 0x55AA55AA
+    cache = torch.full((nb + 1, BS, H, D // 32), fill, dtype=torch.int32, device="cuda")
+    enc.compute_hash_from_paged_cache(kv, ids, T, cache, block_size=BS)
+    assert _lib.last_encode() == "encode_run<%d,1>" % D
+    t = np.unique(np.concatenate([np.arange(min(T, 300)), [T - 1, T - min(T, 40)], rng_for(T).integers(0, T, 3000)]))
+    t = t[used[t // BS] >= 0]
+    blk, tok = used[t // BS], t % BS
+    b_t, k_t = torch.from_numpy(blk).long().cuda(), torch.from_numpy(tok).cuda()
+    got, x = cache[b_t, k_t].cpu().numpy(), kv[b_t, k_t].float().cpu().numpy()
+    nan = np.isnan(x).any(axis=(1, 2))
+    assert not got[nan].any()
+    for h in range(H):
+        assert_codes_match(np.ascontiguousarray(got[~nan, h]).view(np.uint8), x[~nan, h], W.float().numpy())
+    untouched = torch.ones(nb + 1, BS, dtype=torch.bool, device="cuda")
+    full = torch.from_numpy(used[:nb - 1][used[:nb - 1] >= 0]).long().cuda()
+    untouched[full] = False
+    if used[nb - 1] >= 0:
+        untouched[int(used[nb - 1]), :T - (nb - 1) * BS] = False
+    assert (cache[untouched] == fill).all()
+
+
+@pytest.mark.parametrize("D,H,T,slots,side,route", [
+    (128, 8, 1301, "i64", 0, "encode_run<128,0>"), (128, 3, 9001, "i32", 0, "encode_run<128,0>"),  # rows that 32 does not divide
+    (64, 1, 30001, "i64", 1, "encode_run<64,0>"),    # codes that are not aligned
+    (128, 1, 65536, "dense", 0, "encode_run<128,0>"), (128, 1, 65537, "i64", 0, "encode_mfma<4,1,1>"),  # a tile to every wave, one more
+])
+def test_rows_side_by_side_by_slot(D, H, T, slots, side, route):
+    from ucm_amd import _lib
+
+    BS = 48
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + D)
+    x = torch.randn(T, H, D, generator=g, device="cuda", dtype=torch.bfloat16)
+    W = torch.from_numpy(rng_for(D + T).standard_normal((D, D)).astype(np.float32)).to(torch.bfloat16)
+    enc = make_encoder(D, D, torch.bfloat16, W)
+    nb = -(-T // BS)
+    slot = rng_for(T).permutation(nb * BS)[:T].astype(np.int64)
+    if slots == "dense":
+        got = enc.compute_hash(x, per_head=True).cpu().numpy().reshape(T, H, D // 8)
+        slot[:] = 0
+    else:
+        slot[5::9] = -1
+        cache = torch.zeros((nb, BS, H, D // 32 + side), dtype=torch.int32, device="cuda")
+        enc.compute_hash_and_cache(x, torch.from_numpy(slot).to(torch.int64 if slots == "i64" else torch.int32).cuda(),
+                                   cache[..., side:], block_size=BS)
+        flat = cache.cpu().numpy().reshape(nb * BS, H, D // 32 + side)
+        assert not flat[np.setdiff1d(np.arange(nb * BS), slot)].any() and not flat[..., :side].any()
+        got = np.ascontiguousarray(flat[np.maximum(slot, 0)][..., side:]).view(np.uint8)
+    assert _lib.last_encode() == route
+    keep = np.flatnonzero(slot >= 0)
+    keep = np.unique(np.concatenate([keep[:500], keep[-100:], rng_for(T + 1).choice(keep, 2000)]))
+    xs = x.float().cpu().numpy()[keep]
+    for h in range(H):
+        assert_codes_match(np.ascontiguousarray(got[keep, h]), xs[:, h], W.float().numpy())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("slot_dtype", [torch.int32, torch.int64])
 def test_compute_hash_and_cache(dtype, slot_dtype):

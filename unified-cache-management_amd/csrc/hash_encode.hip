@@ -1779,6 +1779,224 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(1,
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// Rows that lie side by side in blocks of a paged cache (a prefix that is hashed where it lies), as many hash bits as
+// channels: 32 rows are one run of memory, and so are their codes.
+//
+// What bounds it is memory, so it is built to have it busy from the start: every wave streams tiles of 32 rows
+// through two slots of its own in LDS (load-to-LDS, whole lines, 128 KiB on their way in a compute unit) and meets
+// the others once, when the projection is there; its operands then stay in registers.  Rows change the place of their
+// 16-byte pieces so that the operand reads find every bank once.  Before (encode_mfma_kernel, whose workgroups transpose
+// the projection through registers in front of their first rows) and now: 16,384 rows of 128 channels 5.0 and 3.3 us,
+// 65,536 rows 6.7 and 5.5, 261,528 rows 20.2 and 16.0 (4.2 TB/s), 1,048,000 rows 64.4 and 60.9; 64 channels, 65,536 rows 5.5
+// and 3.1, 262,144 rows 9.9 and 8.6.  By slot, 16,384 rows of 128 channels 4.8 and 3.5, of 64 channels 65,536 rows 5.4 and 3.3.
+// ---------------------------------------------------------------------------------------
+constexpr int kRunWaves = 8;
+constexpr int kRunSlots = 2;
+constexpr int run_tile_bytes(int ks) { return 32 * ks * 32; }
+constexpr int run_lds(int ks) { return kRunWaves * kRunSlots * run_tile_bytes(ks) + ks * 16 * ks * 32; }
+
+// Four loads of 16 bytes a lane to 4 KiB of LDS, from 4 KiB at base in four orders of a lane's pieces.
+__device__ __forceinline__ void run_load4(uint32_t lds, uint64_t base, const uint32_t (&o)[4])
+{
+    uint32_t keep;
+    asm volatile("s_mov_b32 %[keep], m0\n\ts_mov_b32 m0, %[lds]\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %[o0], %[base]\n\t"
+                 "global_load_lds_dwordx4 %[o1], %[base] offset:1024\n\t"
+                 "global_load_lds_dwordx4 %[o2], %[base] offset:2048\n\t"
+                 "global_load_lds_dwordx4 %[o3], %[base] offset:3072\n\t"
+                 "s_mov_b32 m0, %[keep]\n\t"
+                 : [keep] "=&s"(keep)
+                 : [lds] "s"(lds), [base] "s"(base), [o0] "v"(o[0]), [o1] "v"(o[1]), [o2] "v"(o[2]), [o3] "v"(o[3])
+                 : "memory");
+}
+
+// The same with lane offsets that hold all of the distance from base.
+__device__ __forceinline__ void run_load4_from(uint32_t lds, uint64_t base, const uint32_t (&o)[4])
+{
+    pipe_load(lds, base, o[0], base, o[1]);
+    pipe_load(lds + 2048, base, o[2], base, o[3]);
+}
+
+// PAGED: block_tiles tiles to a block of a paged input; otherwise rows that lie side by side from x on, one tile to a wave,
+// whose codes go where the slots say.
+template <typename V, int KS, bool PAGED>
+__global__ __launch_bounds__(64 * kRunWaves) __attribute__((amdgpu_waves_per_eu(KS == 8 ? 2 : 4, KS == 8 ? 2 : 4))) void encode_run_kernel(EncArgs a, uint32_t tiles, uint32_t block_tiles, uint32_t wg_tiles, uint32_t wave_tiles)
+{
+    constexpr int K = KS * 16, NT = KS / 2, kTile = run_tile_bytes(KS), kLoads = kTile / 1024;
+    constexpr int kPieces = KS * 2;  // of a row
+    static_assert(KS == 8 || KS == 4, "128 or 64 channels");
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* tr_ptr;
+    typedef __attribute__((address_space(3))) const V* row_ptr;
+    typedef uint32_t Code __attribute__((ext_vector_type(NT)));
+    extern __shared__ __align__(16) uint16_t wt[];
+    warm_args(a);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)wt);
+    const uint32_t wlds = lds0 + kRunWaves * kRunSlots * kTile;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, kb = lane >> 5;
+    const uint32_t step = gridDim.x * kRunWaves;
+    uint32_t first = blockIdx.x * wg_tiles + wave * wave_tiles;  // of up to 64 tiles whose block ids the lanes hold
+    uint32_t ids = 0, in_block = 0;
+    auto look_up = [&]() __attribute__((always_inline)) {
+        uint32_t t = first + (uint32_t)lane * step;
+        t = t < tiles && t >= first ? t : tiles - 1;
+        const uint32_t bi = t / block_tiles;
+        in_block = t - bi * block_tiles;
+        ids = (uint32_t)a.src_blocks[bi];
+    };
+    const int64_t rows = a.T * a.H;
+    if (PAGED) look_up();
+    const int64_t my_row = (int64_t)first * 32 + r;
+    int64_t my_t = my_row < rows ? my_row : rows - 1;
+    int my_h = 0;
+    if (!PAGED) {
+        if (a.h_shift >= 0) {
+            my_h = (int)(my_t & (a.H - 1));
+            my_t >>= a.h_shift;
+        } else {
+            const uint32_t t = (uint32_t)my_t / (uint32_t)a.H;  // 2,048 tiles at most
+            my_h = (int)((uint32_t)my_t - t * (uint32_t)a.H);
+            my_t = t;
+        }
+    }
+    {
+        // the projection: rows of 2 N bytes, 64-byte units changed over by k % 4 (128 columns) or k / 2 % 2 (64)
+        constexpr int kRowLanes = NT * 4, kPer = 64 / kRowLanes, kWLoads = KS * 16 / kPer / kRunWaves;
+        const int k = lane / kRowLanes, p = lane % kRowLanes;
+        const int turn = NT == 4 ? (k & 3) : ((k >> 1) & 1);
+        const uint32_t off = (uint32_t)(k * NT * 64 + (p ^ (turn << 2)) * 16);
+        const uint64_t from = (uint64_t)(uintptr_t)a.w + (uint64_t)wave * (kWLoads * 1024);
+        if constexpr (kWLoads == 4) {
+            const uint32_t o[4] = {off, off, off, off};
+            run_load4(wlds + wave * 4096, from, o);
+        } else {
+            static_assert(kWLoads == 1 || kWLoads == 4, "the waves share the projection's loads");
+            uint32_t keep;
+            asm volatile("s_mov_b32 %[keep], m0\n\ts_mov_b32 m0, %[lds]\n\ts_nop 0\n\t"
+                         "global_load_lds_dwordx4 %[o], %[base]\n\t"
+                         "s_mov_b32 m0, %[keep]\n\t"
+                         : [keep] "=&s"(keep)
+                         : [lds] "s"(wlds + wave * 1024), [base] "s"(from), [o] "v"(off)
+                         : "memory");
+        }
+    }
+    // piece p of row i lies at place p ^ i % 16 (of sixteen pieces) or p ^ i / 2 % 8 (of eight)
+    uint32_t xoff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = i * (64 / kPieces) + lane / kPieces;
+        const int turn = KS == 8 ? row & 15 : (row >> 1) & 7;
+        xoff[i] = (uint32_t)(lane / kPieces * K * 2 + ((lane % kPieces) ^ turn) * 16);
+    }
+    const uint32_t ring = lds0 + wave * (kRunSlots * kTile);
+    auto issue = [&](int n) __attribute__((always_inline)) {  // tile `first + n step`, n < 64
+        if (!PAGED) {
+            const uint64_t base = uniform64((uint64_t)(uintptr_t)a.x + (uint64_t)first * kTile);
+            const int64_t left = rows - (int64_t)first * 32;
+            if (left >= 32) {
+#pragma unroll
+                for (int i = 0; i < kLoads; i += 4) run_load4(ring + i * 1024, base + i * 1024, xoff);
+            } else {  // rows past the last one read that one again; their codes are not stored
+#pragma unroll
+                for (int i = 0; i < kLoads; i += 4) {
+                    uint32_t o[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const int row = (i + c) * (64 / kPieces) + lane / kPieces;
+                        o[c] = (uint32_t)(row < left ? row : (int)left - 1) * (K * 2) + xoff[c] % (K * 2);
+                    }
+                    run_load4_from(ring + i * 1024, base, o);
+                }
+            }
+            return;
+        }
+        int64_t blk = (int32_t)__builtin_amdgcn_readlane(ids, n);
+        if (blk < 0 || blk >= a.NBsrc) blk = 0;  // dropped when its codes are stored
+        const uint64_t base = uniform64((uint64_t)(uintptr_t)((const uint16_t*)a.x + blk * a.xs_block) +
+                                        (uint64_t)(uint32_t)__builtin_amdgcn_readlane(in_block, n) * kTile);
+#pragma unroll
+        for (int i = 0; i < kLoads; i += 4) run_load4(ring + (n & 1) * kTile + i * 1024, base + i * 1024, xoff);
+    };
+    // tiles of this wave among the 64
+    auto mine = [&]() { return first < tiles ? (int)((tiles - 1 - first) / step + 1 < 64 ? (tiles - 1 - first) / step + 1 : 64) : 0; };
+    int count = mine();
+    if (count > 0) issue(0);
+    if (count > 1) issue(1);
+    // the projection's loads are older than the rows'
+    if (count > 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * kLoads) : "memory");
+    else if (count > 0) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (count == 0) return;
+    V bv[NT][KS];
+    {
+        const int tk = (lane >> 2) & 3;
+        const uint32_t at = wlds + (kb * 8 + tk) * (NT * 64) + ((NT == 4 ? tk : tk >> 1) << 6) + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                s16x4 half[2];
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+                    half[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(uintptr_t)((at ^ (q << 6)) + (ks * 16 + p * 4) * (NT * 64)));
+                __builtin_memcpy(&bv[q][ks], half, 16);
+            }
+    }
+    const uint32_t xat = ring + r * (K * 2) + ((kb ^ (KS == 8 ? r & 15 : (r >> 1) & 7)) << 4);
+    RawSlot raw{0, 0};
+    if (!PAGED) raw = fetch_slot(a, my_t);
+    while (true) {
+        for (int n = 0; n < count; ++n) {
+            if (n + 1 < count) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            V x[KS];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) x[ks] = *(row_ptr)(uintptr_t)((xat ^ (ks << 5)) + (n & 1) * kTile);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (n + 2 < count) issue(n + 2);
+            Code words;
+#pragma unroll
+            for (int q = 0; q < NT; q += 2) {
+                f32x16 acc0 = acc_start(), acc1 = acc_start();
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    acc0 = Mfma<V>::run(bv[q][ks], x[ks], acc0);
+                    acc1 = Mfma<V>::run(bv[q + 1][ks], x[ks], acc1);
+                }
+                const uint32_t h0 = pack_half(acc0), h1 = pack_half(acc1);
+                words[q] = join_halves(kb ? h0 << 4 : h0);
+                words[q + 1] = join_halves(kb ? h1 << 4 : h1);
+            }
+            if constexpr (!PAGED) {
+                uint32_t* dst = lane < 32 && my_row < rows ? slot_dst(a, slot_value(a, raw, my_t), my_h) : nullptr;
+                if (dst) {
+                    if (((uintptr_t)dst & (sizeof(Code) - 1)) == 0) {
+                        *reinterpret_cast<Code*>(dst) = words;
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < NT; ++q) dst[q] = words[q];
+                    }
+                }
+                return;
+            }
+            const int64_t blk = (int32_t)__builtin_amdgcn_readlane(ids, n);
+            const uint32_t at = (uint32_t)__builtin_amdgcn_readlane(in_block, n) * 32 + r;  // the row in its block
+            const int64_t row = (int64_t)(first + (uint32_t)n * step) * 32 + r;
+            if (lane < 32 && row < rows && blk >= 0 && blk < a.NBsrc && blk < a.NB)
+                *reinterpret_cast<Code*>(a.cache + blk * a.cs_block + (int64_t)at * NT) = words;
+        }
+        if (tiles - first <= (uint64_t)step * 64) break;
+        first += step * 64;
+        look_up();
+        count = mine();
+        issue(0);
+        if (count > 1) issue(1);
+    }
+}
+
 // Latency path for a handful of rows (decode): one wave per (job, head, 32 hash columns,
 // 32 rows).  No LDS and no persistent loop: the B operand is assembled straight from the
 // row-major projection matrix with eight 2-byte loads per k-step, all issued up front, so the
@@ -2949,6 +3167,54 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype, bool alone = tru
     return small_us < lds_floor_us;
 }
 
+// Rows that lie side by side: all of them, a tile of 32 to a wave at most and more than the latency path's, or those of a
+// paged input's blocks with their codes, of any number (64 to 130 rows of 128 channels x 8 heads 3.1 against 3.4 us of the
+// small-row kernel).
+bool run_eligible(const EncArgs& a, int x_dtype, int w_dtype)
+{
+    if (!mfma_eligible(a, x_dtype, w_dtype)) return false;
+    if (!((a.K == 128 && a.N == 128) || (a.K == 64 && a.N == 64))) return false;
+    const int words = a.N / 32;
+    if (!(a.n_w == 1 || a.heads_per_w <= 0 || a.heads_per_w >= a.H)) return false;
+    if ((a.H > 1 && a.x_stride_h != a.K) || a.x_stride_t != (int64_t)a.H * a.K) return false;
+    if (!a.src_blocks) return a.T * a.H <= (int64_t)stream_workgroups() * kRunWaves * 32;
+    if ((a.H > 1 && a.cs_head != words) || a.cs_token != (int64_t)a.H * words) return false;
+    if (((uintptr_t)a.cache & (4 * words - 1)) || a.cs_block % words) return false;
+    return a.T * a.H < ((int64_t)1 << 35);  // tiles are counted in 32 bits
+}
+
+template <typename V, int KS, bool PAGED>
+int launch_run_ks(const EncArgs& a, hipStream_t st)
+{
+    constexpr int lds = run_lds(KS);
+    static int opted = 0;  // 0 = not tried, 1 = allowed, -1 = refused by the runtime
+    if (opted == 0) {
+        const hipError_t e = hipFuncSetAttribute((const void*)encode_run_kernel<V, KS, PAGED>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) (void)hipGetLastError();
+        opted = (e == hipSuccess) ? 1 : -1;
+    }
+    if (opted < 0) return UCM_EUNSUPPORTED;
+    const int64_t tiles = ucm::ceil_div(a.T * a.H, 32);
+    const int64_t most = (int64_t)stream_workgroups() * (PAGED && KS == 4 ? 2 : 1);  // as many as its LDS lets a compute unit hold
+    // Few tiles go to as many compute units as there are, one wave of each after the other; many to the waves of a
+    // workgroup side by side, whose codes then meet in one L2.  16,384 rows of 128 channels by slot 3.5 against 4.4 us side by
+    // side, 40,000 rows 4.6 and 5.0, 64,000 rows 6.2 and 5.8.
+    const bool side_by_side = tiles > 6 * (int64_t)stream_workgroups();
+    const int64_t want = side_by_side ? ucm::ceil_div(tiles, kRunWaves) : tiles;
+    const int64_t wgs = want < most ? want : most;
+    note_encode("encode_run", KS * 16, PAGED);
+    hipLaunchKernelGGL((encode_run_kernel<V, KS, PAGED>), dim3((unsigned)wgs), dim3(64 * kRunWaves), lds, st, a, (uint32_t)tiles,
+                       (uint32_t)((int64_t)a.BS * a.H / 32), side_by_side ? kRunWaves : 1u, side_by_side ? 1u : (uint32_t)wgs);
+    return ucm::launch_status("encode_run_kernel");
+}
+
+template <typename V>
+int launch_run(const EncArgs& a, hipStream_t st)
+{
+    if (a.src_blocks) return a.K == 128 ? launch_run_ks<V, 8, true>(a, st) : launch_run_ks<V, 4, true>(a, st);
+    return a.K == 128 ? launch_run_ks<V, 8, false>(a, st) : launch_run_ks<V, 4, false>(a, st);
+}
+
 // ---- the streaming kernel's time-out latch ----
 // A wave of the streaming kernel whose bounded wait gave up sets a word in pinned host memory (one
 // per device, allocated with the first streaming launch on it).  Every encode entry point reads that
@@ -3021,7 +3287,8 @@ int encode_common(EncArgs a, int x_dtype, int w_dtype, hipStream_t st)
     if (rc != UCM_OK) return rc;
     if (a.T == 0) return UCM_OK;
 
-    if (small_eligible(a, x_dtype, w_dtype)) {
+    const bool run = run_eligible(a, x_dtype, w_dtype);
+    if (!(run && a.src_blocks) && small_eligible(a, x_dtype, w_dtype)) {
         EncJobs js{};
         js.job[0] = a;
         js.job[1] = a;
@@ -3037,6 +3304,11 @@ int encode_common(EncArgs a, int x_dtype, int w_dtype, hipStream_t st)
     if (stream_eligible(a, x_dtype, w_dtype)) {
         a.timeout_flag = stream_latch_flag();
         rc = x_dtype == UCM_DT_BF16 ? launch_stream<bf16x8>(a, st) : launch_stream<f16x8>(a, st);
+        if (rc != UCM_EUNSUPPORTED) return rc;  // no large-LDS opt-in: the tiled kernel below
+        ucm::clear_error();
+    }
+    if (run) {
+        rc = x_dtype == UCM_DT_BF16 ? launch_run<bf16x8>(a, st) : launch_run<f16x8>(a, st);
         if (rc != UCM_EUNSUPPORTED) return rc;  // no large-LDS opt-in: the tiled kernel below
         ucm::clear_error();
     }
