@@ -120,6 +120,27 @@ def test_generic_path_matches_oracle(seed, B, Hq, Hkv, Wd, BS, lens, k):
     check(q, kc, table, lens, k, reduce_heads=True, score_order=True)
 
 
+@pytest.mark.parametrize("Hq,Hkv,BS,lens,k", [
+    (2, 2, 8, [64, 30], 4), (8, 4, 48, [1000, 5, 0, 333], 6), (32, 8, 128, [5000, 4097, 128], 12),
+    (64, 8, 64, [3000, 2990], 9), (16, 16, 16, [700, 17], 8), (64, 32, 32, [900], 5), (4, 2, 4096, [9000, 4100], 2),
+    (32, 8, 32, [20000, 9000], 100),  # a longer row for the selection
+])
+def test_64_bit_codes_of_several_heads(Hq, Hkv, BS, lens, k):
+    """A wave to a block: blocks of less than a load, ragged ends, forced and unusable blocks, lists per head and one
+    for all."""
+    from ucm_amd import _lib
+
+    q, kc, table, lens = make_paged_case(Hq * 101 + Hkv + BS, len(lens), Hq, Hkv, 2, BS, lens, table_pad=1)
+    table[0, 1] = -1
+    if table.shape[1] > 4:
+        table[0, 3] = kc.shape[0]
+    for sink, recent in ((0, 0), (BS, 2 * BS)):
+        check(q, kc, table, lens, k, sink, recent)
+        assert _lib.last_dispatch().startswith("block_score_half<%d>+" % (Hq // Hkv))
+        check(q, kc, table, lens, k, sink, recent, reduce_heads=True, return_physical=True)
+        check(q, kc, table, lens, k, sink, recent, reduce_heads=True, score_order=True)
+
+
 def test_head_major_cache_layout():
     q, kc, table, lens = make_paged_case(301, 2, 32, 8, 4, 128, [700, 1500])
     check(q, kc, table, lens, 4, head_major=True)

@@ -2076,6 +2076,87 @@ __global__ __launch_bounds__(kStripWaves * kWave) __attribute__((amdgpu_waves_pe
 }
 
 // ---------------------------------------------------------------------------------------
+// 64-bit codes of an even number of KV heads (64-dimensional heads): a 16-byte piece is the codes of two heads of a
+// token, a wave scores a block by itself - a lane keeps its pair of heads, so that its query codes stay in
+// registers and the minima meet in shuffles, without LDS or a barrier - and requests eight pieces a lane at a
+// time.  Blocks whose score is settled read nothing.  What bounds it is memory and the launches around it.  The whole step
+// with block_score_generic, which took these (a thread to a code, word by word, an LDS atomic for each), and
+// with this: 32 x 32,768 tokens x 8 heads 29.6 and 18.0 us, 22 x up to 44,810 tokens in blocks of 32 33.9 and 25.1, 16 x up to
+// 65,856 tokens with 8 query heads to each 43.2 and 26.6, 2 x 65,856 tokens with 4 14.1 and 13.0.
+// ---------------------------------------------------------------------------------------
+template <int G>
+__global__ __launch_bounds__(kThreads) void block_score_half(ScoreArgs a, int pair_shift)
+{
+    constexpr int kAhead = 8;
+    const int b = blockIdx.y, j = blockIdx.x * (kThreads / kWave) + wave_id();
+    const int lane = lane_id();
+    const int len = a.lens[b];
+    const int jc = j < a.max_blocks ? j : a.max_blocks - 1;
+    const int64_t pb = physical_block(a, b, jc);
+    const int pairs = 1 << pair_shift, pair = lane & (pairs - 1);
+    uint32_t q[2][G][2];
+    {
+        const uint32_t* qp = a.q + b * a.q_stride_b + (int64_t)(2 * pair * G) * a.q_stride_h;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int w = 0; w < 2; ++w) q[h][g][w] = qp[(h * G + g) * a.q_stride_h + w];
+    }
+    const int pos0 = jc * a.BS;
+    if (j >= a.max_blocks || pos0 >= len) return;
+    const int full = G * 64;
+    const int p1 = pos0 + a.BS < len ? pos0 + a.BS : len;
+    const bool forced = pos0 < a.sink || p1 > len - a.recent;
+    int m[2] = {kInf, kInf};
+    if (pb >= 0 && !forced) {
+        const int pieces = a.BS << pair_shift;
+        const u32x4* base = reinterpret_cast<const u32x4*>(a.kc + pb * a.ks_block);
+        for (int i0 = lane; i0 < pieces; i0 += kWave * kAhead) {
+            u32x4 kv[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) kv[u] = code_load(base + (i0 + u * kWave < pieces ? i0 + u * kWave : i0));
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int i = i0 + u * kWave;
+                const bool seen = i < pieces && pos0 + (i >> pair_shift) < len;
+                int d0 = 0, d1 = 0;
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    d0 = popc_add(kv[u].y ^ q[0][g][1], popc_add(kv[u].x ^ q[0][g][0], d0));
+                    d1 = popc_add(kv[u].w ^ q[1][g][1], popc_add(kv[u].z ^ q[1][g][0], d1));
+                }
+                m[0] = seen && d0 < m[0] ? d0 : m[0];
+                m[1] = seen && d1 < m[1] ? d1 : m[1];
+            }
+        }
+    }
+    for (int st = pairs; st < kWave; st <<= 1) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int o = __shfl_xor(m[h], st);
+            m[h] = o < m[h] ? o : m[h];
+        }
+    }
+    if (a.reduce_out) {
+        // one list per request: the best head
+        int best = m[0] < m[1] ? m[0] : m[1];
+        for (int st = 1; st < pairs; st <<= 1) {
+            const int o = __shfl_xor(best, st);
+            best = o < best ? o : best;
+        }
+        if (lane == 0) a.scores[(int64_t)b * a.max_blocks + j] = pb < 0 ? -1 : (forced ? full : full - best);
+        return;
+    }
+    if (lane < pairs) {
+        int32_t* out = a.scores + (int64_t)b * a.Hkv * a.max_blocks + (int64_t)j * a.sc_j;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) out[(int64_t)(2 * lane + h) * a.sc_h] = pb < 0 ? -1 : (forced ? full : full - m[h]);
+    }
+}
+
+// ---------------------------------------------------------------------------------------
 // Generic block scorer: any strides, code width, head count and group size.  One thread per
 // (token, head) code, word-by-word loads; query codes staged in LDS.
 // ---------------------------------------------------------------------------------------
@@ -3007,6 +3088,14 @@ bool pairs_layout(const ScoreArgs& a, const uint32_t* k_cache)
            a.ks_block % 2 == 0 && (reinterpret_cast<uintptr_t>(k_cache) & 7) == 0;
 }
 
+// 64-bit codes of 2 to 32 heads side by side, for block_score_half (whose waves take a block each: up to 64 KiB)
+bool half_layout(const ScoreArgs& a, const uint32_t* k_cache)
+{
+    return a.Wd == 2 && a.Hkv >= 2 && a.Hkv <= 32 && is_pow2(a.Hkv) && (a.G == 1 || a.G == 2 || a.G == 4 || a.G == 8) &&
+           a.ks_head == 2 && a.ks_token == (int64_t)a.Hkv * 2 && a.ks_block % 4 == 0 &&
+           (reinterpret_cast<uintptr_t>(k_cache) & 15) == 0 && (int64_t)a.BS * a.Hkv <= 8192;
+}
+
 int common_checks(const uint32_t* q, const uint32_t* kc, const int32_t* lens, int64_t NB, int BS,
                   int Hkv, int Wd, int B, int Hq, int max_blocks)
 {
@@ -3119,6 +3208,22 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
         rc = ucm::encode_and_score(*fused, sc, st);
         if (rc != UCM_OK) return rc;
         reduced_scores = true;
+    } else if (half_layout(a, k_cache)) {
+        note_score("block_score_half", a.G);
+        a.reduce_out = (flags & UCM_TOPK_REDUCE_HEADS) ? 1 : 0;
+        reduced_scores = a.reduce_out != 0;
+        if (wave_select && !a.reduce_out) {
+            a.sc_h = 1;
+            a.sc_j = Hkv;
+        }
+        int pair_shift = 0;
+        while ((2 << pair_shift) < Hkv) ++pair_shift;
+        const dim3 hgrid((unsigned)ucm::ceil_div(max_blocks, kThreads / kWave), (unsigned)B);
+        if (a.G == 1) launch_score(block_score_half<1>, hgrid, 0, st, a, pair_shift);
+        else if (a.G == 2) launch_score(block_score_half<2>, hgrid, 0, st, a, pair_shift);
+        else if (a.G == 4) launch_score(block_score_half<4>, hgrid, 0, st, a, pair_shift);
+        else launch_score(block_score_half<8>, hgrid, 0, st, a, pair_shift);
+        a.reduce_out = 0;
     } else if (fast && !one_head_planes) {
         int pmax = planes_for_group(a.G);
         const bool direct = a.G == 1 || a.G == 2 || a.G == 4;

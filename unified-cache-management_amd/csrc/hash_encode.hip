@@ -3516,11 +3516,11 @@ int build_pair(const PairSpec& p, EncArgs& kk, EncArgs& kq, bool& has_keys)
 }
 
 // Blocks of a step up to which its scoring workgroups hash the queries themselves: about as many as are on the chip at
-// once (three workgroups to a compute unit with 128-bit codes, six with 64), every further generation hashes
+// once (three workgroups to a compute unit with 128-bit codes, four with 64), every further generation hashes
 // again.  Step with that kernel and with the separate launches, 8 heads, blocks of 128 tokens: 128 bits, 64 blocks 7.8 and
-// 9.9 us, 512 blocks 9.2 and 10.4, 768 blocks 11.4 and 11.2, 1,024 blocks 15.4 and 12.0; 64 bits, 64 blocks 7.3 and 10.9, 512
-// blocks 8.0 and 11.7, 1,024 blocks 9.6 and 13.8, 2,048 blocks 14.8 and 16.0 (4 heads x 64 tokens 12.8 and 12.5).
-int64_t step_most_blocks(int words) { return words == 4 ? (int64_t)stream_workgroups() * 5 / 2 : (int64_t)stream_workgroups() * 6; }
+// 9.9 us, 512 blocks 9.2 and 10.4, 768 blocks 11.4 and 11.2, 1,024 blocks 15.4 and 12.0; 64 bits, 64 blocks 7.5 and 10.4,
+// 1,024 blocks 9.4 and 10.3, 2,048 blocks 14.5 and 11.9.
+int64_t step_most_blocks(int words) { return (int64_t)stream_workgroups() * (words == 4 ? 5 : 9) / 2; }
 
 bool pair_is_small(const PairSpec& p, const EncArgs& kk, const EncArgs& kq, bool has_keys)
 {
