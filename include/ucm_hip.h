@@ -97,8 +97,9 @@ int ucm_hash_encode_set_stream_threshold(int64_t rows);
 /*
  * Test hook, no counterpart in the reference.  Writes the name of the kernel that the last ucm_hash_encode,
  * ucm_hash_encode_cache or ucm_hash_encode_paged on the calling thread launched, e.g. "encode_small",
- * "encode_mfma<4,1,8>" (column tiles per group, groups per slice, row tiles per workgroup) or
- * "encode_slice<2>" (column tiles per slice), cut to cap - 1 characters.  Returns the full length.  The kernels
+ * "encode_mfma<4,1,8>" (column tiles per group, groups per slice, row tiles per workgroup), "encode_slice<2>"
+ * (column tiles per slice), "encode_pipe<4,8>" (column tiles, waves) or "encode_run<128,1>" (dimensions, paged
+ * input), cut to cap - 1 characters.  Returns the full length.  The kernels
  * give the same codes at very different speeds; this lets a test pin which one a shape takes.
  */
 int64_t ucm_hash_encode_last_dispatch(char* buf, size_t cap);
@@ -305,7 +306,7 @@ int ucm_hamming_topk_set_clock_probe(void* two_u64_in_device_memory);
  * ucm_hamming_score call on the calling thread launched, e.g.
  * "block_score_one<1,8,1,4,1>+select_wave_kernel<4>" or
  * "plane_kernel+block_score_lanes<4,0,8>+select_wave_kernel<4>" (family, then its template
- * arguments), cut to cap - 1 characters.  Returns the full length.  Several kernel families give
+ * arguments; "encode_score<4>" where a decode step hashes and scores in one kernel), cut to cap - 1 characters.  Returns the full length.  Several kernel families give
  * the same results at very different speeds; this lets a test pin which one a shape takes.
  */
 int64_t ucm_hamming_last_dispatch(char* buf, size_t cap);
@@ -374,7 +375,8 @@ int ucm_sparse_decode_step_mla(const void* new_nope, int64_t nope_stride_t,
  * form its attention backend reads: replaces GSAOnDevice.attention_begin at decode
  * (ucm/sparse/gsa_on_device/gsa_on_device.py:564-572 cache_k_hash_gqa_cuda, :396-412 hash_code,
  * :773-811 update_decode_topk_gqa_cuda) and cuda_hamming_topk / update_seq_lens
- * (hamming_topk.py:7-54) — a dozen framework launches there, three kernel launches here.
+ * (hamming_topk.py:7-54) — a dozen framework launches there, three kernel launches here, two for
+ * steps of few blocks.
  *
  *   1. the codes of the step's new keys go to the paged code cache (as ucm_hash_encode_cache);
  *   2. the queries of every KV head's group are averaged (fp32 sum, times 1/G, rounded to the
