@@ -313,3 +313,74 @@ def test_small_step_scores_and_hashes_in_one_launch(B, Hq, Hkv, D, BS, nblk, T, 
         expect[b, :n] = oi[b, 0, :n]
     assert np.array_equal(new_table.cpu().numpy(), expect)
     assert np.array_equal(new_lens.cpu().numpy(), c_api.update_seq_lens(lens, topk_tok, BS))
+
+
+def _step_with_planted_keys(B, Hq, Hkv, D, BS, nblk, per):
+    """A step whose list depends on the codes of its new keys: request b's new keys fill `per` slots each of two blocks
+    outside the windows, all other codes of which are as far from the query as can be.  In one the slots hold the query's own
+    code and the new keys are as far from it as can be (read too early, the block is the best there is), in the other
+    the first of the new keys is the mean query itself.  The second request's table names a block of the first one."""
+    from ucm_amd.sparse import HashEncoder
+
+    dtype = torch.bfloat16
+    rng = rng_for(B * 7919 + Hq * 31 + Hkv + D + BS + per)
+    W, NB, G = D // 32, B * nblk, Hq // Hkv
+    w = torch.from_numpy(rng.standard_normal((D, D)).astype(np.float32)).to(dtype).cuda()
+    cache = torch.from_numpy(rng.integers(0, 2**32, size=(NB, BS, Hkv, W), dtype=np.uint32).view(np.int32)).cuda()
+    tab = rng.permutation(NB).astype(np.int32).reshape(B, nblk)
+    lens = np.full(B, nblk * BS, np.int32)
+    q = torch.from_numpy(rng.standard_normal((B, Hq, D)).astype(np.float32)).to(dtype).cuda()
+    mean = q.view(B, Hkv, G, D)[:, :, 0].float()
+    for g in range(1, G):
+        mean = mean + q.view(B, Hkv, G, D)[:, :, g].float()
+    mean = (mean * torch.tensor(1.0 / G, dtype=torch.float32)).to(dtype)
+    enc = HashEncoder(D, D, dtype, torch.device("cuda:0"))
+    enc.set_hash_weight(w)
+    code = enc.compute_hash(mean).view(torch.int32).view(B, Hkv, W)
+    keys, slots = [], []
+    for b in range(B):
+        stale, found = int(tab[b, 2 + b % 3]), int(tab[b, 6 + b % 2])
+        cache[stale] = ~code[b]
+        cache[found] = ~code[b]
+        at = rng.choice(BS, size=(2, per), replace=False) if 2 * per <= BS else np.stack([rng.permutation(BS)[:per]] * 2)
+        for i in range(per):
+            cache[stale, int(at[0, i])] = code[b]
+            keys += [-mean[b], mean[b] if i == 0 else -mean[b]]
+            slots += [stale * BS + int(at[0, i]), found * BS + int(at[1, i])]
+    if B > 1:
+        tab[1, 4] = tab[0, 2]
+    order = torch.from_numpy(rng.permutation(len(keys)))
+    return w, enc, q, torch.stack(keys)[order.cuda()].contiguous(), torch.tensor(slots)[order].cuda(), cache, tab, lens
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,BS,nblk,per,one", [
+    (1, 32, 8, 128, 128, 40, 1, True), (2, 8, 8, 128, 64, 40, 2, True), (1, 32, 8, 128, 32, 40, 14, True),  # up to 224 rows
+    (3, 12, 1, 128, 128, 30, 32, True), (1, 32, 32, 128, 16, 40, 3, True),    # a head, as many as there may be
+    (1, 32, 8, 64, 128, 40, 32, True), (2, 8, 2, 64, 1024, 14, 64, True),      # 64 bits: up to 512 rows
+    (1, 32, 8, 128, 128, 40, 15, False), (1, 32, 8, 64, 128, 40, 33, False), (2, 64, 32, 128, 128, 40, 2, False),  # more
+])
+def test_new_keys_decide_which_blocks_are_listed(B, Hq, Hkv, D, BS, nblk, per, one):
+    """Keys that the step writes itself count with their new codes, and the codes they replace not at all, in the kernel that
+    hashes and scores at once and beyond the number of new keys up to which it is taken."""
+    from ucm_amd import _lib
+    from ucm_amd.sparse import GSADecodeStep
+
+    w, enc, q, newk, slots, cache, tab, lens = _step_with_planted_keys(B, Hq, Hkv, D, BS, nblk, per)
+    stale = cache.clone()
+    expect_cache = cache.clone()
+    enc.compute_hash_and_cache(newk, slots, expect_cache, block_size=BS)
+    step = GSADecodeStep(w, Hq, Hkv, B, nblk, 6 * BS, block_size=BS, sink_token=BS, recent_token=2 * BS)
+    table, _ = step.step(newk, slots, q, cache, torch.from_numpy(tab).cuda(), torch.from_numpy(lens).cuda())
+    assert _lib.last_dispatch().startswith("encode_score<%d>+" % (D // 32)) == one
+    assert torch.equal(cache, expect_cache)
+
+    def listed(codes):
+        oi, _ = c_api.hamming_topk(step.q_codes.cpu().numpy().view(np.uint32).reshape(B, Hkv, D // 32),
+                                   codes.cpu().numpy().view(np.uint32), tab, lens, 6, BS, 2 * BS,
+                                   flags=c_api.F_REDUCE_HEADS | c_api.F_PHYSICAL)
+        return oi[:, 0]
+
+    expect = listed(cache)
+    assert np.array_equal(table.cpu().numpy()[:, :6], expect)
+    # every request's list would be another one with the codes from before the step
+    assert (listed(stale) != expect).any(axis=1).all()

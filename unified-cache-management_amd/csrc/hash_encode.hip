@@ -2345,9 +2345,9 @@ __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3,
     typedef uint32_t Code __attribute__((ext_vector_type(WD)));
     __shared__ __align__(16) uint16_t wt[WD][32 * KP];
     __shared__ __align__(16) uint16_t rows[32 * KP];
-    __shared__ __align__(16) Code qcode[32], ncode[32];
+    __shared__ __align__(16) Code qcode[32];
     __shared__ uint32_t fresh[kStepMostBS / 32];
-    __shared__ int hits[kStepTokens];
+    __shared__ int2 hits[kStepTokens];  // a new key in this block and its token there
     __shared__ int nhits;
     __shared__ int low[kStepThreads / 64];
     warm_args(js);
@@ -2428,17 +2428,12 @@ __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3,
     if (tid == 0) nhits = 0;
     if (tid < kStepMostBS / 32) fresh[tid] = 0;
     __syncthreads();
-    auto slot_of = [&](int64_t t, int64_t& blk, int64_t& tok) {
-        const int64_t s = slot_value(kk, fetch_slot(kk, t), t);
-        blk = -1;
-        tok = 0;
-        if (s >= 0) split_token(kk, s, blk, tok);
-    };
     if (read && tid < js.tokens) {
-        int64_t blk, tok;
-        slot_of(tid, blk, tok);
+        const int64_t s = slot_value(kk, fetch_slot(kk, tid), tid);
+        int64_t blk = -1, tok = 0;
+        if (s >= 0) split_token(kk, s, blk, tok);
         if (blk == entry) {
-            hits[atomicAdd(&nhits, 1)] = tid;
+            hits[atomicAdd(&nhits, 1)] = make_int2(tid, (int)tok);
             atomicOr(&fresh[tok >> 5], 1u << (tok & 31));
         }
     }
@@ -2461,19 +2456,16 @@ __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3,
             bv[ks] = *reinterpret_cast<const V*>(wt[wave] + (lane & 31) * KP + ks * 16 + (lane >> 5) * 8);
     }
     // codes of the staged rows, one a head (rows past the heads hold anything and are not stored)
-    auto hash = [&](Code* out) __attribute__((always_inline)) {
-        if (wave < WD) {
-            f32x16 acc = acc_start();
+    if (wave < WD) {
+        f32x16 acc = acc_start();
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                acc = Mfma<V>::run(bv[ks], *reinterpret_cast<const V*>(rows + (lane & 31) * KP + ks * 16 + (lane >> 5) * 8), acc);
-            const uint32_t half = pack_half(acc);
-            const uint32_t word = join_halves(lane >> 5 ? half << 4 : half);
-            if (lane < heads) reinterpret_cast<uint32_t*>(out + lane)[wave] = word;
-        }
-        __syncthreads();
-    };
-    hash(qcode);
+        for (int ks = 0; ks < KS; ++ks)
+            acc = Mfma<V>::run(bv[ks], *reinterpret_cast<const V*>(rows + (lane & 31) * KP + ks * 16 + (lane >> 5) * 8), acc);
+        const uint32_t half = pack_half(acc);
+        const uint32_t word = join_halves(lane >> 5 ? half << 4 : half);
+        if (lane < heads) reinterpret_cast<uint32_t*>(qcode + lane)[wave] = word;
+    }
+    __syncthreads();
     const uint32_t* words = reinterpret_cast<const uint32_t*>(qcode);
     if (is_key) {
         if (tid < heads * WD) {
@@ -2489,16 +2481,12 @@ __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3,
         return;
     }
     int best = 0x7fffffff;
-    auto distance = [&](const Code& c, int h) {
+    const int seen = nhits;
+    auto add = [&](const Code& c, int i) {
+        const int tok = i >> h_shift, h = i & (heads - 1);
         int d = 0;
 #pragma unroll
         for (int w = 0; w < WD; ++w) d += __popc(c[w] ^ qcode[h][w]);
-        return d;
-    };
-    const int seen = nhits;
-    auto add = [&](const Code& c, int i) {
-        const int tok = i >> h_shift;
-        const int d = distance(c, i & (heads - 1));
         if (pos0 + tok < len && !(seen > 0 && ((fresh[tok >> 5] >> (tok & 31)) & 1)) && d < best) best = d;
     };
 #pragma unroll
@@ -2507,17 +2495,31 @@ __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3,
         if (i < codes) add(kv[u], i);
     }
     for (int i = kAhead * kStepThreads + tid; i < codes; i += kStepThreads) add(base[i], i);
-    for (int n = 0; n < seen; ++n) {
-        const int t = __builtin_amdgcn_readfirstlane(hits[n]);
-        stage(kk, t, false);
-        __syncthreads();
-        hash(ncode);
-        int64_t blk, tok;
-        slot_of(t, blk, tok);
-        if (tid < heads && pos0 + tok < len) {
-            const int d = distance(ncode[tid], tid);
-            best = d < best ? d : best;
+    // the new keys of this block: 32 rows a wave, straight from memory, against the projection in LDS (one request, 128
+    // bits, 8 heads, 1, 8, 16, 32 and 128 keys in a block: 8.5, 8.6, 9.1, 10.0 and 16.1 us; a key at a time with two
+    // barriers each 8.6, 14.4, 21.4, 34.7 and 114)
+    const int new_rows = seen << h_shift;
+    for (int r0 = wave * 32; r0 < new_rows; r0 += kStepThreads / 64 * 32) {
+        const int row = r0 + (lane & 31) < new_rows ? r0 + (lane & 31) : new_rows - 1;
+        const int2 hit = hits[row >> h_shift];
+        const int h = row & (heads - 1);
+        const uint16_t* src = (const uint16_t*)kk.x + (int64_t)hit.x * kk.x_stride_t + (int64_t)h * kk.x_stride_h + (lane >> 5) * 8;
+        V x[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) x[ks] = *reinterpret_cast<const V*>(src + ks * 16);
+        int d = 0;
+        int at = (lane & 31) * KP + (lane >> 5) * 8;
+        asm volatile("" : "+v"(at));  // opaque: the loop's operands would be kept in 128 registers, and spilled
+#pragma unroll
+        for (int q = 0; q < WD; ++q) {
+            f32x16 acc = acc_start();
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                acc = Mfma<V>::run(*reinterpret_cast<const V*>(wt[q] + at + ks * 16), x[ks], acc);
+            const uint32_t half = pack_half(acc);
+            d += __popc(join_halves(lane >> 5 ? half << 4 : half) ^ words[h * WD + q]);
         }
+        if (pos0 + hit.y < len && d < best) best = d;
     }
 #pragma unroll
     for (int st = 1; st < 64; st <<= 1) {
@@ -3522,6 +3524,12 @@ int build_pair(const PairSpec& p, EncArgs& kk, EncArgs& kq, bool& has_keys)
 // 1,024 blocks 9.4 and 10.3, 2,048 blocks 14.5 and 11.9.
 int64_t step_most_blocks(int words) { return (int64_t)stream_workgroups() * (words == 4 ? 5 : 9) / 2; }
 
+// New keys of such a step: one a request, which fall into blocks of their own, or as many as cost less than the launch they save
+// where all of them fall into one block that is read.  Rows (key, head) of one block, this kernel and the separate launches:
+// 128 bits, 8 heads, 128 rows 9.1 and 9.7 us, 256 rows 10.0 and 9.6; 32 heads, 256 rows 12.9 and 14.3, 512 rows 14.9 and 14.5;
+// 64 bits, 8 heads, 512 rows 9.1 and 9.3, 1,024 rows 11.6 and 9.3.
+bool step_takes_keys(const PairSpec& p) { return p.T <= kStepTokens && (p.T <= p.B || p.T * p.Hkv <= (p.N_bits == 128 ? 224 : 512)); }
+
 bool pair_is_small(const PairSpec& p, const EncArgs& kk, const EncArgs& kq, bool has_keys)
 {
     return has_keys && p.B > 0 && small_eligible(kk, p.x_dtype, p.w_dtype, false) &&
@@ -3585,7 +3593,7 @@ int step_is_fused(const PairSpec& p, const StepScore& s, bool& fused)
     const bool heads = p.Hkv <= 32 && (p.Hkv & (p.Hkv - 1)) == 0;
     const bool rows = p.cs_head == wd && p.cs_token == (int64_t)p.Hkv * wd && p.cs_block % wd == 0 &&
                       ((uintptr_t)p.cache & (4 * wd - 1)) == 0;
-    fused = p.q_group_mean && bits && heads && rows && p.n_w == 1 && p.B > 0 && p.B <= 65535 && p.T <= kStepTokens &&
+    fused = p.q_group_mean && bits && heads && rows && p.n_w == 1 && p.B > 0 && p.B <= 65535 && step_takes_keys(p) &&
             p.BS <= kStepMostBS && s.max_blocks > 0 && (int64_t)p.B * s.max_blocks <= step_most_blocks(wd) &&
             small_eligible(kq, p.x_dtype, p.w_dtype, false) && (!has_keys || small_eligible(kk, p.x_dtype, p.w_dtype, false));
     return UCM_OK;
