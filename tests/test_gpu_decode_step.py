@@ -384,3 +384,33 @@ def test_new_keys_decide_which_blocks_are_listed(B, Hq, Hkv, D, BS, nblk, per, o
     assert np.array_equal(table.cpu().numpy()[:, :6], expect)
     # every request's list would be another one with the codes from before the step
     assert (listed(stale) != expect).any(axis=1).all()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,BS,nblk,one", [
+    (8, 8, 128, 128, 12, True), (4, 4, 128, 257, 12, True), (8, 8, 128, 383, 12, True), (2, 2, 128, 1024, 12, True),  # 1,024 codes and on
+    (8, 8, 128, 1024, 9, True), (32, 32, 128, 1024, 9, True), (16, 16, 128, 512, 10, True),
+    (16, 16, 128, 513, 10, False), (16, 16, 128, 1024, 9, False), (8, 8, 128, 1025, 9, False),
+    (4, 2, 64, 511, 12, True), (16, 16, 64, 1024, 9, True), (32, 32, 64, 129, 12, True),
+])
+def test_codes_of_a_block_of_a_small_step(Hq, Hkv, D, BS, nblk, one):
+    """Blocks of as many codes as a workgroup requests at first, a few more, and as many as there may be; lengths that end
+    inside a block."""
+    from ucm_amd import _lib
+    from ucm_amd.sparse import GSADecodeStep
+
+    rng = rng_for(Hq * 31 + Hkv + D + BS)
+    B, W, dtype = 2, D // 32, torch.bfloat16
+    w = torch.from_numpy(rng.standard_normal((D, D)).astype(np.float32)).to(dtype).cuda()
+    cache = torch.from_numpy(rng.integers(0, 2**32, size=(B * nblk, BS, Hkv, W), dtype=np.uint32).view(np.int32)).cuda()
+    tab = rng.permutation(B * nblk).astype(np.int32).reshape(B, nblk)
+    lens = np.array([nblk * BS - 1, (nblk - 1) * BS - BS // 3], np.int32)
+    q = torch.from_numpy(rng.standard_normal((B, Hq, D)).astype(np.float32)).to(dtype).cuda()
+    newk = torch.from_numpy(rng.standard_normal((B, Hkv, D)).astype(np.float32)).to(dtype).cuda()
+    at = [2 * BS + BS - 1, 3 * BS]  # the last token of a block, the first of one
+    slots = torch.tensor([int(tab[b, at[b] // BS]) * BS + at[b] % BS for b in range(B)])
+    step = GSADecodeStep(w, Hq, Hkv, B, nblk, 5 * BS, block_size=BS, sink_token=0, recent_token=1)
+    table, _ = step.step(newk, slots.cuda(), q, cache, torch.from_numpy(tab).cuda(), torch.from_numpy(lens).cuda())
+    assert _lib.last_dispatch().startswith("encode_score<%d>+" % W) == one
+    oi, _ = c_api.hamming_topk(step.q_codes.cpu().numpy().view(np.uint32).reshape(B, Hkv, W), cache.cpu().numpy().view(np.uint32),
+                               tab, lens, 5, 0, 1, flags=c_api.F_REDUCE_HEADS | c_api.F_PHYSICAL)
+    assert np.array_equal(table.cpu().numpy()[:, :5], oi[:, 0])

@@ -2489,12 +2489,23 @@ __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3,
         for (int w = 0; w < WD; ++w) d += __popc(c[w] ^ qcode[h][w]);
         if (pos0 + tok < len && !(seen > 0 && ((fresh[tok >> 5] >> (tok & 31)) & 1)) && d < best) best = d;
     };
+    // each kAhead codes while the next ones travel
+    for (int i0 = tid;;) {
+        const int next = i0 + kAhead * kStepThreads;
+        const bool more = next - tid < codes;
+        Code after[kAhead];
+        if (more) {
 #pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-        const int i = u * kStepThreads + tid;
-        if (i < codes) add(kv[u], i);
+            for (int u = 0; u < kAhead; ++u) after[u] = base[next + u * kStepThreads < codes ? next + u * kStepThreads : tid];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (i0 + u * kStepThreads < codes) add(kv[u], i0 + u * kStepThreads);
+        if (!more) break;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) kv[u] = after[u];
+        i0 = next;
     }
-    for (int i = kAhead * kStepThreads + tid; i < codes; i += kStepThreads) add(base[i], i);
     // the new keys of this block: 32 rows a wave, straight from memory, against the projection in LDS (one request, 128
     // bits, 8 heads, 1, 8, 16, 32 and 128 keys in a block: 8.5, 8.6, 9.1, 10.0 and 16.1 us; a key at a time with two
     // barriers each 8.6, 14.4, 21.4, 34.7 and 114)
@@ -3524,6 +3535,13 @@ int build_pair(const PairSpec& p, EncArgs& kk, EncArgs& kq, bool& has_keys)
 // 1,024 blocks 9.4 and 10.3, 2,048 blocks 14.5 and 11.9.
 int64_t step_most_blocks(int words) { return (int64_t)stream_workgroups() * (words == 4 ? 5 : 9) / 2; }
 
+// Codes of a block that its workgroup reads, 1,024 in front of the hashing and the rest four a thread at a time (one by one
+// they were as many round trips: 64 blocks of 1,024 tokens x 8 heads 16.9 us, with the separate launches 15.1).  Now and with the
+// separate launches, 128 bits: 8 heads, 64 blocks of 1,024 tokens 14.1 and 15.1 us, 640 of them 19.9 and 21.9; 32 heads, 64 blocks of
+// 512 tokens 21.8 and 27.8, 256 of 1,024 tokens 45.4 and 53.1; 16 heads, whose own scorer streams a block best, 64 blocks of 512 tokens
+// 14.9 and 14.9, of 1,024 tokens 22.1 and 21.1, 512 of them 30.7 and 27.7.  64 bits, 32 heads, 64 blocks of 256 tokens 11.5 and 13.8.
+bool step_takes_codes(const PairSpec& p) { return p.BS <= kStepMostBS && !(p.N_bits == 128 && p.Hkv == 16 && p.BS > 512); }
+
 // New keys of such a step: one a request, which fall into blocks of their own, or as many as cost less than the launch they save
 // where all of them fall into one block that is read.  Rows (key, head) of one block, this kernel and the separate launches:
 // 128 bits, 8 heads, 128 rows 9.1 and 9.7 us, 256 rows 10.0 and 9.6; 32 heads, 256 rows 12.9 and 14.3, 512 rows 14.9 and 14.5;
@@ -3594,7 +3612,7 @@ int step_is_fused(const PairSpec& p, const StepScore& s, bool& fused)
     const bool rows = p.cs_head == wd && p.cs_token == (int64_t)p.Hkv * wd && p.cs_block % wd == 0 &&
                       ((uintptr_t)p.cache & (4 * wd - 1)) == 0;
     fused = p.q_group_mean && bits && heads && rows && p.n_w == 1 && p.B > 0 && p.B <= 65535 && step_takes_keys(p) &&
-            p.BS <= kStepMostBS && s.max_blocks > 0 && (int64_t)p.B * s.max_blocks <= step_most_blocks(wd) &&
+            step_takes_codes(p) && s.max_blocks > 0 && (int64_t)p.B * s.max_blocks <= step_most_blocks(wd) &&
             small_eligible(kq, p.x_dtype, p.w_dtype, false) && (!has_keys || small_eligible(kk, p.x_dtype, p.w_dtype, false));
     return UCM_OK;
 }
