@@ -145,10 +145,12 @@ def test_few_tokens_many_heads_one_projection(B, H, K, N, n_w):
     (224, 1, 512, 512, 1), (225, 1, 512, 512, 1), (256, 1, 256, 128, 1),  # seven row tiles, eight
     (8, 33, 512, 64, 1), (16, 33, 256, 96, 1),   # nine and seventeen row tiles of pairs; columns no power of two
     (40, 8, 512, 128, 8), (5, 12, 256, 64, 4),   # a projection per head or per three heads: two row tiles each, one
+    (1, 1, 512, 512, 1), (21, 1, 512, 96, 1), (22, 1, 512, 512, 1), (3, 7, 512, 64, 1), (21, 8, 512, 128, 8),  # few rows in a tile
+    (1, 3, 256, 96, 3), (27, 1, 256, 128, 1), (28, 1, 256, 64, 1), (2, 14, 256, 128, 1),
 ])
 def test_split_row_tiles(dtype, B, H, K, N, n_w):
-    """Rows of 256 and 512 values, few enough for the kernel whose waves share a row tile: the order in which row
-    and column tiles go out, rows past the last, rows that lie apart (a strided view)."""
+    """Rows of 256 and 512 values, few enough for the kernel whose waves share a row tile: both ways of reading the
+    rows, the order in which row and column tiles go out, rows past the last, rows that lie apart (a strided view)."""
     rng = rng_for(B * 131 + H * 7 + K + N)
     wide = torch.from_numpy(rng.standard_normal((B, H, K + 24)).astype(np.float32)).to(dtype)
     W = torch.from_numpy(rng.standard_normal((n_w, K, N)).astype(np.float32)).to(dtype)

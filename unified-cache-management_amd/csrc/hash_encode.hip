@@ -20,6 +20,7 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -2028,7 +2029,7 @@ __host__ __device__ __forceinline__ bool small_rows_are_pairs(const EncArgs& a)
 // `lds` is the tile's: small_lds(KS, SPLIT) values.
 constexpr int small_lds(int KS, int SPLIT) { return SPLIT * 32 * (KS / SPLIT * 16 + kPad); }
 
-template <typename V, int KS, int SPLIT = 1>
+template <typename V, int KS, int SPLIT = 1, bool kByRow = false>
 __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv, uint16_t* lds)
 {
     static_assert(KS % SPLIT == 0, "the row's k-steps divide evenly over the waves of a tile");
@@ -2046,7 +2047,7 @@ __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv, uint
     // goes out column first, and so do tiles of one wave, whose rows are 128 or 256 bytes.
     const int units = pairs ? (int)((a.T * a.H + kRowsPerWave - 1) / kRowsPerWave)
                             : (int)((a.T + kRowsPerWave - 1) / kRowsPerWave) * a.H;
-    if (SPLIT > 1 && a.nt_shift >= 0 && (wv >> (a.nt_shift + 3)) < (units >> 3)) {
+    if (kByRow && a.nt_shift >= 0 && (wv >> (a.nt_shift + 3)) < (units >> 3)) {
         nt = (wv >> 3) & (ntiles - 1);
         wv = (wv >> (a.nt_shift + 3)) * 8 + (wv & 7);
     } else if (a.nt_shift >= 0) {
@@ -2095,7 +2096,6 @@ __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv, uint
     // layout each of an instruction's 64 pieces of 16 bytes lies on a line of its own, and a compute unit looks up
     // one line a cycle.  The encode launch of a latent-attention step: 16 requests x 64 means of two rows of 512 values
     // (594 workgroups) 10.2 -> 8.9 us, 2 x 64, where it is latency, 6.6 -> 6.2.
-    constexpr bool kByRow = SPLIT > 1;
     constexpr int kRowLanes = KL / 8;           // lanes on one row's slice
     constexpr int kRowsPerLoad = 64 / kRowLanes;
     static_assert(!kByRow || KSL * kRowsPerLoad == kRowsPerWave, "as many row loads as k-steps");
@@ -2275,14 +2275,14 @@ __device__ __forceinline__ void encode_small_body(const EncArgs& a, int wv, uint
 // waves that share a tile: rows of 256 values and more are split four ways
 constexpr int small_split(int KS) { return KS >= 16 ? 4 : 1; }
 
-template <typename V, int KS>
+template <typename V, int KS, bool kByRow = false>
 __global__ __launch_bounds__(64 * small_split(KS)) __attribute__((amdgpu_waves_per_eu(small_split(KS) > 1 ? 3 : 1, 8))) void encode_small_kernel(EncJobs js)
 {
     warm_args(js);
     __shared__ __align__(16) uint16_t lds[small_lds(KS, small_split(KS))];
     const bool second = (int)blockIdx.x >= js.waves0;
-    encode_small_body<V, KS, small_split(KS)>(second ? js.job[1] : js.job[0],
-                                              second ? blockIdx.x - js.waves0 : blockIdx.x, lds);
+    encode_small_body<V, KS, small_split(KS), kByRow>(second ? js.job[1] : js.job[0],
+                                                      second ? blockIdx.x - js.waves0 : blockIdx.x, lds);
 }
 
 // Four jobs in one launch, two of input width 16 * KSA and two of 16 * KSB (the two parts of a
@@ -2292,7 +2292,7 @@ struct EncJobs4 {
     int end[4];  // first wave index past job i
 };
 
-template <typename V, int KSA, int KSB>
+template <typename V, int KSA, int KSB, bool kByRow>
 __global__ __launch_bounds__(64 * small_split(KSA)) __attribute__((amdgpu_waves_per_eu(3, 8))) void encode_small_mixed_kernel(EncJobs4 js)
 {
     static_assert(small_split(KSB) == 1, "the narrow jobs' tiles take one wave of the workgroup");
@@ -2302,7 +2302,7 @@ __global__ __launch_bounds__(64 * small_split(KSA)) __attribute__((amdgpu_waves_
     const int w = blockIdx.x;
     if (w < js.end[1]) {
         const int j = w >= js.end[0] ? 1 : 0;
-        encode_small_body<V, KSA, small_split(KSA)>(js.job[j], j ? w - js.end[0] : w, lds);
+        encode_small_body<V, KSA, small_split(KSA), kByRow>(js.job[j], j ? w - js.end[0] : w, lds);
     } else {
         if (threadIdx.x >= 64) return;  // a narrow tile is one wave's work
         const int j = w >= js.end[2] ? 3 : 2;
@@ -2997,16 +2997,34 @@ int64_t small_waves(const EncArgs& a)
     return ucm::ceil_div(a.T, kRowsPerWave) * a.H * (a.N / 32);
 }
 
+// Whether a launch of split tiles reads its rows line by line: where one of its jobs has a tile of this many rows.  The turn
+// through LDS and the order of the tiles are a chain of 0.3 to 0.5 us in front of the products, which fewer rows, on fewer lines,
+// do not make up for.  Operand layout and line by line: 512 -> 512 bits, 1 row 3.83 and 4.31 us, 20 rows 4.33 and 4.36, 24 rows 4.41
+// and 4.34, 32 rows 4.60 and 4.36; 256 -> 128 bits, 1 row 3.42 and 3.72, 24 rows 3.70 and 3.77, 28 rows 3.68 and 3.69, 32 rows 3.78 and 3.74;
+// a latent step of 8 query rows 13.3 and 13.7, of 32 rows 13.1 and 12.9.
+bool rows_by_line(const EncArgs& a, const EncArgs& b)
+{
+    auto tile_rows = [](const EncArgs& j) { return small_rows_are_pairs(j) ? j.T * j.H : j.T; };
+    return std::max(tile_rows(a), tile_rows(b)) >= (a.K == 512 ? 22 : 28);
+}
+
 template <typename V>
 int launch_small(const EncJobs& js, int64_t waves, int K, hipStream_t st)
 {
     const dim3 grid((unsigned)waves);
+    const bool by_line = rows_by_line(js.job[0], js.job[1]);
     note_encode("encode_small");
     switch (K) {
         case 64: hipLaunchKernelGGL((encode_small_kernel<V, 4>), grid, dim3(64), 0, st, js); break;
         case 128: hipLaunchKernelGGL((encode_small_kernel<V, 8>), grid, dim3(64), 0, st, js); break;
-        case 256: hipLaunchKernelGGL((encode_small_kernel<V, 16>), grid, dim3(64 * small_split(16)), 0, st, js); break;
-        case 512: hipLaunchKernelGGL((encode_small_kernel<V, 32>), grid, dim3(64 * small_split(32)), 0, st, js); break;
+        case 256:
+            if (by_line) hipLaunchKernelGGL((encode_small_kernel<V, 16, true>), grid, dim3(64 * small_split(16)), 0, st, js);
+            else hipLaunchKernelGGL((encode_small_kernel<V, 16>), grid, dim3(64 * small_split(16)), 0, st, js);
+            break;
+        case 512:
+            if (by_line) hipLaunchKernelGGL((encode_small_kernel<V, 32, true>), grid, dim3(64 * small_split(32)), 0, st, js);
+            else hipLaunchKernelGGL((encode_small_kernel<V, 32>), grid, dim3(64 * small_split(32)), 0, st, js);
+            break;
         default: return ucm::fail(UCM_ERROR, "internal: K %d has no small-row kernel", K);
     }
     return ucm::launch_status("encode_small_kernel");
@@ -3554,6 +3572,15 @@ bool pair_is_small(const PairSpec& p, const EncArgs& kk, const EncArgs& kq, bool
            small_eligible(kq, p.x_dtype, p.w_dtype, false);
 }
 
+template <typename V>
+int launch_small_mixed(const EncJobs4& js, hipStream_t st)
+{
+    const dim3 grid((unsigned)js.end[3]), threads(64 * small_split(32));
+    if (rows_by_line(js.job[0], js.job[1])) hipLaunchKernelGGL((encode_small_mixed_kernel<V, 32, 4, true>), grid, threads, 0, st, js);
+    else hipLaunchKernelGGL((encode_small_mixed_kernel<V, 32, 4, false>), grid, threads, 0, st, js);
+    return ucm::launch_status("encode_small_mixed_kernel");
+}
+
 // The queries alone through the small-row kernel (the only one that averages query groups).
 int launch_queries_small(const PairSpec& p, EncArgs& kq, hipStream_t st)
 {
@@ -3686,11 +3713,7 @@ int encode_two_pairs(const PairSpec& pa, const PairSpec& pb, hipStream_t st)
             js.end[i] = (int)end;
         }
         if (end <= 0x7fffffff) {
-            if (pa.x_dtype == UCM_DT_BF16)
-                hipLaunchKernelGGL((encode_small_mixed_kernel<bf16x8, 32, 4>), dim3((unsigned)end), dim3(64 * small_split(32)), 0, st, js);
-            else
-                hipLaunchKernelGGL((encode_small_mixed_kernel<f16x8, 32, 4>), dim3((unsigned)end), dim3(64 * small_split(32)), 0, st, js);
-            return ucm::launch_status("encode_small_mixed_kernel");
+            return pa.x_dtype == UCM_DT_BF16 ? launch_small_mixed<bf16x8>(js, st) : launch_small_mixed<f16x8>(js, st);
         }
     }
     rc = launch_pair(pa, ka, qa, ha, st);
