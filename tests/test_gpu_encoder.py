@@ -169,6 +169,12 @@ def test_split_row_tiles(dtype, B, H, K, N, n_w):
     (20000, 384, 1, 64, torch.float16, "4,8"),   # streams that eight does not divide, a second tile for some
     (50001, 512, 1, 64, torch.bfloat16, "8,8"),  # a second row tile for some of the streams, the last one of a few rows
     (65535, 512, 1, 32, torch.bfloat16, "8,8"),  # two for all, one row short
+    # streams that eight does not divide, dealt out with their slices over all heads
+    (1500, 384, 6, 64, torch.bfloat16, "4,4"),   # twelve, a tile each
+    (3001, 384, 6, 48, torch.float16, "4,8"),    # twelve, the last tile of some rows
+    (4609, 640, 4, 64, torch.bfloat16, "4,8"),   # twelve, a second tile for most, the last one of one row
+    (2305, 640, 8, 64, torch.bfloat16, "4,8"),   # six, two tiles for most
+    (1153, 384, 16, 64, torch.float16, "4,8"),   # five, a tile each, more heads
 ])
 def test_rows_of_512_values_by_tile_shape(T, N, H, BS, dtype, route):
     """Every shape of the tile; one or several row tiles per workgroup; a strided view of the rows, rows that are

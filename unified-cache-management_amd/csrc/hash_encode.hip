@@ -639,8 +639,8 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v)
            (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
-template <typename V, int NT, int kWaves>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void encode_pipe_kernel(EncArgs a, int streams)
+template <typename V, int NT, int kWaves, bool kRuns>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void encode_pipe_kernel(EncArgs a, int streams, int run)
 {
     static_assert((NT == 2 && kWaves == 4) || NT == 4 || (NT == 8 && kWaves == 8), "64, 128 or 256 columns");
     constexpr int kRows = pipe_rows(kWaves), kPipeRing = pipe_ring(NT, kWaves);
@@ -654,19 +654,24 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
     char* lds = reinterpret_cast<char*>(wt);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)wt);
     warm_args(a);
-    const int h = blockIdx.z;
     // The slices of a row tile are workgroups of one XCD (consecutive ones go to the eight XCDs in turn), so that
-    // its rows come past that XCD's L2 once: streams in eights, each eight slice by slice.  What fills the last
-    // eight has nothing to do.  Fewer than eight streams take all XCDs for each.
+    // its rows come past that XCD's L2 once: streams in eights, each eight slice by slice, what fills the last eight having
+    // nothing to do; or, where the number of streams is no multiple of eight, `run` neighbours among all heads'
+    // streams and their slices on each XCD.
     const int slices = a.N / (NT * 32);
-    int stream, n0;
-    if (streams >= 8) {
+    int h, stream, n0;
+    if constexpr (kRuns) {
+        int u = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+        if (u >= streams * slices * a.H) return;
+        n0 = u % slices * (NT * 32);
+        u /= slices;
+        stream = u % streams;
+        h = u / streams;
+    } else {
+        h = blockIdx.z;
         stream = (int)blockIdx.x / (8 * slices) * 8 + (blockIdx.x & 7);
         n0 = (int)(blockIdx.x >> 3) % slices * (NT * 32);
         if (stream >= streams) return;
-    } else {
-        stream = (int)blockIdx.x % streams;
-        n0 = (int)blockIdx.x / streams * (NT * 32);
     }
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2689,40 +2694,56 @@ int launch_mfma(EncArgs a, hipStream_t st)
     return ucm::fail(UCM_EUNSUPPORTED, "no LDS slice fits K=%d", K);
 }
 
-// Row tiles that are walked at the same time: a workgroup to a compute unit, and as many streams on every XCD (three
-// slices, 85 streams: five XCDs had 33 workgroups for their 32 compute units; 24,000 rows 25.0 us, 80 streams 18.8).
-int64_t pipe_streams(const EncArgs& a, int nt, int waves)
+// Row tiles that are walked at the same time: a workgroup to a compute unit, in eights where that costs no generation of
+// workgroups (run = 0; as many streams on every XCD, each with all its slices), otherwise as many as there is room for, dealt out
+// to the XCDs in runs.  384 columns x 6 heads, 128-row tiles: 8 streams of the 14 that there is room for, 16,000 rows 86 us, 14 in
+// runs 53 (14 with a tile's slices on any XCD 58); 640 x 4, 256-row tiles, 16,000 rows 58 and 48; 5 streams of 64 columns,
+// 512 x 8 heads, 16,000 rows 117 on any XCD and 91 in runs.  Where the generations are as many the eights are ahead (512 columns, 60,000
+// rows 29.6 and 30.9 us).
+struct PipeStreams { int64_t count, run; };
+PipeStreams pipe_streams(const EncArgs& a, int nt, int waves)
 {
     const int64_t tiles = ucm::ceil_div(a.T, pipe_rows(waves));
     const int64_t units = (int64_t)(a.N / (32 * nt)) * a.H;
-    int64_t streams = (int64_t)stream_workgroups() / units;
-    if (streams > 8) streams &= ~(int64_t)7;
-    return streams < 1 ? 1 : (streams < tiles ? streams : tiles);
+    const int64_t room = std::max<int64_t>(stream_workgroups() / units, 1);
+    const int64_t all = std::min(room, tiles), eights = std::min(room & ~(int64_t)7, tiles);
+    if (eights >= 8 && ucm::ceil_div(tiles, eights) == ucm::ceil_div(tiles, all)) return {eights, 0};
+    return {all, ucm::ceil_div(all * units, 8)};
 }
 
-template <typename V, int NT, int WAVES>
-int launch_pipe_nt(const EncArgs& a, hipStream_t st)
+template <typename V, int NT, int WAVES, bool RUNS>
+int launch_pipe_nt(const EncArgs& a, const PipeStreams& s, hipStream_t st)
 {
     constexpr int lds = pipe_lds(NT, WAVES);
     static int opted = 0;  // 0 = not tried, 1 = allowed, -1 = refused by the runtime
     if (opted == 0) {
-        const hipError_t e = hipFuncSetAttribute((const void*)encode_pipe_kernel<V, NT, WAVES>,
+        const hipError_t e = hipFuncSetAttribute((const void*)encode_pipe_kernel<V, NT, WAVES, RUNS>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) (void)hipGetLastError();
         opted = (e == hipSuccess) ? 1 : -1;
     }
     if (opted < 0) return UCM_EUNSUPPORTED;
-    const int64_t streams = pipe_streams(a, NT, WAVES);
+    const int slices = a.N / (32 * NT);
+    const dim3 grid = RUNS ? dim3((unsigned)(8 * s.run)) : dim3((unsigned)(ucm::ceil_div(s.count, 8) * 8 * slices), 1, (unsigned)a.H);
     note_encode("encode_pipe", NT, WAVES);
-    hipLaunchKernelGGL((encode_pipe_kernel<V, NT, WAVES>), dim3((unsigned)((streams < 8 ? streams : ucm::ceil_div(streams, 8) * 8) * (a.N / (32 * NT))), 1, (unsigned)a.H),
-                       dim3(64 * WAVES), lds, st, a, (int)streams);
+    hipLaunchKernelGGL((encode_pipe_kernel<V, NT, WAVES, RUNS>), grid, dim3(64 * WAVES), lds, st, a, (int)s.count, (int)s.run);
     return ucm::launch_status("encode_pipe_kernel");
+}
+
+template <typename V, int NT, int WAVES>
+int launch_pipe_nt(const EncArgs& a, hipStream_t st)
+{
+    const PipeStreams s = pipe_streams(a, NT, WAVES);
+    return s.run ? launch_pipe_nt<V, NT, WAVES, true>(a, s, st) : launch_pipe_nt<V, NT, WAVES, false>(a, s, st);
 }
 
 // The tile: each shape's time is a start of 2.4 to 3.2 us and so much for every generation of workgroups (tenths of a
 // microsecond, measured at 256 and 512 columns with every compute unit at work), whose last one is paid in full.
 // 512 columns, the four shapes in their order: 4,096 rows 6.0, 7.3, 9.0 and 13.1 us; 8,192 rows 9.7, 8.2, 9.9, 13.8;
 // 16,384 rows 16.4, 13.6, 11.1, 14.6; 32,768 rows 29.0, 23.7, 19.4, 16.4; 65,536 rows 54.7, 42.2, 34.5, 29.7.
+// They serve other column counts and several heads too: at 128 to 1,024 columns, 1 to 8 heads and 700 to 65,000 rows no choice is
+// slower than the slices of 128 columns that had these calls before (384 x 6 heads, 3,000 rows 17.2 and 11.1 us; 128 x 6, 16,000 rows
+// 25.2 and 22.5; 640 x 4, 24,000 rows 89 and 84).
 template <typename V>
 int launch_pipe(const EncArgs& a, hipStream_t st)
 {
@@ -2733,7 +2754,8 @@ int launch_pipe(const EncArgs& a, hipStream_t st)
         if (a.N % (32 * shapes[i].nt)) continue;
         const int64_t tiles = ucm::ceil_div(a.T, pipe_rows(shapes[i].waves));
         const int64_t units = ucm::ceil_div((int64_t)(a.N / (32 * shapes[i].nt)) * a.H, stream_workgroups());
-        const int64_t cost = ucm::ceil_div(tiles, pipe_streams(a, shapes[i].nt, shapes[i].waves)) * units * shapes[i].cost;
+        const PipeStreams s = pipe_streams(a, shapes[i].nt, shapes[i].waves);
+        const int64_t cost = ucm::ceil_div(tiles, s.count) * units * shapes[i].cost * (s.run && s.count >= 8 && a.N > 32 * shapes[i].nt ? 9 : 8);  // slices of more than seven in runs: up to an eighth slower
         if (i == 0 || cost < best_cost) {
             best = i;
             best_cost = cost;
