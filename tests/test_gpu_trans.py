@@ -217,7 +217,9 @@ def test_errors(device):
 
 
 @pytest.mark.parametrize("n_cols,col_bytes,n_ids", [
-    (2, 4096, 1), (2, 4096, 496), (2, 4096, 497), (2, 48, 1984), (2, 48, 1985),  # a launch, two, four, the table
+    (2, 4096, 1), (2, 4096, 496), (2, 4096, 497), (2, 48, 1984), (2, 48, 1985),  # a launch, two, the table
+    (2, 48, 992), (2, 48, 993), (15, 64, 941), (16, 64, 1872), (16, 64, 1873),   # two, the table; of small columns up to four
+    (16, 2048, 469), (16, 2048, 1405), (16, 2049, 937),
     (1, 70001, 7), (3, 4112, 5), (3, 100, 9),          # tails, columns that start at any byte
     (128, 64, 244), (128, 64, 245), (129, 64, 4),      # the most columns the arguments hold, and one more
 ])

@@ -114,7 +114,9 @@ __global__ __launch_bounds__(kThreads) void paged_copy_kernel(const uint64_t* __
 // (int32) behind them.  2 KiB of arguments cost 0.1 to 0.3 us of host time more than a few bytes.
 constexpr size_t kArgWords = 250;
 constexpr size_t kArgCols = 128;    // columns at most: half of the words stay for ids
-constexpr size_t kArgLaunches = 4;  // launches at most
+constexpr size_t kArgLaunches = 2;  // launches at most,
+constexpr size_t kArgSmallLaunches = 4;  // or this many where rows are kSmallCols columns and more of kSmallBytes at most
+constexpr size_t kSmallCols = 16, kSmallBytes = 2048;
 constexpr size_t kArgBytes = (size_t)512 << 20;  // bytes at most
 
 struct ColumnArgs {
@@ -499,7 +501,12 @@ extern "C" int ucm_trans_paged_copy(ucm_trans_stream_t* s, const uint64_t* base,
     }
     const bool host_end = is_host_memory(flat);
     // Columns of one size between device memory, few enough for the arguments of a few launches.  Beyond that
-    // the upload, paid once, is the cheaper form; a host end is bound by its link.  From 512 MiB on the form
+    // the upload, paid once, is the cheaper form; a host end is bound by its link.  The runtime takes some 30 us more
+    // from the eighth command on that is issued without a wait, and the upload is three commands: 64 copies of 2 columns of
+    // 256 bytes without one between them, 490 blocks (a launch each) 427 us and with the table 803, 990 (two) 665 and 794, 1,480 (three) 909
+    // and 802, 1,980 (four) 1,164 and 846.  Rows of many small columns, a workgroup's piece each, are what the table's form is slow
+    // at: out and back, 1,405 blocks x 16 columns of 256 bytes (four) 50 and 66 us, 1,117 x 64 of 1 KiB 97 and 146, of
+    // 2 KiB 134 and 153; 1,309 x 32 of 4 KiB 151 and 146.  From 512 MiB on the form
     // with the table is the faster one: its workgroups come to their loads later, and with fewer of them in
     // flight the memory turns less often between reads and writes (1 GiB of 64 columns each way: 319 and 345 us
     // out and back, column_copy_kernel 348 and 366, with five of its workgroups to a unit instead of eight 332
@@ -510,7 +517,8 @@ extern "C" int ucm_trans_paged_copy(ucm_trans_stream_t* s, const uint64_t* base,
     if (equal && !host_end && (size_t)n_cols <= kArgCols && segs_per_col <= (1u << 20) &&
         (size_t)n_blocks <= kArgBytes / row_bytes) {
         const size_t per_launch = (kArgWords - n_cols) * 2;
-        if ((size_t)n_blocks <= per_launch * kArgLaunches) {
+        const bool small = (size_t)n_cols >= kSmallCols && col_bytes[0] <= kSmallBytes;
+        if ((size_t)n_blocks <= per_launch * (small ? kArgSmallLaunches : kArgLaunches)) {
             ColumnArgs a;
             a.col_bytes = col_bytes[0]; a.row_bytes = row_bytes; a.n_cols = n_cols; a.to_cache = to_cache;
             std::memcpy(a.words, base, (size_t)n_cols * 8);
