@@ -169,6 +169,8 @@ def test_split_row_tiles(dtype, B, H, K, N, n_w):
     (20000, 384, 1, 64, torch.float16, "4,8"),   # streams that eight does not divide, a second tile for some
     (50001, 512, 1, 64, torch.bfloat16, "8,8"),  # a second row tile for some of the streams, the last one of a few rows
     (65535, 512, 1, 32, torch.bfloat16, "8,8"),  # two for all, one row short
+    (545, 512, 1, 32, torch.bfloat16, "2,4"),    # the fewest rows: five row tiles, the last of one row
+    (289, 1024, 1, 64, torch.float16, "2,4"),    # three
     # streams that eight does not divide, dealt out with their slices over all heads
     (1500, 384, 6, 64, torch.bfloat16, "4,4"),   # twelve, a tile each
     (3001, 384, 6, 48, torch.float16, "4,8"),    # twelve, the last tile of some rows
@@ -644,6 +646,16 @@ def test_column_counts_without_a_one_tile_form_keep_the_small_kernel(K, N, T):
 def test_small_kernel_up_to_where_the_tiled_one_is_as_fast(K, N, H, T, small):
     """Sizes on both sides of the equal times, some way off them."""
     assert (_encode_route(K, N, H, T) == "encode_small") == small
+
+
+@pytest.mark.parametrize("N,H,T,small", [
+    (512, 1, 448, True), (512, 1, 640, False), (512, 1, 1000, False), (256, 1, 960, True), (256, 1, 1200, False),
+    (128, 1, 1900, True), (128, 1, 2500, False), (1024, 1, 224, True), (1024, 1, 300, False), (512, 8, 56, True), (512, 8, 90, False),
+    (192, 1, 1300, True), (192, 1, 4000, False), (64, 1, 8000, True),
+])
+def test_small_kernel_up_to_where_rows_of_512_values_stream(N, H, T, small):
+    """A tile to a compute unit where the other kernel is the ring of chunks; more where it is the slices."""
+    assert (_encode_route(512, N, H, T) == "encode_small") == small
 
 
 @pytest.mark.parametrize("K,N,H,T,tiles", [

@@ -3198,8 +3198,11 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
 // Where the kernel is not pipelined (rows of 256 values; slices of other than 32, 64, 128 and 256 columns,
 // see launch_mfma_q) it runs four tiles a workgroup: 6 us plus 0.13 us per KiB (256 -> 256 with 4 heads: equal at
 // ~5000-6000 rows; 128 -> 192, 8 heads: 1000 tokens 6.0 against 12.2 us, 4000 14.0 against 13.9; 128 -> 512: 1000
-// 9.8 against 21.9, 3000 20.2 against 23.5).  Rows of 512 values have the slice kernel: 7 us until
-// it fills the chip (512 -> 512: equal at ~1100 rows; 1000: 6.3 against 6.8 us, 1500: 8.3 against 7.0 us).
+// 9.8 against 21.9, 3000 20.2 against 23.5).  Rows of 512 values have encode_pipe_kernel where 128 divides the columns, 5.3 us
+// until it fills the chip: the wave-per-tile kernel stays ahead while every tile has a compute unit to itself (512 -> 512: 512 rows
+// 4.6 against 5.3 us, 544 rows 5.5 and 5.3, 1000 rows 5.8 and 5.3; -> 256: 1024 rows 4.6 and 5.3, 1056 rows 5.5 and 5.3; -> 128: 2048
+// rows 4.5 and 5.3, 2600 rows 5.5 and 5.3).  Otherwise they have the slice kernel: 7 us until it fills the chip (512 -> 192: 2000
+// rows 6.6 against 6.6 us, 2700 rows 7.3 and 7.1, 4000 rows 8.6 and 6.7; -> 64: 10,000 rows 6.6 and 7.1; -> 32: 20,000 rows 7.6 and 6.8).
 //
 // alone = false: a job of a decode step, where the other kernels are a launch more for every job (new keys
 // and queries of one or two projections share one here) and a group's mean is this kernel's anyway: it
@@ -3212,6 +3215,7 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype, bool alone = tru
     const int bn = pick_slice(a.N, a.K, (size_t)160 * 1024 - kStage);
     if (bn == 0) return true;
     const double slice_kib = (double)bn * (a.K + kPad) * 2 / 1024.0;
+    if (alone && a.K == 512 && a.N % 128 == 0) return small_waves(a) <= stream_workgroups();
     double lds_floor_us = 6.0 + 0.13 * slice_kib;
     if (alone && a.K == 16 * kSliceKS) lds_floor_us = 7.5;
     else if (alone && one_tile_form(a.K, bn))
