@@ -617,6 +617,46 @@ def test_row_tiles_per_workgroup(K, N, H, T, paged):
         assert_codes_match(got[:, h], xs[:, h], W.float().numpy())
 
 
+@pytest.mark.parametrize("K,N,H,T,paged,route", [
+    (128, 128, 8, 1025, True, "4,1,1"), (128, 128, 8, 12500, True, "4,1,4"), (128, 128, 8, 65700, True, "4,1,8"),
+    (64, 64, 8, 5000, True, "2,1,1"), (64, 64, 8, 10001, True, "2,1,1"),
+    (128, 128, 8, 8193, False, "4,1,1"), (128, 128, 8, 12400, False, "4,1,4"), (128, 128, 8, 65700, False, "4,1,8"),
+    (64, 64, 8, 9001, False, "2,1,1"), (64, 128, 8, 65700, False, "4,1,8"), (128, 256, 1, 66000, False, "4,2,4"),
+])
+def test_row_tiles_of_the_tiled_kernel(K, N, H, T, paged, route):
+    """The codes of each number of row tiles where that kernel is the one that runs: by slot beyond a tile a wave of the
+    streaming one, paged inputs whose rows lie apart."""
+    from ucm_amd import _lib
+
+    rng = rng_for(T * 3 + N)
+    BS, nb = 64, -(-T // 64)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(nb * BS, H, K + 8, generator=g, device="cuda").to(torch.bfloat16)[..., 8:]
+    W = torch.from_numpy(rng.standard_normal((K, N)).astype(np.float32)).to(torch.bfloat16)
+    enc = make_encoder(K, N, torch.bfloat16, W)
+    ids = torch.from_numpy(rng.permutation(nb).astype(np.int32)).cuda()
+    cache = torch.zeros((nb, BS, H, N // 32), dtype=torch.int32, device="cuda")
+    t = torch.arange(T, device="cuda")
+    slot = ids[t // BS].long() * BS + t % BS
+    if paged:
+        enc.compute_hash_from_paged_cache(x.unflatten(0, (nb, BS)), ids, T, cache, block_size=BS)
+        x = x[slot]
+    else:
+        x = x[:T].contiguous()
+        enc.compute_hash_and_cache(x, slot, cache, block_size=BS)
+    assert _lib.last_encode() == "encode_mfma<%s>" % route
+    flat = cache.view(nb * BS, H, N // 32)
+    rest = torch.ones(nb * BS, dtype=torch.bool, device="cuda")
+    rest[slot] = False
+    assert not flat[rest].any()
+    rows = np.unique(np.concatenate([np.arange(130), T - 1 - np.arange(130), rng.integers(0, T, 1500)]))
+    pick = torch.from_numpy(rows).cuda()
+    got = flat[slot[pick]].cpu().numpy().view(np.uint8)
+    xs = x[pick].float().cpu().numpy()
+    for h in range(H):
+        assert_codes_match(got[:, h], xs[:, h], W.float().numpy())
+
+
 def _encode_route(K, N, H, T):
     """The kernel that a plain encode into a paged cache takes."""
     from ucm_amd import _lib
