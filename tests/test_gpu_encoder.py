@@ -619,7 +619,7 @@ def test_row_tiles_per_workgroup(K, N, H, T, paged):
 
 @pytest.mark.parametrize("K,N,H,T,paged,route", [
     (128, 128, 8, 1025, True, "4,1,1"), (128, 128, 8, 12500, True, "4,1,4"), (128, 128, 8, 65700, True, "4,1,8"),
-    (64, 64, 8, 5000, True, "2,1,1"), (64, 64, 8, 10001, True, "2,1,1"),
+    (64, 64, 8, 10001, True, "2,1,1"), (64, 64, 4, 20001, True, "2,1,1"),
     (128, 128, 8, 8193, False, "4,1,1"), (128, 128, 8, 12400, False, "4,1,4"), (128, 128, 8, 65700, False, "4,1,8"),
     (64, 64, 8, 9001, False, "2,1,1"), (64, 128, 8, 65700, False, "4,1,8"), (128, 256, 1, 66000, False, "4,2,4"),
 ])
