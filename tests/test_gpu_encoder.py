@@ -690,7 +690,8 @@ def test_small_kernel_up_to_where_the_tiled_one_is_as_fast(K, N, H, T, small):
 
 @pytest.mark.parametrize("N,H,T,small", [
     (512, 1, 448, True), (512, 1, 640, False), (512, 1, 1000, False), (256, 1, 960, True), (256, 1, 1200, False),
-    (128, 1, 1900, True), (128, 1, 2500, False), (1024, 1, 224, True), (1024, 1, 300, False), (512, 8, 56, True), (512, 8, 90, False),
+    (128, 1, 1900, True), (128, 1, 2500, False), (1024, 1, 224, True), (1024, 1, 300, False), (512, 8, 56, True), (512, 8, 90, False), (512, 32, 20, False),
+    (512, 64, 16, True), (1024, 64, 8, True), (256, 128, 16, True),
     (192, 1, 1300, True), (192, 1, 4000, False), (64, 1, 8000, True),
 ])
 def test_small_kernel_up_to_where_rows_of_512_values_stream(N, H, T, small):

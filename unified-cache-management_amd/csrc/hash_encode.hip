@@ -3201,7 +3201,8 @@ int launch_tiled(const EncArgs& a, hipStream_t st)
 // 9.8 against 21.9, 3000 20.2 against 23.5).  Rows of 512 values have encode_pipe_kernel where 128 divides the columns, 5.3 us
 // until it fills the chip: the wave-per-tile kernel stays ahead while every tile has a compute unit to itself (512 -> 512: 512 rows
 // 4.6 against 5.3 us, 544 rows 5.5 and 5.3, 1000 rows 5.8 and 5.3; -> 256: 1024 rows 4.6 and 5.3, 1056 rows 5.5 and 5.3; -> 128: 2048
-// rows 4.5 and 5.3, 2600 rows 5.5 and 5.3).  Otherwise they have the slice kernel: 7 us until it fills the chip (512 -> 192: 2000
+// rows 4.5 and 5.3, 2600 rows 5.5 and 5.3) - and longer where a few rows of many heads make more of the other's tiles, which are
+// one head's, than fit at once (512 -> 512, 16 rows of 64 heads 5.6 and 6.9).  Otherwise they have the slice kernel: 7 us until it fills the chip (512 -> 192: 2000
 // rows 6.6 against 6.6 us, 2700 rows 7.3 and 7.1, 4000 rows 8.6 and 6.7; -> 64: 10,000 rows 6.6 and 7.1; -> 32: 20,000 rows 7.6 and 6.8).
 //
 // alone = false: a job of a decode step, where the other kernels are a launch more for every job (new keys
@@ -3215,7 +3216,8 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype, bool alone = tru
     const int bn = pick_slice(a.N, a.K, (size_t)160 * 1024 - kStage);
     if (bn == 0) return true;
     const double slice_kib = (double)bn * (a.K + kPad) * 2 / 1024.0;
-    if (alone && a.K == 512 && a.N % 128 == 0) return small_waves(a) <= stream_workgroups();
+    if (alone && a.K == 512 && a.N % 128 == 0 && ucm::ceil_div(a.T, pipe_rows(4)) * (a.N / 64) * a.H <= stream_workgroups())
+        return small_waves(a) <= stream_workgroups();
     double lds_floor_us = 6.0 + 0.13 * slice_kib;
     if (alone && a.K == 16 * kSliceKS) lds_floor_us = 7.5;
     else if (alone && one_tile_form(a.K, bn))
