@@ -414,3 +414,30 @@ def test_codes_of_a_block_of_a_small_step(Hq, Hkv, D, BS, nblk, one):
     oi, _ = c_api.hamming_topk(step.q_codes.cpu().numpy().view(np.uint32).reshape(B, Hkv, W), cache.cpu().numpy().view(np.uint32),
                                tab, lens, 5, 0, 1, flags=c_api.F_REDUCE_HEADS | c_api.F_PHYSICAL)
     assert np.array_equal(table.cpu().numpy()[:, :5], oi[:, 0])
+
+
+@pytest.mark.parametrize("D,Hq,B,nblk,one", [
+    (128, 4, 4, 160, True), (128, 4, 4, 161, False), (64, 4, 4, 256, True), (64, 4, 4, 257, False), (64, 1, 9, 128, False),
+    (64, 12, 9, 128, True), (64, 12, 5, 231, False),
+])
+def test_blocks_up_to_which_a_step_scores_and_hashes_at_once(D, Hq, B, nblk, one):
+    """One generation of workgroups: 640 blocks of 128-bit codes, 1,024 of 64-bit ones on 256 compute units, 1,152 where the
+    group's mean takes the encoder's launch longer."""
+    from ucm_amd import _lib
+    from ucm_amd.sparse import GSADecodeStep
+
+    rng = rng_for(D + B + nblk)
+    BS, W = 16, D // 32
+    w = torch.from_numpy(rng.standard_normal((D, D)).astype(np.float32)).to(torch.bfloat16).cuda()
+    cache = torch.from_numpy(rng.integers(0, 2**32, size=(B * nblk, BS, 1, W), dtype=np.uint32).view(np.int32)).cuda()
+    tab = rng.permutation(B * nblk).astype(np.int32).reshape(B, nblk)
+    lens = np.array([nblk * BS - 3 * b for b in range(B)], np.int32)
+    q = torch.from_numpy(rng.standard_normal((B, Hq, D)).astype(np.float32)).to(torch.bfloat16).cuda()
+    newk = torch.from_numpy(rng.standard_normal((B, 1, D)).astype(np.float32)).to(torch.bfloat16).cuda()
+    slots = torch.tensor([int(tab[b, 7]) * BS + b for b in range(B)]).cuda()
+    step = GSADecodeStep(w, Hq, 1, B, nblk, 12 * BS, block_size=BS)
+    table, _ = step.step(newk, slots, q, cache, torch.from_numpy(tab).cuda(), torch.from_numpy(lens).cuda())
+    assert _lib.last_dispatch().startswith("encode_score<%d>+" % W) == one
+    oi, _ = c_api.hamming_topk(step.q_codes.cpu().numpy().view(np.uint32).reshape(B, 1, W), cache.cpu().numpy().view(np.uint32),
+                               tab, lens, 12, BS, 4 * BS, flags=c_api.F_REDUCE_HEADS | c_api.F_PHYSICAL)
+    assert np.array_equal(table.cpu().numpy()[:, :12], oi[:, 0])

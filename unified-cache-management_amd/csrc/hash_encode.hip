@@ -3584,9 +3584,16 @@ int build_pair(const PairSpec& p, EncArgs& kk, EncArgs& kq, bool& has_keys)
 // Blocks of a step up to which its scoring workgroups hash the queries themselves: about as many as are on the chip at
 // once (three workgroups to a compute unit with 128-bit codes, four with 64), every further generation hashes
 // again.  Step with that kernel and with the separate launches, 8 heads, blocks of 128 tokens: 128 bits, 64 blocks 7.8 and
-// 9.9 us, 512 blocks 9.2 and 10.4, 768 blocks 11.4 and 11.2, 1,024 blocks 15.4 and 12.0; 64 bits, 64 blocks 7.5 and 10.4,
-// 1,024 blocks 9.4 and 10.3, 2,048 blocks 14.5 and 11.9.
-int64_t step_most_blocks(int words) { return (int64_t)stream_workgroups() * (words == 4 ? 5 : 9) / 2; }
+// 9.9 us, 512 blocks 9.2 and 10.4, 768 blocks 11.4 and 11.2, 1,024 blocks 15.4 and 12.0; 64 bits, 64 blocks 7.3 and 9.2,
+// 1,024 blocks 8.9 and 9.4, 1,152 blocks 11.1 and 10.0; 64 bits of one head, 1,024 blocks 9.0 and 9.1, 1,152 blocks 10.6 and 9.3.
+// Groups whose means the encoder's launch adds row by row (it has 2, 4 and 8 rows written out) pay for longer: 32 query heads to
+// one head of 64 bits, 1,152 blocks 13.2 and 26.9.
+int64_t step_most_blocks(const PairSpec& p)
+{
+    const int group = p.Hq / p.Hkv;
+    const int halves = p.N_bits == 128 ? 5 : (group == 1 || group == 2 || group == 4 || group == 8 ? 8 : 9);
+    return (int64_t)stream_workgroups() * halves / 2;
+}
 
 // Codes of a block that its workgroup reads, 1,024 in front of the hashing and the rest four a thread at a time (one by one
 // they were as many round trips: 64 blocks of 1,024 tokens x 8 heads 16.9 us, with the separate launches 15.1).  Now and with the
@@ -3674,7 +3681,7 @@ int step_is_fused(const PairSpec& p, const StepScore& s, bool& fused)
     const bool rows = p.cs_head == wd && p.cs_token == (int64_t)p.Hkv * wd && p.cs_block % wd == 0 &&
                       ((uintptr_t)p.cache & (4 * wd - 1)) == 0;
     fused = p.q_group_mean && bits && heads && rows && p.n_w == 1 && p.B > 0 && p.B <= 65535 && step_takes_keys(p) &&
-            step_takes_codes(p) && s.max_blocks > 0 && (int64_t)p.B * s.max_blocks <= step_most_blocks(wd) &&
+            step_takes_codes(p) && s.max_blocks > 0 && (int64_t)p.B * s.max_blocks <= step_most_blocks(p) &&
             small_eligible(kq, p.x_dtype, p.w_dtype, false) && (!has_keys || small_eligible(kk, p.x_dtype, p.w_dtype, false));
     return UCM_OK;
 }
