@@ -2082,7 +2082,9 @@ __global__ __launch_bounds__(kStripWaves * kWave) __attribute__((amdgpu_waves_pe
 // time.  Blocks whose score is settled read nothing.  What bounds it is memory and the launches around it.  The whole step
 // with block_score_generic, which took these (a thread to a code, word by word, an LDS atomic for each), and
 // with this: 32 x 32,768 tokens x 8 heads 29.6 and 18.0 us, 22 x up to 44,810 tokens in blocks of 32 33.9 and 25.1, 16 x up to
-// 65,856 tokens with 8 query heads to each 43.2 and 26.6, 2 x 65,856 tokens with 4 14.1 and 13.0.
+// 65,856 tokens with 8 query heads to each 43.2 and 26.6, 2 x 65,856 tokens with 4 14.1 and 13.0.  Few long blocks, a wave each, too: one
+// request of 8 blocks x 1,024 tokens x 8 heads 25.6 and 16.3 (one query head each 19.6 and 13.8), 32 blocks x 256 x 32 heads 19.6 and 13.8,
+// 8 blocks x 4,096 x 2 heads 19.4 and 13.8.
 // ---------------------------------------------------------------------------------------
 template <int G>
 __global__ __launch_bounds__(kThreads) void block_score_half(ScoreArgs a, int pair_shift)

@@ -562,17 +562,18 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 // ---------------------------------------------------------------------------------------
-// Rows of 512 values (latent vectors) to hash columns in multiples of 64, any row count above the latency path's.
+// Rows of 512 values (latent vectors) to hash columns in multiples of 128, any row count above the latency path's.
 //
-// A workgroup's tile is 128 rows by 32 NT columns; a wave multiplies 64 rows by 16 NT columns.  Rows and projection
-// come in chunks of 64 values of k, straight from memory into a ring of four chunks in LDS (load-to-LDS, 16 bytes a
-// lane, neighbouring lanes on one line), so that nothing but the first chunk stands in front of the first matrix
+// A workgroup's tile is 32 rows a wave (four waves 128, eight 256) by 32 NT columns (64, 128 or 256); a wave multiplies 64
+// rows by 16 NT columns.  Rows and projection come in chunks of 64 values of k, straight from memory into a ring in LDS of
+// four chunks (four waves) or two (eight; load-to-LDS, 16 bytes a lane, neighbouring lanes on one line), so that nothing but the first chunk stands in front of the first matrix
 // instruction, no register holds a value on its way, and the next tile's chunks travel while this one's are
 // multiplied.  The projection keeps its row-major layout; its operands are read with the transposing LDS read.
 // Pieces of a row change places inside it (the lane picks the piece it fetches), so that both kinds of operand
-// reads find every bank once.  A wave asks for its operands two k-steps ahead; the one barrier of a chunk - all
-// waves have read chunk c, all loads of chunk c + 1 have landed - stands two k-steps in front of the first
-// operand it protects, beside matrix instructions that need none of it.
+// reads find every bank once.  A wave asks for its operands two k-steps ahead (one with 256 columns, whose registers are
+// full); the one barrier of a chunk - all waves have read chunk c, all loads of chunk c + 1 have landed - stands as many
+// k-steps in front of the first operand it protects, beside matrix instructions that need none of it.  24 to 44 scalar
+// registers (addresses of the chunk loads) go through lanes of a vector register; no vector register is spilled.
 //
 // What bounds it: the first chunk's way (some 3 us with the launch), then LDS - 64 x 64 products a wave read 4 KiB of
 // operands for four matrix instructions of 32 cycles, 128 bytes a cycle from four waves, beside 64 that the loads
@@ -585,12 +586,12 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2,
 constexpr int kPipeKS = 32;     // k-steps of 16: rows of 512 values
 constexpr int kPipeChunk = 64;  // values of k to a chunk
 constexpr int pipe_rows(int waves) { return waves * 32; }
-constexpr int pipe_ring(int nt, int waves) { return waves == 8 ? 2 : 4; }  // chunks in LDS
+constexpr int pipe_ring(int waves) { return waves == 8 ? 2 : 4; }  // chunks in LDS
 constexpr int pipe_stage_bytes(int nt, int waves) { return (pipe_rows(waves) + nt * 32) * kPipeChunk * 2; }
 constexpr int pipe_slot_bytes(int waves) { return pipe_rows(waves) * 8; }  // a tile's raw slots: low words, then high words
 constexpr int pipe_lds(int nt, int waves)
 {
-    return pipe_ring(nt, waves) * pipe_stage_bytes(nt, waves) + 2 * pipe_slot_bytes(waves);
+    return pipe_ring(waves) * pipe_stage_bytes(nt, waves) + 2 * pipe_slot_bytes(waves);
 }
 
 // Touches every 64-byte line of a kernel-argument struct at once.  The compiler fetches a field
@@ -609,7 +610,7 @@ __device__ __forceinline__ void warm_args(const T& args)
     asm volatile("" ::"s"(t));
 }
 
-// N loads of 16 bytes a lane, each to 1 KiB of LDS behind the last: bases in scalar registers, lane offsets off.
+// Two loads of 16 bytes a lane, to 1 KiB of LDS each, one behind the other: bases in scalar registers, offsets in lanes.
 __device__ __forceinline__ void pipe_load(uint32_t lds, uint64_t b0, uint32_t o0, uint64_t b1, uint32_t o1)
 {
     uint32_t keep;
@@ -643,7 +644,7 @@ template <typename V, int NT, int kWaves, bool kRuns>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void encode_pipe_kernel(EncArgs a, int streams, int run)
 {
     static_assert((NT == 2 && kWaves == 4) || NT == 4 || (NT == 8 && kWaves == 8), "64, 128 or 256 columns");
-    constexpr int kRows = pipe_rows(kWaves), kPipeRing = pipe_ring(NT, kWaves);
+    constexpr int kRows = pipe_rows(kWaves), kPipeRing = pipe_ring(kWaves);
     constexpr int kPipeRowBytes = kRows * kPipeChunk * 2, kPipeSlotBytes = pipe_slot_bytes(kWaves);
     constexpr int kStage = pipe_stage_bytes(NT, kWaves), kCols = NT / 2;  // kCols: column tiles of 32 of a wave
     constexpr int kWLoads = NT * 4 / kWaves, kLoads = 4 + kWLoads;         // of a wave, per chunk
@@ -1786,8 +1787,9 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(1,
 }
 
 // ---------------------------------------------------------------------------------------
-// Rows that lie side by side in blocks of a paged cache (a prefix that is hashed where it lies), as many hash bits as
-// channels: 32 rows are one run of memory, and so are their codes.
+// Rows that lie side by side, as many hash bits as channels: 32 of them are one run of memory.  Either blocks of a paged cache (a
+// prefix that is hashed where it lies; the codes are runs of memory too), any number of rows; or rows by slot or dense, a tile to
+// a wave at most: their slots are read once, in front of the wave's only tile.
 //
 // What bounds it is memory, so it is built to have it busy from the start: every wave streams tiles of 32 rows
 // through two slots of its own in LDS (load-to-LDS, whole lines, 128 KiB on their way in a compute unit) and meets
@@ -1795,7 +1797,8 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(1,
 // 16-byte pieces so that the operand reads find every bank once.  Before (encode_mfma_kernel, whose workgroups transpose
 // the projection through registers in front of their first rows) and now: 16,384 rows of 128 channels 5.0 and 3.3 us,
 // 65,536 rows 6.7 and 5.5, 261,528 rows 20.2 and 16.0 (4.2 TB/s), 1,048,000 rows 64.4 and 60.9; 64 channels, 65,536 rows 5.5
-// and 3.1, 262,144 rows 9.9 and 8.6.  By slot, 16,384 rows of 128 channels 4.8 and 3.5, of 64 channels 65,536 rows 5.4 and 3.3.
+// and 3.1, 262,144 rows 9.9 and 8.6.  By slot, 16,384 rows of 128 channels 4.8 and 3.5, 64,000 rows 7.2 and 5.8, of 64 channels 65,536
+// rows 5.4 and 3.3.
 // ---------------------------------------------------------------------------------------
 constexpr int kRunWaves = 8;
 constexpr int kRunSlots = 2;
@@ -3233,9 +3236,9 @@ bool small_eligible(const EncArgs& a, int x_dtype, int w_dtype, bool alone = tru
     return small_us < lds_floor_us;
 }
 
-// Rows that lie side by side: all of them, a tile of 32 to a wave at most and more than the latency path's, or those of a
-// paged input's blocks with their codes, of any number (64 to 130 rows of 128 channels x 8 heads 3.1 against 3.4 us of the
-// small-row kernel).
+// Rows that lie side by side: all of them, a tile of 32 to a wave at most (the by-slot form has no second one) and more than the
+// latency path's, or those of a paged input's blocks with their codes, of any number (16 to 512 tokens of 8 heads, 128 channels 3.0
+// to 3.1 against 3.2 to 3.9 us of the small-row kernel, 64 channels 2.3 to 2.5 against 3.0 to 3.3).
 bool run_eligible(const EncArgs& a, int x_dtype, int w_dtype)
 {
     if (!mfma_eligible(a, x_dtype, w_dtype)) return false;
