@@ -200,6 +200,39 @@ def test_against_float64_formulation_at_llama_shape():
     assert gs.sum() <= 8 * 32 * (1 + 1e-5)
 
 
+@pytest.mark.parametrize("X,Hq,Hkv,d,n,M", [
+    (1, 1, 1, 64, 1, 16), (2, 8, 8, 32, 3, 16),       # half a tile of representatives; one and a half
+    (1, 6, 3, 128, 5, 16), (3, 6, 3, 64, 33, 32),     # an odd number of row tiles; of tiles of representatives
+    (9, 32, 8, 32, 256, 16), (2, 4, 4, 32, 257, 32),   # a row's blocks in eight loads of the merging threads, one more
+    (1, 8, 8, 32, 512, 16), (1, 8, 8, 32, 513, 16),
+    (1, 8, 8, 32, 1024, 16), (1, 8, 8, 32, 1025, 16),  # the most blocks of 16 taken once, and one more
+    (1, 2, 1, 32, 1025, 32), (1, 2, 1, 32, 2048, 64), (1, 2, 1, 32, 2049, 64),  # loaded twice; the most that are ranked
+    (17, 8, 4, 128, 40, 64), (2, 4, 2, 64, 21, 128), (2, 4, 2, 32, 65, 256), (2, 4, 2, 32, 9, 320),
+])
+def test_blocks_whose_scores_are_taken_once(X, Hq, Hkv, d, n, M):
+    """Against float64: 16, 32, 64, 128 and 256 representatives on both sides of where such blocks leave the
+    general path.  Half of the blocks lie e^-60 below the others."""
+    q, k = make(X + n + M + d, X, Hq, Hkv, d, n, M)
+    q[..., 0] = 8.0
+    k[..., 0] = np.where(np.arange(n) % 2 == 1, -7.5, 0.0)[:, None, None]
+    gi, gs = run_gpu(q, k, None, n)
+    ref = brute.kvstar_block_scores(q, k)
+    assert sorted(gi.tolist()) == list(range(n)) and np.all(np.diff(gs) <= 0)
+    assert np.all(np.abs(gs - ref[gi]) <= RTOL * ref[gi] + 2e-45)
+
+
+@pytest.mark.parametrize("M", [16, 32, 128])
+@pytest.mark.parametrize("what", ["nan", "+inf", "-inf", "nan_lane", "all_-inf"])
+def test_infinite_and_undefined_scores_taken_once(what, M):
+    test_infinite_and_undefined_scores(what, 300, M, 32)
+
+
+@pytest.mark.parametrize("base", [-3.2e8, 4.0e9])
+@pytest.mark.parametrize("d,M", [(32, 16), (64, 32), (128, 64)])
+def test_scores_of_any_finite_size_taken_once(base, d, M):
+    test_scores_of_any_finite_size(base, d, M)
+
+
 def test_long_rows_in_two_batches_of_statistics():
     # 2560 query rows; against float64, as the checker adds a block's 102,400 probabilities one by one
     q, k = make(40, 40, 64, 2, 130, 9, 40, scale=0.5)

@@ -4,6 +4,8 @@
 // score, so a row is one word per candidate.  Included by the translation units that launch it.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -47,6 +49,8 @@ struct SortArgs {
     int max_n, topk, cap;   // cap: entries the search orders in LDS, a power of two
     int32_t* out_idx;       // [B][topk]
     float* out_score;       // [B][topk]
+    const float* sums;      // topk_rank_sums_kernel, one row: [n_sums][max_n] parts of the scores, instead of keys
+    int n_sums;
 };
 
 // Maximum over the 64 lanes, in every lane: exchanges inside a row of 16 lanes, then the last lane
@@ -644,20 +648,24 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
 
 // Short rows: every candidate counts those that come before it in the output order (larger key, or equal key
 // and earlier position) and writes itself at that rank.  Its time does not depend on the values.  A workgroup
-// ranks 64 candidates; its four waves compare them with every fourth 64 entries of the row, which a wave holds
+// ranks 64 candidates; its waves compare them with every so many 64 entries of the row, which a wave holds
 // in a register and hands round lane by lane.  grid = (rows, ceil(max_n / 64)).
-constexpr int kRankRow = 512;
-__global__ __launch_bounds__(256) void topk_rank_kernel(SortArgs a)
+template <int WAVES>
+struct RankShared {
+    int part[WAVES][64], valid[WAVES];
+};
+
+// mine: the lane's candidate of the workgroup; first: of the wave's first 64, where has_first says that it is known.
+template <int WAVES, typename Key>
+__device__ __forceinline__ void rank_places(const SortArgs& a, int waves, uint32_t mine, uint32_t first, bool has_first,
+                                            Key key_of, RankShared<WAVES>& sh)
 {
-    __shared__ int part[4][64], valid[4];
     const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, mine_at = blockIdx.y;
-    const uint32_t* keys = a.keys + b * a.pitch;
     const int pos = mine_at * 64 + lane;
-    const uint32_t mine = pos < a.max_n ? keys[pos] : 0u;
     const int32_t id = w == 0 && a.idx && pos < a.max_n ? a.idx[(int64_t)b * a.max_n + pos] : pos;
     int rank = 0, have = 0;
-    for (int piece = w; piece * 64 < a.max_n; piece += 4) {
-        const uint32_t k = piece * 64 + lane < a.max_n ? keys[piece * 64 + lane] : 0u;
+    for (int piece = w; piece * 64 < a.max_n; piece += waves) {
+        const uint32_t k = has_first && piece == w ? first : key_of(piece * 64 + lane);
         have += __popcll(__ballot(k != 0u));
         if (piece == mine_at) {
 #pragma unroll
@@ -672,19 +680,79 @@ __global__ __launch_bounds__(256) void topk_rank_kernel(SortArgs a)
             for (int j = 0; j < 64; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)k, j) > above;
         }
     }
-    part[w][lane] = rank;
-    if (lane == 0) valid[w] = have;
+    sh.part[w][lane] = rank;
+    if (lane == 0) sh.valid[w] = have;
     __syncthreads();
     if (w != 0) return;
-    rank = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+    rank = 0;
+    int n_valid = 0;
+#pragma unroll
+    for (int i = 0; i < WAVES; ++i) {
+        if (i >= waves) break;
+        rank += sh.part[i][lane];
+        n_valid += sh.valid[i];
+    }
     if (mine != 0u && rank < a.topk) {
         a.out_idx[(int64_t)b * a.topk + rank] = id;
         a.out_score[(int64_t)b * a.topk + rank] = out_of(mine);
     }
-    for (int t = valid[0] + valid[1] + valid[2] + valid[3] + pos; t < a.topk; t += 64 * (int)gridDim.y) {
+    for (int t = n_valid + pos; t < a.topk; t += 64 * (int)gridDim.y) {
         a.out_idx[(int64_t)b * a.topk + t] = -1;
         a.out_score[(int64_t)b * a.topk + t] = 0.0f;
     }
+}
+
+constexpr int kRankRow = 512;
+__global__ __launch_bounds__(256) void topk_rank_kernel(SortArgs a)
+{
+    __shared__ RankShared<4> sh;
+    const uint32_t* keys = a.keys + blockIdx.x * a.pitch;
+    const int pos = blockIdx.y * 64 + (threadIdx.x & 63);
+    const uint32_t mine = pos < a.max_n ? keys[pos] : 0u;
+    rank_places<4>(a, 4, mine, 0u, false, [&](int at) { return at < a.max_n ? keys[at] : 0u; }, sh);
+}
+
+// The same for one row of up to kRankSums candidates whose scores are still in n_sums parts, which every workgroup
+// adds by itself, in the same order.  A wave for every 64 candidates up to sixteen: the parts of a wave's 64 and those
+// of the workgroup's own 64 are one round trip (253 candidates of 16 parts: 4.7 us, requested a
+// few at a time 5.0; 1024 of them 3 us less than in four waves with a branch at every part).
+constexpr int kRankSums = 2048;
+__global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SortArgs a)
+{
+    __shared__ RankShared<16> sh;
+    auto keys_of = [&](auto n_, const int (&at)[decltype(n_)::value], uint32_t (&key)[decltype(n_)::value]) {
+        constexpr int N = decltype(n_)::value;
+        float s[N] = {};
+        uint32_t off[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) off[n] = at[n] < a.max_n ? at[n] : a.max_n - 1;
+        for (int i = 0; i < a.n_sums; i += 16) {
+            float v[N][16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float* p = a.sums + (int64_t)(i + e < a.n_sums ? i + e : 0) * a.max_n;
+#pragma unroll
+                for (int n = 0; n < N; ++n) v[n][e] = p[off[n]];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // all requested before the first is waited for
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+#pragma unroll
+                for (int n = 0; n < N; ++n) s[n] += i + e < a.n_sums ? v[n][e] : 0.0f;
+        }
+#pragma unroll
+        for (int n = 0; n < N; ++n) key[n] = at[n] < a.max_n ? score_key(s[n]) : 0u;
+    };
+    const int lane = threadIdx.x & 63;
+    const int at[2] = {(int)blockIdx.y * 64 + lane, (int)threadIdx.x};
+    uint32_t key[2];
+    keys_of(std::integral_constant<int, 2>{}, at, key);
+    rank_places<16>(a, blockDim.x / 64, key[0], key[1], true, [&](int p) {
+        const int one[1] = {p};
+        uint32_t k[1];
+        keys_of(std::integral_constant<int, 1>{}, one, k);
+        return k[0];
+    }, sh);
 }
 
 // LDS of topk_kernel: bins and winners, as the two paths lay them out.
@@ -740,6 +808,14 @@ inline int launch_topk_as(SortArgs s, int rows, hipStream_t st)
     static_assert(search_lds(NT, kMaxTopk) + 512 <= 64 * 1024 && direct_lds(NT) + 512 <= 64 * 1024, "");
     hipLaunchKernelGGL((topk_kernel<NT, PER>), dim3((unsigned)rows, (unsigned)split), dim3(NT), need > direct ? need : direct, st, s);
     return ucm::launch_status("topk_kernel");
+}
+
+// One row of up to kRankSums candidates whose scores are in parts.
+inline int launch_rank_sums(const SortArgs& s, hipStream_t st)
+{
+    const unsigned pieces = (unsigned)ucm::ceil_div(s.max_n, 64);
+    hipLaunchKernelGGL(topk_rank_sums_kernel, dim3(1, pieces), dim3(64 * (pieces < 16 ? pieces : 16)), 0, st, s);
+    return ucm::launch_status("topk_rank_sums_kernel");
 }
 
 // Rows of up to 512 candidates are ranked: as fast as the direct path on an even row (two rows, whole call: 253

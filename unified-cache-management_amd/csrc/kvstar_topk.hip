@@ -10,15 +10,17 @@
 //      <= 1e-9, as the reference does);
 //   4. block score[n] = sum over x, H and the M representatives of block n;
 //   5. the topk blocks by descending score.
-// Kernels: kvstar_stats_kernel (q.k on the matrix cores; maximum and sum of exponentials of every
-// (x, H) row over one chunk of the representatives), kvstar_mass_kernel (the chunks' pairs merged,
-// q.k once more, probabilities summed over rows and a block's representatives) and the shared top-k
-// selection.  The [X Hq, S] score matrix is never stored: writing it and reading it back twice moved
-// seven times the bytes of the keys themselves, and computing q.k a second time costs two matrix
-// instructions per 32 x 32 scores of 32 channels.  At 8 query tokens x 32 heads, 253 blocks x 64
-// representatives and 32 channels the four kernels that stored it took 33.1 us (13.6 q.k, 8.6 row
-// statistics, 6.1 block sums, 5.7 selection); these three take 18.3 us
-// (7.4, 8.8, 3.2; 1.2 and 1.0 of the first two for the exponentials: what is left is launches and round trips).
+// Two ways, by the shape of the blocks; the [X Hq, S] score matrix is stored by neither (writing it and reading it
+// back twice moved seven times the bytes of the keys themselves).
+//   * Blocks of 16, 32 or up to four times 64 representatives of 32, 64 or 128 channels, up to kRankSums of them:
+//     kvstar_unit_kernel (q.k on the matrix cores; maximum and sum of exponentials of every row and block),
+//     kvstar_merge_kernel (probabilities of them, summed over sixteen rows) and the ranking, which adds the last sums.
+//   * Everything else: kvstar_stats_kernel (maximum and sum of exponentials of every row over one chunk of the
+//     representatives), kvstar_mass_kernel (the chunks' pairs merged, q.k once more, probabilities summed over rows
+//     and a block's representatives) and the shared top-k selection.
+// 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 15.1 us (6.0, 4.3 and 4.7 of the three
+// kernels: launches and round trips; the products and exponentials are about 1.5), 18.8 the second way
+// (7.5, 9.0, 3.7); 1024 blocks, 128 channels: 42.9 and 70.4, the second way reads the keys twice.
 // Sums are taken in a different order than the reference's loops, the same one on every call (no
 // atomics); the tolerance is stated where the results are compared.  Equal scores come out in
 // ascending block order (the reference's heap pops them in descending block order).
@@ -42,6 +44,9 @@ constexpr int kLongDim = 128;       // above it loads take more of both kernels'
 constexpr int kMaxChunks = 64;      // partial statistics per row
 constexpr int kMassRows = 2048;     // rows whose statistics the mass kernel holds in LDS at a time
 constexpr int kMassGroups = 512;    // its workgroups at most
+constexpr int kMergeRows = 16;      // query rows of a workgroup of the merge kernel
+constexpr int kUnitGroups = 512;    // workgroups of the unit kernel at most
+constexpr int64_t kUnitBytes = 64 << 20;  // its pairs at most
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -67,8 +72,10 @@ struct KvArgs {
     int chunks;
     int dp;                 // d in whole steps of 16 channels
     _Float16* qp;           // [items][32][dp] query rows, channels pruned, zeros behind the last row and channel
-    Stat* part;             // [chunks][items * 32] sum of exponentials over a chunk
+    Stat* part;             // [chunks][items * 32] sum of exponentials over a chunk, or [units][items * 32] over a unit
     uint32_t* keys;         // [n_blocks]
+    float* sums;            // [items * 32 / kMergeRows][units] probabilities of a unit, summed over so many rows
+    int units;              // a unit is a block, where all of a row's fit (0: chunks instead)
     int group_blocks;       // blocks a workgroup of the mass kernel handles together
     int groups;
 };
@@ -123,6 +130,7 @@ __device__ __forceinline__ f16x8 load_q(const QRow& q, int c, int d, int d_orig)
 }
 
 constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596303e-8f;  // log2(e) in two pieces
+constexpr float kLn2 = 0.693147182f;
 
 // exp(x) for x far from overflow (here x <= 0 but for rounding): 2^(x log2 e) with log2 e in two pieces and the
 // product's rounding error carried along (Dekker's exact product, by a fused multiply-add), whole and fractional
@@ -134,6 +142,18 @@ __device__ __forceinline__ float exp_small(float x)
     const float n = __builtin_rintf(t);
     const float r = __builtin_fmaf(x, kLog2eLow, __builtin_fmaf(x, kLog2e, -t));
     return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - n) + r), (int)n);
+}
+
+// exp(x) as a term of a sum that holds a 1, in seven instructions instead of twelve (the unit kernel's launch of the
+// example's shape 5.9 us with it, 6.7 with exp_small): what lies below 2^-126 may be 0.  exp2's argument is rounded, and what
+// the rounding took (x - t ln 2, by a fused multiply-add) is put back to first order; ln 2's own rounding moves a
+// result by 1.9e-9 |t| of itself.
+__device__ __forceinline__ float exp_term(float x)
+{
+    x = __builtin_elementwise_maximum(x, -200.0f);
+    const float t = x * kLog2e;
+    const float e = __builtin_amdgcn_exp2f(t);
+    return __builtin_fmaf(e, __builtin_fmaf(-t, kLn2, x), e);
 }
 
 // What a part's maximum is measured from: 0 where the largest one is minus infinity, whose exponentials are 0.
@@ -217,6 +237,22 @@ __global__ __launch_bounds__(kThreads) void kvstar_pack_kernel(KvArgs a)
     *reinterpret_cast<f16x8*>(a.qp + row * a.dp + c) = load_q(q_row(a, (int)(row >> 5), (int)(row & 31)), c, a.d, a.d_orig);
 }
 
+// The query rows of a workgroup's two items into LDS, eight threads per row, each taking every eighth channel.
+template <int KS>
+__device__ __forceinline__ void gather_rows(const KvArgs& a, _Float16* qt, int pitch)
+{
+    const int rl = threadIdx.x >> 3;  // 0 .. 63: row rl % 32 of the workgroup's item rl / 32
+    const QRow q = q_row(a, blockIdx.y * stat_items(KS) + (rl >> 5), rl & 31);
+    int64_t src[2 * KS];
+    _Float16 v[2 * KS];
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i) src[i] = q_channel(q, (threadIdx.x & 7) + 8 * i, a.d_orig);
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i) v[i] = q.row[src[i]];
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i) qt[rl * pitch + (threadIdx.x & 7) + 8 * i] = q.ok ? v[i] : (_Float16)0;
+}
+
 // grid = (chunks, ceil(items / kItems)).  Wave w serves row tile w % kItems and every
 // kSubs-th tile of representatives of the chunk.  Representatives are the A operand (lane:
 // representative lane % 32, channels 8 (lane / 32) .. + 7 of the k-step), query rows the B operand:
@@ -261,17 +297,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
     };
     if constexpr (KS > 0) {
         load_tiles(t0 < a.tiles_k ? t0 : 0);
-        // eight threads per query row, each taking every eighth channel
-        const int rl = threadIdx.x >> 3;  // 0 .. 63: row rl % 32 of the workgroup's item rl / 32
-        const QRow q = q_row(a, blockIdx.y * kItems + (rl >> 5), rl & 31);
-        int64_t src[2 * KS];
-        _Float16 v[2 * KS];
-#pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) src[i] = q_channel(q, (threadIdx.x & 7) + 8 * i, a.d_orig);
-#pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) v[i] = q.row[src[i]];
-#pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) qt[rl * pitch + (threadIdx.x & 7) + 8 * i] = q.ok ? v[i] : (_Float16)0;
+        gather_rows<KS>(a, qt, pitch);
     } else if constexpr (KS == kAnyDim) {
         const _Float16* row = k_row(t0 < a.tiles_k ? t0 : 0);
 #pragma unroll
@@ -564,6 +590,176 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
     }
 }
 
+// Blocks whose q.k is taken once.  This kernel leaves the maximum and the sum of exponentials of every (row, block), and kvstar_merge_kernel, which
+// sees all of a row's blocks, makes probabilities of them.
+// grid = (parts of the blocks, ceil(items / 2)).  Operands as in kvstar_stats_kernel.  A wave takes a block, or as many
+// small ones as two tiles hold (one tile of 128 channels: registers), at a time.
+template <int KS, int UNIT>
+__global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(KvArgs a)
+{
+    constexpr int kItems = stat_items(KS), kSubs = kThreads / 64 / kItems;
+    constexpr int U = UNIT == 64 || KS <= 4 ? 2 : 1;
+    constexpr int pitch = KS * 16 + 8;
+    __shared__ __align__(16) _Float16 qt[kItems * 32 * pitch];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = wave % kItems, sub = wave / kItems;
+    const int item = blockIdx.y * kItems + li;
+    const int h = item < a.items ? item / a.tiles_q : 0;
+    const int kb = (lane >> 5) * 8;
+    const int rows = a.items * 32;
+    const int per = UNIT == 64 ? a.M / 64 : 1;  // steps of two tiles to a block
+    const int steps = item < a.items ? (UNIT == 64 ? a.units : (a.tiles_k + U - 1) / U) : 0;
+    const int p0 = blockIdx.x * kSubs + sub;
+    f16x8 kk[U][KS];
+    auto load_tiles = [&](int p) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            int64_t s = (int64_t)(p * U + u) * 32 + (lane & 31);
+            s = s < a.S ? s : a.S - 1;
+            const _Float16* row = a.k + (s * a.Hkv + h) * (KS * 16);
+#pragma unroll
+            for (int c = 0; c < KS; ++c) kk[u][c] = *reinterpret_cast<const f16x8*>(row + c * 16 + kb);
+        }
+    };
+    load_tiles(p0 < steps ? p0 * per : 0);
+    gather_rows<KS>(a, qt, pitch);
+    __syncthreads();
+    Stat* out = a.part + item * 32 + (lane & 31);
+    Stat sofar{-INFINITY, 0.0f};
+    for (int p = p0, q = 0; p < steps; q + 1 < per ? ++q : (p += gridDim.x * kSubs, q = 0)) {
+        if (p != p0 || q != 0) load_tiles(p * per + q);
+        f32x16 acc[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc[u] = f32x16{0};
+        const _Float16* qrow = qt + (li * 32 + (lane & 31)) * pitch + kb;
+#pragma unroll
+        for (int c = 0; c < KS; ++c) {
+            const f16x8 qq = *reinterpret_cast<const f16x8*>(qrow + c * 16);
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kk[u][c], qq, acc[u], 0, 0, 0);
+        }
+        // a unit's tile values lo .. hi - 1 of both lane halves; a unit is whole (S is a whole number of them)
+        auto pair_of = [&](auto get, int n) {
+            float m = -INFINITY;
+#pragma unroll
+            for (int v = 0; v < n; ++v) m = fmaxf(m, get(v));
+            m = fmaxf(m, __shfl_xor(m, 32));
+            // minus infinities alone measure from 0 and add 0; a NaN, which the maximum passes over, makes the sum one
+            const float base = stat_base(m);
+            float s = 0.0f;
+#pragma unroll
+            for (int v = 0; v < n; ++v) s += exp_term(get(v) - base);
+            return Stat{m, s + __shfl_xor(s, 32)};
+        };
+        if constexpr (UNIT == 64) {
+            const Stat st = pair_of([&](int v) { return acc[v / 16][v % 16]; }, 32);
+            if (per > 1) {
+                const Stat other[1] = {st};
+                sofar = merge(q == 0 ? Stat{-INFINITY, 0.0f} : sofar, other);
+            } else {
+                sofar = st;
+            }
+            if (lane < 32 && q == per - 1) out[(int64_t)p * rows] = sofar;
+        } else {
+            constexpr int N = UNIT / 2, kPer = 32 / UNIT;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < kPer; ++i) {
+                    const int unit = (p * U + u) * kPer + i;
+                    const Stat st = pair_of([&](int v) { return acc[u][i * N + v]; }, N);
+                    if (lane < 32 && unit < a.units) out[(int64_t)unit * rows] = st;
+                }
+        }
+    }
+}
+
+// The other half: grid = items * 32 / kMergeRows, a workgroup per kMergeRows query rows of an item.  A thread holds
+// R units of one row at a time: the row's maximum and sum over all units meet through the lanes and LDS, then every
+// unit's probability is its sum times exp(its maximum - the row's) over the row's sum, added up over the rows by the
+// sixteen lanes that hold them.
+template <int NT, int R>
+__global__ __launch_bounds__(NT) void kvstar_merge_kernel(KvArgs a)
+{
+    constexpr int kGroups = NT / kMergeRows, kWaves = NT / 64;
+    static_assert(kMergeRows == 16 && kWaves % 4 == 0, "a row of lanes");
+    __shared__ Stat red[kWaves][kMergeRows];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = threadIdx.x % kMergeRows, grp = threadIdx.x / kMergeRows;
+    const int rows = a.items * 32, r0 = blockIdx.x * kMergeRows;
+    const int item = r0 / 32;
+    // rows of the item that exist: X * g of the KV head are cut into its tiles
+    const bool real = (item % a.tiles_q) * 32 + r0 % 32 + r < a.X * a.g;
+    const Stat* p = a.part + r0 + r;
+    Stat v[R];
+    auto load = [&](int u0) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int u = u0 + grp + i * kGroups;
+            v[i] = p[(int64_t)(u < a.units ? u : a.units - 1) * rows];
+        }
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (u0 + grp + i * kGroups >= a.units) v[i] = Stat{-INFINITY, 0.0f};
+    };
+    Stat st{-INFINITY, 0.0f};
+    // one load: v[i].s becomes the unit's sum measured from the thread's own largest score
+    const bool held = a.units <= R * kGroups;
+    if (held) {
+        load(0);
+#pragma unroll
+        for (int i = 0; i < R; ++i) st.m = fmaxf(st.m, v[i].m);
+        const float base = stat_base(st.m);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            v[i].s *= exp_small(v[i].m - base);
+            st.s += v[i].s;
+        }
+    } else {
+        for (int u0 = 0; u0 < a.units; u0 += R * kGroups) {
+            load(u0);
+            st = merge(st, v);
+        }
+    }
+    const float own = st.m;
+    auto meet = [&] {  // the four threads of a wave that share a row
+#pragma unroll
+        for (int o = kMergeRows; o < 64; o <<= 1) {
+            const Stat other[1] = {Stat{__shfl_xor(st.m, o), __shfl_xor(st.s, o)}};
+            st = merge(st, other);
+        }
+    };
+    meet();
+    if (lane < kMergeRows) red[wave][lane] = st;
+    __syncthreads();
+    // every thread a quarter of the waves: exponentials are what this kernel issues most of
+    Stat all[kWaves / 4];
+#pragma unroll
+    for (int w = 0; w < kWaves / 4; ++w) all[w] = red[lane / kMergeRows * (kWaves / 4) + w][r];
+    st = merge(Stat{-INFINITY, 0.0f}, all);
+    meet();
+    // the reference normalises only when the sum exceeds 1e-9
+    float inv = st.s > 1e-9f ? 1.0f / st.s : 1.0f;
+    if (st.m == -INFINITY) inv = NAN;  // a row of minus infinities has no probabilities
+    const float scale = own == st.m ? 1.0f : exp_small(own - st.m);
+    for (int u0 = 0; u0 < a.units; u0 += R * kGroups) {
+        if (!held) load(u0);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int u = u0 + grp + i * kGroups;
+            float e = real ? v[i].s * (held ? scale : exp_small(v[i].m - st.m)) * inv : 0.0f;
+            auto add = [&](auto ctl) {
+                e += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(e), decltype(ctl)::value, 0xf, 0xf, false));
+            };
+            add(std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+            add(std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+            add(std::integral_constant<int, 0x141>{});  // row_half_mirror
+            add(std::integral_constant<int, 0x140>{});  // row_mirror
+            if (r == 0 && u < a.units) a.sums[(int64_t)blockIdx.x * a.units + u] = e;
+        }
+    }
+}
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 constexpr int kMaxDim = 1024;
@@ -589,17 +785,32 @@ void plan_chunks(KvArgs& a)
     a.groups = (int)ucm::ceil_div(a.n_blocks, a.group_blocks);
 }
 
+// Whether the blocks are units: whole halves, ones or pairs of tiles, so that a wave has all of a block's scores.
+// A pair is 8 bytes for every row, written and read, where the second way reads a block's keys and takes its products
+// again: at 16 representatives of 32 channels that is even (256 rows, 1024 blocks 20.5 and 21.4 us, 2040: 27.7 and
+// 27.5), at 64 it never is (2000: 39.3 and 53.8).  Blocks of 48 in units of 16: 20.5 and 18.0.  `rows` bounds the padded query rows for every number of KV heads, so that the
+// workspace's size decides like the call.
+void plan_units(KvArgs& a, int64_t rows)
+{
+    const bool whole = a.M == 16 || a.M == 32 || (a.M % 64 == 0 && a.M <= 256);
+    const int most = a.M == 16 ? 1024 : kRankSums;
+    a.units = whole && a.n_blocks <= most && a.n_blocks * rows * 8 <= kUnitBytes ? a.n_blocks : 0;
+}
+
 // Addresses of the workspace's parts; the sizes hold for every number of KV heads and every head
 // dimension (the caller asks with neither).
 size_t carve_kvstar(KvArgs& a, void* base)
 {
     const size_t rows = (size_t)a.Hq * (a.X + 31);  // at most 31 rows of padding per KV head
+    plan_units(a, (int64_t)rows);
     char* p = (char*)base;
     size_t off = 0;
     a.qp = (_Float16*)(p + off);
     off += align256(rows * kMaxDim * 2);
     a.part = (Stat*)(p + off);
-    off += align256((size_t)a.chunks * rows * 8);
+    off += align256((size_t)(a.chunks > a.units ? a.chunks : a.units) * rows * 8);
+    a.sums = (float*)(p + off);
+    off += align256(ucm::ceil_div((int64_t)rows, kMergeRows) * (size_t)a.units * 4);
     a.keys = (uint32_t*)(p + off);
     off += align256((size_t)key_pitch(a.n_blocks) * 4);
     return off;
@@ -628,6 +839,29 @@ int launch_kvstar(const KvArgs& a, hipStream_t st)
     else
         hipLaunchKernelGGL((kvstar_mass_kernel<(KS > 0 ? KS : kAnyDim), false>), groups, dim3(kThreads), 0, st, a);
     return ucm::launch_status("kvstar_mass_kernel");
+}
+
+template <int KS, int UNIT>
+int launch_units(const KvArgs& a, hipStream_t st)
+{
+    constexpr int U = UNIT == 64 || KS <= 4 ? 2 : 1, kSubs = kThreads / 64 / stat_items(KS);
+    const int64_t heads = ucm::ceil_div(a.items, stat_items(KS)), most = kUnitGroups / heads;
+    const int64_t need = ucm::ceil_div(UNIT == 64 ? a.units : ucm::ceil_div(a.tiles_k, U), kSubs);
+    const int64_t parts = need < most ? need : (most < 1 ? 1 : most);
+    hipLaunchKernelGGL((kvstar_unit_kernel<KS, UNIT>), dim3((unsigned)parts, (unsigned)heads), dim3(kThreads), 0, st, a);
+    int rc = ucm::launch_status("kvstar_unit_kernel");
+    if (rc != UCM_OK) return rc;
+    const dim3 grid((unsigned)(a.items * (32 / kMergeRows)));
+    if (a.units <= 256) hipLaunchKernelGGL((kvstar_merge_kernel<512, 8>), grid, dim3(512), 0, st, a);
+    else if (a.units <= 512) hipLaunchKernelGGL((kvstar_merge_kernel<1024, 8>), grid, dim3(1024), 0, st, a);
+    else hipLaunchKernelGGL((kvstar_merge_kernel<1024, 16>), grid, dim3(1024), 0, st, a);
+    return ucm::launch_status("kvstar_merge_kernel");
+}
+
+template <int KS>
+int launch_units(const KvArgs& a, hipStream_t st)
+{
+    return a.M == 16 ? launch_units<KS, 16>(a, st) : a.M == 32 ? launch_units<KS, 32>(a, st) : launch_units<KS, 64>(a, st);
 }
 
 }  // namespace
@@ -674,14 +908,23 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     a.items = Hkv * a.tiles_q;
     plan_chunks(a);
     carve_kvstar(a, workspace);
+    SortArgs s{};
+    s.max_n = (int)n_blocks; s.topk = topk;
+    s.out_idx = out_idx; s.out_score = out_score;
+    // few row tiles leave the merging to few workgroups (four, 600 blocks of 16 x 32 channels: 18.6 and 17.0 us)
+    const bool few = M == 16 && d == 32 && a.items < 8;
+    if (a.units > 0 && !few && (d == 32 || d == 64 || d == 128)) {
+        const int rc = d == 32 ? launch_units<2>(a, st) : d == 64 ? launch_units<4>(a, st) : launch_units<8>(a, st);
+        if (rc != UCM_OK) return rc;
+        s.sums = a.sums; s.n_sums = a.items * (32 / kMergeRows);
+        return launch_rank_sums(s, st);
+    }
     const int rc = d == 32 ? launch_kvstar<2>(a, st)
                  : d == 64 ? launch_kvstar<4>(a, st)
                  : d == 128 ? launch_kvstar<8>(a, st)
                                    : d <= kAnyDimMost ? launch_kvstar<kAnyDim>(a, st)
                                  : launch_kvstar<kPacked>(a, st);
     if (rc != UCM_OK) return rc;
-    SortArgs s{};
-    s.keys = a.keys; s.pitch = key_pitch(n_blocks); s.max_n = (int)n_blocks; s.topk = topk;
-    s.out_idx = out_idx; s.out_score = out_score;
+    s.keys = a.keys; s.pitch = key_pitch(n_blocks);
     return launch_topk(s, 1, st);
 }
