@@ -191,6 +191,82 @@ def test_fused_latent_attention_step_equals_separate_operators_and_oracle(Hq, T)
         assert torch.equal(st.out_idx, idx) and torch.equal(st.out_score, sc)
 
 
+@pytest.mark.parametrize("B,Hq,R,T,dt", [
+    (1, 1, 1, 1, torch.bfloat16), (1, 2, 2, 1, torch.float16),    # one row; the mean of two
+    (2, 32, 2, 3, torch.bfloat16), (5, 16, 1, 5, torch.bfloat16),  # a whole row tile; two and a half
+    (4, 128, 2, 33, torch.float16), (9, 64, 2, 40, torch.bfloat16),  # eight row tiles; nine, two tiles of keys
+    (3, 48, 2, 2, torch.bfloat16), (2, 64, 4, 2, torch.bfloat16),  # 24 heads, means of four: the kernel of every form
+])
+@pytest.mark.parametrize("slots_i64", [False, True])
+def test_latent_step_hashes_every_row(B, Hq, R, T, dt, slots_i64):
+    """Codes of queries (means of R heads) and new keys against float64: a bit may differ only where the projection is
+    within 1e-5 of its row's length of zero (sums of 512 products in fp32 are within 512 * 2^-24 = 3e-5 of the sum of
+    their sizes, 0.8 / sqrt(512) of that bound for a random sign pattern).  Rows with gaps, a slot outside the cache."""
+    from oracle import brute
+    from ucm_amd.sparse.decode_step import GSADecodeStepMLA
+
+    rng = rng_for(17 * B + Hq + R + T)
+    BS, nblk = 64, 12
+    NB = B * nblk + 2
+    f = lambda *shape: torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).to(dt).cuda()
+    wn, wr, keys, qs = f(512, 512), f(64, 64), f(T, 640), f(B, Hq, 640)
+    cache = torch.from_numpy(rng.integers(-2**31, 2**31 - 1, size=(NB, BS, 18), dtype=np.int64).astype(np.int32)).cuda()
+    before = cache.cpu().numpy().view(np.uint32).reshape(NB * BS, 18)
+    table = torch.from_numpy(rng.permutation(NB)[: B * nblk].astype(np.int32).reshape(B, nblk)).cuda()
+    lens = torch.full((B,), nblk * BS, dtype=torch.int32, device="cuda")
+    where = rng.permutation(NB * BS)[:T].astype(np.int64)
+    if T > 1:
+        where[T // 2] = -1 if slots_i64 else NB * BS
+    slots = torch.from_numpy(where if slots_i64 else where.astype(np.int32)).cuda()
+    st = GSADecodeStepMLA(wn, wr, Hq, R, B, nblk, 6 * BS, block_size=BS)
+    st.step(keys[:, :512], keys[:, 512:576], slots, qs[..., :512], qs[..., 512:576], cache, table, lens)
+    torch.cuda.synchronize()
+
+    def agree(got, rows, first, w):
+        x, W = rows.double().cpu().numpy(), w.double().cpu().numpy()
+        diff = np.unpackbits((got[:, first:first + W.shape[1] // 32] ^ brute.hash_encode(x, W)).view(np.uint8), axis=-1, bitorder="little")
+        assert not np.any(diff.astype(bool) & (brute.margins(x, W) >= 1e-5 * np.sqrt(x.shape[1])))
+
+    means = qs.float().view(B, R, Hq // R, 640).mean(1).to(dt).view(-1, 640)
+    codes = st.q_codes.cpu().numpy().view(np.uint32).reshape(-1, 18)
+    agree(codes, means[:, :512], 0, wn)
+    agree(codes, means[:, 512:576], 16, wr)
+    after = cache.cpu().numpy().view(np.uint32).reshape(NB * BS, 18)
+    ok = (where >= 0) & (where < NB * BS)
+    agree(after[where[ok]], keys[torch.from_numpy(ok)][:, :512], 0, wn)
+    agree(after[where[ok]], keys[torch.from_numpy(ok)][:, 512:576], 16, wr)
+    rest = np.ones(NB * BS, bool)
+    rest[where[ok]] = False
+    assert np.array_equal(after[rest], before[rest])
+
+
+@pytest.mark.parametrize("nblk", [257, 512, 700, 2049])
+@pytest.mark.parametrize("kind", ["ties", "spread", "outlier", "kept"])
+def test_selection_of_long_rows(nblk, kind):
+    """Rows of every number of scores a thread, whose scores are all equal, anywhere in the range, close together but
+    for one far below, and blocks that equal the query beside those that are always kept (fewer and more than k)."""
+    from ucm_amd.sparse import hamming_topk
+
+    rng = rng_for(nblk)
+    B, BS, Wd, G = 2, 64, 18, 64
+    q = np.broadcast_to(rng.integers(0, 2**32, (B, 1, Wd), dtype=np.uint32), (B, G, Wd)).copy()
+    blocks = np.broadcast_to(q[:1, :1], (nblk, BS, Wd)).copy()  # every token of a block is the same
+    flips = {"ties": np.full(nblk, 40), "spread": rng.integers(0, 577, nblk),
+             "outlier": np.where(np.arange(nblk) == 77, 576, rng.integers(200, 205, nblk)),
+             "kept": np.where(np.arange(nblk) % 5 == 2, 0, rng.integers(1, 300, nblk))}[kind]
+    for j in range(nblk):
+        bits = np.zeros(576, np.uint8)
+        bits[rng.permutation(576)[: flips[j]]] = 1
+        blocks[j] ^= np.packbits(bits, bitorder="little").view(np.uint32)
+    table = np.stack([rng.permutation(nblk), rng.permutation(nblk)]).astype(np.int32)
+    lens = np.array([nblk * BS, (nblk - 3) * BS - 5], np.int32)
+    t = lambda a: torch.from_numpy(a.view(np.int32)).cuda()
+    for k in (1, 4, nblk // 3):
+        gi, gs = hamming_topk(t(q), t(blocks).unsqueeze(2), t(table), t(lens), k, BS, 4 * BS, return_physical=True)
+        oi, osc = c_api.hamming_topk(q, blocks[:, :, None], table, lens, k, BS, 4 * BS, flags=c_api.F_PHYSICAL)
+        assert np.array_equal(gi.cpu().numpy(), oi) and np.array_equal(gs.cpu().numpy(), osc)
+
+
 @pytest.mark.parametrize("G", [4, 8])
 def test_separate_operators_under_graph_capture(G):
     """The operators a serving engine captures one by one (encode-and-cache, query hash, block

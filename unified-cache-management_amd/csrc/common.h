@@ -45,6 +45,24 @@ inline int launch_status(const char* kernel)
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+#ifdef __HIPCC__
+// Touches every 64-byte line of a kernel-argument struct at once.  The compiler fetches a field
+// where the code first needs it, behind the branches of the row addressing - a dozen scalar reads
+// one after the other in a kernel that lives for a few microseconds; with the lines already in the
+// scalar cache those reads are short.  (Copying the struct through pinned registers instead makes
+// its pointers lose their address space: every access becomes a flat one.)
+template <class T>
+__device__ __forceinline__ void warm_args(const T& args)
+{
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(&args);
+    uint32_t t = 0;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; i += 16) t |= src[i];
+    t |= src[sizeof(T) / 4 - 1];
+    asm volatile("" ::"s"(t));
+}
+#endif
+
 // hash_encode.hip: one (new keys -> paged cache, queries -> codes) pair of a decode step.
 // Strides of keys and queries in elements, of the cache and of q_codes in 32-bit words.
 struct PairSpec {

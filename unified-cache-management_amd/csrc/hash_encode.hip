@@ -594,22 +594,6 @@ constexpr int pipe_lds(int nt, int waves)
     return pipe_ring(waves) * pipe_stage_bytes(nt, waves) + 2 * pipe_slot_bytes(waves);
 }
 
-// Touches every 64-byte line of a kernel-argument struct at once.  The compiler fetches a field
-// where the code first needs it, behind the branches of the row addressing - a dozen scalar reads
-// one after the other in a kernel that lives for a few microseconds; with the lines already in the
-// scalar cache those reads are short.  (Copying the struct through pinned registers instead makes
-// its pointers lose their address space: every access becomes a flat one.)
-template <class T>
-__device__ __forceinline__ void warm_args(const T& args)
-{
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&args);
-    uint32_t t = 0;
-#pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 4; i += 16) t |= src[i];
-    t |= src[sizeof(T) / 4 - 1];
-    asm volatile("" ::"s"(t));
-}
-
 // Two loads of 16 bytes a lane, to 1 KiB of LDS each, one behind the other: bases in scalar registers, offsets in lanes.
 __device__ __forceinline__ void pipe_load(uint32_t lds, uint64_t b0, uint32_t o0, uint64_t b1, uint32_t o1)
 {
@@ -654,7 +638,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWa
     extern __shared__ __align__(16) uint16_t wt[];
     char* lds = reinterpret_cast<char*>(wt);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)wt);
-    warm_args(a);
+    ucm::warm_args(a);
     // The slices of a row tile are workgroups of one XCD (consecutive ones go to the eight XCDs in turn), so that
     // its rows come past that XCD's L2 once: streams in eights, each eight slice by slice, what fills the last eight having
     // nothing to do; or, where the number of streams is no multiple of eight, `run` neighbours among all heads'
@@ -1840,7 +1824,7 @@ __global__ __launch_bounds__(64 * kRunWaves) __attribute__((amdgpu_waves_per_eu(
     typedef __attribute__((address_space(3))) const V* row_ptr;
     typedef uint32_t Code __attribute__((ext_vector_type(NT)));
     extern __shared__ __align__(16) uint16_t wt[];
-    warm_args(a);
+    ucm::warm_args(a);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)wt);
     const uint32_t wlds = lds0 + kRunWaves * kRunSlots * kTile;
     const int lane = threadIdx.x & 63;
@@ -2286,7 +2270,7 @@ constexpr int small_split(int KS) { return KS >= 16 ? 4 : 1; }
 template <typename V, int KS, bool kByRow = false>
 __global__ __launch_bounds__(64 * small_split(KS)) __attribute__((amdgpu_waves_per_eu(small_split(KS) > 1 ? 3 : 1, 8))) void encode_small_kernel(EncJobs js)
 {
-    warm_args(js);
+    ucm::warm_args(js);
     __shared__ __align__(16) uint16_t lds[small_lds(KS, small_split(KS))];
     const bool second = (int)blockIdx.x >= js.waves0;
     encode_small_body<V, KS, small_split(KS), kByRow>(second ? js.job[1] : js.job[0],
@@ -2306,7 +2290,7 @@ __global__ __launch_bounds__(64 * small_split(KSA)) __attribute__((amdgpu_waves_
     static_assert(small_split(KSB) == 1, "the narrow jobs' tiles take one wave of the workgroup");
     static_assert(small_lds(KSB, 1) <= small_lds(KSA, small_split(KSA)), "one area for both");
     __shared__ __align__(16) uint16_t lds[small_lds(KSA, small_split(KSA))];
-    warm_args(js);
+    ucm::warm_args(js);
     const int w = blockIdx.x;
     if (w < js.end[1]) {
         const int j = w >= js.end[0] ? 1 : 0;
@@ -2315,6 +2299,224 @@ __global__ __launch_bounds__(64 * small_split(KSA)) __attribute__((amdgpu_waves_
         if (threadIdx.x >= 64) return;  // a narrow tile is one wave's work
         const int j = w >= js.end[2] ? 3 : 2;
         encode_small_body<V, KSB>(js.job[j], w - js.end[j - 1], lds);
+    }
+}
+
+// The encodes of a latent-attention step, rows of 512 and of 64 values, as the plugin has them: one projection, mean of no
+// or two rows, powers of two for the heads, the columns and the cache's block.  encode_small_mixed_kernel, which takes every
+// form of them, is a chain of arguments, a prologue of branches, rows, columns of W behind them, LDS and partial sums, and
+// reads a row tile's rows again for every 32 columns (96 KiB a workgroup).  Here W and the rows are asked for together, a
+// workgroup takes 64 columns of a row tile (the same 64 KiB of rows), each of its eight waves a quarter of the row's values
+// and half of the columns, and what the prologue need not decide is not in the code.  The sums are taken in the
+// same order as there, so that a key has the same code from either.
+// Launches of a step, the other kernel and this one: 2 requests x 64 means of two rows (128 query rows) 6.2 and 5.7 us, 16 x 64
+// 8.6 and 8.0; whole steps of 1 to 32 requests and 8 to 128 query rows each 1 to 7 % shorter.  What is left of it, at 2,400 cycles
+// to the microsecond: 2,000 cycles for arguments and 128 KiB through a compute unit's L1 at 64 bytes a cycle, 1,500 for
+// the means (9 instructions for two values), 2,400 for turning W through LDS and the products, 1,700 for the partial sums.
+struct LatentJob {
+    const void* x;
+    const void* w;
+    const void* slot;  // null: row t is slot t
+    uint32_t* cache;
+    int64_t xs_t, xs_h, xs_g;  // element strides of the input; xs_g between the two rows of a mean
+    int64_t slots, cs_block, cs_token, cs_head;
+    int rows, h_shift, mean, slot_is_i64, bs_shift;
+    int first;  // first tile (of 32 rows x 64 or 32 columns) of the job
+};
+
+struct LatentJobs {
+    LatentJob job[4];         // keys and queries of 512 values, keys and queries of 64
+    int wide, narrow;         // tiles of either width
+    int wide_shift, nt_shift;  // log2 of the tiles that a row tile's columns make
+};
+
+constexpr int kLatentWaves = 8;
+constexpr int kLatentPitch = 128 + kPad;    // values of an LDS row of the wide tiles
+constexpr int kLatentPart = 20;             // floats of a lane's partial sums in LDS: 16 and padding against bank conflicts
+static_assert(64 * kLatentPart * 4 <= 32 * kLatentPitch * 2, "a wave's columns make room for its sums");
+static_assert(32 * (64 + kPad) <= 32 * kLatentPitch, "a narrow tile fits a wave's area");
+
+// Row p of a job, the last one for a place behind it.
+__device__ __forceinline__ void latent_row(const LatentJob& a, int p, int& t, int& h)
+{
+    p = p < a.rows ? p : a.rows - 1;
+    t = p >> a.h_shift;
+    h = p & ((1 << a.h_shift) - 1);
+}
+
+// Where the code words of row (t, h) go, or null; the raw words were read with latent_slot.
+__device__ __forceinline__ RawSlot latent_slot(const LatentJob& a, int t)
+{
+    const char* q = a.slot ? (const char*)a.slot + ((int64_t)t << (a.slot_is_i64 ? 3 : 2)) : (const char*)a.x;
+    RawSlot s;
+    s.lo = *(const uint32_t*)q;
+    s.hi = *(const uint32_t*)(q + (a.slot && a.slot_is_i64 ? 4 : 0));
+    return s;
+}
+
+__device__ __forceinline__ uint32_t* latent_dst(const LatentJob& a, RawSlot raw, int t, int h)
+{
+    int64_t s = t;
+    if (a.slot) s = a.slot_is_i64 ? (int64_t)(((uint64_t)raw.hi << 32) | raw.lo) : (int64_t)(int32_t)raw.lo;
+    if (s < 0 || s >= a.slots) return nullptr;
+    return a.cache + (s >> a.bs_shift) * a.cs_block + (s & ((1 << a.bs_shift) - 1)) * a.cs_token + h * a.cs_head;
+}
+
+// Four loads of whole row pieces of 16 bytes a lane, kLanes of them to a row, from row p0 on; the second one of a mean too.
+template <typename V, int G, int kLanes>
+__device__ __forceinline__ void latent_load(const LatentJob& a, int p0, int k0, V (&v)[4][G])
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        int t, h;
+        latent_row(a, p0 + i * (64 / kLanes) + lane / kLanes, t, h);
+        const uint16_t* src = (const uint16_t*)a.x + (t * a.xs_t + h * a.xs_h + k0 + lane % kLanes * 8);
+#pragma unroll
+        for (int g = 0; g < G; ++g) v[i][g] = *reinterpret_cast<const V*>(src + g * a.xs_g);
+    }
+}
+
+// fp32 sum of the rows in order, times a half, rounded to the input type.
+template <typename V, int G>
+__device__ __forceinline__ V latent_mean(const LatentJob& a, const V (&v)[G])
+{
+    if (G == 1 || !a.mean) return v[0];
+    V m;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m[i] = (typename Mfma<V>::elem)(((float)v[0][i] + (float)v[G - 1][i]) * 0.5f);
+    return m;
+}
+
+// Patch (kq, j) of W, 8 values of k by 8 columns, in operand layout: column 8 j + c of the tile at row 8 j + c of LDS.
+template <int kPitch>
+__device__ __forceinline__ void latent_turn(const u32x4 (&row)[8], uint16_t* wt, int kq, int j)
+{
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
+        u32x4 o;
+        o.x = __builtin_amdgcn_perm(row[1][c >> 1], row[0][c >> 1], sel);
+        o.y = __builtin_amdgcn_perm(row[3][c >> 1], row[2][c >> 1], sel);
+        o.z = __builtin_amdgcn_perm(row[5][c >> 1], row[4][c >> 1], sel);
+        o.w = __builtin_amdgcn_perm(row[7][c >> 1], row[6][c >> 1], sel);
+        *reinterpret_cast<u32x4*>(wt + (8 * j + c) * kPitch + kq * 8) = o;
+    }
+}
+
+template <typename V, int G>
+__global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_eu(4, 8))) void encode_latent_kernel(LatentJobs js)
+{
+    __shared__ __align__(16) uint16_t lds[kLatentWaves * 32 * kLatentPitch];
+    ucm::warm_args(js);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, kb = lane >> 5;
+    uint16_t* const wt = lds + wave * 32 * kLatentPitch;
+    if ((int)blockIdx.x >= js.wide) {  // a narrow tile is one wave's work
+        const int tile = ((int)blockIdx.x - js.wide) * kLatentWaves + wave;
+        if (tile >= js.narrow) return;
+        const LatentJob& a = js.job[tile >= js.job[3].first ? 3 : 2];
+        const int wv = tile - a.first, nt = wv & ((1 << js.nt_shift) - 1), p0 = (wv >> js.nt_shift) * 32;
+        const int N = 32 << js.nt_shift;
+        constexpr int kPitch = 64 + kPad;
+        u32x4 row[8];
+        const int kq = (lane & 31) >> 2, j = lane & 3;  // the upper lanes repeat the lower ones' patches
+        const uint16_t* src = (const uint16_t*)a.w + (int64_t)kq * 8 * N + nt * 32 + 8 * j;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) row[i] = *reinterpret_cast<const u32x4*>(src + i * N);
+        V v[4][G];
+        latent_load<V, G, 8>(a, p0, 0, v);
+        int t, h;
+        latent_row(a, p0 + r, t, h);
+        const RawSlot raw = latent_slot(a, t);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<V*>(wt + (i * 8 + lane / 8) * kPitch + lane % 8 * 8) = latent_mean<V, G>(a, v[i]);
+        __builtin_amdgcn_wave_barrier();
+        V av[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) av[ks] = *reinterpret_cast<const V*>(wt + r * kPitch + ks * 16 + kb * 8);
+        __builtin_amdgcn_wave_barrier();
+        latent_turn<kPitch>(row, wt, kq, j);
+        __builtin_amdgcn_wave_barrier();
+        f32x16 acc = acc_start();
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+            acc = Mfma<V>::run(*reinterpret_cast<const V*>(wt + r * kPitch + ks * 16 + kb * 8), av[ks], acc);
+        const uint32_t half = pack_half(acc);
+        const uint32_t word = join_halves(kb ? half << 4 : half);
+        if (lane < 32 && p0 + r < a.rows) {
+            uint32_t* dst = latent_dst(a, raw, t, h);
+            if (dst) dst[nt] = word;
+        }
+        return;
+    }
+    const LatentJob& a = js.job[(int)blockIdx.x >= js.job[1].first ? 1 : 0];
+    int wv = (int)blockIdx.x - a.first, nt;
+    // eight row tiles at a time go out row tile first, so that a row tile's workgroups are on one XCD and its rows come
+    // past that XCD's L2 once (consecutive workgroups go to the eight XCDs in turn)
+    if ((wv >> (js.wide_shift + 3)) < (((a.rows + 31) >> 5) >> 3)) {
+        nt = (wv >> 3) & ((1 << js.wide_shift) - 1);
+        wv = (wv >> (js.wide_shift + 3)) * 8 + (wv & 7);
+    } else {
+        nt = wv & ((1 << js.wide_shift) - 1);
+        wv >>= js.wide_shift;
+    }
+    const int p0 = wv * 32, N = 64 << js.wide_shift;
+    const int slice = wave >> 1, ct = wave & 1;
+    u32x4 row[8];
+    const int kq = lane >> 2, j = lane & 3;
+    const uint16_t* src = (const uint16_t*)a.w + (int64_t)(slice * 128 + kq * 8) * N + nt * 64 + ct * 32 + 8 * j;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) row[i] = *reinterpret_cast<const u32x4*>(src + i * N);
+    V v[4][G];
+    latent_load<V, G, 16>(a, p0 + ct * 16, slice * 128, v);
+    int t, h;
+    latent_row(a, p0 + r, t, h);
+    const RawSlot raw = latent_slot(a, t);
+    // the two waves of a slice share its rows, sixteen in the area of each
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<V*>(wt + (i * 4 + lane / 16) * kLatentPitch + lane % 16 * 8) = latent_mean<V, G>(a, v[i]);
+    __syncthreads();
+    V av[8];
+    {
+        const uint16_t* rows = lds + (slice * 2 + (r >> 4)) * 32 * kLatentPitch + (r & 15) * kLatentPitch + kb * 8;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) av[ks] = *reinterpret_cast<const V*>(rows + ks * 16);
+    }
+    __syncthreads();
+    latent_turn<kLatentPitch>(row, wt, kq, j);
+    __builtin_amdgcn_wave_barrier();
+    f32x16 acc = acc_start();
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+        acc = Mfma<V>::run(*reinterpret_cast<const V*>(wt + r * kLatentPitch + ks * 16 + kb * 8), av[ks], acc);
+    __builtin_amdgcn_wave_barrier();
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    float* const part = reinterpret_cast<float*>(lds);
+    constexpr int kArea = 32 * kLatentPitch / 2;  // floats of a wave's area
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(part + wave * kArea + lane * kLatentPart + 4 * i) = f32x4{acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]};
+    __syncthreads();
+    // The slices' sums meet in slice order, four accumulators to a wave: eight columns of its half, a byte of the rows'
+    // words.  Every slice starts from the same small negative number, which vanishes in any sum that is not exactly zero
+    // and keeps a row of zeros negative; a row with a NaN has NaN in every accumulator, so the first one tells.
+    f32x4 sum = *reinterpret_cast<const f32x4*>(part + ct * kArea + lane * kLatentPart + 4 * slice);
+    float first = part[ct * kArea + lane * kLatentPart];
+#pragma unroll
+    for (int sl = 1; sl < 4; ++sl) {
+        const float* p = part + (sl * 2 + ct) * kArea + lane * kLatentPart;
+        sum += *reinterpret_cast<const f32x4*>(p + 4 * slice);
+        first += p[0];
+    }
+    uint32_t bits = 0;
+#pragma unroll
+    for (int i = 3; i >= 0; --i) bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(sum[i]), 31);
+    bits = first != first ? 0u : (bits ^ 15u);
+    bits = join_halves(kb ? bits << 4 : bits);
+    if (lane < 32 && p0 + r < a.rows) {
+        uint32_t* dst = latent_dst(a, raw, t, h);
+        if (dst) reinterpret_cast<uint8_t*>(dst + nt * 2 + ct)[slice] = (uint8_t)bits;
     }
 }
 
@@ -2358,7 +2560,7 @@ __global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(3,
     __shared__ int2 hits[kStepTokens];  // a new key in this block and its token there
     __shared__ int nhits;
     __shared__ int low[kStepThreads / 64];
-    warm_args(js);
+    ucm::warm_args(js);
     const int lane = threadIdx.x & 63, tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const EncArgs& kk = js.kk;
@@ -3617,9 +3819,50 @@ bool pair_is_small(const PairSpec& p, const EncArgs& kk, const EncArgs& kq, bool
            small_eligible(kq, p.x_dtype, p.w_dtype, false);
 }
 
+// A job of encode_latent_kernel, or false where it has a form that the kernel does not take.
+bool latent_job(const EncArgs& a, LatentJob& j)
+{
+    const bool rows = a.T * a.H <= INT32_MAX && a.h_shift >= 0 && a.n_w == 1 && !a.src_blocks && a.bs_shift >= 0;
+    const bool mean = a.gmean == 2;
+    if (!rows || (a.gmean > 1 && !mean) || a.x_stride_g % 8 != 0) return false;
+    j.x = a.x; j.w = a.w; j.slot = a.slot; j.cache = a.cache;
+    j.xs_t = a.x_stride_t; j.xs_h = a.x_stride_h; j.xs_g = mean ? a.x_stride_g : 0;
+    j.slots = a.NB * (int64_t)a.BS; j.cs_block = a.cs_block; j.cs_token = a.cs_token; j.cs_head = a.cs_head;
+    j.rows = (int)(a.T * a.H); j.h_shift = a.h_shift; j.mean = mean; j.slot_is_i64 = a.slot_is_i64; j.bs_shift = a.bs_shift;
+    return j.rows > 0;
+}
+
+// The four jobs of a latent-attention step for encode_latent_kernel, or false.
+bool latent_jobs(const EncJobs4& js, LatentJobs& out)
+{
+    for (int i = 0; i < 4; ++i)
+        if (!latent_job(js.job[i], out.job[i])) return false;
+    const EncArgs &wide = js.job[0], &narrow = js.job[2];
+    if (wide.nt_shift < 1 || narrow.nt_shift < 0) return false;
+    out.wide_shift = wide.nt_shift - 1;
+    out.nt_shift = narrow.nt_shift;
+    auto row_tiles = [&](int i) { return ucm::ceil_div(out.job[i].rows, kRowsPerWave); };
+    const int64_t w0 = row_tiles(0) << out.wide_shift, n0 = row_tiles(2) << out.nt_shift;
+    const int64_t w = w0 + (row_tiles(1) << out.wide_shift), n = n0 + (row_tiles(3) << out.nt_shift);
+    if (w + n > INT32_MAX) return false;
+    out.job[1].first = (int)w0;
+    out.job[3].first = (int)n0;
+    out.wide = (int)w;
+    out.narrow = (int)n;
+    return true;
+}
+
 template <typename V>
 int launch_small_mixed(const EncJobs4& js, hipStream_t st)
 {
+    LatentJobs lean{};
+    if (latent_jobs(js, lean)) {
+        const dim3 grid((unsigned)(lean.wide + ucm::ceil_div(lean.narrow, kLatentWaves))), threads(64 * kLatentWaves);
+        const bool mean = lean.job[1].mean || lean.job[3].mean || lean.job[0].mean || lean.job[2].mean;
+        if (mean) hipLaunchKernelGGL((encode_latent_kernel<V, 2>), grid, threads, 0, st, lean);
+        else hipLaunchKernelGGL((encode_latent_kernel<V, 1>), grid, threads, 0, st, lean);
+        return ucm::launch_status("encode_latent_kernel");
+    }
     const dim3 grid((unsigned)js.end[3]), threads(64 * small_split(32));
     if (rows_by_line(js.job[0], js.job[1])) hipLaunchKernelGGL((encode_small_mixed_kernel<V, 32, 4, true>), grid, threads, 0, st, js);
     else hipLaunchKernelGGL((encode_small_mixed_kernel<V, 32, 4, false>), grid, threads, 0, st, js);
