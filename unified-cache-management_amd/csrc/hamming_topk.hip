@@ -2211,6 +2211,7 @@ struct SelectArgs {
     int table_stride, max_blocks;
     const int32_t* lens;
     int BS, Hkv, Ho, k, full, key_bits;
+    int bs_shift;        // log2(BS), -1 where BS is no power of two
     uint32_t flags;
     int32_t* out_idx;    // [B][Ho][k]
     int32_t* out_score;  // may be null
@@ -2224,6 +2225,11 @@ struct SelectArgs {
     int thr_len, topk_tok;
 };
 
+__device__ __forceinline__ int blocks_of(const SelectArgs& a, int tokens)
+{
+    return a.bs_shift >= 0 ? (tokens + a.BS - 1) >> a.bs_shift : (tokens + a.BS - 1) / a.BS;
+}
+
 // The first part of that epilogue, shared by the selection kernels: `tid` of `nthreads` threads
 // own a row.  Returns true when the row is complete (short request or no blocks) and the
 // selection can be skipped; otherwise entries [kk, max_blocks) are zeroed and the caller
@@ -2236,7 +2242,7 @@ __device__ __forceinline__ bool plugin_row_prologue(const SelectArgs& a, int b, 
     if (tid == 0) {
         int over = len - a.topk_tok;
         over = over < 0 ? 0 : over;
-        a.new_lens[b] = keep ? len : len - ((over + a.BS - 1) / a.BS) * a.BS;
+        a.new_lens[b] = keep ? len : len - blocks_of(a, over) * a.BS;
     }
     if (keep) {
         const int32_t* src = a.table + (int64_t)b * a.table_stride;
@@ -2447,13 +2453,6 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SelectArgs a)
 // value with ballot counts finds the k-th largest score, two wave prefix sums place the winners
 // in ascending index order, ties to the lower index.  Same results as select_kernel.
 // ---------------------------------------------------------------------------------------
-__device__ __forceinline__ int wave_excl_scan(int v, int* total)
-{
-    const int inc = wave_incl_scan(v);
-    *total = __builtin_amdgcn_readlane(inc, kWave - 1);
-    return inc - v;
-}
-
 template <int EL>
 __global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int rows_total)
 {
@@ -2461,14 +2460,14 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int
     // kernel's arguments would be fetched in two rounds, the row count first)
     const int rowid_raw = blockIdx.x * (kThreads / kWave) + wave_id();
     const int rowid = rowid_raw < rows_total ? rowid_raw : rows_total - 1;
-    const int b = rowid / a.Ho, ho = rowid % a.Ho;
+    const int b = a.Ho == 1 ? rowid : rowid / a.Ho, ho = rowid - b * a.Ho;
     const int lane = lane_id();
     const int len = a.lens[b];
     // the row's scores go out before the length is known (in-range positions only, masked
     // below): one round trip to memory instead of two
     int raw[EL];
+    const bool red = (a.flags & UCM_TOPK_REDUCE_HEADS) && a.Hkv > 1;
     {
-        const bool red = (a.flags & UCM_TOPK_REDUCE_HEADS) && a.Hkv > 1;
         const int32_t* r0 = a.scores + (int64_t)b * a.Hkv * a.max_blocks + (int64_t)(red ? 0 : ho) * a.sc_h;
 #pragma unroll
         for (int e = 0; e < EL; ++e) {
@@ -2492,7 +2491,7 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int
         for (int e = 0; e < EL; ++e) tab[e] = physical ? b * a.max_blocks + lane * EL + e : lane * EL + e;
     }
     if (rowid_raw >= rows_total) return;
-    int n = len > 0 ? (len + a.BS - 1) / a.BS : 0;
+    int n = len > 0 ? blocks_of(a, len) : 0;
     if (n > a.max_blocks) n = a.max_blocks;
     int32_t* oi = a.out_idx + ((int64_t)b * a.Ho + ho) * a.k;
     int32_t* os = a.out_score ? a.out_score + ((int64_t)b * a.Ho + ho) * a.k : nullptr;
@@ -2508,12 +2507,11 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int
         }
         if (n == 0) return;
     }
-    const bool reduce = (a.flags & UCM_TOPK_REDUCE_HEADS) && a.Hkv > 1;
-    const int32_t* row = a.scores + (int64_t)b * a.Hkv * a.max_blocks + (int64_t)(reduce ? 0 : ho) * a.sc_h;
+    const int32_t* row = a.scores + (int64_t)b * a.Hkv * a.max_blocks + (int64_t)(red ? 0 : ho) * a.sc_h;
     int v[EL];
 #pragma unroll
     for (int e = 0; e < EL; ++e) v[e] = raw[e];
-    if (reduce) {
+    if (red) {
         // maximum over the KV heads, CH heads at a time with all of their loads in flight
         // (heads past the last re-read head 0, which changes nothing)
         constexpr int CH = EL <= 4 ? 8 : 2;
@@ -2553,32 +2551,30 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int
     }
     lo = __builtin_amdgcn_readlane(wave_min_lane63(lo), 63);
     hi = __builtin_amdgcn_readlane(wave_max_lane63(hi), 63);
+    int above = 0;  // scores above hi, fewer than kk
     while (lo < hi) {
         const int mid = lo + ((hi - lo + 1) >> 1);
-        if (count_ge(mid) >= kk) lo = mid;
-        else hi = mid - 1;
+        const int c = count_ge(mid);
+        if (c >= kk) {
+            lo = mid;
+        } else {
+            hi = mid - 1;
+            above = c;
+        }
     }
     const int thr = lo;
-    const int need = kk - count_ge(thr + 1);  // ties at thr to take, lowest indices first
-    int eq = 0, gt = 0;
+    const int need = kk - above;  // ties at thr to take, lowest indices first
+    // one prefix sum for both: scores equal to thr in the upper half, greater ones in the lower (a row has 1024 at most)
+    int both = 0;
 #pragma unroll
-    for (int e = 0; e < EL; ++e) {
-        eq += (v[e] == thr);
-        gt += (v[e] > thr);
-    }
-    int tot;
-    const int eq_before = wave_excl_scan(eq, &tot);
-    int eq_take = need - eq_before;
-    eq_take = eq_take < 0 ? 0 : (eq_take > eq ? eq : eq_take);
-    int pos = wave_excl_scan(gt + eq_take, &tot);
-    int eq_seen = 0;
+    for (int e = 0; e < EL; ++e) both += (v[e] == thr ? 1 << 16 : 0) + (v[e] > thr);
+    const int before = wave_incl_scan(both) - both;
+    int eq_seen = before >> 16;  // equal scores of lower positions: the first `need` of them are taken
+    int pos = (before & 0xffff) + (eq_seen < need ? eq_seen : need);
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
         bool take = v[e] > thr;
-        if (v[e] == thr) {
-            take = eq_seen < eq_take;
-            ++eq_seen;
-        }
+        if (v[e] == thr) take = eq_seen++ < need;
         if (take && pos < a.k) {
             oi[pos] = tab[e];
             if (os) os[pos] = (a.flags & UCM_TOPK_DISTANCE) ? a.full - v[e] : v[e];
@@ -2590,17 +2586,24 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int
 // Rows of 257 to 4096 block scores, index-ordered output: one workgroup per row, EL = 2 to 16
 // scores per thread.  Same algorithm as select_wave_kernel<16>, but a wave there runs some 2000
 // instructions back to back for its row (7 us, however few rows there are); here each wave has
-// a quarter of the row and the four partial counts of a search step meet in LDS (two buffers
-// in turn, one barrier per step).
+// a quarter of the row and the search counts in LDS: kBins bins of the row's range, so that nearly every row's threshold
+// is found in two steps of a barrier, some 450 cycles each (halving the range took a step of 450 cycles for every bit of it, with
+// seven thresholds a step 1,130 for every three).  The launch: 2 rows of 313 scores 4.6 and 2.7 us, 16 of 1,024 5.4 and 3.9, 64 of 1,024
+// in a range of 52 4.0 and 3.8.  What is left is the chain of arguments, scores, extremes, threshold, places and stores.
 template <int EL>
 __global__ __launch_bounds__(kThreads) void select_group_kernel(SelectArgs a)
 {
     constexpr int kWaves = kThreads / kWave;
-    __shared__ int cnt[2][kWaves];
-    __shared__ int ext[2][kWaves];
+    constexpr int kBins = 512;
+    __shared__ __align__(16) int hist[2][kBins];
+    __shared__ int ext[3][kWaves];
     __shared__ int wsum[kWaves];
-    const int b = blockIdx.x / a.Ho, ho = blockIdx.x % a.Ho;
+    ucm::warm_args(a);
+    // (divisions stand in front of the first load, or between the loads and the search: forty instructions each)
+    const int b = a.Ho == 1 ? blockIdx.x : blockIdx.x / a.Ho, ho = blockIdx.x - b * a.Ho;
     const int tid = threadIdx.x, lane = lane_id(), wid = wave_id();
+    hist[0][tid] = hist[0][tid + kThreads] = 0;
+    hist[1][tid] = hist[1][tid + kThreads] = 0;
     const bool reduce = (a.flags & UCM_TOPK_REDUCE_HEADS) && a.Hkv > 1;
     const int32_t* row = a.scores + ((int64_t)b * a.Hkv + (reduce ? 0 : ho)) * a.max_blocks;
     const int len = a.lens[b];  // asked for with the scores: one round trip to memory
@@ -2622,7 +2625,7 @@ __global__ __launch_bounds__(kThreads) void select_group_kernel(SelectArgs a)
 #pragma unroll
         for (int e = 0; e < EL; ++e) tab[e] = physical ? b * a.max_blocks + tid * EL + e : tid * EL + e;
     }
-    int n = len > 0 ? (len + a.BS - 1) / a.BS : 0;
+    int n = len > 0 ? blocks_of(a, len) : 0;
     if (n > a.max_blocks) n = a.max_blocks;
     int32_t* oi = a.out_idx + ((int64_t)b * a.Ho + ho) * a.k;
     int32_t* os = a.out_score ? a.out_score + ((int64_t)b * a.Ho + ho) * a.k : nullptr;
@@ -2656,65 +2659,93 @@ __global__ __launch_bounds__(kThreads) void select_group_kernel(SelectArgs a)
                 for (int e = 0; e < EL; ++e) v[e] = o[u][e] > v[e] ? o[u][e] : v[e];
         }
     }
-    int lo = 0x7fffffff, hi = -0x7fffffff;
+    int lo = 0x7fffffff, hi = -0x7fffffff, n_full = 0;
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
         if (tid * EL + e >= n) v[e] = -0x7fffffff;  // below every real score (>= -1): never selected
         else lo = v[e] < lo ? v[e] : lo;
-        hi = v[e] > hi ? v[e] : hi;
+        const bool top = v[e] == a.full;
+        n_full += __popcll(__ballot(top));
+        if (!top) hi = v[e] > hi ? v[e] : hi;
     }
     lo = wave_min_lane63(lo);
     hi = wave_max_lane63(hi);
     if (lane == kWave - 1) {
         ext[0][wid] = lo;
         ext[1][wid] = hi;
+        ext[2][wid] = n_full;
     }
     __syncthreads();
+    n_full = 0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
         lo = ext[0][w] < lo ? ext[0][w] : lo;
         hi = ext[1][w] > hi ? ext[1][w] : hi;
+        n_full += ext[2][w];
     }
     lo = __builtin_amdgcn_readfirstlane(lo);
     hi = __builtin_amdgcn_readfirstlane(hi);
-    // count of scores >= t over the whole row; `step` alternates the LDS buffer
-    int step = 0;
-    auto count_ge = [&](int t) {
-        int c = 0;
+    // The blocks that are always kept have the largest possible score and stand far above the others: they are
+    // counted apart, so that the bins divide the range of the others.
+    n_full = __builtin_amdgcn_readfirstlane(n_full);
+    int above = n_full;
+    if (n_full >= kk) {
+        lo = hi = a.full;
+        above = 0;
+    }
+    // kBins bins over [lo, hi], counted in LDS: nine bits of the threshold a step.  count(>= lo) >= kk holds always,
+    // above = count(> hi) < kk.
+    for (int step = 0; lo < hi; ++step) {
+        int* const h = hist[step & 1];
+        if (step > 1) {  // every wave has read the step before last
+            h[tid] = h[tid + kThreads] = 0;
+            __syncthreads();
+        }
+        const int shift = 23 - __builtin_clz((uint32_t)(hi - lo) | (kBins - 1));
 #pragma unroll
-        for (int e = 0; e < EL; ++e) c += __popcll(__ballot(v[e] >= t));
-        int* buf = cnt[step & 1];
-        ++step;
-        if (lane == 0) buf[wid] = c;
+        for (int e = 0; e < EL; ++e)
+            if (v[e] >= lo && v[e] <= hi) atomicAdd(&h[(uint32_t)(v[e] - lo) >> shift], 1);
         __syncthreads();
-        return buf[0] + buf[1] + buf[2] + buf[3];
-    };
-    while (lo < hi) {  // count_ge(lo) >= kk always holds
-        const int mid = lo + ((hi - lo + 1) >> 1);
-        if (count_ge(mid) >= kk) lo = mid;
-        else hi = mid - 1;
+        // a lane has eight bins: the counts above them, and with them from the top
+        const int4 c0 = *reinterpret_cast<const int4*>(&h[8 * lane]), c1 = *reinterpret_cast<const int4*>(&h[8 * lane + 4]);
+        const int bin[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        int mine = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) mine += bin[i];
+        const int inc = wave_incl_scan(mine);
+        int from = above + __builtin_amdgcn_readlane(inc, kWave - 1) - inc, up = 0, over = from;
+        const bool below = from < kk;
+#pragma unroll
+        for (int i = 7; i >= 0; --i) {
+            if (from < kk) {
+                up = i;
+                over = from;
+            }
+            from += bin[i];
+        }
+        const int owner = __builtin_ctzll(__ballot(below && from >= kk));  // one lane's: the counts only grow downwards
+        above = __builtin_amdgcn_readlane(over, owner);
+        lo = (int)((uint32_t)lo + ((uint32_t)(8 * owner + __builtin_amdgcn_readlane(up, owner)) << shift));
+        const uint32_t width = (1u << shift) - 1;
+        if ((uint32_t)(hi - lo) > width) hi = lo + (int)width;
     }
     const int thr = lo;
-    const int need = kk - count_ge(thr + 1);  // ties at thr to take, lowest indices first
-    int eq = 0, gt = 0;
+    const int need = kk - above;  // ties at thr to take, lowest indices first
+    // one prefix sum for both: scores equal to thr in the upper half, greater ones in the lower (a row has 4096 at most)
+    int both = 0;
 #pragma unroll
-    for (int e = 0; e < EL; ++e) {
-        eq += (v[e] == thr);
-        gt += (v[e] > thr);
-    }
-    int tot;
-    const int eq_before = block_exclusive_scan(eq, wsum, &tot);
-    int eq_take = need - eq_before;
-    eq_take = eq_take < 0 ? 0 : (eq_take > eq ? eq : eq_take);
-    int pos = block_exclusive_scan(gt + eq_take, wsum, &tot);
-    int eq_seen = 0;
+    for (int e = 0; e < EL; ++e) both += (v[e] == thr ? 1 << 16 : 0) + (v[e] > thr);
+    const int inc = wave_incl_scan(both);
+    if (lane == kWave - 1) wsum[wid] = inc;
+    __syncthreads();
+    int before = inc - both;
+    for (int w = 0; w < wid; ++w) before += wsum[w];
+    int eq_seen = before >> 16;  // equal scores of lower positions: the first `need` of them are taken
+    int pos = (before & 0xffff) + (eq_seen < need ? eq_seen : need);
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
         bool take = v[e] > thr;
-        if (v[e] == thr) {
-            take = eq_seen < eq_take;
-            ++eq_seen;
-        }
+        if (v[e] == thr) take = eq_seen++ < need;
         if (take && pos < a.k) {
             oi[pos] = tab[e];
             if (os) os[pos] = (a.flags & UCM_TOPK_DISTANCE) ? a.full - v[e] : v[e];
@@ -3384,6 +3415,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
     s.table_stride = table_stride; s.max_blocks = max_blocks; s.lens = seq_lens; s.BS = BS;
     s.Hkv = reduced_scores ? 1 : Hkv; s.Ho = (flags & UCM_TOPK_REDUCE_HEADS) ? 1 : Hkv; s.k = k;
     s.full = a.G * 32 * Wd;
+    s.bs_shift = (BS & (BS - 1)) == 0 ? __builtin_ctz((unsigned)BS) : -1;
     s.key_bits = 1;
     while ((1ll << s.key_bits) <= (int64_t)s.full + 1) ++s.key_bits;
     s.flags = flags; s.out_idx = out_idx; s.out_score = out_score;
