@@ -59,6 +59,14 @@ struct ScoreArgs {
     unsigned long long* clock_probe;  // strip scorers: see ucm_hamming_topk_set_clock_probe(); else null
 };
 
+// What the strip scorers' first loads take, as arguments in front of the struct: the build has the hardware put a kernel's
+// leading scalar arguments into registers before its waves start, where the fields of a struct are read from memory
+// by every wave, 0.4 to 0.5 us before its first load.  (Fourteen registers in all, 8-byte arguments first.)
+#define STRIP_EARLY                                                                                                   \
+    const int32_t *lens, const int32_t *table, const uint32_t *q, int64_t q_stride_b, int64_t q_stride_h, int table_stride, \
+        int max_blocks, int TB, int G
+#define STRIP_EARLY_OF(a) (a).lens, (a).table, (a).q, (a).q_stride_b, (a).q_stride_h, (a).table_stride, (a).max_blocks, (a).TB, (a).G
+
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
@@ -2064,8 +2072,10 @@ __device__ __forceinline__ void strip_body(const ScoreArgs& a, int max_seq_len, 
 }
 
 template <int WD>
-__global__ __launch_bounds__(kStripWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void block_score_strip(ScoreArgs a)
+__global__ __launch_bounds__(kStripWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void block_score_strip(STRIP_EARLY, ScoreArgs a)
 {
+    a.lens = lens; a.table = table; a.q = q; a.q_stride_b = q_stride_b; a.q_stride_h = q_stride_h;
+    a.table_stride = table_stride; a.max_blocks = max_blocks; a.TB = TB; a.G = G;
     strip_body<WD, 0>(a, 0, nullptr);
 }
 
@@ -2224,6 +2234,15 @@ struct SelectArgs {
     int32_t* new_lens;
     int thr_len, topk_tok;
 };
+
+// What the selection kernels' first loads take, as arguments of their own: the build has the hardware put a kernel's
+// leading scalar arguments into registers before its waves start, where a struct's fields are read from memory by
+// every wave (2 rows of 313 scores 2.5 and 2.3 us, and 0.5 us of a step of 32 x 32,768 tokens).
+#define SELECT_EARLY                                                                                              \
+    const int32_t *scores, const int32_t *lens, const int32_t *table, int table_stride, int max_blocks, int Ho,      \
+        int Hkv, uint32_t flags, int sc_h, int sc_j
+#define SELECT_EARLY_OF(s) \
+    (s).scores, (s).lens, (s).table, (s).table_stride, (s).max_blocks, (s).Ho, (s).Hkv, (s).flags, (s).sc_h, (s).sc_j
 
 __device__ __forceinline__ int blocks_of(const SelectArgs& a, int tokens)
 {
@@ -2454,41 +2473,41 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SelectArgs a)
 // in ascending index order, ties to the lower index.  Same results as select_kernel.
 // ---------------------------------------------------------------------------------------
 template <int EL>
-__global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int rows_total)
+__global__ __launch_bounds__(kThreads) void select_wave_kernel(SELECT_EARLY, int rows_total, SelectArgs a)
 {
     // (a wave past the last row reads the last row and leaves below: with the exit up here the
     // kernel's arguments would be fetched in two rounds, the row count first)
     const int rowid_raw = blockIdx.x * (kThreads / kWave) + wave_id();
     const int rowid = rowid_raw < rows_total ? rowid_raw : rows_total - 1;
-    const int b = a.Ho == 1 ? rowid : rowid / a.Ho, ho = rowid - b * a.Ho;
+    const int b = Ho == 1 ? rowid : rowid / Ho, ho = rowid - b * Ho;
     const int lane = lane_id();
-    const int len = a.lens[b];
+    const int len = lens[b];
     // the row's scores go out before the length is known (in-range positions only, masked
     // below): one round trip to memory instead of two
     int raw[EL];
-    const bool red = (a.flags & UCM_TOPK_REDUCE_HEADS) && a.Hkv > 1;
+    const bool red = (flags & UCM_TOPK_REDUCE_HEADS) && Hkv > 1;
     {
-        const int32_t* r0 = a.scores + (int64_t)b * a.Hkv * a.max_blocks + (int64_t)(red ? 0 : ho) * a.sc_h;
+        const int32_t* r0 = scores + (int64_t)b * Hkv * max_blocks + (int64_t)(red ? 0 : ho) * sc_h;
 #pragma unroll
         for (int e = 0; e < EL; ++e) {
             const int j = lane * EL + e;
-            raw[e] = r0[(int64_t)(j < a.max_blocks ? j : 0) * a.sc_j];
+            raw[e] = r0[(int64_t)(j < max_blocks ? j : 0) * sc_j];
         }
     }
     // physical block ids of the whole row, fetched alongside the scores: the output loop then
     // has no load (and no round trip to memory) per selected element
-    const bool physical = (a.flags & UCM_TOPK_RETURN_PHYSICAL) != 0;
+    const bool physical = (flags & UCM_TOPK_RETURN_PHYSICAL) != 0;
     int tab[EL];
-    if (physical && a.table) {
-        const int32_t* t0 = a.table + (int64_t)b * a.table_stride;
+    if (physical && table) {
+        const int32_t* t0 = table + (int64_t)b * table_stride;
 #pragma unroll
         for (int e = 0; e < EL; ++e) {
             const int j = lane * EL + e;
-            tab[e] = t0[j < a.max_blocks ? j : 0];
+            tab[e] = t0[j < max_blocks ? j : 0];
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < EL; ++e) tab[e] = physical ? b * a.max_blocks + lane * EL + e : lane * EL + e;
+        for (int e = 0; e < EL; ++e) tab[e] = physical ? b * max_blocks + lane * EL + e : lane * EL + e;
     }
     if (rowid_raw >= rows_total) return;
     int n = len > 0 ? blocks_of(a, len) : 0;
@@ -2588,42 +2607,41 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SelectArgs a, int
 // instructions back to back for its row (7 us, however few rows there are); here each wave has
 // a quarter of the row and the search counts in LDS: kBins bins of the row's range, so that nearly every row's threshold
 // is found in two steps of a barrier, some 450 cycles each (halving the range took a step of 450 cycles for every bit of it, with
-// seven thresholds a step 1,130 for every three).  The launch: 2 rows of 313 scores 4.6 and 2.7 us, 16 of 1,024 5.4 and 3.9, 64 of 1,024
+// seven thresholds a step 1,130 for every three).  The launch: 2 rows of 313 scores 4.6 and 2.3 us, 16 of 1,024 5.4 and 3.9, 64 of 1,024
 // in a range of 52 4.0 and 3.8.  What is left is the chain of arguments, scores, extremes, threshold, places and stores.
 template <int EL>
-__global__ __launch_bounds__(kThreads) void select_group_kernel(SelectArgs a)
+__global__ __launch_bounds__(kThreads) void select_group_kernel(SELECT_EARLY, SelectArgs a)
 {
     constexpr int kWaves = kThreads / kWave;
     constexpr int kBins = 512;
     __shared__ __align__(16) int hist[2][kBins];
     __shared__ int ext[3][kWaves];
     __shared__ int wsum[kWaves];
-    ucm::warm_args(a);
     // (divisions stand in front of the first load, or between the loads and the search: forty instructions each)
-    const int b = a.Ho == 1 ? blockIdx.x : blockIdx.x / a.Ho, ho = blockIdx.x - b * a.Ho;
+    const int b = Ho == 1 ? blockIdx.x : blockIdx.x / Ho, ho = blockIdx.x - b * Ho;
     const int tid = threadIdx.x, lane = lane_id(), wid = wave_id();
     hist[0][tid] = hist[0][tid + kThreads] = 0;
     hist[1][tid] = hist[1][tid + kThreads] = 0;
-    const bool reduce = (a.flags & UCM_TOPK_REDUCE_HEADS) && a.Hkv > 1;
-    const int32_t* row = a.scores + ((int64_t)b * a.Hkv + (reduce ? 0 : ho)) * a.max_blocks;
-    const int len = a.lens[b];  // asked for with the scores: one round trip to memory
+    const bool reduce = (flags & UCM_TOPK_REDUCE_HEADS) && Hkv > 1;
+    const int32_t* row = scores + ((int64_t)b * Hkv + (reduce ? 0 : ho)) * max_blocks;
+    const int len = lens[b];  // asked for with the scores: one round trip to memory
     int v[EL], tab[EL];
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
         const int j = tid * EL + e;
-        v[e] = row[j < a.max_blocks ? j : 0];
+        v[e] = row[j < max_blocks ? j : 0];
     }
-    const bool physical = (a.flags & UCM_TOPK_RETURN_PHYSICAL) != 0;
-    if (physical && a.table) {
-        const int32_t* t0 = a.table + (int64_t)b * a.table_stride;
+    const bool physical = (flags & UCM_TOPK_RETURN_PHYSICAL) != 0;
+    if (physical && table) {
+        const int32_t* t0 = table + (int64_t)b * table_stride;
 #pragma unroll
         for (int e = 0; e < EL; ++e) {
             const int j = tid * EL + e;
-            tab[e] = t0[j < a.max_blocks ? j : 0];
+            tab[e] = t0[j < max_blocks ? j : 0];
         }
     } else {
 #pragma unroll
-        for (int e = 0; e < EL; ++e) tab[e] = physical ? b * a.max_blocks + tid * EL + e : tid * EL + e;
+        for (int e = 0; e < EL; ++e) tab[e] = physical ? b * max_blocks + tid * EL + e : tid * EL + e;
     }
     int n = len > 0 ? blocks_of(a, len) : 0;
     if (n > a.max_blocks) n = a.max_blocks;
@@ -3364,7 +3382,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
             note_score("block_score_strip8");
             a.TB = strip_blocks(8, B, max_blocks, false);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
-            launch_score_threads(block_score_strip<8>, g64, kStripWaves * kWave, 0, st, a);
+            launch_score_threads(block_score_strip<8>, g64, kStripWaves * kWave, 0, st, STRIP_EARLY_OF(a), a);
         } else if (planes_inside) {
             // one nibble digit of the per-bit counts up to 15 query heads, two up to 255
             const int nd = a.G <= 15 ? 1 : 2;
@@ -3383,7 +3401,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
             note_score("block_score_strip18");
             a.TB = strip_blocks(18, B, max_blocks, false);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
-            launch_score_threads(block_score_strip<18>, g64, kStripWaves * kWave, 0, st, a);
+            launch_score_threads(block_score_strip<18>, g64, kStripWaves * kWave, 0, st, STRIP_EARLY_OF(a), a);
         } else if (planes_in_lanes) {
             note_score("block_score_lanes_run", Wd / 2, pmax);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, (kThreads / kWave) * kLanesRunBlocks), (unsigned)B);
@@ -3430,20 +3448,20 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
         // up to 256 blocks a wave per row stays ahead of a workgroup per row (config 2 step:
         // 32.7 against 33.3 us)
         note_select("select_wave_kernel", 4);
-        hipLaunchKernelGGL(select_wave_kernel<4>, wgrid, dim3(kThreads), 0, st, s, rows_total);
+        hipLaunchKernelGGL(select_wave_kernel<4>, wgrid, dim3(kThreads), 0, st, SELECT_EARLY_OF(s), rows_total, s);
         return ucm::launch_status("select_wave_kernel");
     }
     if (!(flags & UCM_TOPK_SCORE_ORDER) && max_blocks <= 4096) {
         const dim3 rgrid((unsigned)rows_total);
         note_select("select_group_kernel", max_blocks <= 512 ? 2 : (max_blocks <= 1024 ? 4 : (max_blocks <= 2048 ? 8 : 16)));
         if (max_blocks <= 512)
-            hipLaunchKernelGGL(select_group_kernel<2>, rgrid, dim3(kThreads), 0, st, s);
+            hipLaunchKernelGGL(select_group_kernel<2>, rgrid, dim3(kThreads), 0, st, SELECT_EARLY_OF(s), s);
         else if (max_blocks <= 1024)
-            hipLaunchKernelGGL(select_group_kernel<4>, rgrid, dim3(kThreads), 0, st, s);
+            hipLaunchKernelGGL(select_group_kernel<4>, rgrid, dim3(kThreads), 0, st, SELECT_EARLY_OF(s), s);
         else if (max_blocks <= 2048)
-            hipLaunchKernelGGL(select_group_kernel<8>, rgrid, dim3(kThreads), 0, st, s);
+            hipLaunchKernelGGL(select_group_kernel<8>, rgrid, dim3(kThreads), 0, st, SELECT_EARLY_OF(s), s);
         else
-            hipLaunchKernelGGL(select_group_kernel<16>, rgrid, dim3(kThreads), 0, st, s);
+            hipLaunchKernelGGL(select_group_kernel<16>, rgrid, dim3(kThreads), 0, st, SELECT_EARLY_OF(s), s);
         return ucm::launch_status("select_group_kernel");
     }
     note_select("select_kernel");

@@ -2309,10 +2309,10 @@ __global__ __launch_bounds__(64 * small_split(KSA)) __attribute__((amdgpu_waves_
 // workgroup takes 64 columns of a row tile (the same 64 KiB of rows), each of its eight waves a quarter of the row's values
 // and half of the columns, and what the prologue need not decide is not in the code.  The sums are taken in the
 // same order as there, so that a key has the same code from either.
-// Launches of a step, the other kernel and this one: 2 requests x 64 means of two rows (128 query rows) 6.2 and 5.7 us, 16 x 64
-// 8.6 and 8.0; whole steps of 1 to 32 requests and 8 to 128 query rows each 1 to 7 % shorter.  What is left of it, at 2,400 cycles
-// to the microsecond: 2,000 cycles for arguments and 128 KiB through a compute unit's L1 at 64 bytes a cycle, 1,500 for
-// the means (9 instructions for two values), 2,400 for turning W through LDS and the products, 1,700 for the partial sums.
+// Launches of a step, the other kernel and this one: 2 requests x 64 means of two rows (128 query rows) 6.2 and 5.2 us, 16 x 64
+// 8.6 and 7.6 (5.7 and 8.0 with all arguments in the struct).  What is left of it, at 2,100 cycles to the microsecond: 128 KiB
+// through a compute unit's L1 at 64 bytes a cycle, 1,500 cycles for the means (9 instructions for two values), 2,400 for
+// turning W through LDS and the products, 1,700 for the partial sums.
 struct LatentJob {
     const void* x;
     const void* w;
@@ -2326,8 +2326,9 @@ struct LatentJob {
 
 struct LatentJobs {
     LatentJob job[4];         // keys and queries of 512 values, keys and queries of 64
-    int wide, narrow;         // tiles of either width
+    int wide, narrow;          // tiles of either width
     int wide_shift, nt_shift;  // log2 of the tiles that a row tile's columns make
+    uint32_t shifts;
 };
 
 constexpr int kLatentWaves = 8;
@@ -2336,8 +2337,15 @@ constexpr int kLatentPart = 20;             // floats of a lane's partial sums i
 static_assert(64 * kLatentPart * 4 <= 32 * kLatentPitch * 2, "a wave's columns make room for its sums");
 static_assert(32 * (64 + kPad) <= 32 * kLatentPitch, "a narrow tile fits a wave's area");
 
+// The part of a job that its row loads take.
+struct LatentRows {
+    const void* x;
+    int64_t xs_t, xs_h, xs_g;
+    int rows, h_shift, mean;
+};
+
 // Row p of a job, the last one for a place behind it.
-__device__ __forceinline__ void latent_row(const LatentJob& a, int p, int& t, int& h)
+__device__ __forceinline__ void latent_row(const LatentRows& a, int p, int& t, int& h)
 {
     p = p < a.rows ? p : a.rows - 1;
     t = p >> a.h_shift;
@@ -2364,7 +2372,7 @@ __device__ __forceinline__ uint32_t* latent_dst(const LatentJob& a, RawSlot raw,
 
 // Four loads of whole row pieces of 16 bytes a lane, kLanes of them to a row, from row p0 on; the second one of a mean too.
 template <typename V, int G, int kLanes>
-__device__ __forceinline__ void latent_load(const LatentJob& a, int p0, int k0, V (&v)[4][G])
+__device__ __forceinline__ void latent_load(const LatentRows& a, int p0, int k0, V (&v)[4][G])
 {
     const int lane = threadIdx.x & 63;
 #pragma unroll
@@ -2379,7 +2387,7 @@ __device__ __forceinline__ void latent_load(const LatentJob& a, int p0, int k0, 
 
 // fp32 sum of the rows in order, times a half, rounded to the input type.
 template <typename V, int G>
-__device__ __forceinline__ V latent_mean(const LatentJob& a, const V (&v)[G])
+__device__ __forceinline__ V latent_mean(const LatentRows& a, const V (&v)[G])
 {
     if (G == 1 || !a.mean) return v[0];
     V m;
@@ -2404,18 +2412,25 @@ __device__ __forceinline__ void latent_turn(const u32x4 (&row)[8], uint16_t* wt,
     }
 }
 
+// What the wide tiles' rows and columns take, in front of the struct (see the build's flags: leading scalars arrive in
+// registers): the projection and the rows of 512 values, their strides, log2 of the tiles of a row tile, of the heads, and
+// whether queries are means, a byte each.
+#define LATENT_EARLY                                                                                                 \
+    const void *w, const void *q, const void *k, uint32_t shifts, int q_t, int q_h, int q_g, int k_t, int rows_q, int rows_k
+
 template <typename V, int G>
-__global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_eu(4, 8))) void encode_latent_kernel(LatentJobs js)
+__global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_eu(4, 8))) void encode_latent_kernel(LATENT_EARLY, LatentJobs js)
 {
     __shared__ __align__(16) uint16_t lds[kLatentWaves * 32 * kLatentPitch];
-    ucm::warm_args(js);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, kb = lane >> 5;
     uint16_t* const wt = lds + wave * 32 * kLatentPitch;
-    if ((int)blockIdx.x >= js.wide) {  // a narrow tile is one wave's work
-        const int tile = ((int)blockIdx.x - js.wide) * kLatentWaves + wave;
+    const int tiles_k = (rows_k + 31) >> 5, tiles_q = (rows_q + 31) >> 5, wide_shift = shifts & 0xff;
+    if ((int)blockIdx.x >= (tiles_k + tiles_q) << wide_shift) {  // a narrow tile is one wave's work
+        const int tile = ((int)blockIdx.x - ((tiles_k + tiles_q) << wide_shift)) * kLatentWaves + wave;
         if (tile >= js.narrow) return;
         const LatentJob& a = js.job[tile >= js.job[3].first ? 3 : 2];
+        const LatentRows in{a.x, a.xs_t, a.xs_h, a.xs_g, a.rows, a.h_shift, a.mean};
         const int wv = tile - a.first, nt = wv & ((1 << js.nt_shift) - 1), p0 = (wv >> js.nt_shift) * 32;
         const int N = 32 << js.nt_shift;
         constexpr int kPitch = 64 + kPad;
@@ -2425,12 +2440,12 @@ __global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int i = 0; i < 8; ++i) row[i] = *reinterpret_cast<const u32x4*>(src + i * N);
         V v[4][G];
-        latent_load<V, G, 8>(a, p0, 0, v);
+        latent_load<V, G, 8>(in, p0, 0, v);
         int t, h;
-        latent_row(a, p0 + r, t, h);
+        latent_row(in, p0 + r, t, h);
         const RawSlot raw = latent_slot(a, t);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<V*>(wt + (i * 8 + lane / 8) * kPitch + lane % 8 * 8) = latent_mean<V, G>(a, v[i]);
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<V*>(wt + (i * 8 + lane / 8) * kPitch + lane % 8 * 8) = latent_mean<V, G>(in, v[i]);
         __builtin_amdgcn_wave_barrier();
         V av[4];
 #pragma unroll
@@ -2450,32 +2465,35 @@ __global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_
         }
         return;
     }
-    const LatentJob& a = js.job[(int)blockIdx.x >= js.job[1].first ? 1 : 0];
-    int wv = (int)blockIdx.x - a.first, nt;
+    const bool keys = (int)blockIdx.x < tiles_k << wide_shift;
+    const LatentJob& a = js.job[keys ? 0 : 1];
+    const LatentRows in{keys ? k : q, keys ? k_t : q_t, keys ? 0 : q_h, keys ? 0 : q_g, keys ? rows_k : rows_q,
+                        keys ? 0 : (int)(shifts >> 8 & 0xff), keys ? 0 : (int)(shifts >> 16)};
+    int wv = (int)blockIdx.x - (keys ? 0 : tiles_k << wide_shift), nt;
     // eight row tiles at a time go out row tile first, so that a row tile's workgroups are on one XCD and its rows come
     // past that XCD's L2 once (consecutive workgroups go to the eight XCDs in turn)
-    if ((wv >> (js.wide_shift + 3)) < (((a.rows + 31) >> 5) >> 3)) {
-        nt = (wv >> 3) & ((1 << js.wide_shift) - 1);
-        wv = (wv >> (js.wide_shift + 3)) * 8 + (wv & 7);
+    if ((wv >> (wide_shift + 3)) < ((keys ? tiles_k : tiles_q) >> 3)) {
+        nt = (wv >> 3) & ((1 << wide_shift) - 1);
+        wv = (wv >> (wide_shift + 3)) * 8 + (wv & 7);
     } else {
-        nt = wv & ((1 << js.wide_shift) - 1);
-        wv >>= js.wide_shift;
+        nt = wv & ((1 << wide_shift) - 1);
+        wv >>= wide_shift;
     }
-    const int p0 = wv * 32, N = 64 << js.wide_shift;
+    const int p0 = wv * 32, N = 64 << wide_shift;
     const int slice = wave >> 1, ct = wave & 1;
     u32x4 row[8];
     const int kq = lane >> 2, j = lane & 3;
-    const uint16_t* src = (const uint16_t*)a.w + (int64_t)(slice * 128 + kq * 8) * N + nt * 64 + ct * 32 + 8 * j;
+    const uint16_t* src = (const uint16_t*)w + (int64_t)(slice * 128 + kq * 8) * N + nt * 64 + ct * 32 + 8 * j;
 #pragma unroll
     for (int i = 0; i < 8; ++i) row[i] = *reinterpret_cast<const u32x4*>(src + i * N);
     V v[4][G];
-    latent_load<V, G, 16>(a, p0 + ct * 16, slice * 128, v);
+    latent_load<V, G, 16>(in, p0 + ct * 16, slice * 128, v);
     int t, h;
-    latent_row(a, p0 + r, t, h);
+    latent_row(in, p0 + r, t, h);
     const RawSlot raw = latent_slot(a, t);
     // the two waves of a slice share its rows, sixteen in the area of each
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<V*>(wt + (i * 4 + lane / 16) * kLatentPitch + lane % 16 * 8) = latent_mean<V, G>(a, v[i]);
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<V*>(wt + (i * 4 + lane / 16) * kLatentPitch + lane % 16 * 8) = latent_mean<V, G>(in, v[i]);
     __syncthreads();
     V av[8];
     {
@@ -2514,7 +2532,7 @@ __global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_
     for (int i = 3; i >= 0; --i) bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(sum[i]), 31);
     bits = first != first ? 0u : (bits ^ 15u);
     bits = join_halves(kb ? bits << 4 : bits);
-    if (lane < 32 && p0 + r < a.rows) {
+    if (lane < 32 && p0 + r < in.rows) {
         uint32_t* dst = latent_dst(a, raw, t, h);
         if (dst) reinterpret_cast<uint8_t*>(dst + nt * 2 + ct)[slice] = (uint8_t)bits;
     }
@@ -3839,6 +3857,10 @@ bool latent_jobs(const EncJobs4& js, LatentJobs& out)
         if (!latent_job(js.job[i], out.job[i])) return false;
     const EncArgs &wide = js.job[0], &narrow = js.job[2];
     if (wide.nt_shift < 1 || narrow.nt_shift < 0) return false;
+    const LatentJob &k = out.job[0], &q = out.job[1];
+    auto word = [](int64_t v) { return v >= INT32_MIN && v <= INT32_MAX; };
+    if (wide.H != 1 || k.mean || k.w != q.w || !word(k.xs_t) || !word(q.xs_t) || !word(q.xs_h) || !word(q.xs_g)) return false;
+    out.shifts = (uint32_t)(wide.nt_shift - 1) | (uint32_t)q.h_shift << 8 | (uint32_t)q.mean << 16;
     out.wide_shift = wide.nt_shift - 1;
     out.nt_shift = narrow.nt_shift;
     auto row_tiles = [&](int i) { return ucm::ceil_div(out.job[i].rows, kRowsPerWave); };
@@ -3859,8 +3881,13 @@ int launch_small_mixed(const EncJobs4& js, hipStream_t st)
     if (latent_jobs(js, lean)) {
         const dim3 grid((unsigned)(lean.wide + ucm::ceil_div(lean.narrow, kLatentWaves))), threads(64 * kLatentWaves);
         const bool mean = lean.job[1].mean || lean.job[3].mean || lean.job[0].mean || lean.job[2].mean;
-        if (mean) hipLaunchKernelGGL((encode_latent_kernel<V, 2>), grid, threads, 0, st, lean);
-        else hipLaunchKernelGGL((encode_latent_kernel<V, 1>), grid, threads, 0, st, lean);
+        const LatentJob &k = lean.job[0], &q = lean.job[1];
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, threads, 0, st, q.w, q.x, k.x, lean.shifts, (int)q.xs_t, (int)q.xs_h, (int)q.xs_g, (int)k.xs_t,
+                               q.rows, k.rows, lean);
+        };
+        if (mean) launch(encode_latent_kernel<V, 2>);
+        else launch(encode_latent_kernel<V, 1>);
         return ucm::launch_status("encode_latent_kernel");
     }
     const dim3 grid((unsigned)js.end[3]), threads(64 * small_split(32));
