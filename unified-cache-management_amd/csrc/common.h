@@ -46,6 +46,24 @@ inline int launch_status(const char* kernel)
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 #ifdef __HIPCC__
+// What a kernel's first loads take goes into leading arguments of these types: the build has the hardware put the first
+// fourteen words of scalar and vector arguments into registers before the waves start, where the fields of a struct
+// are read from memory by every wave, 0.2 to 0.5 us in front of its first load.  Vectors, as every argument of a launch
+// costs the host some 25 ns (two launches with twelve arguments more: 8.6 and 8.9 us a call that waits for its host).
+typedef uint64_t ArgPair __attribute__((ext_vector_type(2)));
+typedef int32_t ArgInts __attribute__((ext_vector_type(4)));
+inline ArgPair arg_pair(const void* a, const void* b) { return ArgPair{(uint64_t)(uintptr_t)a, (uint64_t)(uintptr_t)b}; }
+inline ArgPair arg_pair(const void* a, uint64_t b) { return ArgPair{(uint64_t)(uintptr_t)a, b}; }
+inline uint64_t arg_words(int lo, int hi) { return (uint32_t)lo | (uint64_t)(uint32_t)hi << 32; }
+__device__ __forceinline__ int arg_lo(uint64_t v) { return (int)(uint32_t)v; }
+__device__ __forceinline__ int arg_hi(uint64_t v) { return (int)(v >> 32); }
+// (by way of the global address space: an address of unknown space would make every access a flat one)
+template <class T>
+__device__ __forceinline__ T* arg_ptr(uint64_t v)
+{
+    return (T*)(__attribute__((address_space(1))) T*)v;
+}
+
 // Touches every 64-byte line of a kernel-argument struct at once.  The compiler fetches a field
 // where the code first needs it, behind the branches of the row addressing - a dozen scalar reads
 // one after the other in a kernel that lives for a few microseconds; with the lines already in the

@@ -59,8 +59,10 @@ __device__ __forceinline__ float wave_sum_last(float v)
 // and the query pieces, which come from the caches, go out in front of them), so the row data cost one
 // round trip; no LDS and no barrier.  2 x 8000 rows of 1024 (65.5 MB): 12.3 us = 5.3 TB/s of the launch;
 // with 4 KiB in flight per wave, behind a barrier for a query staged in LDS, 14.6 us.
-__global__ __launch_bounds__(kDotThreads) void dot_score_kernel(DotArgs a)
+__global__ __launch_bounds__(kDotThreads) void dot_score_kernel(ucm::ArgPair rows, ucm::ArgPair lists, ucm::ArgInts n)
 {
+    const DotArgs a{ucm::arg_ptr<const float>(rows.x), (int64_t)(uint32_t)n.z | (int64_t)n.w << 32, n.x, ucm::arg_ptr<const float>(rows.y),
+                    ucm::arg_ptr<const int32_t>(lists.x), n.y, ucm::arg_ptr<uint32_t>(lists.y), key_pitch(n.y)};
     const int b = blockIdx.y;
     const float* q = a.q + (int64_t)b * a.dim;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -160,7 +162,8 @@ extern "C" int ucm_dot_topk(const float* data, int64_t n_items, int32_t dim, con
     d.pitch = key_pitch(max_n);
     const int rows_per_wg = (kDotThreads / 64) * kRowsPerWave;
     hipLaunchKernelGGL(dot_score_kernel, dim3((unsigned)ucm::ceil_div(max_n, rows_per_wg), (unsigned)B),
-                       dim3(kDotThreads), 0, st, d);
+                       dim3(kDotThreads), 0, st, ucm::arg_pair(d.data, d.q), ucm::arg_pair(d.idx, d.keys),
+                       ucm::ArgInts{dim, max_n, (int)(uint32_t)n_items, (int)(n_items >> 32)});
     int rc = ucm::launch_status("dot_score_kernel");
     if (rc != UCM_OK) return rc;
     SortArgs s{};

@@ -40,7 +40,7 @@ __device__ __forceinline__ float key_place(uint32_t k)
 }
 
 // Keys of a row lie at a pitch of whole 64-byte lines: every thread loads its keys as 16-byte pieces.
-inline int64_t key_pitch(int64_t n) { return (n + 15) & ~(int64_t)15; }
+__host__ __device__ __forceinline__ int64_t key_pitch(int64_t n) { return (n + 15) & ~(int64_t)15; }
 
 struct SortArgs {
     const uint32_t* keys;   // [B] rows of max_n keys, `pitch` apart; 16-byte aligned
@@ -49,9 +49,16 @@ struct SortArgs {
     int max_n, topk, cap;   // cap: entries the search orders in LDS, a power of two
     int32_t* out_idx;       // [B][topk]
     float* out_score;       // [B][topk]
-    const float* sums;      // topk_rank_sums_kernel, one row: [n_sums][max_n] parts of the scores, instead of keys
-    int n_sums;
 };
+
+// The same as leading arguments of a kernel (see ucm::ArgPair).
+#define SORT_ARGS ucm::ArgPair p_in, ucm::ArgPair p_out, ucm::ArgInts n
+#define SORT_ARGS_OF(s) ucm::arg_pair((s).keys, (s).idx), ucm::arg_pair((s).out_idx, (s).out_score), ucm::ArgInts{(s).max_n, (s).topk, (s).cap, 0}
+__device__ __forceinline__ SortArgs sort_args(SORT_ARGS)
+{
+    return SortArgs{ucm::arg_ptr<const uint32_t>(p_in.x), key_pitch(n.x), ucm::arg_ptr<const int32_t>(p_in.y), n.x, n.y, n.z,
+                    ucm::arg_ptr<int32_t>(p_out.x), ucm::arg_ptr<float>(p_out.y)};
+}
 
 // Maximum over the 64 lanes, in every lane: exchanges inside a row of 16 lanes, then the last lane
 // of a row broadcast into the next rows (a few cycles each; a shuffle is a trip through the LDS pipe).
@@ -703,9 +710,10 @@ __device__ __forceinline__ void rank_places(const SortArgs& a, int waves, uint32
 }
 
 constexpr int kRankRow = 512;
-__global__ __launch_bounds__(256) void topk_rank_kernel(SortArgs a)
+__global__ __launch_bounds__(256) void topk_rank_kernel(SORT_ARGS)
 {
     __shared__ RankShared<4> sh;
+    const SortArgs a = sort_args(p_in, p_out, n);
     const uint32_t* keys = a.keys + blockIdx.x * a.pitch;
     const int pos = blockIdx.y * 64 + (threadIdx.x & 63);
     const uint32_t mine = pos < a.max_n ? keys[pos] : 0u;
@@ -714,23 +722,27 @@ __global__ __launch_bounds__(256) void topk_rank_kernel(SortArgs a)
 
 // The same for one row of up to kRankSums candidates whose scores are still in n_sums parts, which every workgroup
 // adds by itself, in the same order.  A wave for every 64 candidates up to sixteen: the parts of a wave's 64 and those
-// of the workgroup's own 64 are one round trip (253 candidates of 16 parts: 4.7 us, requested a
+// of the workgroup's own 64 are one round trip (253 candidates of 16 parts: 4.1 us, with its arguments read from memory 4.7, requested a
 // few at a time 5.0; 1024 of them 3 us less than in four waves with a branch at every part).
 constexpr int kRankSums = 2048;
-__global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SortArgs a)
+__global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SORT_ARGS)
 {
     __shared__ RankShared<16> sh;
+    SortArgs a = sort_args(p_in, p_out, n);
+    const float* const sums = reinterpret_cast<const float*>(a.keys);
+    const int max_n = n.x, n_sums = n.z;
+    a.idx = nullptr;
     auto keys_of = [&](auto n_, const int (&at)[decltype(n_)::value], uint32_t (&key)[decltype(n_)::value]) {
         constexpr int N = decltype(n_)::value;
         float s[N] = {};
         uint32_t off[N];
 #pragma unroll
-        for (int n = 0; n < N; ++n) off[n] = at[n] < a.max_n ? at[n] : a.max_n - 1;
-        for (int i = 0; i < a.n_sums; i += 16) {
+        for (int n = 0; n < N; ++n) off[n] = at[n] < max_n ? at[n] : max_n - 1;
+        for (int i = 0; i < n_sums; i += 16) {
             float v[N][16];
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const float* p = a.sums + (int64_t)(i + e < a.n_sums ? i + e : 0) * a.max_n;
+                const float* p = sums + (int64_t)(i + e < n_sums ? i + e : 0) * max_n;
 #pragma unroll
                 for (int n = 0; n < N; ++n) v[n][e] = p[off[n]];
             }
@@ -738,10 +750,10 @@ __global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SortArgs a)
 #pragma unroll
             for (int e = 0; e < 16; ++e)
 #pragma unroll
-                for (int n = 0; n < N; ++n) s[n] += i + e < a.n_sums ? v[n][e] : 0.0f;
+                for (int n = 0; n < N; ++n) s[n] += i + e < n_sums ? v[n][e] : 0.0f;
         }
 #pragma unroll
-        for (int n = 0; n < N; ++n) key[n] = at[n] < a.max_n ? score_key(s[n]) : 0u;
+        for (int n = 0; n < N; ++n) key[n] = at[n] < max_n ? score_key(s[n]) : 0u;
     };
     const int lane = threadIdx.x & 63;
     const int at[2] = {(int)blockIdx.y * 64 + lane, (int)threadIdx.x};
@@ -762,8 +774,9 @@ constexpr size_t search_lds(int nt, int cap) { return (size_t)nt * 16 + (size_t)
 // grid = (rows, workgroups per row).  Thread t holds list positions t * PER ..
 // t * PER + PER - 1 (consecutive, so that one prefix sum over per-thread counts orders the list).
 template <int NT, int PER>
-__global__ __launch_bounds__(NT) void topk_kernel(SortArgs a)
+__global__ __launch_bounds__(NT) void topk_kernel(SORT_ARGS)
 {
+    const SortArgs a = sort_args(p_in, p_out, n);
     extern __shared__ __align__(16) uint32_t lds[];
     __shared__ int wsum[NT / 64];
     __shared__ uint32_t range[2][NT / 64];
@@ -806,15 +819,16 @@ inline int launch_topk_as(SortArgs s, int rows, hipStream_t st)
     const int split = PER > 0 ? (int)ucm::ceil_div(most, NT) : 1;
     const size_t need = search_lds(NT, cap), direct = PER > 0 ? direct_lds(NT) : 0;
     static_assert(search_lds(NT, kMaxTopk) + 512 <= 64 * 1024 && direct_lds(NT) + 512 <= 64 * 1024, "");
-    hipLaunchKernelGGL((topk_kernel<NT, PER>), dim3((unsigned)rows, (unsigned)split), dim3(NT), need > direct ? need : direct, st, s);
+    hipLaunchKernelGGL((topk_kernel<NT, PER>), dim3((unsigned)rows, (unsigned)split), dim3(NT), need > direct ? need : direct, st, SORT_ARGS_OF(s));
     return ucm::launch_status("topk_kernel");
 }
 
-// One row of up to kRankSums candidates whose scores are in parts.
-inline int launch_rank_sums(const SortArgs& s, hipStream_t st)
+// One row of up to kRankSums candidates whose scores are in n_sums parts, [n_sums][s.max_n].
+inline int launch_rank_sums(const SortArgs& s, const float* sums, int n_sums, hipStream_t st)
 {
     const unsigned pieces = (unsigned)ucm::ceil_div(s.max_n, 64);
-    hipLaunchKernelGGL(topk_rank_sums_kernel, dim3(1, pieces), dim3(64 * (pieces < 16 ? pieces : 16)), 0, st, s);
+    hipLaunchKernelGGL(topk_rank_sums_kernel, dim3(1, pieces), dim3(64 * (pieces < 16 ? pieces : 16)), 0, st,
+                       ucm::arg_pair(sums, nullptr), ucm::arg_pair(s.out_idx, s.out_score), ucm::ArgInts{s.max_n, s.topk, n_sums, 0});
     return ucm::launch_status("topk_rank_sums_kernel");
 }
 
@@ -828,7 +842,7 @@ inline int launch_rank_sums(const SortArgs& s, hipStream_t st)
 inline int launch_topk(const SortArgs& s, int rows, hipStream_t st)
 {
     if (s.max_n <= kRankRow) {
-        hipLaunchKernelGGL(topk_rank_kernel, dim3((unsigned)rows, (unsigned)ucm::ceil_div(s.max_n, 64)), dim3(256), 0, st, s);
+        hipLaunchKernelGGL(topk_rank_kernel, dim3((unsigned)rows, (unsigned)ucm::ceil_div(s.max_n, 64)), dim3(256), 0, st, SORT_ARGS_OF(s));
         return ucm::launch_status("topk_rank_kernel");
     }
     if (s.max_n <= 1024) return launch_topk_as<256, 4>(s, rows, st);

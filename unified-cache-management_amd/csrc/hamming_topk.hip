@@ -59,14 +59,6 @@ struct ScoreArgs {
     unsigned long long* clock_probe;  // strip scorers: see ucm_hamming_topk_set_clock_probe(); else null
 };
 
-// What the strip scorers' first loads take, as arguments in front of the struct: the build has the hardware put a kernel's
-// leading scalar arguments into registers before its waves start, where the fields of a struct are read from memory
-// by every wave, 0.4 to 0.5 us before its first load.  (Fourteen registers in all, 8-byte arguments first.)
-#define STRIP_EARLY                                                                                                   \
-    const int32_t *lens, const int32_t *table, const uint32_t *q, int64_t q_stride_b, int64_t q_stride_h, int table_stride, \
-        int max_blocks, int TB, int G
-#define STRIP_EARLY_OF(a) (a).lens, (a).table, (a).q, (a).q_stride_b, (a).q_stride_h, (a).table_stride, (a).max_blocks, (a).TB, (a).G
-
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
@@ -2072,10 +2064,11 @@ __device__ __forceinline__ void strip_body(const ScoreArgs& a, int max_seq_len, 
 }
 
 template <int WD>
-__global__ __launch_bounds__(kStripWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void block_score_strip(STRIP_EARLY, ScoreArgs a)
+__global__ __launch_bounds__(kStripWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 8))) void block_score_strip(ucm::ArgPair request, ucm::ArgPair query, ucm::ArgInts n, int64_t q_stride_h, ScoreArgs a)
 {
-    a.lens = lens; a.table = table; a.q = q; a.q_stride_b = q_stride_b; a.q_stride_h = q_stride_h;
-    a.table_stride = table_stride; a.max_blocks = max_blocks; a.TB = TB; a.G = G;
+    a.lens = ucm::arg_ptr<const int32_t>(request.x); a.table = ucm::arg_ptr<const int32_t>(request.y);
+    a.q = ucm::arg_ptr<const uint32_t>(query.x); a.q_stride_b = (int64_t)query.y; a.q_stride_h = q_stride_h;
+    a.table_stride = n.x; a.max_blocks = n.y; a.TB = n.z; a.G = n.w;
     strip_body<WD, 0>(a, 0, nullptr);
 }
 
@@ -2222,6 +2215,7 @@ struct SelectArgs {
     const int32_t* lens;
     int BS, Hkv, Ho, k, full, key_bits;
     int bs_shift;        // log2(BS), -1 where BS is no power of two
+    int rows_total;      // select_wave_kernel only: B * Ho
     uint32_t flags;
     int32_t* out_idx;    // [B][Ho][k]
     int32_t* out_score;  // may be null
@@ -2235,14 +2229,17 @@ struct SelectArgs {
     int thr_len, topk_tok;
 };
 
-// What the selection kernels' first loads take, as arguments of their own: the build has the hardware put a kernel's
-// leading scalar arguments into registers before its waves start, where a struct's fields are read from memory by
-// every wave (2 rows of 313 scores 2.5 and 2.3 us, and 0.5 us of a step of 32 x 32,768 tokens).
-#define SELECT_EARLY                                                                                              \
-    const int32_t *scores, const int32_t *lens, const int32_t *table, int table_stride, int max_blocks, int Ho,      \
-        int Hkv, uint32_t flags, int sc_h, int sc_j
-#define SELECT_EARLY_OF(s) \
-    (s).scores, (s).lens, (s).table, (s).table_stride, (s).max_blocks, (s).Ho, (s).Hkv, (s).flags, (s).sc_h, (s).sc_j
+// What the selection kernels' first loads take, as leading arguments (see ucm::ArgPair; 2 rows of 313 scores 2.5 and
+// 2.3 us, a step of 32 x 32,768 tokens 29.1 and 28.6).
+#define SELECT_EARLY ucm::ArgPair row_args, ucm::ArgPair table_heads, ucm::ArgInts n_args, uint64_t strides
+#define SELECT_EARLY_OF(s)                                                                                        \
+    ucm::arg_pair((s).scores, (s).lens), ucm::arg_pair((s).table, ucm::arg_words((s).Ho, (s).Hkv)),                    \
+        ucm::ArgInts{(s).table_stride, (s).max_blocks, (int)(s).flags, (s).rows_total}, ucm::arg_words((s).sc_h, (s).sc_j)
+#define SELECT_EARLY_VARS                                                                                         \
+    const int32_t *const scores = ucm::arg_ptr<const int32_t>(row_args.x), *const lens = ucm::arg_ptr<const int32_t>(row_args.y), \
+                  *const table = ucm::arg_ptr<const int32_t>(table_heads.x);                                          \
+    const int Ho = ucm::arg_lo(table_heads.y), Hkv = ucm::arg_hi(table_heads.y), table_stride = n_args.x, max_blocks = n_args.y; \
+    const uint32_t flags = (uint32_t)n_args.z
 
 __device__ __forceinline__ int blocks_of(const SelectArgs& a, int tokens)
 {
@@ -2473,8 +2470,10 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SelectArgs a)
 // in ascending index order, ties to the lower index.  Same results as select_kernel.
 // ---------------------------------------------------------------------------------------
 template <int EL>
-__global__ __launch_bounds__(kThreads) void select_wave_kernel(SELECT_EARLY, int rows_total, SelectArgs a)
+__global__ __launch_bounds__(kThreads) void select_wave_kernel(SELECT_EARLY, SelectArgs a)
 {
+    SELECT_EARLY_VARS;
+    const int sc_h = ucm::arg_lo(strides), sc_j = ucm::arg_hi(strides), rows_total = n_args.w;
     // (a wave past the last row reads the last row and leaves below: with the exit up here the
     // kernel's arguments would be fetched in two rounds, the row count first)
     const int rowid_raw = blockIdx.x * (kThreads / kWave) + wave_id();
@@ -2612,6 +2611,7 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SELECT_EARLY, int
 template <int EL>
 __global__ __launch_bounds__(kThreads) void select_group_kernel(SELECT_EARLY, SelectArgs a)
 {
+    SELECT_EARLY_VARS;
     constexpr int kWaves = kThreads / kWave;
     constexpr int kBins = 512;
     __shared__ __align__(16) int hist[2][kBins];
@@ -2946,6 +2946,13 @@ template <typename K, typename... Args>
 void launch_score(K kernel, dim3 grid, size_t lds, hipStream_t st, Args... args)
 {
     launch_score_threads(kernel, grid, kThreads, lds, st, args...);
+}
+
+template <typename K>
+void launch_strip(K kernel, const ScoreArgs& a, dim3 grid, hipStream_t st)
+{
+    launch_score_threads(kernel, grid, kStripWaves * kWave, 0, st, ucm::arg_pair(a.lens, a.table), ucm::arg_pair(a.q, (uint64_t)a.q_stride_b),
+                         ucm::ArgInts{a.table_stride, a.max_blocks, a.TB, a.G}, a.q_stride_h, a);
 }
 
 template <int CPU, bool DIRECT, int GP>
@@ -3382,7 +3389,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
             note_score("block_score_strip8");
             a.TB = strip_blocks(8, B, max_blocks, false);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
-            launch_score_threads(block_score_strip<8>, g64, kStripWaves * kWave, 0, st, STRIP_EARLY_OF(a), a);
+            launch_strip(block_score_strip<8>, a, g64, st);
         } else if (planes_inside) {
             // one nibble digit of the per-bit counts up to 15 query heads, two up to 255
             const int nd = a.G <= 15 ? 1 : 2;
@@ -3401,7 +3408,7 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
             note_score("block_score_strip18");
             a.TB = strip_blocks(18, B, max_blocks, false);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, kStripWaves * a.TB), (unsigned)B);
-            launch_score_threads(block_score_strip<18>, g64, kStripWaves * kWave, 0, st, STRIP_EARLY_OF(a), a);
+            launch_strip(block_score_strip<18>, a, g64, st);
         } else if (planes_in_lanes) {
             note_score("block_score_lanes_run", Wd / 2, pmax);
             const dim3 g64((unsigned)ucm::ceil_div(max_blocks, (kThreads / kWave) * kLanesRunBlocks), (unsigned)B);
@@ -3442,13 +3449,13 @@ int hamming_topk_run(const uint32_t* q_codes, int64_t q_stride_b, int64_t q_stri
     s.new_lens = step_out ? step_out->new_lens : nullptr;
     s.thr_len = step_out ? step_out->thr_len : 0;
     s.topk_tok = step_out ? step_out->topk_tok : 0;
-    const int rows_total = B * s.Ho;
+    const int rows_total = s.rows_total = B * s.Ho;
     const dim3 wgrid((unsigned)ucm::ceil_div(rows_total, kThreads / kWave));
     if (!(flags & UCM_TOPK_SCORE_ORDER) && max_blocks <= 256) {
         // up to 256 blocks a wave per row stays ahead of a workgroup per row (config 2 step:
         // 32.7 against 33.3 us)
         note_select("select_wave_kernel", 4);
-        hipLaunchKernelGGL(select_wave_kernel<4>, wgrid, dim3(kThreads), 0, st, SELECT_EARLY_OF(s), rows_total, s);
+        hipLaunchKernelGGL(select_wave_kernel<4>, wgrid, dim3(kThreads), 0, st, SELECT_EARLY_OF(s), s);
         return ucm::launch_status("select_wave_kernel");
     }
     if (!(flags & UCM_TOPK_SCORE_ORDER) && max_blocks <= 4096) {

@@ -2412,15 +2412,14 @@ __device__ __forceinline__ void latent_turn(const u32x4 (&row)[8], uint16_t* wt,
     }
 }
 
-// What the wide tiles' rows and columns take, in front of the struct (see the build's flags: leading scalars arrive in
-// registers): the projection and the rows of 512 values, their strides, log2 of the tiles of a row tile, of the heads, and
-// whether queries are means, a byte each.
-#define LATENT_EARLY                                                                                                 \
-    const void *w, const void *q, const void *k, uint32_t shifts, int q_t, int q_h, int q_g, int k_t, int rows_q, int rows_k
-
 template <typename V, int G>
-__global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_eu(4, 8))) void encode_latent_kernel(LATENT_EARLY, LatentJobs js)
+__global__ __launch_bounds__(64 * kLatentWaves) __attribute__((amdgpu_waves_per_eu(4, 8))) void encode_latent_kernel(ucm::ArgPair wq, ucm::ArgPair early, ucm::ArgInts n, int rows_k, LatentJobs js)
 {
+    // the projection and the rows of 512 values, their strides, and a byte each log2 of the tiles of a row tile and of the
+    // heads, and whether queries are means
+    const void *const w = ucm::arg_ptr<const void>(wq.x), *const q = ucm::arg_ptr<const void>(wq.y), *const k = ucm::arg_ptr<const void>(early.x);
+    const int q_t = ucm::arg_lo(early.y), q_h = ucm::arg_hi(early.y), q_g = n.y, k_t = n.z, rows_q = n.w;
+    const uint32_t shifts = (uint32_t)n.x;
     __shared__ __align__(16) uint16_t lds[kLatentWaves * 32 * kLatentPitch];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, kb = lane >> 5;
@@ -3883,8 +3882,8 @@ int launch_small_mixed(const EncJobs4& js, hipStream_t st)
         const bool mean = lean.job[1].mean || lean.job[3].mean || lean.job[0].mean || lean.job[2].mean;
         const LatentJob &k = lean.job[0], &q = lean.job[1];
         auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, threads, 0, st, q.w, q.x, k.x, lean.shifts, (int)q.xs_t, (int)q.xs_h, (int)q.xs_g, (int)k.xs_t,
-                               q.rows, k.rows, lean);
+            hipLaunchKernelGGL(kernel, grid, threads, 0, st, ucm::arg_pair(q.w, q.x), ucm::arg_pair(k.x, ucm::arg_words((int)q.xs_t, (int)q.xs_h)),
+                               ucm::ArgInts{(int)lean.shifts, (int)q.xs_g, (int)k.xs_t, q.rows}, k.rows, lean);
         };
         if (mean) launch(encode_latent_kernel<V, 2>);
         else launch(encode_latent_kernel<V, 1>);

@@ -18,7 +18,7 @@
 //   * Everything else: kvstar_stats_kernel (maximum and sum of exponentials of every row over one chunk of the
 //     representatives), kvstar_mass_kernel (the chunks' pairs merged, q.k once more, probabilities summed over rows
 //     and a block's representatives) and the shared top-k selection.
-// 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 15.1 us (6.0, 4.3 and 4.7 of the three
+// 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 13.5 us (6.0, 4.0 and 4.1 of the three
 // kernels: launches and round trips; the products and exponentials are about 1.5), 18.8 the second way
 // (7.5, 9.0, 3.7); 1024 blocks, 128 channels: 42.9 and 70.4, the second way reads the keys twice.
 // Sums are taken in a different order than the reference's loops, the same one on every call (no
@@ -595,8 +595,11 @@ __global__ __launch_bounds__(kThreads) void kvstar_mass_kernel(KvArgs a)
 // grid = (parts of the blocks, ceil(items / 2)).  Operands as in kvstar_stats_kernel.  A wave takes a block, or as many
 // small ones as two tiles hold (one tile of 128 channels: registers), at a time.
 template <int KS, int UNIT>
-__global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(KvArgs a)
+__global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(ucm::ArgPair qk, ucm::ArgPair early, ucm::ArgInts n, int X, KvArgs a)
 {
+    a.q = ucm::arg_ptr<const _Float16>(qk.x); a.k = ucm::arg_ptr<const _Float16>(qk.y); a.pruned = ucm::arg_ptr<const int64_t>(early.x);
+    a.S = ucm::arg_lo(early.y); a.Hkv = ucm::arg_hi(early.y); a.Hq = n.x & 0xffff; a.g = n.x >> 16; a.d_orig = n.y;
+    a.tiles_q = n.z; a.items = n.w; a.X = X; a.d = KS * 16; a.tiles_k = (int)(a.S + 31) / 32;
     constexpr int kItems = stat_items(KS), kSubs = kThreads / 64 / kItems;
     constexpr int U = UNIT == 64 || KS <= 4 ? 2 : 1;
     constexpr int pitch = KS * 16 + 8;
@@ -679,32 +682,35 @@ __global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(KvArgs a)
 // unit's probability is its sum times exp(its maximum - the row's) over the row's sum, added up over the rows by the
 // sixteen lanes that hold them.
 template <int NT, int R>
-__global__ __launch_bounds__(NT) void kvstar_merge_kernel(KvArgs a)
+__global__ __launch_bounds__(NT) void kvstar_merge_kernel(ucm::ArgPair in_out, ucm::ArgInts n)
 {
+    const Stat* const part = ucm::arg_ptr<const Stat>(in_out.x);
+    float* const sums = ucm::arg_ptr<float>(in_out.y);
+    const int units = n.x, items = n.y, tiles_q = n.z, real_rows = n.w;
     constexpr int kGroups = NT / kMergeRows, kWaves = NT / 64;
     static_assert(kMergeRows == 16 && kWaves % 4 == 0, "a row of lanes");
     __shared__ Stat red[kWaves][kMergeRows];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = threadIdx.x % kMergeRows, grp = threadIdx.x / kMergeRows;
-    const int rows = a.items * 32, r0 = blockIdx.x * kMergeRows;
+    const int rows = items * 32, r0 = blockIdx.x * kMergeRows;
     const int item = r0 / 32;
     // rows of the item that exist: X * g of the KV head are cut into its tiles
-    const bool real = (item % a.tiles_q) * 32 + r0 % 32 + r < a.X * a.g;
-    const Stat* p = a.part + r0 + r;
+    const bool real = (item % tiles_q) * 32 + r0 % 32 + r < real_rows;
+    const Stat* p = part + r0 + r;
     Stat v[R];
     auto load = [&](int u0) {
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             const int u = u0 + grp + i * kGroups;
-            v[i] = p[(int64_t)(u < a.units ? u : a.units - 1) * rows];
+            v[i] = p[(int64_t)(u < units ? u : units - 1) * rows];
         }
 #pragma unroll
         for (int i = 0; i < R; ++i)
-            if (u0 + grp + i * kGroups >= a.units) v[i] = Stat{-INFINITY, 0.0f};
+            if (u0 + grp + i * kGroups >= units) v[i] = Stat{-INFINITY, 0.0f};
     };
     Stat st{-INFINITY, 0.0f};
     // one load: v[i].s becomes the unit's sum measured from the thread's own largest score
-    const bool held = a.units <= R * kGroups;
+    const bool held = units <= R * kGroups;
     if (held) {
         load(0);
 #pragma unroll
@@ -716,7 +722,7 @@ __global__ __launch_bounds__(NT) void kvstar_merge_kernel(KvArgs a)
             st.s += v[i].s;
         }
     } else {
-        for (int u0 = 0; u0 < a.units; u0 += R * kGroups) {
+        for (int u0 = 0; u0 < units; u0 += R * kGroups) {
             load(u0);
             st = merge(st, v);
         }
@@ -742,7 +748,7 @@ __global__ __launch_bounds__(NT) void kvstar_merge_kernel(KvArgs a)
     float inv = st.s > 1e-9f ? 1.0f / st.s : 1.0f;
     if (st.m == -INFINITY) inv = NAN;  // a row of minus infinities has no probabilities
     const float scale = own == st.m ? 1.0f : exp_small(own - st.m);
-    for (int u0 = 0; u0 < a.units; u0 += R * kGroups) {
+    for (int u0 = 0; u0 < units; u0 += R * kGroups) {
         if (!held) load(u0);
 #pragma unroll
         for (int i = 0; i < R; ++i) {
@@ -755,7 +761,7 @@ __global__ __launch_bounds__(NT) void kvstar_merge_kernel(KvArgs a)
             add(std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
             add(std::integral_constant<int, 0x141>{});  // row_half_mirror
             add(std::integral_constant<int, 0x140>{});  // row_mirror
-            if (r == 0 && u < a.units) a.sums[(int64_t)blockIdx.x * a.units + u] = e;
+            if (r == 0 && u < units) sums[(int64_t)blockIdx.x * units + u] = e;
         }
     }
 }
@@ -848,13 +854,19 @@ int launch_units(const KvArgs& a, hipStream_t st)
     const int64_t heads = ucm::ceil_div(a.items, stat_items(KS)), most = kUnitGroups / heads;
     const int64_t need = ucm::ceil_div(UNIT == 64 ? a.units : ucm::ceil_div(a.tiles_k, U), kSubs);
     const int64_t parts = need < most ? need : (most < 1 ? 1 : most);
-    hipLaunchKernelGGL((kvstar_unit_kernel<KS, UNIT>), dim3((unsigned)parts, (unsigned)heads), dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((kvstar_unit_kernel<KS, UNIT>), dim3((unsigned)parts, (unsigned)heads), dim3(kThreads), 0, st,
+                       ucm::arg_pair(a.q, a.k), ucm::arg_pair(a.pruned, ucm::arg_words((int)a.S, a.Hkv)),
+                       ucm::ArgInts{a.Hq | a.g << 16, a.d_orig, a.tiles_q, a.items}, a.X, a);
     int rc = ucm::launch_status("kvstar_unit_kernel");
     if (rc != UCM_OK) return rc;
     const dim3 grid((unsigned)(a.items * (32 / kMergeRows)));
-    if (a.units <= 256) hipLaunchKernelGGL((kvstar_merge_kernel<512, 8>), grid, dim3(512), 0, st, a);
-    else if (a.units <= 512) hipLaunchKernelGGL((kvstar_merge_kernel<1024, 8>), grid, dim3(1024), 0, st, a);
-    else hipLaunchKernelGGL((kvstar_merge_kernel<1024, 16>), grid, dim3(1024), 0, st, a);
+    auto launch = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, grid, dim3((unsigned)threads), 0, st, ucm::arg_pair(a.part, a.sums),
+                           ucm::ArgInts{a.units, a.items, a.tiles_q, a.X * a.g});
+    };
+    if (a.units <= 256) launch(kvstar_merge_kernel<512, 8>, 512);
+    else if (a.units <= 512) launch(kvstar_merge_kernel<1024, 8>, 1024);
+    else launch(kvstar_merge_kernel<1024, 16>, 1024);
     return ucm::launch_status("kvstar_merge_kernel");
 }
 
@@ -916,8 +928,7 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     if (a.units > 0 && !few && (d == 32 || d == 64 || d == 128)) {
         const int rc = d == 32 ? launch_units<2>(a, st) : d == 64 ? launch_units<4>(a, st) : launch_units<8>(a, st);
         if (rc != UCM_OK) return rc;
-        s.sums = a.sums; s.n_sums = a.items * (32 / kMergeRows);
-        return launch_rank_sums(s, st);
+        return launch_rank_sums(s, a.sums, a.items * (32 / kMergeRows), st);
     }
     const int rc = d == 32 ? launch_kvstar<2>(a, st)
                  : d == 64 ? launch_kvstar<4>(a, st)
