@@ -35,8 +35,7 @@ __device__ __forceinline__ float key_score(uint32_t k)
 __device__ __forceinline__ float key_place(uint32_t k)
 {
     const float big = 1.7e38f;
-    const float v = key_score(k);
-    return k == 1u ? -big : (v > big ? big : (v < -big ? -big : v));
+    return fminf(fmaxf(key_score(k), -big), big);  // a NaN, key 1, goes to the lower end
 }
 
 // Keys of a row lie at a pitch of whole 64-byte lines: every thread loads its keys as 16-byte pieces.
@@ -74,6 +73,18 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v)
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+// op over N neighbouring lanes (N = 4, 8 or 16, aligned), in every lane.
+template <int N, typename Op>
+__device__ __forceinline__ int row_reduce(int v, Op op)
+{
+    static_assert(N == 4 || N == 8 || N == 16, "lanes of a row");
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
+    if (N > 4) v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false));  // row_half_mirror
+    if (N > 8) v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, false));  // row_mirror
+    return v;
+}
+
 // Exclusive prefix sum of one int per thread over a workgroup of NT threads.
 template <int NT>
 __device__ __forceinline__ int scan_wg(int v, int* wsum, int* total)
@@ -89,15 +100,10 @@ __device__ __forceinline__ int scan_wg(int v, int* wsum, int* total)
     __syncthreads();
     if (lane == 63) wsum[w] = inc;
     __syncthreads();
-    int base = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) {
-        const int x = wsum[i];
-        if (i < w) base += x;
-        tot += x;
-    }
-    *total = tot;
-    return base + inc - v;
+    // a wave's sum a lane, the same in every 16 lanes (words in turn by all waves: 64 instructions instead of 16)
+    const int x = wsum[lane % (NT / 64)];
+    *total = row_reduce<NT / 64>(x, [](int p, int q) { return p + q; });
+    return row_reduce<NT / 64>(lane % (NT / 64) < w ? x : 0, [](int p, int q) { return p + q; }) + inc - v;
 }
 
 // What a score is output as: a NaN of one kind, whichever it was.
@@ -115,7 +121,7 @@ struct Bins {
     __device__ __forceinline__ int of(uint32_t k) const
     {
         const float at = (top - key_place(k)) * scale;  // not a number where the scale is infinite: bin 0
-        return at > 0.0f ? (int)(at < (float)(BINS - 1) ? at : (float)(BINS - 1)) : 0;
+        return (int)fminf(fmaxf(at, 0.0f), (float)(BINS - 1));
     }
 };
 
@@ -141,7 +147,8 @@ struct Direct {
     unsigned long long* win;  // NT + kCrowd entries
     int* wsum;
     uint32_t (*range)[NT / 64];
-    int* s_int;               // ends of the bins in front of this workgroup's places and of its own; first and last crowded bin
+    int* s_int;               // ends of the bins in front of this workgroup's places and of its own; first and last crowded bin;
+                              // a bit for every division that has one
     const int b, tid, lane, w;
     // an entry's bin, counted through all divisions, and its place in the bin << 16; in one word where 16 keys
     // leave no registers for two (at 8 keys and less two words are 0.2 us faster)
@@ -183,12 +190,9 @@ struct Direct {
             range[1][w] = l;
         }
         __syncthreads();
-#pragma unroll
-        for (int i = 0; i < NT / 64; ++i) {
-            hi = range[0][i] > hi ? range[0][i] : hi;
-            l = range[1][i] > l ? range[1][i] : l;
-        }
-        lo = ~l;
+        auto most = [](int p, int q) { return (int)max((uint32_t)p, (uint32_t)q); };
+        hi = (uint32_t)row_reduce<NT / 64>((int)range[0][lane % (NT / 64)], most);
+        lo = ~(uint32_t)row_reduce<NT / 64>((int)range[1][lane % (NT / 64)], most);
     }
 
     // The counts of a division's bins turned into (first place << 16 | entries) words; both fit: a row on this
@@ -212,7 +216,9 @@ struct Direct {
         }
         *mine = make_uint4(packed[0], packed[1], packed[2], packed[3]);
         if (division == 0) mark_ends(packed, 0, 1, 0);
-        return __syncthreads_or(crowded);
+        if (crowded) atomicOr(&s_int[4], 1 << division);
+        __syncthreads();
+        return s_int[4] >> division & 1;
     }
 
     // First and last crowded bin of a division, behind a barrier.
@@ -262,11 +268,13 @@ struct Direct {
     {
         int lo_at, hi_at;
         share(lo_at, hi_at);
+        int at_bin[PER];  // all read in front of the first write (a key that is none has some bin, too)
+#pragma unroll
+        for (int e = 0; e < PER; ++e) at_bin[e] = (int)(bins[bin(e)] >> 16);
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            if (kreg[e] == 0u) continue;
-            const int f = (int)(bins[bin(e)] >> 16);
-            if (f >= lo_at && f < hi_at) win[f - lo_at + place_of(e)] = ((unsigned long long)kreg[e] << 32) | (uint32_t)(~(uint32_t)(tid * PER + e));
+            const int f = at_bin[e];
+            if (kreg[e] != 0u && f >= lo_at && f < hi_at) win[f - lo_at + place_of(e)] = ((unsigned long long)kreg[e] << 32) | (uint32_t)(~(uint32_t)(tid * PER + e));
         }
         __syncthreads();
         const int end = s_int[1];
@@ -278,7 +286,13 @@ struct Direct {
             const uint32_t p = bins[bin_of(k)];
             const int f = (int)(p >> 16), n = (int)(p & 0xffffu);
             int rank = f;  // entries of the bin that go before this one come first
-            for (int j = 0; j < n; ++j) rank += win[f - lo_at + j] > x;
+            for (int j = 0; j < n; j += 4) {  // four a round trip, places past the bin's last repeat it
+                unsigned long long o[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) o[u] = win[f - lo_at + (j + u < n ? j + u : n - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) rank += j + u < n && o[u] > x;
+            }
             if (rank < kk) {
                 a.out_idx[(int64_t)b * a.topk + rank] = id;
                 a.out_score[(int64_t)b * a.topk + rank] = out_of(k);
@@ -293,7 +307,7 @@ struct Direct {
     __device__ __forceinline__ bool run()
     {
         reinterpret_cast<uint4*>(bins)[tid] = make_uint4(0u, 0u, 0u, 0u);
-        if (tid < 4) s_int[tid] = tid == 2 ? (1 + kAgain) * kBins : (tid == 3 ? -1 : 0);
+        if (tid < 5) s_int[tid] = tid == 2 ? (1 + kAgain) * kBins : (tid == 3 ? -1 : 0);
         uint32_t hi, lo;
         range_of([](int) { return true; }, hi, lo);
         const Bins<kBins> whole(hi, lo);
@@ -314,9 +328,20 @@ struct Direct {
                 else if (kreg[e] != 0u) set(e, (uint32_t)bin(e), atomicAdd(&bins[bin(e)], 1u));
             }
         } else {
+            bool all = true;
 #pragma unroll
-            for (int e = 0; e < PER; ++e)
-                if (kreg[e] != 0u) set(e, (uint32_t)bin(e), atomicAdd(&bins[bin(e)], 1u));
+            for (int e = 0; e < PER; ++e) all &= kreg[e] != 0u;
+            if (__ballot(all) == ~0ull) {  // no test between the additions: they are one round trip
+                uint32_t place[PER];
+#pragma unroll
+                for (int e = 0; e < PER; ++e) place[e] = atomicAdd(&bins[bin(e)], 1u);
+#pragma unroll
+                for (int e = 0; e < PER; ++e) set(e, (uint32_t)bin(e), place[e]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < PER; ++e)
+                    if (kreg[e] != 0u) set(e, (uint32_t)bin(e), atomicAdd(&bins[bin(e)], 1u));
+            }
         }
         __syncthreads();
         uint32_t packed[4];
@@ -780,7 +805,7 @@ __global__ __launch_bounds__(NT) void topk_kernel(SORT_ARGS)
     extern __shared__ __align__(16) uint32_t lds[];
     __shared__ int wsum[NT / 64];
     __shared__ uint32_t range[2][NT / 64];
-    __shared__ int s_int[4];
+    __shared__ int s_int[5];
     if constexpr (PER > 0) {
         static_assert(PER % 4 == 0, "16-byte loads");
         uint32_t kreg[PER];
