@@ -680,11 +680,11 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
 
 // Short rows: every candidate counts those that come before it in the output order (larger key, or equal key
 // and earlier position) and writes itself at that rank.  Its time does not depend on the values.  A workgroup
-// ranks 64 candidates; its waves compare them with every so many 64 entries of the row, which a wave holds
-// in a register and hands round lane by lane.  grid = (rows, ceil(max_n / 64)).
+// ranks 64 candidates; its waves compare them with every so many 64 entries of the row.  grid = (rows, ceil(max_n / 64)).
 template <int WAVES>
 struct RankShared {
-    int part[WAVES][64], valid[WAVES];
+    __attribute__((aligned(16))) uint32_t key[WAVES][64];
+    uint32_t part[WAVES][64];  // ranks among a wave's entries, and in the upper half how many of them there are
 };
 
 // mine: the lane's candidate of the workgroup; first: of the wave's first 64, where has_first says that it is known.
@@ -699,31 +699,40 @@ __device__ __forceinline__ void rank_places(const SortArgs& a, int waves, uint32
     for (int piece = w; piece * 64 < a.max_n; piece += waves) {
         const uint32_t k = has_first && piece == w ? first : key_of(piece * 64 + lane);
         have += __popcll(__ballot(k != 0u));
-        if (piece == mine_at) {
+        // A wave's keys go round by way of LDS, four to a read that all lanes share (lane by lane through a scalar
+        // register: 0.1 us more), eight to a step of the loop: code is fetched anew by every
+        // launch, and all 64 are 2 to 4 KB of it.
+        sh.key[w][lane] = k;
+        __builtin_amdgcn_wave_barrier();
+        const uint4* all = reinterpret_cast<const uint4*>(sh.key[w]);
+        auto count = [&](auto own_) {
+#pragma unroll 2
+            for (int j = 0; j < 64; j += 4) {
+                const uint4 o4 = all[j / 4];
+                const uint32_t o[4] = {o4.x, o4.y, o4.z, o4.w};
 #pragma unroll
-            for (int j = 0; j < 64; ++j) {
-                const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)k, j);
-                rank += o > mine || (o == mine && j < lane);
+                for (int i = 0; i < 4; ++i) {
+                    if constexpr (decltype(own_)::value) rank += o[i] > mine || (o[i] == mine && j + i < lane);
+                    // equal keys come first where they lie in front: o >= mine is o > mine - 1 (mine is 0 for nothing only)
+                    else rank += o[i] > mine - (piece < mine_at ? 1u : 0u);
+                }
             }
-        } else {
-            // equal keys come first where they lie in front: o >= mine is o > mine - 1 (mine is 0 for nothing only)
-            const uint32_t above = mine - (piece < mine_at ? 1u : 0u);
-#pragma unroll
-            for (int j = 0; j < 64; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)k, j) > above;
-        }
+        };
+        if (piece == mine_at) count(std::true_type{});
+        else count(std::false_type{});
+        __builtin_amdgcn_wave_barrier();
     }
-    sh.part[w][lane] = rank;
-    if (lane == 0) sh.valid[w] = have;
+    sh.part[w][lane] = (uint32_t)rank | (uint32_t)have << 16;
     __syncthreads();
     if (w != 0) return;
-    rank = 0;
-    int n_valid = 0;
+    uint32_t sum = 0;
 #pragma unroll
     for (int i = 0; i < WAVES; ++i) {
-        if (i >= waves) break;
-        rank += sh.part[i][lane];
-        n_valid += sh.valid[i];
+        const uint32_t p = sh.part[i][lane];
+        sum += i < waves ? p : 0u;
     }
+    rank = (int)(sum & 0xffffu);
+    const int n_valid = (int)(sum >> 16);
     if (mine != 0u && rank < a.topk) {
         a.out_idx[(int64_t)b * a.topk + rank] = id;
         a.out_score[(int64_t)b * a.topk + rank] = out_of(mine);

@@ -18,9 +18,9 @@
 //   * Everything else: kvstar_stats_kernel (maximum and sum of exponentials of every row over one chunk of the
 //     representatives), kvstar_mass_kernel (the chunks' pairs merged, q.k once more, probabilities summed over rows
 //     and a block's representatives) and the shared top-k selection.
-// 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 13.5 us (6.0, 4.0 and 4.1 of the three
+// 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 13.0 us (5.9, 4.0 and 3.8 of the three
 // kernels: launches and round trips; the products and exponentials are about 1.5), 18.8 the second way
-// (7.5, 9.0, 3.7); 1024 blocks, 128 channels: 42.9 and 70.4, the second way reads the keys twice.
+// (7.5, 9.0, 3.7); 1024 blocks, 128 channels: 41 and 70.4, the second way reads the keys twice.
 // Sums are taken in a different order than the reference's loops, the same one on every call (no
 // atomics); the tolerance is stated where the results are compared.  Equal scores come out in
 // ascending block order (the reference's heap pops them in descending block order).
@@ -104,11 +104,12 @@ struct QRow {
 
 __device__ __forceinline__ QRow q_row(const KvArgs& a, int item, int r)
 {
-    const int h = item / a.tiles_q;
+    const int h = a.tiles_q == 1 ? item : item / a.tiles_q;
     const int rr = (item - h * a.tiles_q) * 32 + r;
+    const int x = (a.g & (a.g - 1)) == 0 ? rr >> __builtin_ctz(a.g) : rr / a.g;  // (a division is forty instructions)
     QRow q;
     q.ok = item < a.items && rr < a.X * a.g;
-    q.row = a.q + ((int64_t)(q.ok ? rr / a.g : 0) * a.Hq + (q.ok ? h * a.g + rr % a.g : 0)) * a.d_orig;
+    q.row = a.q + ((int64_t)(q.ok ? x : 0) * a.Hq + (q.ok ? h * a.g + rr - x * a.g : 0)) * a.d_orig;
     q.pruned = a.pruned ? a.pruned + (int64_t)(q.ok ? h : 0) * a.d : nullptr;
     return q;
 }
@@ -237,21 +238,32 @@ __global__ __launch_bounds__(kThreads) void kvstar_pack_kernel(KvArgs a)
     *reinterpret_cast<f16x8*>(a.qp + row * a.dp + c) = load_q(q_row(a, (int)(row >> 5), (int)(row & 31)), c, a.d, a.d_orig);
 }
 
-// The query rows of a workgroup's two items into LDS, eight threads per row, each taking every eighth channel.
+// The query rows of a workgroup's two items into LDS, eight threads per row, each taking every eighth channel, in two
+// parts: the channels' numbers are asked for in front of the keys, so that waiting for them is not waiting for those.
 template <int KS>
-__device__ __forceinline__ void gather_rows(const KvArgs& a, _Float16* qt, int pitch)
-{
-    const int rl = threadIdx.x >> 3;  // 0 .. 63: row rl % 32 of the workgroup's item rl / 32
-    const QRow q = q_row(a, blockIdx.y * stat_items(KS) + (rl >> 5), rl & 31);
+struct Gather {
+    QRow q;
+    int rl;
     int64_t src[2 * KS];
-    _Float16 v[2 * KS];
+    __device__ __forceinline__ explicit Gather(const KvArgs& a)
+    {
+        rl = threadIdx.x >> 3;  // 0 .. 63: row rl % 32 of the workgroup's item rl / 32
+        q = q_row(a, blockIdx.y * stat_items(KS) + (rl >> 5), rl & 31);
 #pragma unroll
-    for (int i = 0; i < 2 * KS; ++i) src[i] = q_channel(q, (threadIdx.x & 7) + 8 * i, a.d_orig);
+        for (int i = 0; i < 2 * KS; ++i) {
+            const int j = (threadIdx.x & 7) + 8 * i;
+            src[i] = q.pruned ? q.pruned[j] : j;
+        }
+    }
+    __device__ __forceinline__ void rows(const KvArgs& a, _Float16* qt, int pitch) const
+    {
+        _Float16 v[2 * KS];
 #pragma unroll
-    for (int i = 0; i < 2 * KS; ++i) v[i] = q.row[src[i]];
+        for (int i = 0; i < 2 * KS; ++i) v[i] = q.row[src[i] < 0 ? 0 : (src[i] >= a.d_orig ? a.d_orig - 1 : src[i])];
 #pragma unroll
-    for (int i = 0; i < 2 * KS; ++i) qt[rl * pitch + (threadIdx.x & 7) + 8 * i] = q.ok ? v[i] : (_Float16)0;
-}
+        for (int i = 0; i < 2 * KS; ++i) qt[rl * pitch + (threadIdx.x & 7) + 8 * i] = q.ok ? v[i] : (_Float16)0;
+    }
+};
 
 // grid = (chunks, ceil(items / kItems)).  Wave w serves row tile w % kItems and every
 // kSubs-th tile of representatives of the chunk.  Representatives are the A operand (lane:
@@ -296,8 +308,9 @@ __global__ __launch_bounds__(kThreads) void kvstar_stats_kernel(KvArgs a)
         }
     };
     if constexpr (KS > 0) {
+        const Gather<KS> gather(a);
         load_tiles(t0 < a.tiles_k ? t0 : 0);
-        gather_rows<KS>(a, qt, pitch);
+        gather.rows(a, qt, pitch);
     } else if constexpr (KS == kAnyDim) {
         const _Float16* row = k_row(t0 < a.tiles_k ? t0 : 0);
 #pragma unroll
@@ -607,7 +620,7 @@ __global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(ucm::ArgPair qk, 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = wave % kItems, sub = wave / kItems;
     const int item = blockIdx.y * kItems + li;
-    const int h = item < a.items ? item / a.tiles_q : 0;
+    const int h = item < a.items ? (a.tiles_q == 1 ? item : item / a.tiles_q) : 0;
     const int kb = (lane >> 5) * 8;
     const int rows = a.items * 32;
     const int per = UNIT == 64 ? a.M / 64 : 1;  // steps of two tiles to a block
@@ -624,8 +637,9 @@ __global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(ucm::ArgPair qk, 
             for (int c = 0; c < KS; ++c) kk[u][c] = *reinterpret_cast<const f16x8*>(row + c * 16 + kb);
         }
     };
+    const Gather<KS> gather(a);
     load_tiles(p0 < steps ? p0 * per : 0);
-    gather_rows<KS>(a, qt, pitch);
+    gather.rows(a, qt, pitch);
     __syncthreads();
     Stat* out = a.part + item * 32 + (lane & 31);
     Stat sofar{-INFINITY, 0.0f};
