@@ -768,7 +768,7 @@ __global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SORT_ARGS)
     a.idx = nullptr;
     auto keys_of = [&](auto n_, const int (&at)[decltype(n_)::value], uint32_t (&key)[decltype(n_)::value]) {
         constexpr int N = decltype(n_)::value;
-        float s[N] = {};
+        double s[N] = {};  // sixteen parts one after the other in 32 bits were the largest error of a block's score
         uint32_t off[N];
 #pragma unroll
         for (int n = 0; n < N; ++n) off[n] = at[n] < max_n ? at[n] : max_n - 1;
@@ -784,10 +784,10 @@ __global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SORT_ARGS)
 #pragma unroll
             for (int e = 0; e < 16; ++e)
 #pragma unroll
-                for (int n = 0; n < N; ++n) s[n] += i + e < n_sums ? v[n][e] : 0.0f;
+                for (int n = 0; n < N; ++n) s[n] += i + e < n_sums ? (double)v[n][e] : 0.0;
         }
 #pragma unroll
-        for (int n = 0; n < N; ++n) key[n] = at[n] < max_n ? score_key(s[n]) : 0u;
+        for (int n = 0; n < N; ++n) key[n] = at[n] < max_n ? score_key((float)s[n]) : 0u;
     };
     const int lane = threadIdx.x & 63;
     const int at[2] = {(int)blockIdx.y * 64 + lane, (int)threadIdx.x};

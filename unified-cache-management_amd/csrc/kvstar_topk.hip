@@ -21,6 +21,8 @@
 // 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 13.0 us (5.9, 4.0 and 3.8 of the three
 // kernels: launches and round trips; the products and exponentials are about 1.5), 18.8 the second way
 // (7.5, 9.0, 3.7); 1024 blocks, 128 channels: 41 and 70.4, the second way reads the keys twice.
+// Error against 64 bits at that shape 3.3e-8 of the scores' 2-norm (the second way 4.7e-8), over thirteen others from 24 to
+// 1024 blocks 2.6e-8 to 2.0e-7 (3.7e-8 to 1.9e-7).
 // Sums are taken in a different order than the reference's loops, the same one on every call (no
 // atomics); the tolerance is stated where the results are compared.  Equal scores come out in
 // ascending block order (the reference's heap pops them in descending block order).
