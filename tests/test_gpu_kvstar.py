@@ -221,6 +221,18 @@ def test_blocks_whose_scores_are_taken_once(X, Hq, Hkv, d, n, M):
     assert np.all(np.abs(gs - ref[gi]) <= RTOL * ref[gi] + 2e-45)
 
 
+@pytest.mark.parametrize("Hq,n", [(32767, 4), (32768, 8), (40000, 4), (65535, 3)])
+def test_as_many_heads_to_a_group_as_are_taken(Hq, n):
+    """Group sizes on both sides of 2^15 and the largest, against float64: blocks of very different mass."""
+    q, k = make(Hq, 1, Hq, 1, 32, n, 16)
+    k *= np.arange(1, n + 1, dtype=np.float16)[:, None, None, None] * np.float16(0.5)
+    gi, gs = run_gpu(q, k, None, n)
+    ref = brute.kvstar_block_scores(q, k)
+    assert np.ptp(ref) > 0.1 * ref.mean()
+    assert gi.tolist() == np.argsort(-ref, kind="stable").tolist()
+    assert np.all(np.abs(gs - ref[gi]) <= RTOL * ref[gi])
+
+
 @pytest.mark.parametrize("M", [16, 32, 128])
 @pytest.mark.parametrize("what", ["nan", "+inf", "-inf", "nan_lane", "all_-inf"])
 def test_infinite_and_undefined_scores_taken_once(what, M):

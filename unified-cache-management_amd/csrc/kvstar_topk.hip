@@ -613,7 +613,7 @@ template <int KS, int UNIT>
 __global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(ucm::ArgPair qk, ucm::ArgPair early, ucm::ArgInts n, int X, KvArgs a)
 {
     a.q = ucm::arg_ptr<const _Float16>(qk.x); a.k = ucm::arg_ptr<const _Float16>(qk.y); a.pruned = ucm::arg_ptr<const int64_t>(early.x);
-    a.S = ucm::arg_lo(early.y); a.Hkv = ucm::arg_hi(early.y); a.Hq = n.x & 0xffff; a.g = n.x >> 16; a.d_orig = n.y;
+    a.S = ucm::arg_lo(early.y); a.Hkv = ucm::arg_hi(early.y); a.Hq = n.x & 0xffff; a.g = (int)((uint32_t)n.x >> 16); a.d_orig = n.y;
     a.tiles_q = n.z; a.items = n.w; a.X = X; a.d = KS * 16; a.tiles_k = (int)(a.S + 31) / 32;
     constexpr int kItems = stat_items(KS), kSubs = kThreads / 64 / kItems;
     constexpr int U = UNIT == 64 || KS <= 4 ? 2 : 1;
@@ -872,7 +872,7 @@ int launch_units(const KvArgs& a, hipStream_t st)
     const int64_t parts = need < most ? need : (most < 1 ? 1 : most);
     hipLaunchKernelGGL((kvstar_unit_kernel<KS, UNIT>), dim3((unsigned)parts, (unsigned)heads), dim3(kThreads), 0, st,
                        ucm::arg_pair(a.q, a.k), ucm::arg_pair(a.pruned, ucm::arg_words((int)a.S, a.Hkv)),
-                       ucm::ArgInts{a.Hq | a.g << 16, a.d_orig, a.tiles_q, a.items}, a.X, a);
+                       ucm::ArgInts{(int)((uint32_t)a.Hq | (uint32_t)a.g << 16), a.d_orig, a.tiles_q, a.items}, a.X, a);  // X * Hq <= 65535
     int rc = ucm::launch_status("kvstar_unit_kernel");
     if (rc != UCM_OK) return rc;
     const dim3 grid((unsigned)(a.items * (32 / kMergeRows)));
