@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "exp_sum.h"
 #include "float_topk.h"
 
 namespace {
@@ -133,7 +134,6 @@ __device__ __forceinline__ f16x8 load_q(const QRow& q, int c, int d, int d_orig)
 }
 
 constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596303e-8f;  // log2(e) in two pieces
-constexpr float kLn2 = 0.693147182f;
 
 // exp(x) for x far from overflow (here x <= 0 but for rounding): 2^(x log2 e) with log2 e in two pieces and the
 // product's rounding error carried along (Dekker's exact product, by a fused multiply-add), whole and fractional
@@ -145,18 +145,6 @@ __device__ __forceinline__ float exp_small(float x)
     const float n = __builtin_rintf(t);
     const float r = __builtin_fmaf(x, kLog2eLow, __builtin_fmaf(x, kLog2e, -t));
     return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - n) + r), (int)n);
-}
-
-// exp(x) as a term of a sum that holds a 1, in seven instructions instead of twelve (the unit kernel's launch of the
-// example's shape 5.9 us with it, 6.7 with exp_small): what lies below 2^-126 may be 0.  exp2's argument is rounded, and what
-// the rounding took (x - t ln 2, by a fused multiply-add) is put back to first order; ln 2's own rounding moves a
-// result by 1.9e-9 |t| of itself.
-__device__ __forceinline__ float exp_term(float x)
-{
-    x = __builtin_elementwise_maximum(x, -200.0f);
-    const float t = x * kLog2e;
-    const float e = __builtin_amdgcn_exp2f(t);
-    return __builtin_fmaf(e, __builtin_fmaf(-t, kLn2, x), e);
 }
 
 // What a part's maximum is measured from: 0 where the largest one is minus infinity, whose exponentials are 0.
@@ -182,6 +170,14 @@ __device__ __forceinline__ Stat merge(Stat st, const Stat (&v)[N], int count = N
 #pragma unroll
     for (int i = 0; i < N; ++i) sum += i < count ? v[i].s * part_weight(v[i].m - base) : 0.0f;
     return Stat{m, sum};
+}
+
+// Two parts of a sum that is not a row's but a block's, where its own size is what is asked for: an exact weight.
+__device__ __forceinline__ Stat join(Stat a, Stat b)
+{
+    const float m = fmaxf(a.m, b.m);
+    const float w = exp_small(fminf(a.m, b.m) - stat_base(m));
+    return Stat{m, a.m < b.m ? a.s * w + b.s : a.s + b.s * w};
 }
 
 // Any head dimension: U tiles of representatives against a row tile, up to eight k-steps' loads in flight (16
@@ -665,19 +661,16 @@ __global__ __launch_bounds__(kThreads) void kvstar_unit_kernel(ucm::ArgPair qk, 
             m = fmaxf(m, __shfl_xor(m, 32));
             // minus infinities alone measure from 0 and add 0; a NaN, which the maximum passes over, makes the sum one
             const float base = stat_base(m);
-            float s = 0.0f;
+            ucm::ExpSum sum;
 #pragma unroll
-            for (int v = 0; v < n; ++v) s += exp_term(get(v) - base);
+            for (int v = 0; v < n; ++v)
+                sum.add(__builtin_elementwise_maximum(get(v) - base, -200.0f), [](float t) { return __builtin_amdgcn_exp2f(t); });
+            const float s = sum.sum();
             return Stat{m, s + __shfl_xor(s, 32)};
         };
         if constexpr (UNIT == 64) {
             const Stat st = pair_of([&](int v) { return acc[v / 16][v % 16]; }, 32);
-            if (per > 1) {
-                const Stat other[1] = {st};
-                sofar = merge(q == 0 ? Stat{-INFINITY, 0.0f} : sofar, other);
-            } else {
-                sofar = st;
-            }
+            sofar = q == 0 ? st : join(sofar, st);
             if (lane < 32 && q == per - 1) out[(int64_t)p * rows] = sofar;
         } else {
             constexpr int N = UNIT / 2, kPer = 32 / UNIT;
