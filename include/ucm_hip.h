@@ -567,6 +567,10 @@ int ucm_dot_topk(const float* data, int64_t n_items, int32_t dim, const float* q
  * score[n] = sum of p over x, H and the M representatives of block n.
  * out_idx / out_score  [topk]: blocks by descending score, -1 / 0 past n_blocks; equal scores
  *               in ascending block order.  topk <= 4096, d <= 1024, X * Hq <= 65535.
+ * workspace     The size is a shape's own and does not only grow with it: ask for every shape that is
+ *               called.  A buffer asked for at the largest X, Hq, n_blocks and M is accepted for all
+ *               smaller ones too, but may leave out the faster of the call's two ways where that
+ *               one's parts do not fit (scores then differ by rounding).
  */
 size_t ucm_kvstar_topk_workspace_bytes(int32_t X, int32_t Hq, int64_t n_blocks, int32_t M);
 int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t d_orig,

@@ -245,6 +245,32 @@ def test_scores_of_any_finite_size_taken_once(base, d, M):
     test_scores_of_any_finite_size(base, d, M)
 
 
+@pytest.mark.parametrize("asked,called", [
+    ((8, 32, 2049, 64), (8, 32, 8, 32, 2048, 64)),   # one block less, and the blocks' products are taken once
+    ((8, 32, 2049, 64), (8, 32, 8, 32, 300, 64)), ((8, 32, 513, 48), (8, 32, 8, 32, 513, 32)),
+    ((16, 64, 2000, 64), (1, 64, 8, 32, 2000, 64)),  # fewer query tokens
+    ((8, 32, 2000, 64), (8, 32, 8, 32, 2000, 64)), ((2, 4, 257, 32), (2, 4, 1, 512, 256, 32)),
+    ((2, 4, 129, 64), (2, 4, 2, 256, 128, 64)),      # 65 chunks of four tiles would be asked for, in fives they are 52
+])
+def test_a_buffer_asked_for_at_a_larger_shape(asked, called):
+    """The C call takes it, answers rightly and writes nothing behind it."""
+    from ucm_amd import _lib
+
+    X, Hq, Hkv, d, n, M = called
+    size = _lib.lib().ucm_kvstar_topk_workspace_bytes(*asked)
+    q, k = make(n, X, Hq, Hkv, d, n, M, scale=0.5 if d < 200 else 0.2)
+    tq, tk = torch.from_numpy(q).cuda(), torch.from_numpy(k).cuda()
+    ws = torch.full((size + 4096,), 0x5a, dtype=torch.uint8, device="cuda")
+    idx, sc = torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, dtype=torch.float32, device="cuda")
+    rc = _lib.lib().ucm_kvstar_topk(tq.data_ptr(), X, Hq, d, tk.data_ptr(), n, M, Hkv, d, None, n, idx.data_ptr(), sc.data_ptr(),
+                                    ws.data_ptr(), size, _lib.stream_ptr(tq.device))
+    _lib.check(rc)
+    ref = brute.kvstar_block_scores(q, k)
+    gi, gs = idx.cpu().numpy(), sc.cpu().numpy()
+    assert sorted(gi.tolist()) == list(range(n)) and np.all(np.abs(gs - ref[gi]) <= ATOL + RTOL * ref[gi])
+    assert bool((ws[size:] == 0x5a).all())
+
+
 def test_long_rows_in_two_batches_of_statistics():
     # 2560 query rows; against float64, as the checker adds a block's 102,400 probabilities one by one
     q, k = make(40, 40, 64, 2, 130, 9, 40, scale=0.5)

@@ -45,6 +45,7 @@ constexpr int kEarly = 8;           // k-steps that kernels for any dimension re
 constexpr int kEarlyMost = 256;     // in rows up to this (512 channels, 16 representatives: 0.8 us more with it)
 constexpr int kLongDim = 128;       // above it loads take more of both kernels' time than the statistics' merging
 constexpr int kMaxChunks = 64;      // partial statistics per row
+constexpr int kLeastTiles = 4;      // tiles of a chunk
 constexpr int kMassRows = 2048;     // rows whose statistics the mass kernel holds in LDS at a time
 constexpr int kMassGroups = 512;    // its workgroups at most
 constexpr int kMergeRows = 16;      // query rows of a workgroup of the merge kernel
@@ -792,7 +793,7 @@ void plan_chunks(KvArgs& a)
     // 64 blocks of 16, two heads: 19.2 and 17.0).
     const bool longer = a.d > kLongDim;
     a.per_chunk = (int)ucm::ceil_div(a.tiles_k, kMaxChunks);
-    if (a.per_chunk < (longer ? 4 : 8)) a.per_chunk = longer ? 4 : 8;
+    if (a.per_chunk < (longer ? kLeastTiles : 8)) a.per_chunk = longer ? kLeastTiles : 8;
     a.chunks = (int)ucm::ceil_div(a.tiles_k, a.per_chunk);
     a.group_blocks = a.M >= 32 ? 1 : 32 / a.M;
     if (longer)
@@ -800,35 +801,42 @@ void plan_chunks(KvArgs& a)
     a.groups = (int)ucm::ceil_div(a.n_blocks, a.group_blocks);
 }
 
+// Query rows with their padding, for every number of KV heads: at most 31 rows of it to each.
+int64_t padded_rows(const KvArgs& a) { return (int64_t)a.Hq * (a.X + 31); }
+
 // Whether the blocks are units: whole halves, ones or pairs of tiles, so that a wave has all of a block's scores.
 // A pair is 8 bytes for every row, written and read, where the second way reads a block's keys and takes its products
 // again: at 16 representatives of 32 channels that is even (256 rows, 1024 blocks 20.5 and 21.4 us, 2040: 27.7 and
-// 27.5), at 64 it never is (2000: 39.3 and 53.8).  Blocks of 48 in units of 16: 20.5 and 18.0.  `rows` bounds the padded query rows for every number of KV heads, so that the
-// workspace's size decides like the call.
-void plan_units(KvArgs& a, int64_t rows)
+// 27.5), at 64 it never is (2000: 39.3 and 53.8).  Blocks of 48 in units of 16: 20.5 and 18.0.
+void plan_units(KvArgs& a)
 {
     const bool whole = a.M == 16 || a.M == 32 || (a.M % 64 == 0 && a.M <= 256);
     const int most = a.M == 16 ? 1024 : kRankSums;
-    a.units = whole && a.n_blocks <= most && a.n_blocks * rows * 8 <= kUnitBytes ? a.n_blocks : 0;
+    a.units = whole && a.n_blocks <= most && a.n_blocks * padded_rows(a) * 8 <= kUnitBytes ? a.n_blocks : 0;
 }
 
-// Addresses of the workspace's parts; the sizes hold for every number of KV heads and every head
-// dimension (the caller asks with neither).
-size_t carve_kvstar(KvArgs& a, void* base)
+// Addresses of the workspace's parts, of the second way with `chunks` chunks and of the units for `rows` rows.
+size_t carve_kvstar(KvArgs& a, void* base, int chunks)
 {
-    const size_t rows = (size_t)a.Hq * (a.X + 31);  // at most 31 rows of padding per KV head
-    plan_units(a, (int64_t)rows);
+    const size_t rows = (size_t)padded_rows(a);
     char* p = (char*)base;
     size_t off = 0;
     a.qp = (_Float16*)(p + off);
     off += align256(rows * kMaxDim * 2);
     a.part = (Stat*)(p + off);
-    off += align256((size_t)(a.chunks > a.units ? a.chunks : a.units) * rows * 8);
-    a.sums = (float*)(p + off);
-    off += align256(ucm::ceil_div((int64_t)rows, kMergeRows) * (size_t)a.units * 4);
+    off += align256((size_t)chunks * rows * 8);
     a.keys = (uint32_t*)(p + off);
     off += align256((size_t)key_pitch(a.n_blocks) * 4);
     return off;
+}
+
+size_t carve_units(KvArgs& a, void* base, int64_t rows)
+{
+    char* p = (char*)base;
+    a.part = (Stat*)p;
+    const size_t off = align256((size_t)a.units * rows * 8);
+    a.sums = (float*)(p + off);
+    return off + align256(ucm::ceil_div(rows, kMergeRows) * (size_t)a.units * 4);
 }
 
 template <int KS>
@@ -892,9 +900,12 @@ extern "C" size_t ucm_kvstar_topk_workspace_bytes(int32_t X, int32_t Hq, int64_t
     if (X <= 0 || Hq <= 0 || n_blocks <= 0 || M <= 0) return 256;
     if (n_blocks > INT32_MAX || n_blocks * M > INT32_MAX) return 256;  // refused by the call
     KvArgs a{};
-    a.X = X; a.Hq = Hq; a.n_blocks = (int)n_blocks; a.M = M; a.d = kMaxDim;
-    plan_chunks(a);
-    return carve_kvstar(a, nullptr);
+    a.X = X; a.Hq = Hq; a.n_blocks = (int)n_blocks; a.M = M;
+    plan_units(a);
+    // the most chunks that any dimension has for as many representatives or fewer
+    const int64_t chunks = ucm::ceil_div(ucm::ceil_div(n_blocks * M, 32), kLeastTiles);
+    const size_t general = carve_kvstar(a, nullptr, (int)(chunks < kMaxChunks ? chunks : kMaxChunks)), units = carve_units(a, nullptr, padded_rows(a));
+    return general > units ? general : units;
 }
 
 extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t d_orig,
@@ -917,8 +928,6 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     const int64_t rows = (int64_t)X * Hq;
     // row tiles are a grid dimension; the second bound is the entry point's own, no index comes near it
     UCM_REQUIRE(rows <= 65535 && rows * M <= INT32_MAX, "too many query rows");
-    UCM_REQUIRE(workspace && workspace_bytes >= ucm_kvstar_topk_workspace_bytes(X, Hq, n_blocks, M),
-                "workspace too small");
     UCM_REQUIRE((((uintptr_t)blk_repre | (uintptr_t)workspace) & 15) == 0, "block representatives must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
     KvArgs a{};
@@ -927,18 +936,24 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     a.n_blocks = (int)n_blocks; a.M = M;
     a.tiles_q = (int)ucm::ceil_div((int64_t)X * a.g, 32);
     a.items = Hkv * a.tiles_q;
+    plan_units(a);
+    a.d = kMaxDim;  // as much for every dimension
     plan_chunks(a);
-    carve_kvstar(a, workspace);
+    UCM_REQUIRE(workspace && workspace_bytes >= carve_kvstar(a, nullptr, a.chunks), "workspace too small");
+    a.d = d;
+    plan_chunks(a);
     SortArgs s{};
     s.max_n = (int)n_blocks; s.topk = topk;
     s.out_idx = out_idx; s.out_score = out_score;
     // few row tiles leave the merging to few workgroups (four, 600 blocks of 16 x 32 channels: 18.6 and 17.0 us)
     const bool few = M == 16 && d == 32 && a.items < 8;
-    if (a.units > 0 && !few && (d == 32 || d == 64 || d == 128)) {
+    // (a buffer that only the second way fits into, one asked for at another shape, is taken by it)
+    if (a.units > 0 && !few && (d == 32 || d == 64 || d == 128) && carve_units(a, workspace, (int64_t)a.items * 32) <= workspace_bytes) {
         const int rc = d == 32 ? launch_units<2>(a, st) : d == 64 ? launch_units<4>(a, st) : launch_units<8>(a, st);
         if (rc != UCM_OK) return rc;
         return launch_rank_sums(s, a.sums, a.items * (32 / kMergeRows), st);
     }
+    carve_kvstar(a, workspace, a.chunks);
     const int rc = d == 32 ? launch_kvstar<2>(a, st)
                  : d == 64 ? launch_kvstar<4>(a, st)
                  : d == 128 ? launch_kvstar<8>(a, st)

@@ -53,7 +53,8 @@ class SetupParam:
 def kvstar_topk(query_group, blk_repre, pruned_index, topk, workspace=None):
     """query_group fp16 [x, Hq, d_orig], blk_repre fp16 [n, M, Hkv, d], pruned_index int64
     [Hkv, d] or None, all on one GPU -> (block numbers int32 [min(topk, n)], scores fp32) on
-    torch's current stream."""
+    torch's current stream.  workspace: uint8 of ucm_kvstar_topk_workspace_bytes for this shape or
+    more; a smaller one is not used."""
     out = _lib.native().kvstar_topk(query_group, blk_repre, pruned_index, topk, workspace)
     if out is not None:
         if type(out) is int:
