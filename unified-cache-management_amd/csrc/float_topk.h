@@ -688,7 +688,8 @@ struct RankShared {
 };
 
 // mine: the lane's candidate of the workgroup; first: of the wave's first 64, where has_first says that it is known.
-template <int WAVES, typename Key>
+// UNROLL: reads of four keys to a step of the loop over a wave's 64.
+template <int WAVES, int UNROLL, typename Key>
 __device__ __forceinline__ void rank_places(const SortArgs& a, int waves, uint32_t mine, uint32_t first, bool has_first,
                                             Key key_of, RankShared<WAVES>& sh)
 {
@@ -699,14 +700,12 @@ __device__ __forceinline__ void rank_places(const SortArgs& a, int waves, uint32
     for (int piece = w; piece * 64 < a.max_n; piece += waves) {
         const uint32_t k = has_first && piece == w ? first : key_of(piece * 64 + lane);
         have += __popcll(__ballot(k != 0u));
-        // A wave's keys go round by way of LDS, four to a read that all lanes share (lane by lane through a scalar
-        // register: 0.1 us more), eight to a step of the loop: code is fetched anew by every
-        // launch, and all 64 are 2 to 4 KB of it.
+        // A wave's keys go round by way of LDS, four to a read that all lanes share.
         sh.key[w][lane] = k;
         __builtin_amdgcn_wave_barrier();
         const uint4* all = reinterpret_cast<const uint4*>(sh.key[w]);
         auto count = [&](auto own_) {
-#pragma unroll 2
+#pragma unroll UNROLL
             for (int j = 0; j < 64; j += 4) {
                 const uint4 o4 = all[j / 4];
                 const uint32_t o[4] = {o4.x, o4.y, o4.z, o4.w};
@@ -743,6 +742,8 @@ __device__ __forceinline__ void rank_places(const SortArgs& a, int waves, uint32
     }
 }
 
+// All 64 keys in a row, as a wave has up to two pieces: 8 and 32 rows of 400 candidates 4.4 and 4.5 us, eight keys to a step 4.7 and 4.9,
+// lane by lane through a scalar register 4.5 and 4.55 (one row of 253: 3.3, 3.3 and 3.5).
 constexpr int kRankRow = 512;
 __global__ __launch_bounds__(256) void topk_rank_kernel(SORT_ARGS)
 {
@@ -751,13 +752,14 @@ __global__ __launch_bounds__(256) void topk_rank_kernel(SORT_ARGS)
     const uint32_t* keys = a.keys + blockIdx.x * a.pitch;
     const int pos = blockIdx.y * 64 + (threadIdx.x & 63);
     const uint32_t mine = pos < a.max_n ? keys[pos] : 0u;
-    rank_places<4>(a, 4, mine, 0u, false, [&](int at) { return at < a.max_n ? keys[at] : 0u; }, sh);
+    rank_places<4, 16>(a, 4, mine, 0u, false, [&](int at) { return at < a.max_n ? keys[at] : 0u; }, sh);
 }
 
 // The same for one row of up to kRankSums candidates whose scores are still in n_sums parts, which every workgroup
 // adds by itself, in the same order.  A wave for every 64 candidates up to sixteen: the parts of a wave's 64 and those
 // of the workgroup's own 64 are one round trip (253 candidates of 16 parts: 4.1 us, with its arguments read from memory 4.7, requested a
-// few at a time 5.0; 1024 of them 3 us less than in four waves with a branch at every part).
+// few at a time 5.0; 1024 of them 3 us less than in four waves with a branch at every part).  Eight keys to a step of the ranking's
+// loop: code is fetched anew by every launch, and sixteen waves in straight line wait for it (253 candidates 3.9 and 4.4 us, 1024: 5.3 and 6.2).
 constexpr int kRankSums = 2048;
 __global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SORT_ARGS)
 {
@@ -793,7 +795,7 @@ __global__ __launch_bounds__(1024) void topk_rank_sums_kernel(SORT_ARGS)
     const int at[2] = {(int)blockIdx.y * 64 + lane, (int)threadIdx.x};
     uint32_t key[2];
     keys_of(std::integral_constant<int, 2>{}, at, key);
-    rank_places<16>(a, blockDim.x / 64, key[0], key[1], true, [&](int p) {
+    rank_places<16, 2>(a, blockDim.x / 64, key[0], key[1], true, [&](int p) {
         const int one[1] = {p};
         uint32_t k[1];
         keys_of(std::integral_constant<int, 1>{}, one, k);
