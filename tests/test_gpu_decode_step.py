@@ -240,23 +240,17 @@ def test_latent_step_hashes_every_row(B, Hq, R, T, dt, slots_i64):
     assert np.array_equal(after[rest], before[rest])
 
 
-@pytest.mark.parametrize("nblk", [257, 512, 700, 2049])
-@pytest.mark.parametrize("kind", ["ties", "spread", "outlier", "kept"])
-def test_selection_of_long_rows(nblk, kind):
-    """Rows of every number of scores a thread, whose scores are all equal, anywhere in the range, close together but
-    for one far below, and blocks that equal the query beside those that are always kept (fewer and more than k)."""
+def select_long_rows(nblk, flips, BS, G, Wd=18):
+    """Rows whose scores are G * (32 Wd - flips): every token of a block is the same, the query with as many bits turned."""
     from ucm_amd.sparse import hamming_topk
 
     rng = rng_for(nblk)
-    B, BS, Wd, G = 2, 64, 18, 64
+    B = 2
     q = np.broadcast_to(rng.integers(0, 2**32, (B, 1, Wd), dtype=np.uint32), (B, G, Wd)).copy()
-    blocks = np.broadcast_to(q[:1, :1], (nblk, BS, Wd)).copy()  # every token of a block is the same
-    flips = {"ties": np.full(nblk, 40), "spread": rng.integers(0, 577, nblk),
-             "outlier": np.where(np.arange(nblk) == 77, 576, rng.integers(200, 205, nblk)),
-             "kept": np.where(np.arange(nblk) % 5 == 2, 0, rng.integers(1, 300, nblk))}[kind]
+    blocks = np.broadcast_to(q[:1, :1], (nblk, BS, Wd)).copy()
     for j in range(nblk):
-        bits = np.zeros(576, np.uint8)
-        bits[rng.permutation(576)[: flips[j]]] = 1
+        bits = np.zeros(32 * Wd, np.uint8)
+        bits[rng.permutation(32 * Wd)[: flips[j]]] = 1
         blocks[j] ^= np.packbits(bits, bitorder="little").view(np.uint32)
     table = np.stack([rng.permutation(nblk), rng.permutation(nblk)]).astype(np.int32)
     lens = np.array([nblk * BS, (nblk - 3) * BS - 5], np.int32)
@@ -265,6 +259,20 @@ def test_selection_of_long_rows(nblk, kind):
         gi, gs = hamming_topk(t(q), t(blocks).unsqueeze(2), t(table), t(lens), k, BS, 4 * BS, return_physical=True)
         oi, osc = c_api.hamming_topk(q, blocks[:, :, None], table, lens, k, BS, 4 * BS, flags=c_api.F_PHYSICAL)
         assert np.array_equal(gi.cpu().numpy(), oi) and np.array_equal(gs.cpu().numpy(), osc)
+
+
+@pytest.mark.parametrize("nblk", [257, 512, 700, 2049])
+@pytest.mark.parametrize("kind", ["ties", "spread", "outlier", "kept", "two", "64", "65"])
+def test_selection_of_long_rows(nblk, kind):
+    """Rows of every number of scores a thread, whose scores are all equal, anywhere in the range, close together but
+    for one far below, blocks that equal the query beside those that are always kept (fewer and more than k), and few
+    values: two, and on both sides of as many as have several bins each."""
+    rng = rng_for(nblk + 1)
+    flips = {"ties": np.full(nblk, 40), "spread": rng.integers(0, 577, nblk),
+             "outlier": np.where(np.arange(nblk) == 77, 576, rng.integers(200, 205, nblk)),
+             "kept": np.where(np.arange(nblk) % 5 == 2, 0, rng.integers(1, 300, nblk)),
+             "two": 100 + np.arange(nblk) // 3 % 2, "64": 100 + np.arange(nblk) % 64, "65": 100 + np.arange(nblk) % 65}[kind]
+    select_long_rows(nblk, flips, 64, 64 if kind in ("ties", "spread", "outlier", "kept") else 1)
 
 
 @pytest.mark.parametrize("G", [4, 8])
