@@ -240,6 +240,48 @@ def test_latent_step_hashes_every_row(B, Hq, R, T, dt, slots_i64):
     assert np.array_equal(after[rest], before[rest])
 
 
+@pytest.mark.parametrize("R", [1, 2])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Nn,Nr", [(512, 64), (64, 32), (128, 32), (256, 128), (512, 256), (1024, 512)])
+def test_latent_step_of_any_width_and_rows_without_a_sign(R, dt, Nn, Nr):
+    """Every number of column tiles of both parts, and rows of zeros, with a NaN and with an infinity among the keys and
+    the queries (in their wide part, their narrow part or both): no bit set in the first two, and every code the one that
+    the separate encoders give, which take the sums in the same order."""
+    from ucm_amd.sparse import HashEncoder
+    from ucm_amd.sparse.decode_step import GSADecodeStepMLA
+
+    rng = rng_for(Nn + Nr + R)
+    B, Hq, T, BS, nblk = 3, 32, 9, 64, 12
+    NB, Wn = B * nblk, Nn // 32
+    f = lambda *shape: torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).to(dt).cuda()
+    wn, wr = f(512, Nn), f(64, Nr)
+    parts = {512: (f(T, 512), f(B, R, Hq // R, 512)), 64: (f(T, 64), f(B, R, Hq // R, 64))}
+    special = {512: (0, 1, 2), 64: (0, 3, 4)}  # rows of zeros, with a NaN, with an infinity
+    for K, (k, q) in parts.items():
+        zero, nan, inf = special[K]
+        k[zero], q[1, :, zero] = 0, 0
+        k[nan, K - 3] = q[0, R - 1, nan, 17] = float("nan")
+        k[inf, 40] = q[2, R - 1, inf, K - 1] = float("inf")
+    cache = torch.zeros((NB, BS, Wn + Nr // 32), dtype=torch.int32, device="cuda")
+    table = torch.arange(NB, dtype=torch.int32, device="cuda").view(B, nblk)
+    lens = torch.full((B,), nblk * BS, dtype=torch.int32, device="cuda")
+    slots = torch.from_numpy(rng.permutation(NB * BS)[:T].astype(np.int64)).cuda()
+    st = GSADecodeStepMLA(wn, wr, Hq, R, B, nblk, 6 * BS, block_size=BS)
+    st.step(parts[512][0], parts[64][0], slots, parts[512][1].view(B, Hq, 512), parts[64][1].view(B, Hq, 64), cache, table, lens)
+    torch.cuda.synchronize()
+    codes = st.q_codes.view(B, Hq // R, -1)
+    keys = cache.view(NB * BS, -1)[slots]
+    for K, w, words in ((512, wn, slice(0, Wn)), (64, wr, slice(Wn, None))):
+        k, q = parts[K]
+        enc = HashEncoder(K, w.shape[1], dt, torch.device("cuda:0"))
+        enc.set_hash_weight(w)
+        zero, nan, _ = special[K]
+        assert not keys[[zero, nan], words].any() and not codes[1, zero, words].any() and not codes[0, nan, words].any()
+        assert torch.equal(keys[:, words], enc.compute_hash(k).view(torch.int32))
+        means = (q.float().sum(1) / R).to(dt)
+        assert torch.equal(codes[..., words], enc.compute_hash(means).view(torch.int32))
+
+
 def select_long_rows(nblk, flips, BS, G, Wd=18):
     """Rows whose scores are G * (32 Wd - flips): every token of a block is the same, the query with as many bits turned."""
     from ucm_amd.sparse import hamming_topk
@@ -273,6 +315,15 @@ def test_selection_of_long_rows(nblk, kind):
              "kept": np.where(np.arange(nblk) % 5 == 2, 0, rng.integers(1, 300, nblk)),
              "two": 100 + np.arange(nblk) // 3 % 2, "64": 100 + np.arange(nblk) % 64, "65": 100 + np.arange(nblk) % 65}[kind]
     select_long_rows(nblk, flips, 64, 64 if kind in ("ties", "spread", "outlier", "kept") else 1)
+
+
+@pytest.mark.parametrize("nblk", [300, 1100])
+def test_selection_of_long_rows_in_three_steps(nblk):
+    """240 heads of 1,536 bits: a range above 2^18, of which a step of 512 bins leaves 1,024 values and the next one two, so
+    that the third counts in the first one's bins again."""
+    flips = rng_for(nblk).integers(1, 1537, nblk)
+    assert 240 * int(np.max(flips) - np.min(flips)) >= 2**18
+    select_long_rows(nblk, flips, 16, 240, 48)
 
 
 @pytest.mark.parametrize("G", [4, 8])

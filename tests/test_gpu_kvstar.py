@@ -221,6 +221,23 @@ def test_blocks_whose_scores_are_taken_once(X, Hq, Hkv, d, n, M):
     assert np.all(np.abs(gs - ref[gi]) <= RTOL * ref[gi] + 2e-45)
 
 
+@pytest.mark.parametrize("X,Hq,Hkv,d,d_orig,n,M", [
+    (8, 32, 8, 32, 128, 253, 64),                      # 32k tokens, a quarter of the channels
+    (5, 28, 4, 64, 100, 40, 32), (8, 28, 4, 32, 45, 70, 16), (3, 6, 2, 128, 130, 21, 192),  # seven and three heads to a group
+    (2, 14, 2, 32, 64, 33, 192), (9, 20, 4, 64, 64, 25, 16), (1, 12, 1, 128, 160, 17, 256), (8, 8, 8, 32, 33, 9, 128),
+])
+def test_pruned_channels_and_any_group_taken_once(X, Hq, Hkv, d, d_orig, n, M):
+    """Against float64: channels in any order, some twice, and some outside the query row, which count as its ends."""
+    rng = np.random.default_rng(n + d)
+    q, k = make(X * 7 + n, X, Hq, Hkv, d, n, M, scale=0.5 if d < 128 else 0.3, d_orig=d_orig)
+    pr = rng.integers(0, d_orig, (Hkv, d))
+    pr[:, 3], pr[-1, d // 2], pr[0, d - 1] = -2, d_orig, d_orig + 1000
+    gi, gs = run_gpu(q, k, pr, n)
+    ref = brute.kvstar_block_scores(q, k, np.clip(pr, 0, d_orig - 1))
+    assert sorted(gi.tolist()) == list(range(n)) and np.all(np.diff(gs) <= 0)
+    assert np.all(np.abs(gs - ref[gi]) <= RTOL * ref[gi])
+
+
 @pytest.mark.parametrize("Hq,n", [(32767, 4), (32768, 8), (40000, 4), (65535, 3)])
 def test_as_many_heads_to_a_group_as_are_taken(Hq, n):
     """Group sizes on both sides of 2^15 and the largest, against float64: blocks of very different mass."""
@@ -236,11 +253,11 @@ def test_as_many_heads_to_a_group_as_are_taken(Hq, n):
 @pytest.mark.parametrize("M", [16, 32, 128])
 @pytest.mark.parametrize("what", ["nan", "+inf", "-inf", "nan_lane", "all_-inf"])
 def test_infinite_and_undefined_scores_taken_once(what, M):
-    test_infinite_and_undefined_scores(what, 300, M, 32)
+    test_infinite_and_undefined_scores(what, 300, M, 64 if M == 16 else 32)  # (two row tiles of 16 x 32 take the general path)
 
 
 @pytest.mark.parametrize("base", [-3.2e8, 4.0e9])
-@pytest.mark.parametrize("d,M", [(32, 16), (64, 32), (128, 64)])
+@pytest.mark.parametrize("d,M", [(64, 16), (128, 16), (32, 32), (64, 32), (128, 64)])
 def test_scores_of_any_finite_size_taken_once(base, d, M):
     test_scores_of_any_finite_size(base, d, M)
 
