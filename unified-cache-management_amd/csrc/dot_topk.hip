@@ -33,8 +33,7 @@ struct DotArgs {
     const float* q;        // [B][dim]
     const int32_t* idx;    // [B][max_n], -1 = no candidate
     int max_n;
-    uint32_t* keys;        // [B] rows, `pitch` apart
-    int64_t pitch;
+    uint32_t* keys;        // [B] rows, key_pitch(max_n) apart
 };
 
 // Sum over the 64 lanes, in lane 63.
@@ -62,7 +61,7 @@ __device__ __forceinline__ float wave_sum_last(float v)
 __global__ __launch_bounds__(kDotThreads) void dot_score_kernel(ucm::ArgPair rows, ucm::ArgPair lists, ucm::ArgInts n)
 {
     const DotArgs a{ucm::arg_ptr<const float>(rows.x), (int64_t)(uint32_t)n.z | (int64_t)n.w << 32, n.x, ucm::arg_ptr<const float>(rows.y),
-                    ucm::arg_ptr<const int32_t>(lists.x), n.y, ucm::arg_ptr<uint32_t>(lists.y), key_pitch(n.y)};
+                    ucm::arg_ptr<const int32_t>(lists.x), n.y, ucm::arg_ptr<uint32_t>(lists.y)};
     const int b = blockIdx.y;
     const float* q = a.q + (int64_t)b * a.dim;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -127,7 +126,7 @@ __global__ __launch_bounds__(kDotThreads) void dot_score_kernel(ucm::ArgPair row
     for (int r = 0; r < kRowsPerWave; ++r) {
         const float t = wave_sum_last(acc[r]);
         const int j = first + r;
-        if (lane == 63 && j < a.max_n) a.keys[b * a.pitch + j] = ok[r] ? score_key(t) : 0u;
+        if (lane == 63 && j < a.max_n) a.keys[b * key_pitch(a.max_n) + j] = ok[r] ? score_key(t) : 0u;
     }
 }
 
@@ -159,7 +158,6 @@ extern "C" int ucm_dot_topk(const float* data, int64_t n_items, int32_t dim, con
     DotArgs d{};
     d.data = data; d.n_items = n_items; d.dim = dim; d.q = query; d.idx = indexes; d.max_n = max_n;
     d.keys = (uint32_t*)workspace;
-    d.pitch = key_pitch(max_n);
     const int rows_per_wg = (kDotThreads / 64) * kRowsPerWave;
     hipLaunchKernelGGL(dot_score_kernel, dim3((unsigned)ucm::ceil_div(max_n, rows_per_wg), (unsigned)B),
                        dim3(kDotThreads), 0, st, ucm::arg_pair(d.data, d.q), ucm::arg_pair(d.idx, d.keys),
@@ -167,7 +165,7 @@ extern "C" int ucm_dot_topk(const float* data, int64_t n_items, int32_t dim, con
     int rc = ucm::launch_status("dot_score_kernel");
     if (rc != UCM_OK) return rc;
     SortArgs s{};
-    s.keys = d.keys; s.pitch = d.pitch; s.idx = indexes; s.max_n = max_n; s.topk = topk;
+    s.keys = d.keys; s.idx = indexes; s.max_n = max_n; s.topk = topk;
     s.out_idx = out_idx; s.out_score = out_score;
     return launch_topk(s, B, st);
 }

@@ -38,12 +38,11 @@ __device__ __forceinline__ float key_place(uint32_t k)
     return fminf(fmaxf(key_score(k), -big), big);  // a NaN, key 1, goes to the lower end
 }
 
-// Keys of a row lie at a pitch of whole 64-byte lines: every thread loads its keys as 16-byte pieces.
+// Keys of a row lie at this pitch, whole 64-byte lines: every thread loads its keys as 16-byte pieces.
 __host__ __device__ __forceinline__ int64_t key_pitch(int64_t n) { return (n + 15) & ~(int64_t)15; }
 
 struct SortArgs {
-    const uint32_t* keys;   // [B] rows of max_n keys, `pitch` apart; 16-byte aligned
-    int64_t pitch;
+    const uint32_t* keys;   // [B] rows of max_n keys, key_pitch(max_n) apart; 16-byte aligned
     const int32_t* idx;     // [B][max_n] what a list position stands for, or null: the position itself
     int max_n, topk, cap;   // cap: entries the search orders in LDS, a power of two
     int32_t* out_idx;       // [B][topk]
@@ -55,7 +54,7 @@ struct SortArgs {
 #define SORT_ARGS_OF(s) ucm::arg_pair((s).keys, (s).idx), ucm::arg_pair((s).out_idx, (s).out_score), ucm::ArgInts{(s).max_n, (s).topk, (s).cap, 0}
 __device__ __forceinline__ SortArgs sort_args(SORT_ARGS)
 {
-    return SortArgs{ucm::arg_ptr<const uint32_t>(p_in.x), key_pitch(n.x), ucm::arg_ptr<const int32_t>(p_in.y), n.x, n.y, n.z,
+    return SortArgs{ucm::arg_ptr<const uint32_t>(p_in.x), ucm::arg_ptr<const int32_t>(p_in.y), n.x, n.y, n.z,
                     ucm::arg_ptr<int32_t>(p_out.x), ucm::arg_ptr<float>(p_out.y)};
 }
 
@@ -422,7 +421,7 @@ __device__ void topk_search(const SortArgs& a, const uint32_t (&kreg)[PER ? PER 
     int* bfill = bcount + kBuckets;
     int* bbase = bfill + kBuckets;
     const int b = blockIdx.x;
-    const uint32_t* keys = a.keys + b * a.pitch;
+    const uint32_t* keys = a.keys + b * key_pitch(a.max_n);
     const int tid = threadIdx.x, lane = tid & 63;
     // f(chunk, key) over the thread's keys; uniform control flow.  Without registers chunk e covers
     // list positions e * NT + tid.
@@ -749,7 +748,7 @@ __global__ __launch_bounds__(256) void topk_rank_kernel(SORT_ARGS)
 {
     __shared__ RankShared<4> sh;
     const SortArgs a = sort_args(p_in, p_out, n);
-    const uint32_t* keys = a.keys + blockIdx.x * a.pitch;
+    const uint32_t* keys = a.keys + blockIdx.x * key_pitch(a.max_n);
     const int pos = blockIdx.y * 64 + (threadIdx.x & 63);
     const uint32_t mine = pos < a.max_n ? keys[pos] : 0u;
     rank_places<4, 16>(a, 4, mine, 0u, false, [&](int at) { return at < a.max_n ? keys[at] : 0u; }, sh);
@@ -820,7 +819,7 @@ __global__ __launch_bounds__(NT) void topk_kernel(SORT_ARGS)
     if constexpr (PER > 0) {
         static_assert(PER % 4 == 0, "16-byte loads");
         uint32_t kreg[PER];
-        const uint32_t* keys = a.keys + blockIdx.x * a.pitch;
+        const uint32_t* keys = a.keys + blockIdx.x * key_pitch(a.max_n);
         const int first = threadIdx.x * PER;
 #pragma unroll
         for (int e = 0; e < PER; e += 4) {

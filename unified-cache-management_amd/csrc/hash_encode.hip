@@ -2325,10 +2325,9 @@ struct LatentJob {
 };
 
 struct LatentJobs {
-    LatentJob job[4];         // keys and queries of 512 values, keys and queries of 64
-    int wide, narrow;          // tiles of either width
-    int wide_shift, nt_shift;  // log2 of the tiles that a row tile's columns make
-    uint32_t shifts;
+    LatentJob job[4];  // keys and queries of 512 values, keys and queries of 64
+    int narrow;        // tiles of the narrow jobs
+    int nt_shift;      // log2 of their tiles that a row tile's columns make
 };
 
 constexpr int kLatentWaves = 8;
@@ -3849,8 +3848,8 @@ bool latent_job(const EncArgs& a, LatentJob& j)
     return j.rows > 0;
 }
 
-// The four jobs of a latent-attention step for encode_latent_kernel, or false.
-bool latent_jobs(const EncJobs4& js, LatentJobs& out)
+// The four jobs of a latent-attention step for encode_latent_kernel, the number of wide tiles and the kernel's `shifts`, or false.
+bool latent_jobs(const EncJobs4& js, LatentJobs& out, int& wide_tiles, uint32_t& shifts)
 {
     for (int i = 0; i < 4; ++i)
         if (!latent_job(js.job[i], out.job[i])) return false;
@@ -3859,16 +3858,16 @@ bool latent_jobs(const EncJobs4& js, LatentJobs& out)
     const LatentJob &k = out.job[0], &q = out.job[1];
     auto word = [](int64_t v) { return v >= INT32_MIN && v <= INT32_MAX; };
     if (wide.H != 1 || k.mean || k.w != q.w || !word(k.xs_t) || !word(q.xs_t) || !word(q.xs_h) || !word(q.xs_g)) return false;
-    out.shifts = (uint32_t)(wide.nt_shift - 1) | (uint32_t)q.h_shift << 8 | (uint32_t)q.mean << 16;
-    out.wide_shift = wide.nt_shift - 1;
+    shifts = (uint32_t)(wide.nt_shift - 1) | (uint32_t)q.h_shift << 8 | (uint32_t)q.mean << 16;
+    const int wide_shift = wide.nt_shift - 1;
     out.nt_shift = narrow.nt_shift;
     auto row_tiles = [&](int i) { return ucm::ceil_div(out.job[i].rows, kRowsPerWave); };
-    const int64_t w0 = row_tiles(0) << out.wide_shift, n0 = row_tiles(2) << out.nt_shift;
-    const int64_t w = w0 + (row_tiles(1) << out.wide_shift), n = n0 + (row_tiles(3) << out.nt_shift);
+    const int64_t w0 = row_tiles(0) << wide_shift, n0 = row_tiles(2) << out.nt_shift;
+    const int64_t w = w0 + (row_tiles(1) << wide_shift), n = n0 + (row_tiles(3) << out.nt_shift);
     if (w + n > INT32_MAX) return false;
     out.job[1].first = (int)w0;
     out.job[3].first = (int)n0;
-    out.wide = (int)w;
+    wide_tiles = (int)w;
     out.narrow = (int)n;
     return true;
 }
@@ -3877,13 +3876,15 @@ template <typename V>
 int launch_small_mixed(const EncJobs4& js, hipStream_t st)
 {
     LatentJobs lean{};
-    if (latent_jobs(js, lean)) {
-        const dim3 grid((unsigned)(lean.wide + ucm::ceil_div(lean.narrow, kLatentWaves))), threads(64 * kLatentWaves);
+    int wide;
+    uint32_t shifts;
+    if (latent_jobs(js, lean, wide, shifts)) {
+        const dim3 grid((unsigned)(wide + ucm::ceil_div(lean.narrow, kLatentWaves))), threads(64 * kLatentWaves);
         const bool mean = lean.job[1].mean || lean.job[3].mean || lean.job[0].mean || lean.job[2].mean;
         const LatentJob &k = lean.job[0], &q = lean.job[1];
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, threads, 0, st, ucm::arg_pair(q.w, q.x), ucm::arg_pair(k.x, ucm::arg_words((int)q.xs_t, (int)q.xs_h)),
-                               ucm::ArgInts{(int)lean.shifts, (int)q.xs_g, (int)k.xs_t, q.rows}, k.rows, lean);
+                               ucm::ArgInts{(int)shifts, (int)q.xs_g, (int)k.xs_t, q.rows}, k.rows, lean);
         };
         if (mean) launch(encode_latent_kernel<V, 2>);
         else launch(encode_latent_kernel<V, 1>);

@@ -960,6 +960,6 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
                                    : d <= kAnyDimMost ? launch_kvstar<kAnyDim>(a, st)
                                  : launch_kvstar<kPacked>(a, st);
     if (rc != UCM_OK) return rc;
-    s.keys = a.keys; s.pitch = key_pitch(n_blocks);
+    s.keys = a.keys;
     return launch_topk(s, 1, st);
 }
