@@ -756,7 +756,7 @@ __global__ __launch_bounds__(256) void topk_rank_kernel(SORT_ARGS)
 
 // The same for one row of up to kRankSums candidates whose scores are still in n_sums parts, which every workgroup
 // adds by itself, in the same order.  A wave for every 64 candidates up to sixteen: the parts of a wave's 64 and those
-// of the workgroup's own 64 are one round trip (253 candidates of 16 parts: 4.1 us, with its arguments read from memory 4.7, requested a
+// of the workgroup's own 64 are one round trip (253 candidates of 16 parts: 3.9 us, with its arguments read from memory 4.7, requested a
 // few at a time 5.0; 1024 of them 3 us less than in four waves with a branch at every part).  Eight keys to a step of the ranking's
 // loop: code is fetched anew by every launch, and sixteen waves in straight line wait for it (253 candidates 3.9 and 4.4 us, 1024: 5.3 and 6.2).
 constexpr int kRankSums = 2048;

@@ -2466,7 +2466,7 @@ __global__ __launch_bounds__(kThreads) void select_kernel(SelectArgs a)
 // ---------------------------------------------------------------------------------------
 // Wave-level selection for rows of at most 64*EL block scores (index-ordered output only).
 // One wave per (request, KV head) row, no LDS and no barriers: a binary search on the score
-// value with ballot counts finds the k-th largest score, two wave prefix sums place the winners
+// value with ballot counts finds the k-th largest score, one wave prefix sum places the winners
 // in ascending index order, ties to the lower index.  Same results as select_kernel.
 // ---------------------------------------------------------------------------------------
 template <int EL>
@@ -2582,7 +2582,7 @@ __global__ __launch_bounds__(kThreads) void select_wave_kernel(SELECT_EARLY, Sel
     }
     const int thr = lo;
     const int need = kk - above;  // ties at thr to take, lowest indices first
-    // one prefix sum for both: scores equal to thr in the upper half, greater ones in the lower (a row has 1024 at most)
+    // one prefix sum for both: scores equal to thr in the upper half, greater ones in the lower (a row has 256 at most)
     int both = 0;
 #pragma unroll
     for (int e = 0; e < EL; ++e) both += (v[e] == thr ? 1 << 16 : 0) + (v[e] > thr);

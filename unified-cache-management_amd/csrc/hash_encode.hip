@@ -3251,7 +3251,8 @@ int64_t small_waves(const EncArgs& a)
 // through LDS and the order of the tiles are a chain of 0.3 to 0.5 us in front of the products, which fewer rows, on fewer lines,
 // do not make up for.  Operand layout and line by line: 512 -> 512 bits, 1 row 3.83 and 4.31 us, 20 rows 4.33 and 4.36, 24 rows 4.41
 // and 4.34, 32 rows 4.60 and 4.36; 256 -> 128 bits, 1 row 3.42 and 3.72, 24 rows 3.70 and 3.77, 28 rows 3.68 and 3.69, 32 rows 3.78 and 3.74;
-// a latent step of 8 query rows 13.3 and 13.7, of 32 rows 13.1 and 12.9.
+// a latent step through encode_small_mixed_kernel (those of the plugin's form have a kernel of their own) of 8 query rows 13.3 and 13.7, of
+// 32 rows 13.1 and 12.9.
 bool rows_by_line(const EncArgs& a, const EncArgs& b)
 {
     auto tile_rows = [](const EncArgs& j) { return small_rows_are_pairs(j) ? j.T * j.H : j.T; };
@@ -3848,6 +3849,9 @@ bool latent_job(const EncArgs& a, LatentJob& j)
     return j.rows > 0;
 }
 
+// The kernel of every form is no faster at any number of rows, so none of them is a bound; launches, that kernel and this one: 1 query row 4.7
+// and 4.5 us, 4 rows 4.9 and 4.5, 8 means of two 5.8 and 5.1, 16 rows 5.2 and 4.6, 128 5.4 and 4.7, 512 6.6 and 5.1, 2,048 10.6 and 10.7, 4,096
+// 16.2 and 13.4.
 // The four jobs of a latent-attention step for encode_latent_kernel, the number of wide tiles and the kernel's `shifts`, or false.
 bool latent_jobs(const EncJobs4& js, LatentJobs& out, int& wide_tiles, uint32_t& shifts)
 {

@@ -18,11 +18,11 @@
 //   * Everything else: kvstar_stats_kernel (maximum and sum of exponentials of every row over one chunk of the
 //     representatives), kvstar_mass_kernel (the chunks' pairs merged, q.k once more, probabilities summed over rows
 //     and a block's representatives) and the shared top-k selection.
-// 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 13.0 us (5.9, 4.0 and 3.8 of the three
+// 8 query tokens x 32 heads, 253 blocks x 64 representatives, 32 channels: 13.0 to 13.3 us (6.2, 3.9 and 3.9 of the three
 // kernels: launches and round trips; the products and exponentials are about 1.5), 18.8 the second way
-// (7.5, 9.0, 3.7); 1024 blocks, 128 channels: 41 and 70.4, the second way reads the keys twice.
-// Error against 64 bits at that shape 3.3e-8 of the scores' 2-norm (the second way 4.7e-8), over thirteen others from 24 to
-// 1024 blocks 2.6e-8 to 2.0e-7 (3.7e-8 to 1.9e-7).
+// (7.5, 9.0, 3.7); 1024 blocks, 128 channels: 36.1 and 70.4, the second way reads the keys twice.
+// Error against 64 bits at that shape 3.3e-8 of the scores' 2-norm (the second way 4.8e-8), over 34 others of like
+// values (1 to 16 tokens, 24 to 1000 blocks of 16 to 256, 32 to 128 channels) 2.8e-8 to 3.8e-7 (3.5e-8 to 3.9e-7).
 // Sums are taken in a different order than the reference's loops, the same one on every call (no
 // atomics); the tolerance is stated where the results are compared.  Equal scores come out in
 // ascending block order (the reference's heap pops them in descending block order).
@@ -945,7 +945,9 @@ extern "C" int ucm_kvstar_topk(const void* query, int32_t X, int32_t Hq, int32_t
     SortArgs s{};
     s.max_n = (int)n_blocks; s.topk = topk;
     s.out_idx = out_idx; s.out_score = out_score;
-    // few row tiles leave the merging to few workgroups (four, 600 blocks of 16 x 32 channels: 18.6 and 17.0 us)
+    // Few row tiles leave the merging to few workgroups.  Four tiles, 600 blocks of 16 x 32 channels: 18.6 and the second way 17.0 us;
+    // larger blocks have more to gain: one tile, 300 of 16 x 64 channels 15.4 and 17.0, 253 of 32 x 32 13.0 and 14.4, 24 of 32 x 32 12.9
+    // and 14.1, 1500 of 32 x 32 23.9 and 24.5; eight tiles, 600 of 16 x 32 16.8 and 19.0.
     const bool few = M == 16 && d == 32 && a.items < 8;
     // (a buffer that only the second way fits into, one asked for at another shape, is taken by it)
     if (a.units > 0 && !few && (d == 32 || d == 64 || d == 128) && carve_units(a, workspace, (int64_t)a.items * 32) <= workspace_bytes) {
